@@ -1,6 +1,6 @@
-// Register/LDS-resident evaluation kernels:
-//   k_cell_local  one thread per Dirac: power cell clipped in place in LDS
-//                 (at most kMaxFast vertices) by the Diracs of the
+// Register-resident evaluation kernels:
+//   k_cell_local  16 lanes per Dirac: power cell clipped in place, one vertex
+//                 per lane (at most kMaxFast), by the Diracs of the
 //                 surrounding bins, certified ring by ring or through the
 //                 max-weight pyramid, written once to HBM;
 //   k_pairs       (cell, triangle) pairs whose bounding boxes meet;
@@ -29,7 +29,6 @@
 
 namespace ma {
 
-constexpr int kCellBlock = 64;
 constexpr int kNodeDiracs = 8;    // pyramid nodes with at most this many Diracs are taken whole
 // Starting box half-width, in bins: wide enough for the large cells of sparse
 // regions at converged weights (targets spread over a lognormal range, 1/20 of
@@ -74,7 +73,7 @@ struct CellArgs {
   double dom[4];     // domain bounding box
   const TriData *tri;
   const float4 *tbox;  // FP32 outward-rounded triangle bounding boxes
-  double *px, *py;   // FP64 cell vertices (local to the Dirac), [v * n + k]
+  double *px, *py;   // FP64 cell vertices (local to the Dirac), [k * kMaxFast + v]
   float *pxf, *pyf;  // FP32 cell vertices (mixed mode)
   int32_t *plab;     // neighbour across edge v -> v+1 (-1: domain edge)
   int32_t *pn;       // vertex count, -1 = handled by the general kernel
@@ -83,7 +82,7 @@ struct CellArgs {
   double *mass, *intg, *mom;  // mom: local first moments, interleaved (x, y)
   double *mom2;      // local second moments (xx, yy, xy) per Dirac (mode 3)
   int32_t *ovf, *novf;  // pairs left to k_frag_wide, and their count
-  double *eacc;      // edge integrals int rho ds, [v * n + k]; -0.0 until an edge is seen
+  double *eacc;      // edge integrals int rho ds, [k * kMaxFast + v]; -0.0 until an edge is seen
   float *eaccf;      // FP32 edge integrals (mixed mode)
   const int32_t *triv;  // triangle vertex ids (counter-clockwise, as in tri)
   double *dval;      // adjoint w.r.t. vertex density values (mode 2)
@@ -92,7 +91,7 @@ struct CellArgs {
   int force_general;  // route every cell to the general kernel (testing)
   int walk_budget;    // pyramid nodes a cell may visit before the bin path
   unsigned long long *stripes;  // striped event counters (EvalBuffers::stripes)
-  int32_t *ptri;      // first kPadTri candidate triangles of each cell, [c * n + k]
+  int32_t *ptri;      // first kPadTri candidate triangles of each cell, [k * kPadTri + c]
   FragOut fo;         // fragment polygons (mode 1, when fo.count is set)
   // per Dirac: 1 if its cell took the bin path (far from its Dirac) in the
   // last evaluation of the same Diracs; with use_far such cells go to the
@@ -117,36 +116,124 @@ struct CellBuf<float> {
   __device__ static float *eacc(const CellArgs &a) { return a.eaccf; }
 };
 
-// The LDS polygon of one thread.
+// ---------------------------------------------------------------------------
+// Groups of 16 lanes (one DPP row of the wave) build one cell together: lane
+// l holds polygon vertex l in registers, tests one candidate, one bin or one
+// pyramid node at a time, and all control flow is uniform in the group.
+// Candidates, bins and nodes are loaded 16 at a time, reductions and
+// broadcasts are DPP moves, and no LDS limits the waves in flight; what bounds
+// k_cell_local is VALU issue (84 % busy, 61 % of the lanes active).  One
+// thread per cell with its polygon in LDS waited instead on dependent gathers
+// and its wave's slowest lane (24 % of the lanes active, 1.4 - 1.8 waves per
+// SIMD).  Measured, before and after: 1M Diracs at w = 0 in FP32 2.49 and
+// 1.55 ms, 1M in FP64 at weights up to 1.6 bins off 8.5 and 3.0 ms, 2M on an
+// annulus in FP64 13.0 and 2.8 ms, 1000 Diracs (too few threads before) 278
+// and 33 us.
+// ---------------------------------------------------------------------------
+constexpr int kGroup = 16;
+constexpr int kCellThreads = 256;                    // threads of the cell kernels
+constexpr int kCellGroups = kCellThreads / kGroup;   // cells per workgroup
+constexpr int kCellXcdRun = 64;                      // workgroups of an XCD's run (1024 cells)
+static_assert(kMaxFast == kGroup, "one polygon vertex per lane");
+
+constexpr int kDppShr = 0x110, kDppRor = 0x120, kDppBcast = 0x150;  // row_shr, row_ror, row_newbcast
+template <int CTRL>
+__device__ inline int dpp(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ inline float dpp(float v) {
+  return __int_as_float(dpp<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ inline double dpp(double v) {
+  return __hiloint2double(dpp<CTRL>(__double2hiint(v)), dpp<CTRL>(__double2loint(v)));
+}
+template <class T>
+__device__ inline T row_max(T v) {
+  v = fmax(v, dpp<kDppRor + 8>(v));
+  v = fmax(v, dpp<kDppRor + 4>(v));
+  v = fmax(v, dpp<kDppRor + 2>(v));
+  return fmax(v, dpp<kDppRor + 1>(v));
+}
+template <class T>
+__device__ inline T row_min(T v) {
+  return -row_max(-v);
+}
+__device__ inline unsigned row_min(unsigned v) {
+  v = min(v, (unsigned)dpp<kDppRor + 8>((int)v));
+  v = min(v, (unsigned)dpp<kDppRor + 4>((int)v));
+  v = min(v, (unsigned)dpp<kDppRor + 2>((int)v));
+  return min(v, (unsigned)dpp<kDppRor + 1>((int)v));
+}
+// largest of non-negative floats (their bit patterns order like integers)
+__device__ inline float row_max_nonneg(float f) {
+  int v = __float_as_int(f);
+  v = max(v, dpp<kDppRor + 8>(v));
+  v = max(v, dpp<kDppRor + 4>(v));
+  v = max(v, dpp<kDppRor + 2>(v));
+  return __int_as_float(max(v, dpp<kDppRor + 1>(v)));
+}
+__device__ inline int row_sum(int v) {
+  v += dpp<kDppRor + 8>(v);
+  v += dpp<kDppRor + 4>(v);
+  v += dpp<kDppRor + 2>(v);
+  return v + dpp<kDppRor + 1>(v);
+}
+// inclusive prefix sum over the row
+__device__ inline int row_scan(int v) {
+  v += dpp<kDppShr + 1>(v);
+  v += dpp<kDppShr + 2>(v);
+  v += dpp<kDppShr + 4>(v);
+  return v + dpp<kDppShr + 8>(v);
+}
+// values of lane `src` of the row; base4 = 4 x the row's first lane
+__device__ inline int row_get(int v, int base4, int src) {
+  return __builtin_amdgcn_ds_bpermute(base4 + 4 * src, v);
+}
+__device__ inline float row_get(float v, int base4, int src) {
+  return __int_as_float(row_get(__float_as_int(v), base4, src));
+}
+__device__ inline double row_get(double v, int base4, int src) {
+  return __hiloint2double(row_get(__double2hiint(v), base4, src),
+                          row_get(__double2loint(v), base4, src));
+}
+
+// a / b: a reciprocal and one correction (within an ulp), FP64 as the compiler does it
+__device__ inline float ratio(float a, float b) {
+  const float r = __builtin_amdgcn_rcpf(b), q = a * r;
+  return fmaf(fmaf(-b, q, a), r, q);
+}
+__device__ inline double ratio(double a, double b) { return a / b; }
+
+// The polygon of one group.  Lanes past the last vertex hold vertex 0.
+// Half-plane of competitor j seen from Dirac k, in coordinates local to y_k:
+// X stays in the cell of k iff kk - 2 X.Y > 0 (strict: ties are outside),
+// Y = y_j - y_k, kk = |Y|^2 + w_k - w_j.
 template <class R>
-struct CellLDS {
-  R (*sx)[kCellBlock];
-  R (*sy)[kCellBlock];
-  int (*sl)[kCellBlock];
-  int t;
-  __device__ double rho2(int n) const {
-    R r = R(0);
-    for (int v = 0; v < n; v++) r = fmax(r, sx[v][t] * sx[v][t] + sy[v][t] * sy[v][t]);
-    return (double)r * (1.0 + Tol<R>::pad);
-  }
-  // Disc holding the polygon: centre (cx, cy) = centre of its bounding box,
-  // returns the squared radius about it (padded like rho2)
-  __device__ double disc(int n, double &cx, double &cy) const {
-    double x0 = kInf, x1 = -kInf, y0 = kInf, y1 = -kInf;
-    for (int v = 0; v < n; v++) {
-      x0 = fmin(x0, (double)sx[v][t]);
-      x1 = fmax(x1, (double)sx[v][t]);
-      y0 = fmin(y0, (double)sy[v][t]);
-      y1 = fmax(y1, (double)sy[v][t]);
-    }
-    cx = 0.5 * (x0 + x1);
-    cy = 0.5 * (y0 + y1);
-    double r = 0.0;
-    for (int v = 0; v < n; v++) {
-      const double dx = (double)sx[v][t] - cx, dy = (double)sy[v][t] - cy;
-      r = fmax(r, dx * dx + dy * dy);
-    }
-    return r * (1.0 + Tol<R>::pad) + 1e-24 * (cx * cx + cy * cy);
+struct Cell {
+  int l;       // lane in the group
+  int base;    // first lane of the group in its wave
+  double ih, h2;  // 1 / bin side, its square's inverse
+  R x = R(0), y = R(0);  // vertex l
+  int lab = -1;          // edge vertex l -> l + 1
+  int n = 0;             // vertices (uniform in the group)
+  float rb = 0.0f;       // radius of the polygon about the Dirac, squared, in bins (upper bound)
+  bool cut = false;      // the starting box cut the domain box
+  int nredo = 0;         // FP32 values re-decided in FP64 (this lane)
+
+  __device__ explicit Cell(const Grid &g)
+      : l((int)threadIdx.x & (kGroup - 1)), base((int)threadIdx.x & 48), ih(1.0 / g.h),
+        h2(g.h * g.h) {}
+  // lanes of the group with p set
+  __device__ unsigned mask(bool p) const { return (unsigned)(__ballot(p) >> base) & 0xffffu; }
+  template <class T>
+  __device__ T get(T v, int src) const { return row_get(v, 4 * base, src); }
+  __device__ double rho2() const { return (double)rb * h2; }
+
+  __device__ void update_radius() {
+    const float xb = (float)(x * (R)ih), yb = (float)(y * (R)ih);
+    rb = row_max_nonneg(xb * xb + yb * yb) * (1.0f + 1e-6f + (float)Tol<R>::pad);
   }
   // Box [X0,X1] x [Y0,Y1] (local coordinates) with the labels of its bottom,
   // right, top and left edges, cut to a few bins around the Dirac (edges
@@ -163,226 +250,336 @@ struct CellLDS {
     if (Y0 < -half) { Y0 = -half; lb = kBoxLabel; }
     if (Y1 > half) { Y1 = half; lt = kBoxLabel; }
     cut = (lb == kBoxLabel) || (lr == kBoxLabel) || (lt == kBoxLabel) || (ll == kBoxLabel);
-    if (!(X0 < X1 && Y0 < Y1)) return false;
-    sx[0][t] = (R)X0; sy[0][t] = (R)Y0; sl[0][t] = lb;
-    sx[1][t] = (R)X1; sy[1][t] = (R)Y0; sl[1][t] = lr;
-    sx[2][t] = (R)X1; sy[2][t] = (R)Y1; sl[2][t] = lt;
-    sx[3][t] = (R)X0; sy[3][t] = (R)Y1; sl[3][t] = ll;
-    return true;
+    n = 4;
+    x = (R)((l == 1 || l == 2) ? X1 : X0);
+    y = (R)((l == 2 || l == 3) ? Y1 : Y0);
+    lab = l == 1 ? lr : l == 2 ? lt : l == 3 ? ll : lb;
+    update_radius();
+    return X0 < X1 && Y0 < Y1;
   }
   // true if the finished cell may extend beyond the cut of init(): it still
   // touches the cut, or it came out empty although the box was cut (a cell
   // displaced from its Dirac by more than the box is not seen from inside it)
-  __device__ bool touches_cut(int n) const {
+  __device__ bool touches_cut() const {
     if (n == 0) return cut;
-    for (int v = 0; v < n; v++)
-      if (sl[v][t] == kBoxLabel) return true;
-    return false;
+    return mask(l < n && lab == kBoxLabel) != 0u;
   }
-  bool cut = false;
-};
-
-// Half-plane of competitor j seen from Dirac k, in coordinates local to y_k:
-// X stays in the cell of k iff kk - 2 X.Y > 0 (strict: ties are outside),
-// Y = y_j - y_k, kk = |Y|^2 + w_k - w_j.  Both precisions are carried.
-template <class R>
-struct HalfPlane {
-  R Yx, Yy, kk;
-  double Yx64, Yy64, kk64;
-  int label;
-  // FP32: the error bound of a value, redo x (|kk| + 2 rv (|Yx| + |Yy|)) for
-  // every vertex within distance rv of the Dirac (rv: the polygon's radius
-  // when the clip starts; clipping only adds points inside the polygon)
-  R thr = R(0);
-  __device__ void set_bound(double rv) {
-    if (Tol<R>::redo > R(0))
-      thr = (R)((double)Tol<R>::redo * (fabs(kk64) + 2.0 * rv * (fabs(Yx64) + fabs(Yy64))));
-  }
-  // value at (x, y); an FP32 value within the FP32 error bound of zero is
-  // replaced by the FP64 value at the same (stored) point
-  __device__ R value(R x, R y, int *nredo) const {
-    const R s = kk - R(2) * (x * Yx + y * Yy);
-    if (Tol<R>::redo > R(0) && fabs(s) <= thr) {
-      if (nredo) (*nredo)++;
-      return (R)(kk64 - 2.0 * ((double)x * Yx64 + (double)y * Yy64));
-    }
-    return s;
-  }
-};
-
-// In-place clip of the LDS polygon of thread t by a half-plane.  The
-// surviving vertices form one cyclic run; it is moved to the front, followed
-// by the exit point X (label = new neighbour) and the entry point E (label of
-// the edge it lies on).  Returns the new vertex count; sets fail on overflow
-// or when rounding breaks the single-run structure.
-template <class R>
-__device__ inline int clip_lds(CellLDS<R> &L, int n, const HalfPlane<R> &H, bool &fail,
-                               int &nredo) {
-  const int t = L.t;
-  uint32_t in = 0u;
-  for (int v = 0; v < n; v++)
-    if (H.value(L.sx[v][t], L.sy[v][t], &nredo) > R(0)) in |= 1u << v;
-  const uint32_t full = (1u << n) - 1u;
-  if (in == full) return n;
-  if (in == 0u) return 0;
-  uint32_t nxt = ((in >> 1) | ((in & 1u) << (n - 1))) & full;
-  uint32_t exit_m = in & ~nxt, entry_m = ~in & nxt & full;
-  if (sizeof(R) == sizeof(float) && (__popc(exit_m) != 1 || __popc(entry_m) != 1)) {
-    // FP32 rounding broke the single run: classify every stored vertex in FP64
-    in = 0u;
-    for (int v = 0; v < n; v++) {
-      const double x = (double)L.sx[v][t], y = (double)L.sy[v][t];
-      if (H.kk64 - 2.0 * (x * H.Yx64 + y * H.Yy64) > 0.0) in |= 1u << v;
-    }
-    nredo += n;
-    if (in == full) return n;
-    if (in == 0u) return 0;
-    nxt = ((in >> 1) | ((in & 1u) << (n - 1))) & full;
-    exit_m = in & ~nxt;
-    entry_m = ~in & nxt & full;
-  }
-  if (__popc(exit_m) != 1 || __popc(entry_m) != 1) {
-    fail = true;
-    return n;
-  }
-  const int xk = __ffs(exit_m) - 1, ek = __ffs(entry_m) - 1;
-  const int xk1 = (xk + 1 == n) ? 0 : xk + 1, ek1 = (ek + 1 == n) ? 0 : ek + 1;
-  const int cnt_in = __popc(in);
-  const int m = cnt_in + 2;
-  if (m > kMaxFast) {
-    fail = true;
-    return n;
-  }
-  R ax = L.sx[xk][t], ay = L.sy[xk][t], bx = L.sx[xk1][t], by = L.sy[xk1][t];
-  R sa = H.value(ax, ay, nullptr), sb = H.value(bx, by, nullptr);
-  R tt = sa / (sa - sb);
-  const R Xx = ax + tt * (bx - ax), Xy = ay + tt * (by - ay);
-  ax = L.sx[ek][t]; ay = L.sy[ek][t]; bx = L.sx[ek1][t]; by = L.sy[ek1][t];
-  sa = H.value(ax, ay, nullptr);
-  sb = H.value(bx, by, nullptr);
-  tt = sa / (sa - sb);
-  const R Ex = ax + tt * (bx - ax), Ey = ay + tt * (by - ay);
-  const int El = L.sl[ek][t];
-  const int s0 = ek1;
-  int px, pe;
-  if (s0 <= xk) {
-    for (int i = 0; i < cnt_in; i++) {
-      L.sx[i][t] = L.sx[s0 + i][t];
-      L.sy[i][t] = L.sy[s0 + i][t];
-      L.sl[i][t] = L.sl[s0 + i][t];
-    }
-    px = cnt_in;
-    pe = cnt_in + 1;
-  } else {
-    const int tl = n - s0, dest = xk + 3;
-    if (dest < s0) {
-      for (int i = 0; i < tl; i++) {
-        L.sx[dest + i][t] = L.sx[s0 + i][t];
-        L.sy[dest + i][t] = L.sy[s0 + i][t];
-        L.sl[dest + i][t] = L.sl[s0 + i][t];
-      }
-    } else if (dest > s0) {
-      for (int i = tl - 1; i >= 0; i--) {
-        L.sx[dest + i][t] = L.sx[s0 + i][t];
-        L.sy[dest + i][t] = L.sy[s0 + i][t];
-        L.sl[dest + i][t] = L.sl[s0 + i][t];
+  // Clips by the half-plane that lane c brings: (Yx, Yy, kk), edge label
+  // `label`.  The surviving vertices form one cyclic run; they move to the
+  // front in order, followed by the exit point (label = the new neighbour) and
+  // the entry point (label of the edge it lies on).  FP32: a value within
+  // lane c's error bound thr of zero is replaced by the FP64 value at the same
+  // (stored) point.  Returns whether the polygon changed; sets fail when it
+  // outgrows the lanes or rounding breaks the single-run structure.
+  __device__ bool clip(int c, double lYx, double lYy, double lkk, int label, float thr,
+                       bool &fail) {
+    const R Yx = get((R)lYx, c), Yy = get((R)lYy, c), kk = get((R)lkk, c);
+    const int nlab = get(label, c);
+    R s = kk - R(2) * (x * Yx + y * Yy);
+    if (Tol<R>::redo > R(0)) {
+      const bool redo = fabs(s) <= (R)get(thr, c);
+      if (mask(redo)) {
+        const double Y0 = get(lYx, c), Y1 = get(lYy, c), k0 = get(lkk, c);
+        if (redo) {
+          s = (R)(k0 - 2.0 * ((double)x * Y0 + (double)y * Y1));
+          nredo += l < n;
+        }
       }
     }
-    px = xk + 1;
-    pe = xk + 2;
+    const unsigned full = (1u << n) - 1u;
+    unsigned in = mask(s > R(0)) & full;
+    int kept, s0;  // survivors and the first of their run
+    auto run = [&]() {
+      kept = __popc(in);
+      const int out = 32 - __clz((int)(~in & full));  // one past the last vertex cut off
+      s0 = (in & 1u) ? (out == n ? 0 : out) : __ffs((int)in) - 1;
+      const unsigned t = ((1u << kept) - 1u) << s0;
+      return ((t | (t >> n)) & full) == in;
+    };
+    if (in == full) return false;
+    if (in == 0u) {
+      n = 0;
+      return true;
+    }
+    bool single = run();
+    if (sizeof(R) == sizeof(float) && !single) {
+      // FP32 rounding broke the single run: classify every stored vertex in FP64
+      const double Y0 = get(lYx, c), Y1 = get(lYy, c), k0 = get(lkk, c);
+      in = mask(k0 - 2.0 * ((double)x * Y0 + (double)y * Y1) > 0.0) & full;
+      nredo += l < n;
+      if (in == full) return false;
+      if (in == 0u) {
+        n = 0;
+        return true;
+      }
+      single = run();
+    }
+    if (!single || kept + 2 > kGroup) {
+      fail = true;
+      return false;
+    }
+    // slot l takes survivor s0 + l; slot kept the crossing of the edge out of
+    // the last survivor, slot kept + 1 that of the edge into the first
+    const bool ex = l == kept, en = l == kept + 1;
+    int ia = s0 + (l < kept ? l : ex ? kept - 1 : en ? n - 1 : 0);
+    int ib = s0 + (ex ? kept : 0);
+    ia -= ia >= n ? n : 0;
+    ib -= ib >= n ? n : 0;
+    const R ax = get(x, ia), ay = get(y, ia), bx = get(x, ib), by = get(y, ib);
+    const int al = get(lab, ia);
+    R sa, sb;
+    if (sizeof(R) == sizeof(float)) {
+      sa = get(s, ia);
+      sb = get(s, ib);
+    } else {
+      sa = kk - R(2) * (ax * Yx + ay * Yy);
+      sb = kk - R(2) * (bx * Yx + by * Yy);
+    }
+    const R tt = (ex || en) ? ratio(sa, sa - sb) : R(0);
+    x = ax + tt * (bx - ax);
+    y = ay + tt * (by - ay);
+    lab = ex ? nlab : al;
+    n = kept + 2;
+    return true;
   }
-  L.sx[px][t] = Xx;
-  L.sy[px][t] = Xy;
-  L.sl[px][t] = H.label;
-  L.sx[pe][t] = Ex;
-  L.sy[pe][t] = Ey;
-  L.sl[pe][t] = El;
-  return m;
-}
+};
 
-// Clips the cell of Dirac k by the power half-plane of candidate j.  A cheap
-// distance test first discards candidates that cannot reach the polygon:
-// pi_j - pi_k >= kk - 2 C.Y - 2 r |Y| on a disc of centre C and radius r
-// holding it (Y = y_j - y_k, kk = |Y|^2 + w_k - w_j, local coordinates).
-// CENTRED = false: the disc is centred at the Dirac (r = the polygon's
-// radius about it, which the ring certificate also uses); CENTRED = true:
-// at the centre of the polygon's bounding box (cx, cy kept up to date), the
-// tight choice for a cell far from its Dirac.
-template <bool CENTRED = false, class R>
-__device__ inline void consider(const CellArgs &a, int64_t k, int32_t j, double yx, double yy,
-                                double wk, CellLDS<R> &L, int &n, double &rho2, bool &fail,
-                                int &nredo, double *cx = nullptr, double *cy = nullptr) {
-  if (j == k || n == 0) return;
-  const double Yx = a.pos[2 * j] - yx, Yy = a.pos[2 * j + 1] - yy, wj = a.w[j];
-  const double d2 = Yx * Yx + Yy * Yy;
-  const double dw = wdiff(a.wlo, wk, k, wj, j);  // w_k - w_j
-  if (d2 == 0.0) {
-    // coincident Diracs: the larger weight (then the smaller caller index)
-    // hides the other
-    if (dw < 0.0 || (dw == 0.0 && a.perm[j] < a.perm[k])) n = 0;
+// Clips the polygon C of Dirac k (position (yx, yy), weight wk) by up to 16
+// Diracs, lane l bringing Dirac j (-1: none).  A candidate that cannot reach
+// the disc about the Dirac holding the polygon is discarded at once (pi_j -
+// pi_k >= kk - 2 r |Y|); the others take their half-plane's smallest value
+// over the polygon's vertices, and the deepest cut clips first: every clip
+// then cuts, and 8.5 of them build a cell of 6 edges (taking the nearest
+// bisector first and testing against the disc only: 7.8 clips and 9.4 that
+// cut nothing, at 130 instructions each against 30 for the test).  The test
+// runs in T: float in units of bins with its rounding bounded (near the
+// Dirac), or double (far from it, where that bound would pass everything).
+// SEEN: j may be an edge of the polygon already.
+template <class T, bool SEEN, class R>
+__device__ inline void clip_batch(const CellArgs &a, int64_t k, double yx, double yy, double wk,
+                                  int32_t j, Cell<R> &C, bool &fail) {
+  bool has = j >= 0 && j != (int32_t)k, hide = false;
+  double Yx = 0.0, Yy = 0.0, kk = 1.0, d2 = 1.0;
+  if (has) {
+    const double2 pj = reinterpret_cast<const double2 *>(a.pos)[j];
+    const double wj = a.w[j];
+    Yx = pj.x - yx;
+    Yy = pj.y - yy;
+    d2 = Yx * Yx + Yy * Yy;
+    const double dw = wdiff(a.wlo, wk, k, wj, j);  // w_k - w_j
+    kk = d2 + dw;
+    const double ct = kk - 1e-12 * (d2 + fabs(wk) + fabs(wj));
+    if (d2 == 0.0) {
+      // coincident Diracs: the larger weight (then the smaller caller index)
+      // hides the other
+      hide = dw < 0.0 || (dw == 0.0 && a.perm[j] < a.perm[k]);
+      has = false;
+    } else if (ct > 0.0 && ct * ct > 4.0 * C.rho2() * d2) {
+      has = false;
+    }
+  }
+  if (C.mask(hide)) {
+    C.n = 0;
     return;
   }
-  // j cannot cut the polygon if kk - 2 C.Y - tol > 2 r |Y|, decided on
-  // squares (no square roots)
-  const double cy2 = CENTRED ? 2.0 * (*cx * Yx + *cy * Yy) : 0.0;
-  const double ct = d2 + dw - cy2 - 1e-12 * (d2 + fabs(wk) + fabs(wj) + fabs(cy2));
-  if (ct > 0.0 && ct * ct > 4.0 * rho2 * d2) return;
-  for (int v = 0; v < n; v++)
-    if (L.sl[v][L.t] == j) return;  // already an edge of the cell
-  HalfPlane<R> H;
-  H.Yx64 = Yx;
-  H.Yy64 = Yy;
-  H.kk64 = d2 + dw;
-  H.Yx = (R)Yx;
-  H.Yy = (R)Yy;
-  H.kk = (R)H.kk64;
-  H.label = j;
-  // radius bound of the vertices about the Dirac: rho2 is about the Dirac,
-  // or (CENTRED) about (cx, cy)
-  H.set_bound(CENTRED ? sqrt(*cx * *cx + *cy * *cy) + sqrt(rho2) : sqrt(rho2));
-  n = clip_lds(L, n, H, fail, nredo);
-  if (CENTRED)
-    rho2 = L.disc(n, *cx, *cy);
-  else
-    rho2 = L.rho2(n);
+  // the half-plane in T (float: in bins) and the bound of a value's rounding
+  const double sc = sizeof(T) == sizeof(float) ? C.ih : 1.0;
+  const T Tx = (T)(Yx * sc), Ty = (T)(Yy * sc), Tk = (T)(kk * (sc * sc));
+  const float len = fabsf((float)(Yx * C.ih)) + fabsf((float)(Yy * C.ih));
+  const float err = 1e-6f * (fabsf((float)(kk * (C.ih * C.ih))) +
+                             2.0f * __builtin_amdgcn_sqrtf(C.rb) * len);
+  const float thr = err * (float)C.h2;  // for the FP32 polygon's own values
+  const float inv = __builtin_amdgcn_rcpf(len);
+  // order of the candidates: depth of the cut over |Y|, the lane in the low
+  // bits; kNone for those that do not cut
+  constexpr unsigned kNone = ~0u;
+  auto order = [&]() -> unsigned {
+    const T vx = (T)((double)C.x * sc), vy = (T)((double)C.y * sc);
+    T m = T(-kInf);
+#define MA_VERTEX(v) m = fmax(m, dpp<kDppBcast + v>(vx) * Tx + dpp<kDppBcast + v>(vy) * Ty);
+    MA_VERTEX(0) MA_VERTEX(1) MA_VERTEX(2) MA_VERTEX(3) MA_VERTEX(4) MA_VERTEX(5)
+    if (C.n > 6) {
+      MA_VERTEX(6) MA_VERTEX(7) MA_VERTEX(8)
+      if (C.n > 9) {
+        MA_VERTEX(9) MA_VERTEX(10) MA_VERTEX(11) MA_VERTEX(12) MA_VERTEX(13) MA_VERTEX(14)
+        MA_VERTEX(15)
+      }
+    }
+#undef MA_VERTEX
+    const T d = Tk - T(2) * m;
+    const bool reach = sizeof(T) == sizeof(float) ? !(d > (T)err) : !(d > T(0));
+    const float key = sizeof(T) == sizeof(float) ? (float)d * inv
+                                                 : (float)((double)d * (C.ih * C.ih)) * inv;
+    const int u = __float_as_int(key);
+    const unsigned o = (unsigned)(u ^ ((u >> 31) | (int)0x80000000)) & ~15u;
+    return has && reach ? (o | (unsigned)C.l) : kNone;
+  };
+  if (!C.mask(has)) return;
+  bool any = false;
+  unsigned key = order();
+  while (true) {
+    const unsigned best = row_min(key);
+    if (best == kNone) break;
+    const int c = (int)(best & 15u);
+    if (C.l == c) {
+      has = false;
+      key = kNone;
+    }
+    if (SEEN) {
+      const int cand = C.get((int)j, c);
+      if (C.mask(C.l < C.n && C.lab == cand)) continue;
+    }
+    const bool changed = C.clip(c, Yx, Yy, kk, (int)j, thr, fail);
+    if (fail || C.n == 0) return;
+    if (changed) {
+      any = true;
+      key = order();
+    }
+  }
+  if (any) C.update_radius();
 }
 
-// Writes a finished cell: polygon, bounding box, candidate triangle count.
+// Ranges [lo, lo + cnt) of the group's lanes as one stream: f(q, b, valid) is
+// called for 16 consecutive entries at a time, q the entry and b the lane
+// whose range holds it; more() stops the stream.
+template <class F, class M>
+__device__ inline void for_ranges(int base, int l, int32_t lo, int cnt, M &&more, F &&f) {
+  const int inc = row_scan(cnt);
+  const int ex = inc - cnt, tot = dpp<kDppBcast + 15>(inc);
+  for (int s0 = 0; s0 < tot && more(); s0 += kGroup) {
+    const int s = s0 + l;
+    int b = 0;  // the last lane whose range starts at or before s
+#pragma unroll
+    for (int step = 8; step > 0; step >>= 1)
+      if (row_get(ex, 4 * base, b + step) <= s) b += step;
+    const int32_t q = row_get(lo - ex, 4 * base, b) + s;
+    f(q, b, s < tot);
+  }
+}
+
+// Clips by the Diracs of the lanes' ranges (of `list`, or Diracs themselves).
+template <class T, bool SEEN, class R>
+__device__ inline void clip_ranges(const CellArgs &a, int64_t k, double yx, double yy, double wk,
+                                   int32_t lo, int cnt, const int32_t *list, Cell<R> &C,
+                                   bool &fail) {
+  for_ranges(C.base, C.l, lo, cnt, [&]() { return C.n > 0 && !fail; },
+             [&](int32_t q, int, bool valid) {
+               const int32_t j = valid ? (list ? list[q] : q) : -1;
+               clip_batch<T, SEEN>(a, k, yx, yy, wk, j, C, fail);
+             });
+}
+
+// The triangles whose bounding box meets [px0,px1]x[py0,py1], once each, by
+// the 16 lanes of a group: f(ti, i) for the i-th of them.  A triangle listed
+// in several bins is taken in the bin of the lower-left corner of the overlap
+// of the two boxes, which its bin entries mark (kTriFirstX, kTriFirstY).
+// Returns their number.
+template <class F>
+__device__ inline int group_triangles(const CellArgs &a, int base, int l, double px0, double py0,
+                                      double px1, double py1, F &&f) {
+  const Grid &g = a.g;
+  // lanes 0..3 locate one side each
+  const double side = l == 0 ? px0 : l == 1 ? py0 : l == 2 ? px1 : py1;
+  const int bc = bin_coord(side, (l & 1) ? g.y0 : g.x0, g.h, g.G);
+  const int qx0 = dpp<kDppBcast + 0>(bc), qy0 = dpp<kDppBcast + 1>(bc);
+  const int qx1 = dpp<kDppBcast + 2>(bc), qy1 = dpp<kDppBcast + 3>(bc);
+  const int W = qx1 - qx0 + 1, nb = W * (qy1 - qy0 + 1);
+  const float invW = 1.0f / (float)W;
+  int count = 0;
+  for (int t0 = 0; t0 < nb; t0 += kGroup) {
+    const int t = t0 + l;
+    int ty = (int)((float)t * invW);  // t / W, off by one at most
+    ty += (t >= (ty + 1) * W) - (t < ty * W);
+    const int by = qy0 + ty, bx = qx0 + t - ty * W;
+    int32_t lo = 0;
+    int cnt = 0;
+    if (t < nb) {
+      const int64_t b = morton2((uint32_t)bx, (uint32_t)by);
+      lo = a.tbin_start[b];
+      cnt = a.tbin_start[b + 1] - lo;
+    }
+    const int first = (bx == qx0 ? kTriFirstX : 0) | (by == qy0 ? kTriFirstY : 0);
+    for_ranges(base, l, lo, cnt, []() { return true; }, [&](int32_t q, int b, bool valid) {
+      const int fb = row_get(first, 4 * base, b);
+      bool hit = false;
+      int32_t ti = 0;
+      if (valid) {
+        const int32_t it = a.tbin_items[q];
+        ti = it >> kTriShift;
+        if (((it | fb) & (kTriFirstX | kTriFirstY)) == (kTriFirstX | kTriFirstY)) {
+          const float4 tb = a.tbox[ti];
+          hit = !((double)tb.z < px0 || (double)tb.x > px1 || (double)tb.w < py0 ||
+                  (double)tb.y > py1);
+        }
+      }
+      const unsigned m = (unsigned)(__ballot(hit) >> base) & 0xffffu;
+      if (hit) f(ti, count + __popc(m & ((1u << l) - 1u)));
+      count += __popc(m);
+    });
+  }
+  return count;
+}
+
+// FP32 polygons: the vertices of a finished cell between two neighbours are
+// taken again as the crossing of the two bisectors, in FP64, and rounded once
+// (the clips' own vertices carry the rounding of the far ends of the edges
+// they cut; without this the masses at 1M Diracs are 9.5e-7 off in the 2-norm
+// instead of 6.4e-8).  A vertex that moves by more than 1e-3 of a bin (bisectors
+// nearly parallel) stays.
+__device__ inline void polish(const CellArgs &a, int64_t k, double yx, double yy, double wk,
+                              Cell<float> &C) {
+  const int l = C.l, n = C.n;
+  const int lp = l == 0 ? n - 1 : l - 1;
+  const bool own = l < n && C.lab >= 0;
+  double Yx = 0.0, Yy = 0.0, kk = 0.0;
+  if (own) {
+    const double2 pj = reinterpret_cast<const double2 *>(a.pos)[C.lab];
+    Yx = pj.x - yx;
+    Yy = pj.y - yy;
+    kk = Yx * Yx + Yy * Yy + wdiff(a.wlo, wk, k, a.w[C.lab], C.lab);
+  }
+  const double Px = C.get(Yx, lp & (kGroup - 1)), Py = C.get(Yy, lp & (kGroup - 1));
+  const double kp = C.get(kk, lp & (kGroup - 1));
+  const double det = Px * Yy - Py * Yx;  // zero without two neighbours
+  if (own && det != 0.0) {
+    const double s = 0.5 / det;
+    const double X = (kp * Yy - kk * Py) * s, Y = (Px * kk - Yx * kp) * s;
+    if (fabs(X - (double)C.x) + fabs(Y - (double)C.y) <= 1e-3 * a.g.h) {
+      C.x = (float)X;
+      C.y = (float)Y;
+    }
+  }
+  const float x0 = C.get(C.x, 0), y0 = C.get(C.y, 0);
+  C.x = l < n ? C.x : x0;
+  C.y = l < n ? C.y : y0;
+}
+__device__ inline void polish(const CellArgs &, int64_t, double, double, double, Cell<double> &) {}
+
+// Writes a finished cell: polygon, bounding box, candidate triangles (counted,
+// and the first kPadTri kept for k_pairs).
 template <class R>
 __device__ inline void write_cell(const CellArgs &a, int64_t k, double yx, double yy,
-                                  const CellLDS<R> &L, int n) {
-  const int64_t N = a.n;
-  a.pn[k] = n;
+                                  const Cell<R> &C) {
+  const int l = C.l, n = C.n;
+  if (l == 0) a.pn[k] = n;
   if (n == 0) {
-    a.tcount[k] = 0;
+    if (l == 0) a.tcount[k] = 0;
     return;
   }
-  R *px = CellBuf<R>::px(a), *py = CellBuf<R>::py(a), *eacc = CellBuf<R>::eacc(a);
-  double bx0 = kInf, by0 = kInf, bx1 = -kInf, by1 = -kInf;
-  for (int v = 0; v < n; v++) {
-    const R x = L.sx[v][L.t], y = L.sy[v][L.t];
-    px[v * N + k] = x;
-    py[v * N + k] = y;
-    a.plab[v * N + k] = L.sl[v][L.t];
-    eacc[v * N + k] = R(-0.0);  // "not seen": any contribution (>= 0) clears the sign
-    bx0 = fmin(bx0, (double)x);
-    bx1 = fmax(bx1, (double)x);
-    by0 = fmin(by0, (double)y);
-    by1 = fmax(by1, (double)y);
+  if (l < n) {
+    const int64_t at = k * kMaxFast + l;
+    CellBuf<R>::px(a)[at] = C.x;
+    CellBuf<R>::py(a)[at] = C.y;
+    a.plab[at] = C.lab;
+    CellBuf<R>::eacc(a)[at] = R(-0.0);  // "not seen": any contribution (>= 0) clears the sign
   }
-  bx0 += yx; bx1 += yx; by0 += yy; by1 += yy;
-  a.bbox[4 * k] = bx0;
-  a.bbox[4 * k + 1] = by0;
-  a.bbox[4 * k + 2] = bx1;
-  a.bbox[4 * k + 3] = by1;
-  // candidate triangles: counted, and the first kPadTri kept for k_pairs
-  int cnt = 0;
-  for_each_triangle(a.g, a.tbin_start, a.tbin_items, a.tbox, bx0, by0, bx1, by1, 0, 0,
-                    a.g.G - 1, a.g.G - 1, [&](int32_t ti) {
-                      if (cnt < kPadTri) a.ptri[cnt * N + k] = ti;
-                      cnt++;
-                    });
-  a.tcount[k] = cnt;
+  const double bx0 = (double)row_min(C.x) + yx, by0 = (double)row_min(C.y) + yy;
+  const double bx1 = (double)row_max(C.x) + yx, by1 = (double)row_max(C.y) + yy;
+  if (l < 4) a.bbox[4 * k + l] = l == 0 ? bx0 : l == 1 ? by0 : l == 2 ? bx1 : by1;
+  const int cnt = group_triangles(a, C.base, l, bx0, by0, bx1, by1, [&](int32_t ti, int i) {
+    if (i < kPadTri) a.ptri[k * kPadTri + i] = ti;
+  });
+  if (l == 0) a.tcount[k] = cnt;
 }
 
 __device__ inline void zero_cell_outputs(const CellArgs &a, int64_t k) {
@@ -397,41 +594,57 @@ __device__ inline void zero_cell_outputs(const CellArgs &a, int64_t k) {
   }
 }
 
-// Lower bound of pi_j - pi_k over the polygon (radius rho about y_k) for
-// every Dirac j at distance >= D from y_k with weight <= W; the polygon is
-// safe from such j when it is positive.
-__device__ inline bool far_enough(double D, double rho, double W, double wk) {
-  return D > rho && D * D - 2.0 * rho * D - (W - wk) > 1e-12 * (D * D + fabs(W) + fabs(wk));
+// Lower bound of pi_j - pi_k over the polygon (squared radius rho2 about y_k)
+// for every Dirac j at squared distance >= D2 from y_k with weight <= W: the
+// polygon is safe from such j when D > rho and D^2 - 2 rho D - (W - w_k) > 0,
+// decided on squares (no square roots).
+__device__ inline bool far_enough(double D2, double rho2, double W, double wk) {
+  const double t = D2 - (W - wk) - 1e-12 * (D2 + fabs(W) + fabs(wk));
+  return D2 > rho2 && t > 0.0 && t * t > 4.0 * rho2 * D2;
 }
 
-// Multi-level certificate for the polygon (radius rho about y_k) once the
-// bins within Chebyshev distance r of the Dirac's bin have been visited.  At
-// level l the 3 x 3 block of level-l nodes around the Dirac's node contains
+// Multi-level certificate for the polygon (squared radius rho2 about y_k) once
+// the bins within Chebyshev distance r of the Dirac's bin have been visited.
+// At level l the 3 x 3 block of level-l nodes around the Dirac's node contains
 // the bins within 2^l of its bin; the Diracs of that block not yet covered
-// lie at least as far as the boundary of the covered region and weigh at
-// most the block's maximum (pyr3).  Blocks are nested and the top one is the
-// whole grid, so every unvisited Dirac is bounded once.
+// lie at least as far as the boundary of the covered region (the block one
+// level down, or the visited square) and weigh at most the block's maximum
+// (pyr3).  Blocks are nested and the top one is the whole grid, so every
+// unvisited Dirac is bounded once.  Lane l takes level l.
+template <class R>
 __device__ inline bool certify_levels(const Grid &g, const double *pyr3, const PyrOff &off, int sbx,
-                                      int sby, int r, double yx, double yy, double rho,
+                                      int sby, int r, double yx, double yy, const Cell<R> &C,
                                       double wk) {
-  int x0 = max(sbx - r, 0), x1 = min(sbx + r, g.G - 1);
-  int y0 = max(sby - r, 0), y1 = min(sby + r, g.G - 1);
-  for (int l = 0; l <= g.L; l++) {
-    const int nx = sbx >> l, ny = sby >> l;
-    const int bx0 = max((nx - 1) << l, 0), bx1 = min(((nx + 2) << l) - 1, g.G - 1);
-    const int by0 = max((ny - 1) << l, 0), by1 = min(((ny + 2) << l) - 1, g.G - 1);
-    if (bx0 > x0 || bx1 < x1 || by0 > y0 || by1 < y1) continue;  // does not hold the region yet
+  static_assert(kMaxLevels < kGroup, "one lane per level");
+  const int G = g.G, l = C.l;
+  const int vx0 = max(sbx - r, 0), vx1 = min(sbx + r, G - 1);
+  const int vy0 = max(sby - r, 0), vy1 = min(sby + r, G - 1);
+  auto block = [&](int lev, int &x0, int &y0, int &x1, int &y1) {
+    const int nx = sbx >> lev, ny = sby >> lev;
+    x0 = max((nx - 1) << lev, 0);
+    x1 = min(((nx + 2) << lev) - 1, G - 1);
+    y0 = max((ny - 1) << lev, 0);
+    y1 = min(((ny + 2) << lev) - 1, G - 1);
+    return x0 <= vx0 && x1 >= vx1 && y0 <= vy0 && y1 >= vy1;  // holds the visited square
+  };
+  bool ok = true;
+  int bx0, by0, bx1, by1;
+  if (l <= g.L && block(l, bx0, by0, bx1, by1)) {
+    int x0 = vx0, y0 = vy0, x1 = vx1, y1 = vy1;
+    if (l > 0 && block(l - 1, bx0, by0, bx1, by1)) {
+      x0 = bx0; y0 = by0; x1 = bx1; y1 = by1;
+    }
     double D = kInf;
     if (x0 > 0) D = fmin(D, yx - (g.x0 + x0 * g.h));
-    if (x1 < g.G - 1) D = fmin(D, g.x0 + (x1 + 1) * g.h - yx);
+    if (x1 < G - 1) D = fmin(D, g.x0 + (x1 + 1) * g.h - yx);
     if (y0 > 0) D = fmin(D, yy - (g.y0 + y0 * g.h));
-    if (y1 < g.G - 1) D = fmin(D, g.y0 + (y1 + 1) * g.h - yy);
-    if (D == kInf) return true;  // the covered region is the whole grid
-    const double Wb = pyr3[off.o[l] + morton2((uint32_t)nx, (uint32_t)ny)];
-    if (Wb != -kInf && !far_enough(D, rho, Wb, wk)) return false;
-    x0 = bx0; x1 = bx1; y0 = by0; y1 = by1;
+    if (y1 < G - 1) D = fmin(D, g.y0 + (y1 + 1) * g.h - yy);
+    if (D != kInf) {
+      const double Wb = pyr3[off.o[l] + morton2((uint32_t)(sbx >> l), (uint32_t)(sby >> l))];
+      ok = Wb == -kInf || (D > 0.0 && far_enough(D * D, C.rho2(), Wb, wk));
+    }
   }
-  return true;
+  return C.mask(!ok) == 0u;
 }
 
 // -0.0 exactly (an edge integral no fragment has touched)
@@ -449,284 +662,273 @@ __device__ inline void wave_count(T *dst, bool flag) {
     atomicAdd(dst, (T)__popcll(bal));
 }
 
-// Next bin of Chebyshev ring r around bin (sbx, sby) inside the grid, in row
-// order: every bin of the ring's first and last rows, the two ends of the
-// others (bx = INT_MIN before the first).  Returns false after the last.
-__device__ inline bool ring_next(int sbx, int sby, int G, int r, int &by, int &bx) {
-  while (true) {
-    if (bx == INT_MIN) {
-      by = max(sby - r, 0);
-      bx = sbx - r;
-    } else {
-      const bool edge_row = (by == sby - r) || (by == sby + r);
-      bx += (edge_row || r == 0) ? 1 : 2 * r;
-      if (bx > sbx + r) {
-        by++;
-        bx = sbx - r;
-      }
-    }
-    if (by > min(sby + r, G - 1)) return false;
-    if (bx >= 0 && bx < G) return true;
-  }
-}
-
-// Site-centric construction: the domain box is clipped by the Diracs of the
-// bins in Chebyshev rings 0..rmax around the Dirac's own bin.  After each
-// ring the cell is final if every unvisited Dirac (distance >= D from y_k,
-// weight <= the global maximum) is far_enough.  Otherwise the remaining
-// Diracs are reached through the max-weight pyramid: a depth-first walk in
-// Morton order (stackless: children of node m are 4m..4m+3 one level down)
-// that skips nodes inside the visited square, prunes nodes that are
-// far_enough for their own maximum weight and clips by the Diracs of the
-// bins it reaches.  Pruning uses the polygon radius at the time of the test,
-// which only shrinks, so every pruned Dirac stays unable to cut the final
-// cell.
+// Site-centric construction: the starting box is clipped by the Diracs of the
+// bins in Chebyshev rings 0..rmax around the Dirac's own bin (rings 0 and 1
+// together).  A lane takes a bin; from ring 2 on a bin whose maximum weight
+// and distance cannot reach the polygon is skipped.  After each ring the cell
+// is final if every unvisited Dirac is far_enough (certify_levels).  Otherwise
+// the remaining Diracs are reached through the max-weight pyramid: a
+// depth-first walk that tests the 16 grandchildren of a node at once, skips
+// nodes inside the visited square, prunes nodes that are far_enough for their
+// own maximum weight and clips by the Diracs of the nodes it keeps.  Pruning
+// uses the polygon radius at the time of the test, which only shrinks, so
+// every pruned Dirac stays unable to cut the final cell.
+constexpr int kWalkStack = 64;  // pending nodes of a walk; a fuller one goes to the bin path
 template <class R>
-__global__ void __launch_bounds__(kCellBlock) k_cell_local(CellArgs a, const double *pyr,
-                                                           const double *pyr3, PyrOff off,
-                                                           int rmax) {
-  __shared__ R sx[kMaxFast][kCellBlock];
-  __shared__ R sy[kMaxFast][kCellBlock];
-  __shared__ int sl[kMaxFast][kCellBlock];
-  CellLDS<R> L{sx, sy, sl, (int)threadIdx.x};
-  const int64_t k = xcd_block(blockIdx.x, gridDim.x) * kCellBlock + threadIdx.x;
+__global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const double *pyr,
+                                                             const double *pyr3, PyrOff off,
+                                                             int rmax) {
+  __shared__ uint32_t stacks[kCellGroups][kWalkStack];
+  const int64_t k = xcd_block<kCellXcdRun>(blockIdx.x, gridDim.x) * kCellGroups +
+                    threadIdx.x / kGroup;
   if (k >= a.n) return;
   const Grid &g = a.g;
-  zero_cell_outputs(a, k);
+  Cell<R> C(g);
+  const int l = C.l;
+  const bool lead = l == 0;
+  if (lead) zero_cell_outputs(a, k);
   if (a.force_general) {
-    a.pn[k] = -1;
-    a.tcount[k] = 0;
-    atomicOr(&a.flags[3], 1);
-    if (sizeof(R) == sizeof(double)) a.far[k] = 0;
+    if (lead) {
+      a.pn[k] = -1;
+      a.tcount[k] = 0;
+      atomicOr(&a.flags[3], 1);
+      if (sizeof(R) == sizeof(double)) a.far[k] = 0;
+    }
     return;
   }
-  const double yx = a.pos[2 * k], yy = a.pos[2 * k + 1], wk = a.w[k];
+  const int lane16 = (int)((k >> 6) & 15);
   if (sizeof(R) == sizeof(double) && a.use_far && a.far[k]) {
     // far from its Dirac at the last weights: the per-bin candidate owners
     // build it exactly (the site-centric search would only run over budget)
-    const int lane16 = (int)((k >> 6) & 15);
-    wave_count(&a.stripes[(16 + lane16) * 16], true);
-    a.pn[k] = -2;
-    a.tcount[k] = 0;
+    wave_count(&a.stripes[(16 + lane16) * 16], lead);
+    if (lead) {
+      a.pn[k] = -2;
+      a.tcount[k] = 0;
+    }
     return;
   }
-  int n = 4, nredo = 0;
-  bool fail = !L.init(a.dom[0] - yx, a.dom[1] - yy, a.dom[2] - yx, a.dom[3] - yy,
-                      a.box_half);
+  const double yx = a.pos[2 * k], yy = a.pos[2 * k + 1], wk = a.w[k];
+  bool fail = !C.init(a.dom[0] - yx, a.dom[1] - yy, a.dom[2] - yx, a.dom[3] - yy, a.box_half);
   bool certified = false;
-  double rho2 = L.rho2(4);
-  const double W = pyr[off.o[g.L]];
+  // squared distance of y_k to the box of nodes [x, x + 2^lev) x [y, y + 2^lev)
+  auto dist2 = [&](int x, int y, int lev) {
+    const double X0 = g.x0 + x * g.h, X1 = g.x0 + (x + (1 << lev)) * g.h;
+    const double Y0 = g.y0 + y * g.h, Y1 = g.y0 + (y + (1 << lev)) * g.h;
+    const double dx = fmax(fmax(X0 - yx, yx - X1), 0.0);
+    const double dy = fmax(fmax(Y0 - yy, yy - Y1), 0.0);
+    return dx * dx + dy * dy;
+  };
   const int sbx = bin_coord(yx, g.x0, g.h, g.G), sby = bin_coord(yy, g.y0, g.h, g.G);
-  int r = 0;
-  for (; r <= rmax && n > 0 && !fail; r++) {
-    // the ring's Diracs as one stream per lane: a lane moves on to its next
-    // non-empty bin by itself, so every pass of the loop clips one candidate
-    // on every lane that has one (bin by bin, the wave would wait each time
-    // for its fullest bin); the certificate below stays ring-synchronous
-    int by = 0, bx = INT_MIN;
-    int32_t q = 0, qe = 0;
-    while (n > 0 && !fail) {
-      bool more = true;
-      while (q >= qe && (more = ring_next(sbx, sby, g.G, r, by, bx))) {
-        const int64_t b = morton2((uint32_t)bx, (uint32_t)by);
-        q = a.bin_start[b];
-        qe = a.bin_start[b + 1];
+  int r = min(rmax, 1);
+  for (; r <= rmax && C.n > 0 && !fail; r++) {
+    // positions of the ring, counter-clockwise from its lower-left corner
+    // (r <= 1: the bins of the 3 x 3 block, or the Dirac's own)
+    const int len = r == 0 ? 1 : r == 1 ? 9 : 8 * r;
+    for (int p0 = 0; p0 < len && C.n > 0 && !fail; p0 += kGroup) {
+      const int p = p0 + l;
+      int bx = sbx, by = sby;
+      if (r == 1) {
+        bx += p % 3 - 1;
+        by += p / 3 - 1;
+      } else if (r > 1) {
+        const int sd = (p >= 2 * r) + (p >= 4 * r) + (p >= 6 * r), o = p - sd * 2 * r;
+        bx += sd == 0 ? o - r : sd == 1 ? r : sd == 2 ? r - o : -r;
+        by += sd == 0 ? -r : sd == 1 ? o - r : sd == 2 ? r : r - o;
       }
-      if (!more) break;
-      consider(a, k, q, yx, yy, wk, L, n, rho2, fail, nredo);
-      q++;
+      int32_t lo = 0;
+      int cnt = 0;
+      if (p < len && bx >= 0 && bx < g.G && by >= 0 && by < g.G) {
+        const int64_t b = morton2((uint32_t)bx, (uint32_t)by);
+        if (r <= 1 || !far_enough(dist2(bx, by, 0), C.rho2(), pyr[b], wk)) {
+          lo = a.bin_start[b];
+          cnt = a.bin_start[b + 1] - lo;
+        }
+      }
+      clip_ranges<float, false>(a, k, yx, yy, wk, lo, cnt, nullptr, C, fail);
     }
-    if (n == 0 || fail) break;
-    double D = kInf;
-    if (sbx - r > 0) D = fmin(D, yx - (g.x0 + (sbx - r) * g.h));
-    if (sbx + r < g.G - 1) D = fmin(D, g.x0 + (sbx + r + 1) * g.h - yx);
-    if (sby - r > 0) D = fmin(D, yy - (g.y0 + (sby - r) * g.h));
-    if (sby + r < g.G - 1) D = fmin(D, g.y0 + (sby + r + 1) * g.h - yy);
-    if (D == kInf || far_enough(D, sqrt(rho2), W, wk) ||
-        certify_levels(g, pyr3, off, sbx, sby, r, yx, yy, sqrt(rho2), wk)) {
+    if (C.n == 0 || fail) break;
+    if (certify_levels(g, pyr3, off, sbx, sby, r, yx, yy, C, wk)) {
       certified = true;
       break;
     }
   }
-  const bool walk = !certified && n > 0 && !fail;
+  const bool walk = !certified && C.n > 0 && !fail;
   bool over_budget = false;
   if (walk) {
     // bins [sbx - rr, sbx + rr] x [sby - rr, sby + rr] have been visited
     const int rr = min(r, rmax);
     const int vx0 = sbx - rr, vx1 = sbx + rr, vy0 = sby - rr, vy1 = sby + rr;
-    int l = g.L;
-    uint32_t m = 0;
-    int visits = 0;
-    while (n > 0 && !fail) {
-      if (++visits > a.walk_budget) {
+    uint32_t *stack = stacks[threadIdx.x / kGroup];
+    int sp = 0, visits = 0;
+    uint32_t ent = (uint32_t)g.L << 27;
+    while (true) {
+      const int lev = (int)(ent >> 27), st = min(lev, 2), cl = lev - st;
+      const uint32_t ch = ((ent & ((1u << 27) - 1u)) << (2 * st)) | (uint32_t)l;
+      const int nch = 1 << (2 * st);
+      visits += nch;
+      if (visits > a.walk_budget) {
         // weights with a large spread leave many nodes unprunable: the cell
         // is rebuilt from the per-bin candidate owners instead
         over_budget = true;
         break;
       }
-      const int nx0 = (int)(compact1by1(m) << l), ny0 = (int)(compact1by1(m >> 1) << l);
-      const int nx1 = nx0 + (1 << l) - 1, ny1 = ny0 + (1 << l) - 1;
       bool descend = false;
-      if (!(nx0 >= vx0 && nx1 <= vx1 && ny0 >= vy0 && ny1 <= vy1)) {
-        const double Wn = pyr[off.o[l] + m];
-        if (Wn != -kInf) {
-          const double bx0 = g.x0 + nx0 * g.h, bx1 = g.x0 + (nx1 + 1) * g.h;
-          const double by0 = g.y0 + ny0 * g.h, by1 = g.y0 + (ny1 + 1) * g.h;
-          const double dx = fmax(fmax(bx0 - yx, yx - bx1), 0.0);
-          const double dy = fmax(fmax(by0 - yy, yy - by1), 0.0);
-          if (!far_enough(sqrt(dx * dx + dy * dy), sqrt(rho2), Wn, wk)) {
+      int32_t lo = 0;
+      int cnt = 0;
+      if (l < nch) {
+        const int nx = (int)(compact1by1(ch) << cl), ny = (int)(compact1by1(ch >> 1) << cl);
+        const int sd = 1 << cl;
+        if (!(nx >= vx0 && nx + sd - 1 <= vx1 && ny >= vy0 && ny + sd - 1 <= vy1)) {
+          const double W = pyr[off.o[cl] + ch];
+          if (W != -kInf && !far_enough(dist2(nx, ny, cl), C.rho2(), W, wk)) {
             // the Diracs of a node are one contiguous Morton range: a node
             // holding few of them (sparse regions) is taken whole
-            const int32_t q0 = a.bin_start[(int64_t)m << (2 * l)];
-            const int32_t q1 = a.bin_start[((int64_t)m + 1) << (2 * l)];
-            if (l == 0 || q1 - q0 <= kNodeDiracs) {
-              for (int32_t q = q0; q < q1 && n > 0 && !fail; q++)
-                consider(a, k, q, yx, yy, wk, L, n, rho2, fail, nredo);
-            } else {
+            lo = a.bin_start[(int64_t)ch << (2 * cl)];
+            cnt = a.bin_start[((int64_t)ch + 1) << (2 * cl)] - lo;
+            if (cl > 0 && cnt > kNodeDiracs) {
               descend = true;
+              cnt = 0;
             }
           }
         }
       }
-      if (descend) {
-        l--;
-        m <<= 2;
-        continue;
+      const unsigned dm = C.mask(descend);
+      if (sp + __popc(dm) > kWalkStack) {
+        over_budget = true;
+        break;
       }
-      while (l < g.L && (m & 3u) == 3u) {
-        m >>= 2;
-        l++;
-      }
-      if (l == g.L) break;
-      m++;
+      if (descend) stack[sp + __popc(dm & ((1u << l) - 1u))] = ((uint32_t)cl << 27) | ch;
+      sp += __popc(dm);
+      clip_ranges<float, true>(a, k, yx, yy, wk, lo, cnt, nullptr, C, fail);
+      if (sp == 0 || C.n == 0 || fail) break;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the lanes' stack entries
+      ent = stack[--sp];
     }
   }
   // a cell still touching the starting box is larger than that box (or lies
   // beyond it): in FP64 it is rebuilt from the per-bin candidate owners, in
   // FP32 by the FP64 kernels
-  if (!fail && !over_budget && L.touches_cut(n)) {
+  if (!fail && !over_budget && C.touches_cut()) {
     if (sizeof(R) == sizeof(double))
       over_budget = true;
     else
       fail = true;
   }
-  {
-    const int lane16 = (int)((k >> 6) & 15);
-    wave_count(&a.stripes[lane16 * 16], walk);  // cells that needed the pyramid walk
-    wave_count(&a.stripes[(16 + lane16) * 16], over_budget && !fail);  // left to the bin path
-    wave_count(&a.stripes[(32 + lane16) * 16], fail);  // left to the general kernels
+  wave_count(&a.stripes[lane16 * 16], lead && walk);  // cells that needed the pyramid walk
+  wave_count(&a.stripes[(16 + lane16) * 16], lead && over_budget && !fail);  // left to the bin path
+  wave_count(&a.stripes[(32 + lane16) * 16], lead && fail);  // left to the general kernels
+  if (Tol<R>::redo > R(0)) {
+    const int redo = row_sum(C.nredo);
+    if (lead && redo > 0) atomicAdd(&a.counters[5], (unsigned long long)redo);
   }
-  if (Tol<R>::redo > R(0) && nredo > 0) atomicAdd(&a.counters[5], (unsigned long long)nredo);
-  if (fail) {
-    a.pn[k] = -1;
-    a.tcount[k] = 0;
-    atomicOr(&a.flags[3], 1);
+  if (lead && sizeof(R) == sizeof(double) && !fail) a.far[k] = over_budget ? 1 : 0;
+  if (fail || over_budget) {
+    if (lead) {
+      a.pn[k] = fail ? -1 : -2;
+      a.tcount[k] = 0;
+      if (fail) atomicOr(&a.flags[3], 1);
+    }
     return;
   }
-  if (sizeof(R) == sizeof(double)) a.far[k] = over_budget ? 1 : 0;
-  if (over_budget) {
-    a.pn[k] = -2;
-    a.tcount[k] = 0;
-    return;
-  }
-  write_cell(a, k, yx, yy, L, n);
+  polish(a, k, yx, yy, wk, C);
+  write_cell(a, k, yx, yy, C);
 }
 
 // Bin-candidate construction for the cells listed in `list` (those whose
 // pyramid walk ran over budget): the bin rectangle of the Dirac is clipped by
-// the candidate owners of its bins, nearest rings first.  The rectangle
-// covers every bin where the Dirac may own a point and the owners of every
-// point of these bins are among the candidates, so no certificate is needed.
+// the candidate owners of its bins.  The rectangle covers every bin where the
+// Dirac may own a point and the owners of every point of these bins are among
+// the candidates, so no certificate is needed.
 template <class R>
-__global__ void __launch_bounds__(kCellBlock) k_cell_bins(CellArgs a, const int32_t *list,
-                                                          const int32_t *nlist) {
-  __shared__ R sx[kMaxFast][kCellBlock];
-  __shared__ R sy[kMaxFast][kCellBlock];
-  __shared__ int sl[kMaxFast][kCellBlock];
-  CellLDS<R> L{sx, sy, sl, (int)threadIdx.x};
-  const int64_t idx = blockIdx.x * (int64_t)kCellBlock + threadIdx.x;
+__global__ void __launch_bounds__(kCellThreads) k_cell_bins(CellArgs a, const int32_t *list,
+                                                            const int32_t *nlist) {
+  const int64_t idx = blockIdx.x * (int64_t)kCellGroups + threadIdx.x / kGroup;
   if (idx >= *nlist) return;
-  const int64_t k = list[idx];
   const Grid &g = a.g;
+  Cell<R> C(g);
+  const int l = C.l;
+  const bool lead = l == 0;
+  const int64_t k = list[idx];
   const int rx0 = a.rect[4 * k], ry0 = a.rect[4 * k + 1], rx1 = a.rect[4 * k + 2],
             ry1 = a.rect[4 * k + 3];
   if (rx0 > rx1) {
-    a.pn[k] = 0;
-    a.tcount[k] = 0;
+    if (lead) {
+      a.pn[k] = 0;
+      a.tcount[k] = 0;
+    }
     return;
   }
-  if ((int64_t)(rx1 - rx0 + 1) * (ry1 - ry0 + 1) > kBigRect) {
-    // a long sequential candidate loop: left to the workgroup-per-cell kernel
-    a.pn[k] = -1;
-    a.tcount[k] = 0;
-    atomicOr(&a.flags[3], 1);
+  const int W = rx1 - rx0 + 1;
+  if ((int64_t)W * (ry1 - ry0 + 1) > kBigRect) {
+    // many bins: left to the workgroup-per-cell kernel
+    if (lead) {
+      a.pn[k] = -1;
+      a.tcount[k] = 0;
+      atomicOr(&a.flags[3], 1);
+    }
     return;
   }
+  const int nb = W * (ry1 - ry0 + 1);
   const double yx = a.pos[2 * k], yy = a.pos[2 * k + 1], wk = a.w[k];
-  int n = 4, nredo = 0;
-  bool fail = !L.init(g.x0 + rx0 * g.h - yx, g.y0 + ry0 * g.h - yy,
+  bool fail = !C.init(g.x0 + rx0 * g.h - yx, g.y0 + ry0 * g.h - yy,
                       g.x0 + (rx1 + 1) * g.h - yx, g.y0 + (ry1 + 1) * g.h - yy,
                       sizeof(R) == sizeof(float) ? a.box_half : kInf);  // FP64: the rectangle bounds it
-  double ccx = 0.0, ccy = 0.0;
-  double rho2 = L.disc(4, ccx, ccy);
-  const int sbx = min(max(bin_coord(yx, g.x0, g.h, g.G), rx0), rx1);
-  const int sby = min(max(bin_coord(yy, g.y0, g.h, g.G), ry0), ry1);
-  const int maxr = max(max(sbx - rx0, rx1 - sbx), max(sby - ry0, ry1 - sby));
-  for (int r = 0; r <= maxr && n > 0 && !fail; r++) {
-    for (int by = max(sby - r, ry0); by <= min(sby + r, ry1) && n > 0 && !fail; by++) {
-      const bool edge_row = (by == sby - r) || (by == sby + r);
-      for (int bx = max(sbx - r, rx0); bx <= min(sbx + r, rx1) && n > 0 && !fail; bx++) {
-        if (!edge_row && bx != sbx - r && bx != sbx + r) continue;
-        const int64_t b = morton2((uint32_t)bx, (uint32_t)by);
-        for (int32_t i = a.cand_start[b]; i < a.cand_start[b + 1] && n > 0 && !fail; i++)
-          consider<true>(a, k, a.cand[i], yx, yy, wk, L, n, rho2, fail, nredo, &ccx, &ccy);
-      }
+  for (int t0 = 0; t0 < nb && C.n > 0 && !fail; t0 += kGroup) {
+    const int t = t0 + l;
+    int32_t lo = 0;
+    int cnt = 0;
+    if (t < nb) {
+      const int64_t b = morton2((uint32_t)(rx0 + t % W), (uint32_t)(ry0 + t / W));
+      lo = a.cand_start[b];
+      cnt = a.cand_start[b + 1] - lo;
     }
+    clip_ranges<R, true>(a, k, yx, yy, wk, lo, cnt, a.cand, C, fail);
   }
-  if (Tol<R>::redo > R(0) && nredo > 0) atomicAdd(&a.counters[5], (unsigned long long)nredo);
-  if (!fail && L.touches_cut(n)) fail = true;
+  if (Tol<R>::redo > R(0)) {
+    const int redo = row_sum(C.nredo);
+    if (lead && redo > 0) atomicAdd(&a.counters[5], (unsigned long long)redo);
+  }
+  if (!fail && C.touches_cut()) fail = true;
   if (sizeof(R) == sizeof(double) && !fail) {
     // back within the site-centric search's starting box: the next
     // evaluation tries that search again
-    bool inside = true;
     const double half = a.box_half;
-    for (int v = 0; v < n; v++)
-      inside = inside && fabs((double)L.sx[v][L.t]) < half && fabs((double)L.sy[v][L.t]) < half;
-    a.far[k] = inside ? 0 : 1;
+    const bool out = l < C.n && !(fabs((double)C.x) < half && fabs((double)C.y) < half);
+    const bool any = C.mask(out) != 0u;
+    if (lead) a.far[k] = any ? 1 : 0;
   }
   if (fail) {
-    a.pn[k] = -1;
-    a.tcount[k] = 0;
-    atomicOr(&a.flags[3], 1);
+    if (lead) {
+      a.pn[k] = -1;
+      a.tcount[k] = 0;
+      atomicOr(&a.flags[3], 1);
+    }
     return;
   }
-  write_cell(a, k, yx, yy, L, n);
+  polish(a, k, yx, yy, wk, C);
+  write_cell(a, k, yx, yy, C);
 }
 
 // Exact owners of the bins.  Candidate entry i (Dirac j listed by bin b) is
 // kept only if the part of b (grown by 1e-6 of its side) where j beats every
 // other candidate of b has positive area: the grown bin square clipped by the
 // power half-planes of those candidates (coordinates local to y_j, strict tie
-// rule, the coincident-Dirac rule of consider) is not empty.  The owners of
+// rule, the coincident-Dirac rule of clip_batch) is not empty.  The owners of
 // every point of b are among its candidates, so the kept Diracs are those
 // whose cells meet the grown bin in positive area (entries whose clip
 // overflows or breaks on rounding are kept: a superfluous candidate costs
 // time, not correctness).  A Dirac's bin rectangle then spans only the bins
 // its cell meets, instead of every bin where its power merely comes close to
 // one competitor's.
-__global__ void __launch_bounds__(kCellBlock) k_cand_refine(
-    Grid g, const double *__restrict__ pos, const double *__restrict__ w, const double *wlo,
-    const int32_t *__restrict__ perm, const int32_t *__restrict__ cand_start,
-    const int32_t *__restrict__ cand, const int32_t *__restrict__ cbin, int64_t ncand,
-    int32_t *keep) {
-  __shared__ double sx[kMaxFast][kCellBlock];
-  __shared__ double sy[kMaxFast][kCellBlock];
-  __shared__ int sl[kMaxFast][kCellBlock];
-  CellLDS<double> L{sx, sy, sl, (int)threadIdx.x};
-  const int64_t i = blockIdx.x * (int64_t)kCellBlock + threadIdx.x;
+__global__ void __launch_bounds__(kCellThreads) k_cand_refine(CellArgs a, const int32_t *cbin,
+                                                              int64_t ncand, int32_t *keep) {
+  const int64_t i = xcd_block<kCellXcdRun>(blockIdx.x, gridDim.x) * kCellGroups +
+                    threadIdx.x / kGroup;
   if (i >= ncand) return;
-  const int32_t b = cbin[i], j = cand[i];
-  const double yx = pos[2 * j], yy = pos[2 * j + 1], wj = w[j];
+  const Grid &g = a.g;
+  Cell<double> C(g);
+  const int32_t b = cbin[i], j = a.cand[i];
+  const double yx = a.pos[2 * j], yy = a.pos[2 * j + 1];
   const uint32_t bx = compact1by1((uint32_t)b), by = compact1by1((uint32_t)b >> 1);
   // the bin grown by a margin: a neighbour across an edge of j's cell that
   // lies on a bin side owns a strip of the grown bin, so the bins of j's
@@ -735,34 +937,25 @@ __global__ void __launch_bounds__(kCellBlock) k_cand_refine(
   const double eps = 1e-6 * g.h;
   const double x0 = g.x0 + bx * g.h - eps, y0 = g.y0 + by * g.h - eps;
   const double x1 = g.x0 + (bx + 1) * g.h + eps, y1 = g.y0 + (by + 1) * g.h + eps;
-  int n = 4, nredo = 0;
-  bool fail = !L.init(x0 - yx, y0 - yy, x1 - yx, y1 - yy, kInf);
-  const int32_t q1 = cand_start[b + 1];
-  for (int32_t q = cand_start[b]; q < q1 && n > 0 && !fail; q++) {
-    const int32_t k = cand[q];
-    if (k == j) continue;
-    const double Yx = pos[2 * k] - yx, Yy = pos[2 * k + 1] - yy;
-    const double d2 = Yx * Yx + Yy * Yy;
-    const double dw = wdiff(wlo, wj, j, w[k], k);  // w_j - w_k
-    if (d2 == 0.0) {
-      if (dw < 0.0 || (dw == 0.0 && perm[k] < perm[j])) n = 0;
-      continue;
-    }
-    HalfPlane<double> H;
-    H.Yx64 = H.Yx = Yx;
-    H.Yy64 = H.Yy = Yy;
-    H.kk64 = H.kk = d2 + dw;
-    H.label = k;
-    n = clip_lds(L, n, H, fail, nredo);
-  }
-  keep[i] = (n > 0 || fail) ? 1 : 0;
+  bool fail = !C.init(x0 - yx, y0 - yy, x1 - yx, y1 - yy, kInf);
+  const int32_t q0 = a.cand_start[b];
+  const int cnt = a.cand_start[b + 1] - q0;
+  clip_ranges<double, false>(a, j, yx, yy, a.w[j], q0, C.l == 0 ? cnt : 0, a.cand, C, fail);
+  if (C.l == 0) keep[i] = (C.n > 0 || fail) ? 1 : 0;
 }
 
 ma_status refine_candidates(ma_engine *e, int64_t total) {
   EvalBuffers &B = e->eb;
-  hipLaunchKernelGGL(k_cand_refine, dim3(nblocks(total, kCellBlock)), dim3(kCellBlock), 0,
-                     e->stream, e->grid, e->pos.p, B.w_s.p, B.wlo(), e->perm.p, B.cand_cnt.p,
-                     B.cand.p, B.cbin.p, total, B.ckeep.p);
+  CellArgs a{};
+  a.g = e->grid;
+  a.pos = e->pos.p;
+  a.w = B.w_s.p;
+  a.wlo = B.wlo();
+  a.perm = e->perm.p;
+  a.cand_start = B.cand_cnt.p;
+  a.cand = B.cand.p;
+  hipLaunchKernelGGL(k_cand_refine, dim3(nblocks(total, kCellGroups)), dim3(kCellThreads), 0,
+                     e->stream, a, B.cbin.p, total, B.ckeep.p);
   const int32_t zero = 0;
   MA_HIP_TRY(hipMemcpyAsync(B.ckeep.p + total, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
                             e->stream));
@@ -775,7 +968,8 @@ ma_status refine_candidates(ma_engine *e, int64_t total) {
 // together (coalesced): slot s belongs to the last cell whose offset is <= s
 // (binary search over the 64 offsets in LDS) and takes that cell's kept
 // triangle.  Cells with more than kPadTri candidates were not kept by the
-// cell kernel; their own lane scans the triangle bins again.
+// cell kernel; the wave's four groups scan the triangle bins of four such
+// cells at a time again.
 __global__ void __launch_bounds__(64) k_pairs(CellArgs a, const int32_t *poff, int32_t *pair_cell,
                                               int32_t *pair_tri) {
   __shared__ int32_t soff[65];
@@ -790,15 +984,19 @@ __global__ void __launch_bounds__(64) k_pairs(CellArgs a, const int32_t *poff, i
   if (lane == 0) soff[64] = poff[k0 + nk];
   skeep[lane] = cnt <= kPadTri;
   __syncthreads();
-  if (cnt > kPadTri) {
-    int32_t o = soff[lane];
-    for_each_triangle(a.g, a.tbin_start, a.tbin_items, a.tbox, a.bbox[4 * k], a.bbox[4 * k + 1],
-                      a.bbox[4 * k + 2], a.bbox[4 * k + 3], 0, 0, a.g.G - 1, a.g.G - 1,
-                      [&](int32_t ti) {
-                        pair_cell[o] = (int32_t)k;
-                        pair_tri[o] = ti;
-                        o++;
-                      });
+  const unsigned long long many = __ballot(cnt > kPadTri);
+  for (unsigned long long m = many; m; m &= m - 1, m &= m - 1, m &= m - 1, m &= m - 1) {
+    unsigned long long mine = m;  // this group's cell: the (lane / 16)-th of the next four
+    for (int i = 0; i < lane >> 4; i++) mine &= mine - 1;
+    if (!mine) continue;
+    const int c = __ffsll((long long)mine) - 1;
+    const double *bb = a.bbox + 4 * (k0 + c);
+    const int32_t o = soff[c];
+    group_triangles(a, lane & 48, lane & (kGroup - 1), bb[0], bb[1], bb[2], bb[3],
+                    [&](int32_t ti, int i) {
+                      pair_cell[o + i] = (int32_t)(k0 + c);
+                      pair_tri[o + i] = ti;
+                    });
   }
   const int32_t lo = soff[0], hi = soff[64];
   for (int32_t slot = lo + lane; slot < hi; slot += 64) {
@@ -809,7 +1007,7 @@ __global__ void __launch_bounds__(64) k_pairs(CellArgs a, const int32_t *poff, i
     if (!skeep[j]) continue;
     const int c = slot - soff[j];
     pair_cell[slot] = (int32_t)(k0 + j);
-    pair_tri[slot] = a.ptri[c * N + k0 + j];
+    pair_tri[slot] = a.ptri[(k0 + j) * kPadTri + c];
   }
 }
 
@@ -939,9 +1137,9 @@ struct Integrator {
     return area > Tol<R>::area * ((xhi - xlo) + (yhi - ylo)) * cmax;
   }
   R *eacc;
-  int64_t N, k;
+  int64_t k;
   __device__ void commit(int lab, R r) {
-    atomicAdd(&eacc[lab * N + k], r);
+    atomicAdd(&eacc[k * kMaxFast + lab], r);
   }
   __device__ void edge(const SV<R> &a, const SV<R> &b) {
     if (MODE != 0 || a.lab < 0) return;
@@ -1084,7 +1282,6 @@ __device__ inline void frag_setup(const CellArgs &a, int64_t k, const TriData &t
   I.xhi = I.yhi = R(-kInf);
   I.cmax = R(0);
   I.eacc = CellBuf<R>::eacc(a);
-  I.N = a.n;
   I.k = k;
   if (MODE == 2) {
     // barycentric coordinates of the triangle in coordinates local to the Dirac
@@ -1106,10 +1303,10 @@ struct PolyGlobal {
   const CellArgs &a;
   int64_t k;
   __device__ void operator()(int v, SV<R> &c) const {
-    const int64_t N = a.n;
-    c.x = CellBuf<R>::px(a)[v * N + k];
-    c.y = CellBuf<R>::py(a)[v * N + k];
-    c.lab = (a.plab[v * N + k] >= 0) ? v : -1;
+    const int64_t at = k * kMaxFast + v;
+    c.x = CellBuf<R>::px(a)[at];
+    c.y = CellBuf<R>::py(a)[at];
+    c.lab = (a.plab[at] >= 0) ? v : -1;
   }
 };
 
@@ -1385,10 +1582,11 @@ __global__ void __launch_bounds__(kRowBlock) k_rows(CellArgs a, double *fval_par
     int nr = 0;
     double diag = 0.0;
     for (int v = 0; v < n; v++) {
-      const int32_t j = a.plab[v * N + k];
-      if (j < 0 || is_neg_zero(eacc[v * N + k])) continue;  // edge met by no fragment
+      const int32_t j = a.plab[k * kMaxFast + v];
+      const R ei = eacc[k * kMaxFast + v];
+      if (j < 0 || is_neg_zero(ei)) continue;  // edge met by no fragment
       const double dx = yx - a.pos[2 * j], dy = yy - a.pos[2 * j + 1];
-      const double val = (double)eacc[v * N + k] / (2.0 * sqrt(dx * dx + dy * dy));
+      const double val = (double)ei / (2.0 * sqrt(dx * dx + dy * dy));
       diag += val;
       int p = 0;
       while (p < nr && cols(p) < j) p++;
@@ -1589,10 +1787,10 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   for (int l = 0; l <= e->grid.L; l++) po.o[l] = e->pyr_off[l];
   MA_HIP_TRY(hipEventRecord(e->ev[10], e->stream));
   if (fp32)
-    hipLaunchKernelGGL(k_cell_local<float>, dim3(nblocks(n, kCellBlock)), dim3(kCellBlock), 0,
+    hipLaunchKernelGGL(k_cell_local<float>, dim3(nblocks(n, kCellGroups)), dim3(kCellThreads), 0,
                        e->stream, a, B.pyr.p, B.pyr3.p, po, e->local_rings);
   else
-    hipLaunchKernelGGL(k_cell_local<double>, dim3(nblocks(n, kCellBlock)), dim3(kCellBlock), 0,
+    hipLaunchKernelGGL(k_cell_local<double>, dim3(nblocks(n, kCellGroups)), dim3(kCellThreads), 0,
                        e->stream, a, B.pyr.p, B.pyr3.p, po, e->local_rings);
   MA_HIP_TRY(hipEventRecord(e->ev[11], e->stream));
   {
@@ -1659,12 +1857,12 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
                                   e->stream));
         hipLaunchKernelGGL(k_collect, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, B.pn.p,
                            -2, B.glist.p, B.glist.p + n);
-        const unsigned nb = (unsigned)((ct0[6] + kCellBlock - 1) / kCellBlock);
+        const unsigned nb = nblocks((int64_t)ct0[6], kCellGroups);
         if (fp32)
-          hipLaunchKernelGGL(k_cell_bins<float>, dim3(nb), dim3(kCellBlock), 0, e->stream, a,
+          hipLaunchKernelGGL(k_cell_bins<float>, dim3(nb), dim3(kCellThreads), 0, e->stream, a,
                              B.glist.p, B.glist.p + n);
         else
-          hipLaunchKernelGGL(k_cell_bins<double>, dim3(nb), dim3(kCellBlock), 0, e->stream, a,
+          hipLaunchKernelGGL(k_cell_bins<double>, dim3(nb), dim3(kCellThreads), 0, e->stream, a,
                              B.glist.p, B.glist.p + n);
       }
       MA_HIP_TRY(hipEventRecord(e->ev[9], e->stream));

@@ -100,6 +100,7 @@ constexpr int kWalkBudget = 512;
 constexpr int kPadTri = 24;
 // Polygon capacity of the register/LDS fast path (vertices per cell).
 constexpr int kMaxFast = 16;
+constexpr int kMaxLevels = 12;  // levels of the bin grid above the bins
 constexpr int kRowBlock = 128;  // threads per block of k_rows (its LDS rows)
 
 // Fragment polygons written out by the first-moment kernels while `count` is
@@ -182,7 +183,7 @@ struct EvalBuffers {
   DBuf<float> pxf, pyf, eaccf;   // FP32 polygons and edge integrals (mixed mode)
   DBuf<int32_t> plab, pn, tcount, poff, pair_cell, pair_tri, glist;
   DBuf<int32_t> cstage;  // the first candidates of every bin, kept by the counting walk
-  DBuf<int32_t> ptri;         // kPadTri candidate triangles per cell, [c * n + k]
+  DBuf<int32_t> ptri;         // kPadTri candidate triangles per cell, [k * kPadTri + c]
   DBuf<int32_t> ovf;          // pairs for k_frag_wide (+ count)
   // cells beyond the general kernel (list + count at [n]) and their long rows
   DBuf<int32_t> hlist, hrow_col;

@@ -721,7 +721,7 @@ static void choose_grid(ma_engine *e, const double *X, int64_t n, int layout) {
   int L = (int)std::lround(std::log(std::max(1.0, (double)n / 1.5)) / per4);
   if (e->have_mesh)
     L = std::max(L, (int)std::lround(std::log(std::max(1.0, (double)e->nt / 16.0)) / per4));
-  L = std::max(0, std::min(L, 12));
+  L = std::max(0, std::min(L, kMaxLevels));
   Grid g;
   g.L = L;
   g.G = 1 << L;

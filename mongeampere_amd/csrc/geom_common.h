@@ -46,11 +46,12 @@ static inline unsigned nblocks(int64_t n, int b = kBlock) { return (unsigned)((n
 // balanced between them); the blocks past the last whole round keep their
 // number.  A bijection of [0, nb).
 constexpr int kXcds = 8, kXcdRun = 16;
+template <int RUN = kXcdRun>
 __device__ inline int64_t xcd_block(int64_t b, int64_t nb) {
-  const int64_t full = nb / (kXcds * kXcdRun) * (kXcds * kXcdRun);
+  const int64_t full = nb / (kXcds * RUN) * (kXcds * RUN);
   if (b >= full) return b;
   const int64_t x = b % kXcds, i = b / kXcds;
-  return ((i / kXcdRun) * kXcds + x) * kXcdRun + i % kXcdRun;
+  return ((i / RUN) * kXcds + x) * RUN + i % RUN;
 }
 
 // w_k - w_j for weights carried in two words (w = hi + lo, |lo| <= ulp(hi) / 2,
@@ -120,38 +121,9 @@ __device__ inline void ac6_points(R ax, R ay, R bx, R by, R cx, R cy, AC6T<R> &q
   q.py[5] = ay + s6 * uy + s6 * vy;
 }
 
-// Enumerates, once each, the triangles whose bounding box meets the box
-// [px0,px1]x[py0,py1] (absolute), scanning the bins of that box clipped to
-// the bin rectangle [rx0,rx1]x[ry0,ry1].  A triangle listed in several bins
-// is visited in the bin holding the lower-left corner of the overlap of the
-// two boxes.
-// tbox: per triangle its bounding box (x0, y0, x1, y1) in FP32, rounded
-// outwards (16 B per test instead of the 72 B triangle record).
-template <class F>
-__device__ inline void for_each_triangle(const Grid &g, const int32_t *__restrict__ tbin_start,
-                                         const int32_t *__restrict__ tbin_items,
-                                         const float4 *__restrict__ tbox, double px0, double py0,
-                                         double px1, double py1, int rx0, int ry0, int rx1,
-                                         int ry1, F f) {
-  const int qx0 = max(bin_coord(px0, g.x0, g.h, g.G), rx0);
-  const int qx1 = min(bin_coord(px1, g.x0, g.h, g.G), rx1);
-  const int qy0 = max(bin_coord(py0, g.y0, g.h, g.G), ry0);
-  const int qy1 = min(bin_coord(py1, g.y0, g.h, g.G), ry1);
-  for (int by = qy0; by <= qy1; by++)
-    for (int bx = qx0; bx <= qx1; bx++) {
-      const int64_t b = morton2((uint32_t)bx, (uint32_t)by);
-      for (int32_t q = tbin_start[b]; q < tbin_start[b + 1]; q++) {
-        const int32_t ti = tbin_items[q];
-        const float4 tb = tbox[ti];
-        const double tx0 = tb.x, ty0 = tb.y, tx1 = tb.z, ty1 = tb.w;
-        if (tx1 < px0 || tx0 > px1 || ty1 < py0 || ty0 > py1) continue;
-        const int ox = max(bin_coord(fmax(tx0, px0), g.x0, g.h, g.G), qx0);
-        const int oy = max(bin_coord(fmax(ty0, py0), g.y0, g.h, g.G), qy0);
-        if (ox != bx || oy != by) continue;
-        f(ti);
-      }
-    }
-}
+// Entries of the triangle bins: the triangle, and whether this bin is in the
+// first column / row of bins its box meets (tbin entries sort by triangle).
+constexpr int kTriShift = 2, kTriFirstX = 1, kTriFirstY = 2;
 
 // Fragment output (FragOut): one record per fragment of positive area.
 // frag_reserve: plain atomics, for kernels whose lanes are not converged.

@@ -236,7 +236,7 @@ hipError_t build_dirac_grid(ma_engine *e, const double *d_X, int layout) {
 // ---------------------------------------------------------------------------
 template <bool FILL>
 // A triangle is listed in every bin its FP32 (outward-rounded) bounding box
-// meets: the same box for_each_triangle uses to visit it once.
+// meets (the box group_triangles tests).
 __global__ void k_tbin(const float4 *tbox, int64_t nt, Grid g, int32_t *cnt_or_cursor,
                        int32_t *items) {
   int64_t f = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -250,7 +250,8 @@ __global__ void k_tbin(const float4 *tbox, int64_t nt, Grid g, int32_t *cnt_or_c
       uint32_t b = morton2((uint32_t)bx, (uint32_t)by);
       if (FILL) {
         int32_t s = atomicAdd(&cnt_or_cursor[b], 1);
-        items[s] = (int32_t)f;
+        items[s] = ((int32_t)f << kTriShift) | (bx == bx0 ? kTriFirstX : 0) |
+                   (by == by0 ? kTriFirstY : 0);
       } else {
         atomicAdd(&cnt_or_cursor[b], 1);
       }
@@ -856,7 +857,7 @@ __global__ void __launch_bounds__(kBlock) k_cells_general(
       for (int bx = qx0; bx <= qx1; bx++) {
         const int64_t b = morton2((uint32_t)bx, (uint32_t)by);
         for (int32_t q = tbin_start[b]; q < tbin_start[b + 1]; q++) {
-          const TriData t = tri[tbin_items[q]];
+          const TriData t = tri[tbin_items[q] >> kTriShift];
           double tx0, ty0, tx1, ty1;
           tri_bbox(t, tx0, ty0, tx1, ty1);
           if (tx1 < px0 || tx0 > px1 || ty1 < py0 || ty0 > py1) continue;
@@ -904,7 +905,7 @@ __global__ void __launch_bounds__(kBlock) k_cells_general(
           double dv[3] = {0.0, 0.0, 0.0};
           frag_integrals<MODE>(Q.x, Q.y, m, t, yx, yy, wk, S, dv);
           if (MODE == 2) {
-            const int64_t ti = tbin_items[q];
+            const int64_t ti = tbin_items[q] >> kTriShift;
 #pragma unroll
             for (int v = 0; v < 3; v++) atomicAdd(&dval[triv[3 * ti + v]], dv[v]);
           }
@@ -1366,7 +1367,7 @@ __global__ void __launch_bounds__(kHugeBlock) k_cell_huge(
       const int bx = qx0 + (int)(ib % wx), by = qy0 + (int)(ib / wx);
       const int64_t b = morton2((uint32_t)bx, (uint32_t)by);
       for (int32_t q = tbin_start[b]; q < tbin_start[b + 1]; q++) {
-        const TriData t = tri[tbin_items[q]];
+        const TriData t = tri[tbin_items[q] >> kTriShift];
         double tx0, ty0, tx1, ty1;
         tri_bbox(t, tx0, ty0, tx1, ty1);
         if (tx1 < bx0 || tx0 > bx1 || ty1 < by0 || ty0 > by1) continue;
@@ -1409,12 +1410,12 @@ __global__ void __launch_bounds__(kHugeBlock) k_cell_huge(
           const int md = frag_distinct(m, eps, gx, gy);
           unsigned long long f, v;
           frag_reserve(fo, md, f, v);
-          frag_write(fo, f, v, md, perm[k], tbin_items[q], yx, yy, m, eps, gx, gy);
+          frag_write(fo, f, v, md, perm[k], tbin_items[q] >> kTriShift, yx, yy, m, eps, gx, gy);
         }
         double dv[3] = {0.0, 0.0, 0.0};
         frag_integrals<MODE>(fx, fy, m, t, yx, yy, wk, S, dv);
         if (MODE == 2) {
-          const int64_t ti = tbin_items[q];
+          const int64_t ti = tbin_items[q] >> kTriShift;
           for (int c = 0; c < 3; c++) atomicAdd(&dval[triv[3 * ti + c]], dv[c]);
         }
         if (MODE == 0) {
