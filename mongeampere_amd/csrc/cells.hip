@@ -26,6 +26,7 @@
 #include <climits>
 
 #include "geom_common.h"
+#include "lanes.h"
 
 namespace ma {
 
@@ -130,74 +131,7 @@ struct CellBuf<float> {
 // annulus in FP64 13.0 and 2.8 ms, 1000 Diracs (too few threads before) 278
 // and 33 us.
 // ---------------------------------------------------------------------------
-constexpr int kGroup = 16;
-constexpr int kCellThreads = 256;                    // threads of the cell kernels
-constexpr int kCellGroups = kCellThreads / kGroup;   // cells per workgroup
-constexpr int kCellXcdRun = 64;                      // workgroups of an XCD's run (1024 cells)
 static_assert(kMaxFast == kGroup, "one polygon vertex per lane");
-
-constexpr int kDppShr = 0x110, kDppRor = 0x120, kDppBcast = 0x150;  // row_shr, row_ror, row_newbcast
-template <int CTRL>
-__device__ inline int dpp(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL>
-__device__ inline float dpp(float v) {
-  return __int_as_float(dpp<CTRL>(__float_as_int(v)));
-}
-template <int CTRL>
-__device__ inline double dpp(double v) {
-  return __hiloint2double(dpp<CTRL>(__double2hiint(v)), dpp<CTRL>(__double2loint(v)));
-}
-template <class T>
-__device__ inline T row_max(T v) {
-  v = fmax(v, dpp<kDppRor + 8>(v));
-  v = fmax(v, dpp<kDppRor + 4>(v));
-  v = fmax(v, dpp<kDppRor + 2>(v));
-  return fmax(v, dpp<kDppRor + 1>(v));
-}
-template <class T>
-__device__ inline T row_min(T v) {
-  return -row_max(-v);
-}
-__device__ inline unsigned row_min(unsigned v) {
-  v = min(v, (unsigned)dpp<kDppRor + 8>((int)v));
-  v = min(v, (unsigned)dpp<kDppRor + 4>((int)v));
-  v = min(v, (unsigned)dpp<kDppRor + 2>((int)v));
-  return min(v, (unsigned)dpp<kDppRor + 1>((int)v));
-}
-// largest of non-negative floats (their bit patterns order like integers)
-__device__ inline float row_max_nonneg(float f) {
-  int v = __float_as_int(f);
-  v = max(v, dpp<kDppRor + 8>(v));
-  v = max(v, dpp<kDppRor + 4>(v));
-  v = max(v, dpp<kDppRor + 2>(v));
-  return __int_as_float(max(v, dpp<kDppRor + 1>(v)));
-}
-__device__ inline int row_sum(int v) {
-  v += dpp<kDppRor + 8>(v);
-  v += dpp<kDppRor + 4>(v);
-  v += dpp<kDppRor + 2>(v);
-  return v + dpp<kDppRor + 1>(v);
-}
-// inclusive prefix sum over the row
-__device__ inline int row_scan(int v) {
-  v += dpp<kDppShr + 1>(v);
-  v += dpp<kDppShr + 2>(v);
-  v += dpp<kDppShr + 4>(v);
-  return v + dpp<kDppShr + 8>(v);
-}
-// values of lane `src` of the row; base4 = 4 x the row's first lane
-__device__ inline int row_get(int v, int base4, int src) {
-  return __builtin_amdgcn_ds_bpermute(base4 + 4 * src, v);
-}
-__device__ inline float row_get(float v, int base4, int src) {
-  return __int_as_float(row_get(__float_as_int(v), base4, src));
-}
-__device__ inline double row_get(double v, int base4, int src) {
-  return __hiloint2double(row_get(__double2hiint(v), base4, src),
-                          row_get(__double2loint(v), base4, src));
-}
 
 // a / b: a reciprocal and one correction (within an ulp), FP64 as the compiler does it
 __device__ inline float ratio(float a, float b) {
@@ -439,24 +373,6 @@ __device__ inline void clip_batch(const CellArgs &a, int64_t k, double yx, doubl
   if (any) C.update_radius();
 }
 
-// Ranges [lo, lo + cnt) of the group's lanes as one stream: f(q, b, valid) is
-// called for 16 consecutive entries at a time, q the entry and b the lane
-// whose range holds it; more() stops the stream.
-template <class F, class M>
-__device__ inline void for_ranges(int base, int l, int32_t lo, int cnt, M &&more, F &&f) {
-  const int inc = row_scan(cnt);
-  const int ex = inc - cnt, tot = dpp<kDppBcast + 15>(inc);
-  for (int s0 = 0; s0 < tot && more(); s0 += kGroup) {
-    const int s = s0 + l;
-    int b = 0;  // the last lane whose range starts at or before s
-#pragma unroll
-    for (int step = 8; step > 0; step >>= 1)
-      if (row_get(ex, 4 * base, b + step) <= s) b += step;
-    const int32_t q = row_get(lo - ex, 4 * base, b) + s;
-    f(q, b, s < tot);
-  }
-}
-
 // Clips by the Diracs of the lanes' ranges (of `list`, or Diracs themselves).
 template <class T, bool SEEN, class R>
 __device__ inline void clip_ranges(const CellArgs &a, int64_t k, double yx, double yy, double wk,
@@ -673,7 +589,6 @@ __device__ inline void wave_count(T *dst, bool flag) {
 // own maximum weight and clips by the Diracs of the nodes it keeps.  Pruning
 // uses the polygon radius at the time of the test, which only shrinks, so
 // every pruned Dirac stays unable to cut the final cell.
-constexpr int kWalkStack = 64;  // pending nodes of a walk; a fuller one goes to the bin path
 template <class R>
 __global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const double *pyr,
                                                              const double *pyr3, PyrOff off,
@@ -793,10 +708,6 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const d
         }
       }
       const unsigned dm = C.mask(descend);
-      if (sp + __popc(dm) > kWalkStack) {
-        over_budget = true;
-        break;
-      }
       if (descend) stack[sp + __popc(dm & ((1u << l) - 1u))] = ((uint32_t)cl << 27) | ch;
       sp += __popc(dm);
       clip_ranges<float, true>(a, k, yx, yy, wk, lo, cnt, nullptr, C, fail);
@@ -1682,14 +1593,27 @@ ma_status run_bin_candidates(ma_engine *e, const int32_t *pn, const unsigned cha
 // kernel left to other kernels (pn < 0): the starting box of that kernel
 // (at most kBoxWide) and one more ring.
 constexpr int kMaskBins = (int)kBoxWide + 1;
+// One thread per Dirac finds such cells; the wave's 64 lanes mark the square of
+// one of them at a time (2000 cells of 2M: 167 us when each thread marked its
+// own 35 x 35 bins).
 __global__ void k_mark_bins(Grid g, int64_t n, const double *pos, const int32_t *pn,
                             unsigned char *mask) {
   const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k >= n || pn[k] >= 0) return;
-  const int bx = bin_coord(pos[2 * k], g.x0, g.h, g.G), by = bin_coord(pos[2 * k + 1], g.y0, g.h, g.G);
-  for (int y = max(by - kMaskBins, 0); y <= min(by + kMaskBins, g.G - 1); y++)
-    for (int x = max(bx - kMaskBins, 0); x <= min(bx + kMaskBins, g.G - 1); x++)
-      mask[morton2((uint32_t)x, (uint32_t)y)] = 1;
+  const bool marks = k < n && pn[k] < 0;
+  int bx = 0, by = 0;
+  if (marks) {
+    bx = bin_coord(pos[2 * k], g.x0, g.h, g.G);
+    by = bin_coord(pos[2 * k + 1], g.y0, g.h, g.G);
+  }
+  constexpr int kSide = 2 * kMaskBins + 1;
+  for (unsigned long long m = __ballot(marks); m; m &= m - 1) {
+    const int c = __ffsll((long long)m) - 1;
+    const int cx = __shfl(bx, c, 64) - kMaskBins, cy = __shfl(by, c, 64) - kMaskBins;
+    for (int t = (int)(threadIdx.x & 63); t < kSide * kSide; t += 64) {
+      const int x = cx + t % kSide, y = cy + t / kSide;
+      if (x >= 0 && x < g.G && y >= 0 && y < g.G) mask[morton2((uint32_t)x, (uint32_t)y)] = 1;
+    }
+  }
 }
 // *out = 1 if the bin rectangle of a cell with pn < 0 reaches the outer ring
 // of its own square of marked bins (its cell may extend past the bins whose

@@ -150,7 +150,8 @@ struct EvalBuffers {
   DBuf<int32_t> cbin;        // bin of each candidate entry (before refinement)
   DBuf<int32_t> ckeep;       // keep flags of the entries, then their prefix sums
   DBuf<int32_t> cand2, cstart2;  // refined lists (swapped with cand / cand_cnt)
-  DBuf<double> ubin;         // per bin: min over Diracs of the max power over the bin
+  DBuf<double> plane;        // plane pyramid (4 per node) and its sums, built with the lists
+  DBuf<double> node_sums;
   DBuf<int32_t> owner;       // per bin, best competitor of the last evaluation
   DBuf<int32_t> rect;        // per Dirac: bin rectangle (x0, y0, x1, y1)
   DBuf<double> mass_s, intg_s, fval_part;
@@ -165,7 +166,7 @@ struct EvalBuffers {
   DBuf<int32_t> csr_ptr, csr_col;   // Morton-order CSR
   DBuf<double> csr_val;
   DBuf<double> diag;
-  DBuf<int32_t> flags;       // [0] overflow poly, [1] candidate walk stack overflow,
+  DBuf<int32_t> flags;       // [0] overflow poly,
                              // [3] cells for the general kernels
   DBuf<unsigned long long> counters;  // [0] fragments, [1] candidates, [2] max poly, [3] empty,
                                       // [4] vertices, [5] FP64 re-decisions, [6] bin-path cells,

@@ -14,6 +14,7 @@
 #include <cmath>
 
 #include "geom_common.h"
+#include "lanes.h"
 
 namespace ma {
 
@@ -317,194 +318,321 @@ __global__ void k_pyr_up(const double *lo, double *hi, int64_t nhi) {
 }
 
 // ---------------------------------------------------------------------------
-// Candidate owners of a bin.  A Dirac j can own a point of bin b only if
-//   min_{x in b} pi_j(x) <= U_b := max_{x in b} pi_k(x)   for any competitor k,
-// and only if pi_j - pi_k (affine) is <= 0 at some corner of b.  The search
-// is a depth-first traversal of the max-weight pyramid, nearest nodes first,
-// pruning nodes whose lower bound dist^2(node, b) - max w exceeds U_b; the
-// competitor k is the Dirac with the smallest max over the bin's corners
-// seen so far (warm-started from the previous evaluation).
+// Plane pyramid.  With coordinates about the grid's centre and v_j = |y_j|^2 -
+// w_j, pi_j(x) = |x|^2 + v_j - 2 x.y_j.  A node keeps a gradient a and b = min
+// over its Diracs of v_j - a.y_j (a lower bound of it above level 0), so that
+//   min_j v_j - 2 x.y_j >= b + min over the node's box of (a - 2 x).y.
+// Where the weights vary smoothly a is close to 2 x for the points x that the
+// node's Diracs own, and the bound is tight to the square of the node's side.
+// (The bound of the max-weight pyramid, dist^2(x, node) - max w, is loose by
+// four times the distance from a Dirac to its cell times the node's side:
+// with clustered Diracs a search for the owners of one bin then met about 500
+// Diracs instead of 10.)
+// a = 2 (centre of the node) - gw, gw the gradient of the weights by least
+// squares over the 16 grandchildren of the node's even-level ancestor.
 // ---------------------------------------------------------------------------
-struct BinGeom {
+struct Plane {
+  double ax, ay, b, pad;
+};
+// Diracs of an even-level node: number, sums of y and w.
+struct NodeSums {
+  double n, x, y, w;
+};
+struct NodeBox {
   double x0, y0, x1, y1;
 };
-__device__ inline double pi_max_corners(const BinGeom &B, double yx, double yy, double w) {
-  double ax = fmax(fabs(B.x0 - yx), fabs(B.x1 - yx));
-  double ay = fmax(fabs(B.y0 - yy), fabs(B.y1 - yy));
-  return ax * ax + ay * ay - w;
+__device__ inline NodeBox node_box(const Grid &g, uint32_t m, int lev) {
+  const double side = g.h * (double)(1u << lev), half = 0.5 * g.h * (double)g.G;
+  NodeBox q;
+  q.x0 = compact1by1(m) * side - half;
+  q.y0 = compact1by1(m >> 1) * side - half;
+  q.x1 = q.x0 + side;
+  q.y1 = q.y0 + side;
+  return q;
 }
-__device__ inline double pi_min_rect(const BinGeom &B, double yx, double yy, double w) {
-  double dx = fmax(fmax(B.x0 - yx, yx - B.x1), 0.0);
-  double dy = fmax(fmax(B.y0 - yy, yy - B.y1), 0.0);
-  return dx * dx + dy * dy - w;
+// min of t.y over the box; mag gets the magnitude of its terms
+__device__ inline double box_min(const NodeBox &q, double tx, double ty, double &mag) {
+  const double px = tx > 0.0 ? q.x0 : q.x1, py = ty > 0.0 ? q.y0 : q.y1;
+  mag = fabs(tx * px) + fabs(ty * py);
+  return tx * px + ty * py;
 }
-// true if pi_j - pi_k can be <= 0 somewhere in the bin (min over corners)
-__device__ inline bool may_beat(const BinGeom &B, double jx, double jy, double wj, double kx,
-                                double ky, double wk) {
-  const double cx[4] = {B.x0, B.x1, B.x0, B.x1};
-  const double cy[4] = {B.y0, B.y0, B.y1, B.y1};
+// rounding allowance of a bound: its terms carry errors of a few 1e-16
+constexpr double kPlaneEps = 1e-13;
+// lower bound of v_j - 2 x.y_j over the node's Diracs, rounding allowed for
+__device__ inline double plane_bound(const Plane &p, const NodeBox &q, double x, double y) {
+  double mag;
+  const double m = box_min(q, p.ax - 2.0 * x, p.ay - 2.0 * y, mag);
+  return p.b + m - kPlaneEps * (fabs(p.b) + mag);
+}
+__device__ inline double row_sum(double v) {
+  v += dpp<kDppRor + 8>(v);
+  v += dpp<kDppRor + 4>(v);
+  v += dpp<kDppRor + 2>(v);
+  return v + dpp<kDppRor + 1>(v);
+}
+
+// One group per node of level lev + 2 (lev + 1 when that is the top: step 1);
+// lane c takes its descendant c of level lev.  lev = 0: from the Diracs of the
+// bins; above: from the records of level lev.
+__global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int step,
+                                                        const int32_t *__restrict__ bin_start,
+                                                        const double *__restrict__ pos,
+                                                        const double *__restrict__ w, PyrOff off,
+                                                        Plane *pl, NodeSums *sums) {
+  const int top = lev + step;
+  const int64_t node = blockIdx.x * (int64_t)kCellGroups + threadIdx.x / kGroup;
+  if (node >= (int64_t)1 << (2 * (g.L - top))) return;
+  const int l = (int)threadIdx.x & (kGroup - 1), base4 = 4 * ((int)threadIdx.x & 48);
+  const bool on = l < (1 << (2 * step));
+  const uint32_t m = ((uint32_t)node << (2 * step)) | (uint32_t)(on ? l : 0);
+  const double hx = g.x0 + 0.5 * g.h * g.G, hy = g.y0 + 0.5 * g.h * g.G;
+  NodeSums s{0.0, 0.0, 0.0, 0.0};
+  int32_t q0 = 0, q1 = 0;
+  if (on && lev == 0) {
+    q0 = bin_start[m];
+    q1 = bin_start[m + 1];
+    for (int32_t q = q0; q < q1; q++) {
+      s.x += pos[2 * q] - hx;
+      s.y += pos[2 * q + 1] - hy;
+      s.w += w[q];
+    }
+    s.n = (double)(q1 - q0);
+  } else if (on) {
+    s = sums[off.o[lev] + m];
+  }
+  // gradient of the weights: least squares over the lanes' means
+  const double N = row_sum(s.n), Sx = row_sum(s.x), Sy = row_sum(s.y), Sw = row_sum(s.w);
+  double gx = 0.0, gy = 0.0;
+  {
+    const double in = N > 0.0 ? 1.0 / N : 0.0, im = s.n > 0.0 ? 1.0 / s.n : 0.0;
+    const double dx = s.x * im - Sx * in, dy = s.y * im - Sy * in, dw = s.w * im - Sw * in;
+    const double xx = row_sum(s.n * dx * dx), xy = row_sum(s.n * dx * dy);
+    const double yy = row_sum(s.n * dy * dy);
+    const double xw = row_sum(s.n * dx * dw), yw = row_sum(s.n * dy * dw);
+    const double det = xx * yy - xy * xy;
+    if (det > 1e-6 * xx * yy) {  // else (Diracs on a line, or one): constant weights
+      gx = (xw * yy - yw * xy) / det;
+      gy = (yw * xx - xw * xy) / det;
+    }
+  }
+  auto gradient = [&](const NodeBox &q, Plane &p) {
+    p.ax = (q.x0 + q.x1) - gx;
+    p.ay = (q.y0 + q.y1) - gy;
+    p.pad = 0.0;
+  };
+  Plane p{0.0, 0.0, kInf, 0.0};
+  NodeBox q = node_box(g, m, lev);
+  if (lev == 0) {
+    gradient(q, p);
+    for (int32_t i = q0; i < q1; i++) {
+      const double x = pos[2 * i] - hx, y = pos[2 * i + 1] - hy;
+      const double v = x * x + y * y - w[i], d = p.ax * x + p.ay * y;
+      p.b = fmin(p.b, v - d - kPlaneEps * (x * x + y * y + fabs(w[i]) + fabs(p.ax * x) +
+                                           fabs(p.ay * y)));
+    }
+    if (on) pl[off.o[0] + m] = p;
+  } else if (on) {
+    p = pl[off.o[lev] + m];
+  }
+  // one and two levels up: the children's bounds moved to the parent's gradient
+  uint32_t mm = m;
+  for (int k = 1; k <= step; k++) {
+    mm >>= 2;
+    Plane u{0.0, 0.0, kInf, 0.0};
+    const NodeBox up = node_box(g, mm, lev + k);
+    gradient(up, u);
+    double t = kInf;
+    if (on && p.b < kInf) {
+      double mag;
+      const double d = box_min(q, p.ax - u.ax, p.ay - u.ay, mag);
+      t = p.b + d - kPlaneEps * (fabs(p.b) + mag);
+    }
+    const int st = k == 1 ? 1 : 4;  // lanes of the children: l, l ^ st, ...
+    t = fmin(t, row_get(t, base4, l ^ st));
+    t = fmin(t, row_get(t, base4, l ^ (2 * st)));
+    u.b = t;
+    if (on && (l & (4 * st - 1)) == 0) pl[off.o[lev + k] + mm] = u;
+    p = u;
+    q = up;
+  }
+  if (l == 0) sums[off.o[top] + node] = NodeSums{N, Sx, Sy, Sw};
+}
+
+// true if pi_j - pi_k (affine) can be <= 0 somewhere in the bin (min over
+// corners); corners in absolute coordinates
+__device__ inline bool may_beat(double x0, double y0, double h, double jx, double jy, double wj,
+                                double kx, double ky, double wk) {
   bool ok = false;
 #pragma unroll
   for (int c = 0; c < 4; c++) {
-    double dj = (cx[c] - jx) * (cx[c] - jx) + (cy[c] - jy) * (cy[c] - jy) - wj;
-    double dk = (cx[c] - kx) * (cx[c] - kx) + (cy[c] - ky) * (cy[c] - ky) - wk;
+    const double cx = x0 + (c & 1 ? h : 0.0), cy = y0 + (c & 2 ? h : 0.0);
+    const double dj = (cx - jx) * (cx - jx) + (cy - jy) * (cy - jy) - wj;
+    const double dk = (cx - kx) * (cx - kx) + (cy - ky) * (cy - ky) - wk;
     ok |= (dj - dk) <= 1e-12 * (fabs(dj) + fabs(dk));
   }
   return ok;
 }
-__device__ inline bool above(double lo, double U) {
-  return lo > U + 1e-12 * (fabs(lo) + fabs(U));
-}
 
-// Depth-first walk of the max-weight pyramid for bin B, nearest nodes
-// first, pruning nodes whose lower bound dist^2(node, B) - max w exceeds U
-// (U may decrease while walking); visit(q) is called for every Dirac of the
-// surviving leaves.  Returns false if the fixed-size stack overflowed.
-template <class Visit>
-__device__ inline bool pyr_walk(const Grid &g, const int32_t *bin_start, const double *pyr,
-                                const PyrOff &off, const BinGeom &B, const double &U,
+// Depth-first walk of the plane pyramid by the 16 lanes of a group: the
+// grandchildren of a node are tested at once (keep(plane, box)), nodes of few
+// Diracs are taken whole, and visit(q, valid) gets 16 Diracs at a time.
+constexpr int kWalkTake = 16;
+template <class Keep, class Visit>
+__device__ inline void row_walk(const Grid &g, const int32_t *bin_start, const Plane *pl,
+                                const PyrOff &off, uint32_t *stack, int base, int l, Keep &&keep,
                                 Visit &&visit) {
-  uint32_t stack[64];
   int sp = 0;
-  bool ok = true;
-  stack[sp++] = ((uint32_t)g.L << 27);
-  while (sp > 0) {
-    const uint32_t ent = stack[--sp];
-    const int l = (int)(ent >> 27);
-    const uint32_t m = ent & ((1u << 27) - 1u);
-    if (l == 0) {
-      for (int32_t q = bin_start[m]; q < bin_start[m + 1]; q++) visit(q);
-      continue;
-    }
-    const int cl = l - 1;
-    const uint32_t c0 = m << 2;
-    const double side = g.h * (double)(1u << cl);
-    double lo4[4];
-    uint32_t id4[4];
-    int k4 = 0;
-    for (int c = 0; c < 4; c++) {
-      const uint32_t ch = c0 + (uint32_t)c;
-      const double W = pyr[off.o[cl] + ch];
-      if (W == -kInf) continue;
-      const double nx0 = g.x0 + compact1by1(ch) * side, ny0 = g.y0 + compact1by1(ch >> 1) * side;
-      const double dx = fmax(fmax(nx0 - B.x1, B.x0 - (nx0 + side)), 0.0);
-      const double dy = fmax(fmax(ny0 - B.y1, B.y0 - (ny0 + side)), 0.0);
-      const double lo = dx * dx + dy * dy - W;
-      if (above(lo, U)) continue;
-      int p = k4++;
-      while (p > 0 && lo4[p - 1] < lo) {  // keep descending order: nearest popped first
-        lo4[p] = lo4[p - 1];
-        id4[p] = id4[p - 1];
-        p--;
+  uint32_t ent = (uint32_t)g.L << 27;
+  while (true) {
+    const int lev = (int)(ent >> 27), st = min(lev, 2), cl = lev - st;
+    const uint32_t ch = ((ent & ((1u << 27) - 1u)) << (2 * st)) | (uint32_t)l;
+    bool descend = false;
+    int32_t lo = 0;
+    int cnt = 0;
+    if (l < (1 << (2 * st))) {
+      const Plane p = pl[off.o[cl] + ch];
+      if (p.b < kInf && keep(p, node_box(g, ch, cl))) {
+        lo = bin_start[(int64_t)ch << (2 * cl)];
+        cnt = bin_start[((int64_t)ch + 1) << (2 * cl)] - lo;
+        if (cl > 0 && cnt > kWalkTake) {
+          descend = true;
+          cnt = 0;
+        }
       }
-      lo4[p] = lo;
-      id4[p] = ch;
     }
-    for (int c = 0; c < k4; c++) {
-      if (sp < 64)
-        stack[sp++] = ((uint32_t)cl << 27) | id4[c];
-      else
-        ok = false;
-    }
+    const unsigned dm = (unsigned)(__ballot(descend) >> base) & 0xffffu;
+    if (descend) stack[sp + __popc(dm & ((1u << l) - 1u))] = ((uint32_t)cl << 27) | ch;
+    sp += __popc(dm);
+    for_ranges(base, l, lo, cnt, []() { return true; },
+               [&](int32_t q, int, bool valid) { visit(q, valid); });
+    if (sp == 0) break;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the lanes' stack entries
+    ent = stack[--sp];
   }
-  return ok;
 }
 
-__device__ inline BinGeom bin_geom(const Grid &g, int64_t b) {
-  const uint32_t bx = compact1by1((uint32_t)b), by = compact1by1((uint32_t)(b >> 1));
-  BinGeom B;
-  B.x0 = g.x0 + bx * g.h;
-  B.y0 = g.y0 + by * g.h;
-  B.x1 = B.x0 + g.h;
-  B.y1 = B.y0 + g.h;
-  return B;
-}
-
-// Candidate owners of a bin, in three passes.  A Dirac j can own a point of
-// bin b only if min_{x in b} pi_j(x) <= U_b := min_k max_{x in b} pi_k(x),
-// and only if pi_j - pi_k (affine) is <= 0 at some corner of b for the
-// minimiser k ("owner").  Pass 1 finds U_b and the owner (warm-started from
-// the previous evaluation's owner); passes 2 and 3 count and then write the
-// Diracs passing both tests, into exactly sized CSR lists.
-__global__ void __launch_bounds__(kBlock) k_cand_owner(
-    Grid g, const int32_t *__restrict__ tbin_start, const int32_t *__restrict__ bin_start,
-    const double *__restrict__ pos, const double *__restrict__ w, const double *__restrict__ pyr,
-    PyrOff off, int32_t *owner, double *ubin, int32_t *flags,
-    const unsigned char *__restrict__ mask) {
-  const int64_t b = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (b >= g.nbins) return;
-  if (tbin_start[b + 1] == tbin_start[b] || (mask && !mask[b])) {
-    ubin[b] = -kInf;  // no triangle (or not needed): no candidates
-    return;
-  }
-  const BinGeom B = bin_geom(g, b);
-  int best = owner[b];
-  double U = kInf;
-  if (best >= 0) U = pi_max_corners(B, pos[2 * best], pos[2 * best + 1], w[best]);
-  const bool ok = pyr_walk(g, bin_start, pyr, off, B, U, [&](int32_t q) {
-    const double h = pi_max_corners(B, pos[2 * q], pos[2 * q + 1], w[q]);
-    if (h < U) {
-      U = h;
-      best = q;
-    }
-  });
-  owner[b] = best;
-  ubin[b] = U;
-  if (!ok) atomicOr(&flags[1], 1);
-}
-
-// The counting pass also keeps the first kCandStage candidates of each bin
+// Candidate owners of a bin: with k the owner of the bin's centre, the Diracs
+// j with pi_j <= pi_k at some corner (pi_j - pi_k is affine, so no other Dirac
+// owns a point of the bin).  Counting pass, 16 lanes per bin: a first walk
+// finds k (starting from the previous evaluation's, or from a greedy descent),
+// a second one counts the candidates and keeps the first kCandStage of them
 // (stage[b * kCandStage + i], 512 B per bin, allocated only when lists are
-// built); the filling pass copies those and walks again only for the bins
-// with more (48 left C2's converged cells a third slower).
+// built).  Filling pass, into exactly sized CSR lists: copies those, and walks
+// again only for the bins with more (48 kept candidates left C2's converged
+// cells a third slower).  VALU work of the node tests bounds it.  200k
+// clustered Diracs, 512 x 512 bins: 16.5 ms with one thread per bin walking the
+// max-weight pyramid, 3.1 ms with a group per bin on that pyramid, 0.93 ms
+// with the planes (their five launches take 0.03 ms).
 constexpr int kCandStage = 128;
 template <bool FILL>
-__global__ void __launch_bounds__(kBlock) k_cand_list(
-    Grid g, const int32_t *__restrict__ bin_start, const double *__restrict__ pos,
-    const double *__restrict__ w, const double *__restrict__ pyr, PyrOff off,
-    const int32_t *__restrict__ owner, const double *__restrict__ ubin, int32_t *cand_start,
-    int32_t *cand, int32_t *cbin, int32_t *stage, int32_t *flags,
-    unsigned long long *counters) {
-  const int64_t b = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(kCellThreads) k_cand_list(
+    Grid g, const int32_t *__restrict__ tbin_start, const int32_t *__restrict__ bin_start,
+    const double *__restrict__ pos, const double *__restrict__ w, const Plane *__restrict__ pl,
+    PyrOff off, int32_t *owner, int32_t *cand_start, int32_t *cand, int32_t *cbin, int32_t *stage,
+    unsigned long long *counters, const unsigned char *__restrict__ mask) {
+  __shared__ uint32_t stacks[kCellGroups][kWalkStack];
+  const int64_t b = xcd_block<kCellXcdRun>(blockIdx.x, gridDim.x) * kCellGroups +
+                    threadIdx.x / kGroup;
   if (b >= g.nbins) return;
+  const int l = (int)threadIdx.x & (kGroup - 1), base = (int)threadIdx.x & 48;
+  uint32_t *stack = stacks[threadIdx.x / kGroup];
   if (FILL) {
     const int32_t o = cand_start[b], c = cand_start[b + 1] - o;
     if (c <= kCandStage) {
-      for (int i = 0; i < c; i++) {
+      for (int i = l; i < c; i += kGroup) {
         cand[o + i] = stage[b * kCandStage + i];
         cbin[o + i] = (int32_t)b;
       }
       return;
     }
-  }
-  const double U = ubin[b];
-  if (U == -kInf) {
-    if (!FILL) cand_start[b] = 0;
+  } else if (tbin_start[b + 1] == tbin_start[b] || (mask && !mask[b])) {
+    if (l == 0) cand_start[b] = 0;  // no triangle (or not needed): no candidates
     return;
   }
-  const BinGeom B = bin_geom(g, b);
-  const int best = owner[b];
-  const double bx = pos[2 * best], by = pos[2 * best + 1], bw = w[best];
-  int cnt = 0;
-  int32_t *out = FILL ? cand + cand_start[b] : nullptr;
-  int32_t *obin = FILL ? cbin + cand_start[b] : nullptr;
-  const bool ok = pyr_walk(g, bin_start, pyr, off, B, U, [&](int32_t q) {
-    const double jx = pos[2 * q], jy = pos[2 * q + 1], wj = w[q];
-    if (q != best && (above(pi_min_rect(B, jx, jy, wj), U) || !may_beat(B, jx, jy, wj, bx, by, bw)))
-      return;
-    if (FILL) {
-      out[cnt] = q;
-      obin[cnt] = (int32_t)b;
-    } else if (cnt < kCandStage) {
-      stage[b * kCandStage + cnt] = q;
-    }
-    cnt++;
-  });
+  const NodeBox B = node_box(g, (uint32_t)b, 0);
+  const double hx = g.x0 + 0.5 * g.h * g.G, hy = g.y0 + 0.5 * g.h * g.G;
+  int best = owner[b];
   if (!FILL) {
+    const double mx = 0.5 * (B.x0 + B.x1), my = 0.5 * (B.y0 + B.y1);
+    // v - 2 x.y of a Dirac at the bin's centre x
+    auto value = [&](int32_t q) {
+      const double x = pos[2 * q] - hx, y = pos[2 * q + 1] - hy;
+      return x * x + y * y - w[q] - 2.0 * (mx * x + my * y);
+    };
+    double U = kInf;
+    auto better = [&](int32_t q, bool valid) {
+      const double h = valid ? value(q) : kInf;
+      const double m = row_min(h);
+      if (m < U) {
+        U = m;
+        best = row_get(q, 4 * base, __ffs((unsigned)(__ballot(h == m) >> base) & 0xffffu) - 1);
+      }
+    };
+    if (best >= 0) {
+      U = value(best);
+    } else {
+      // greedy descent to the bin with the smallest lower bound
+      uint32_t m = 0;
+      for (int lev = g.L; lev > 0;) {
+        const int st = min(lev, 2);
+        lev -= st;
+        const uint32_t ch = (m << (2 * st)) | (uint32_t)l;
+        double v = kInf;
+        if (l < (1 << (2 * st))) {
+          const Plane p = pl[off.o[lev] + ch];
+          if (p.b < kInf) v = plane_bound(p, node_box(g, ch, lev), mx, my);
+        }
+        const unsigned eq = (unsigned)(__ballot(v == row_min(v)) >> base) & 0xffffu;
+        m = (m << (2 * st)) | (uint32_t)(eq ? __ffs(eq) - 1 : 0);
+      }
+      const int32_t q0 = bin_start[m], q1 = bin_start[m + 1];
+      for (int32_t q = q0; q < q1; q += kGroup) better(q + l, q + l < q1);
+    }
+    row_walk(g, bin_start, pl, off, stack, base, l,
+             [&](const Plane &p, const NodeBox &q) { return !(plane_bound(p, q, mx, my) > U); },
+             better);
+    if (l == 0) owner[b] = best;
+  }
+  const double kx = pos[2 * best], ky = pos[2 * best + 1], kw = w[best];
+  // the owner's v - 2 x.y at the corners, rounding allowed for
+  double thr[4];
+  {
+    const double x = kx - hx, y = ky - hy, v = x * x + y * y - kw;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const double cx = c & 1 ? B.x1 : B.x0, cy = c & 2 ? B.y1 : B.y0;
+      thr[c] = v - 2.0 * (cx * x + cy * y) +
+               kPlaneEps * (x * x + y * y + fabs(kw) + 2.0 * (fabs(cx * x) + fabs(cy * y)));
+    }
+  }
+  const double ox = B.x0 + hx, oy = B.y0 + hy;  // the bin's lower corner
+  int cnt = 0;
+  const int32_t o = FILL ? cand_start[b] : 0;
+  row_walk(g, bin_start, pl, off, stack, base, l,
+           [&](const Plane &p, const NodeBox &q) {
+             bool any = false;
+#pragma unroll
+             for (int c = 0; c < 4; c++)
+               any |= !(plane_bound(p, q, c & 1 ? B.x1 : B.x0, c & 2 ? B.y1 : B.y0) > thr[c]);
+             return any;
+           },
+           [&](int32_t q, bool valid) {
+             const bool hit = valid && (q == best || may_beat(ox, oy, g.h, pos[2 * q],
+                                                              pos[2 * q + 1], w[q], kx, ky, kw));
+             const unsigned hm = (unsigned)(__ballot(hit) >> base) & 0xffffu;
+             const int at = cnt + __popc(hm & ((1u << l) - 1u));
+             if (hit && FILL) {
+               cand[o + at] = q;
+               cbin[o + at] = (int32_t)b;
+             } else if (hit && at < kCandStage) {
+               stage[b * kCandStage + at] = q;
+             }
+             cnt += __popc(hm);
+           });
+  if (!FILL && l == 0) {
     cand_start[b] = cnt;
     atomicAdd(&counters[1], (unsigned long long)cnt);
   }
-  if (!ok) atomicOr(&flags[1], 1);
 }
 
 // Compaction of the refined candidate lists: pos is the exclusive prefix sum
@@ -1627,54 +1755,47 @@ ma_status refine_candidates(ma_engine *e, int64_t total);
 
 // Candidate owners of every domain bin (of the bins with mask[b] set, when
 // mask is given) and the bin rectangles of the Diracs marked pn < 0 (see
-// k_cand_owner, k_cand_list, k_rect).
+// k_plane, k_cand_list, k_rect).
 ma_status run_bin_candidates(ma_engine *e, const int32_t *pn, const unsigned char *mask) {
   const Grid &g = e->grid;
   const int64_t n = e->n;
   EvalBuffers &B = e->eb;
   PyrOff po{};
   for (int l = 0; l <= g.L; l++) po.o[l] = e->pyr_off[l];
-  MA_HIP_TRY(B.ubin.ensure((size_t)g.nbins));
-  MA_HIP_TRY(B.cand_cnt.ensure((size_t)g.nbins + 1));
-  MA_HIP_TRY(hipMemsetAsync(B.flags.p + 1, 0, sizeof(int32_t), e->stream));
-  const int32_t zero = 0;
-  int32_t total = 0, fl[4] = {0, 0, 0, 0};
-  // count scan of cand_cnt (nbins entries), total and flags to the host
-  auto scan_counts = [&]() -> ma_status {
-    MA_HIP_TRY(hipMemcpyAsync(B.cand_cnt.p + g.nbins, &zero, sizeof(int32_t),
-                              hipMemcpyHostToDevice, e->stream));
-    MA_HIP_TRY(exclusive_scan(e, B.cand_cnt.p, B.cand_cnt.p, g.nbins + 1));
-    MA_HIP_TRY(hipMemcpyAsync(&total, B.cand_cnt.p + g.nbins, sizeof(int32_t),
-                              hipMemcpyDeviceToHost, e->stream));
-    MA_HIP_TRY(hipMemcpyAsync(fl, B.flags.p, sizeof fl, hipMemcpyDeviceToHost, e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
-    if (fl[1]) {
-      e->err = "candidate search stack overflow";
-      return MA_CAPACITY;
-    }
-    return MA_OK;
-  };
-  // walks of the pyramid per bin: the owner bound, then the counts (keeping
-  // the first kCandStage candidates), then the lists of the bins with more
-  // (one walk that records while the bound is still falling, and filters
-  // afterwards, measured slower: it records far more)
-  hipLaunchKernelGGL(k_cand_owner, dim3(nblocks(g.nbins)), dim3(kBlock), 0, e->stream, g,
-                     e->tbin_start.p, e->bin_start.p, e->pos.p, B.w_s.p, B.pyr.p, po, B.owner.p,
-                     B.ubin.p, B.flags.p, mask);
-  MA_HIP_TRY(B.cstage.ensure((size_t)g.nbins * kCandStage));
-  hipLaunchKernelGGL(k_cand_list<false>, dim3(nblocks(g.nbins)), dim3(kBlock), 0, e->stream, g,
-                     e->bin_start.p, e->pos.p, B.w_s.p, B.pyr.p, po, B.owner.p, B.ubin.p,
-                     B.cand_cnt.p, (int32_t *)nullptr, (int32_t *)nullptr, B.cstage.p, B.flags.p,
-                     B.counters.p);
-  {
-    ma_status st = scan_counts();
-    if (st != MA_OK) return st;
+  const int64_t nodes = e->pyr_off[g.L] + 1;
+  MA_HIP_TRY(B.plane.ensure((size_t)(4 * nodes)));
+  MA_HIP_TRY(B.node_sums.ensure((size_t)(4 * nodes)));
+  Plane *pl = reinterpret_cast<Plane *>(B.plane.p);
+  for (int lev = 0; lev < g.L || lev == 0; lev += 2) {
+    const int step = std::min(2, g.L - lev);
+    hipLaunchKernelGGL(k_plane, dim3(nblocks((int64_t)1 << (2 * (g.L - lev - step)), kCellGroups)),
+                       dim3(kCellThreads), 0, e->stream, g, lev, step, e->bin_start.p, e->pos.p,
+                       B.w_s.p, po, pl, reinterpret_cast<NodeSums *>(B.node_sums.p));
   }
+  MA_HIP_TRY(B.cand_cnt.ensure((size_t)g.nbins + 1));
+  const int32_t zero = 0;
+  int32_t total = 0;
+  // walks of the pyramid per bin: owners and counts (keeping the first
+  // kCandStage candidates), then the lists of the bins with more (one walk
+  // that records while the bound is still falling, and filters afterwards,
+  // measured slower: it records far more)
+  const dim3 grid(nblocks(g.nbins, kCellGroups)), block(kCellThreads);
+  MA_HIP_TRY(B.cstage.ensure((size_t)g.nbins * kCandStage));
+  hipLaunchKernelGGL(k_cand_list<false>, grid, block, 0, e->stream, g, e->tbin_start.p,
+                     e->bin_start.p, e->pos.p, B.w_s.p, pl, po, B.owner.p, B.cand_cnt.p,
+                     (int32_t *)nullptr, (int32_t *)nullptr, B.cstage.p, B.counters.p, mask);
+  // offsets, and the total to the host
+  MA_HIP_TRY(hipMemcpyAsync(B.cand_cnt.p + g.nbins, &zero, sizeof(int32_t),
+                            hipMemcpyHostToDevice, e->stream));
+  MA_HIP_TRY(exclusive_scan(e, B.cand_cnt.p, B.cand_cnt.p, g.nbins + 1));
+  MA_HIP_TRY(hipMemcpyAsync(&total, B.cand_cnt.p + g.nbins, sizeof(int32_t),
+                            hipMemcpyDeviceToHost, e->stream));
+  MA_HIP_TRY(hipStreamSynchronize(e->stream));
   MA_HIP_TRY(B.cand.ensure((size_t)total + 1));
   MA_HIP_TRY(B.cbin.ensure((size_t)total + 1));
-  hipLaunchKernelGGL(k_cand_list<true>, dim3(nblocks(g.nbins)), dim3(kBlock), 0, e->stream, g,
-                     e->bin_start.p, e->pos.p, B.w_s.p, B.pyr.p, po, B.owner.p, B.ubin.p,
-                     B.cand_cnt.p, B.cand.p, B.cbin.p, B.cstage.p, B.flags.p, B.counters.p);
+  hipLaunchKernelGGL(k_cand_list<true>, grid, block, 0, e->stream, g, e->tbin_start.p,
+                     e->bin_start.p, e->pos.p, B.w_s.p, pl, po, B.owner.p, B.cand_cnt.p, B.cand.p,
+                     B.cbin.p, B.cstage.p, B.counters.p, mask);
   if (total > 0 && e->refine) {
     // keep only the exact owners of each bin (refine_candidates), then
     // compact the lists

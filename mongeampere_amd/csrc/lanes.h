@@ -1,0 +1,102 @@
+// Groups of 16 lanes: one DPP row of the wave.  All lanes of a group run the
+// same control flow (conditions come from ballots or row reductions), so a
+// group works together on one cell or one bin; the four groups of a wave are
+// independent.
+#pragma once
+
+#include "geom_common.h"
+
+namespace ma {
+
+constexpr int kGroup = 16;
+constexpr int kCellThreads = 256;                    // threads of the group kernels
+constexpr int kCellGroups = kCellThreads / kGroup;   // groups (cells, bins) per workgroup
+constexpr int kCellXcdRun = 64;                      // workgroups of an XCD's run (1024 cells)
+// Pending nodes of a depth-first pyramid walk that expands a node into its 16
+// grandchildren: 15 stay behind at each of the first kMaxLevels / 2 - 1 steps
+// and 16 come from the next, 91 at most (the last step reaches bins).
+constexpr int kWalkStack = 96;
+static_assert((kMaxLevels / 2 - 1) * 15 + 16 <= kWalkStack, "stack of a pyramid walk");
+
+constexpr int kDppShr = 0x110, kDppRor = 0x120, kDppBcast = 0x150;  // row_shr, row_ror, row_newbcast
+template <int CTRL>
+__device__ inline int dpp(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ inline float dpp(float v) {
+  return __int_as_float(dpp<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ inline double dpp(double v) {
+  return __hiloint2double(dpp<CTRL>(__double2hiint(v)), dpp<CTRL>(__double2loint(v)));
+}
+template <class T>
+__device__ inline T row_max(T v) {
+  v = fmax(v, dpp<kDppRor + 8>(v));
+  v = fmax(v, dpp<kDppRor + 4>(v));
+  v = fmax(v, dpp<kDppRor + 2>(v));
+  return fmax(v, dpp<kDppRor + 1>(v));
+}
+template <class T>
+__device__ inline T row_min(T v) {
+  return -row_max(-v);
+}
+__device__ inline unsigned row_min(unsigned v) {
+  v = min(v, (unsigned)dpp<kDppRor + 8>((int)v));
+  v = min(v, (unsigned)dpp<kDppRor + 4>((int)v));
+  v = min(v, (unsigned)dpp<kDppRor + 2>((int)v));
+  return min(v, (unsigned)dpp<kDppRor + 1>((int)v));
+}
+// largest of non-negative floats (their bit patterns order like integers)
+__device__ inline float row_max_nonneg(float f) {
+  int v = __float_as_int(f);
+  v = max(v, dpp<kDppRor + 8>(v));
+  v = max(v, dpp<kDppRor + 4>(v));
+  v = max(v, dpp<kDppRor + 2>(v));
+  return __int_as_float(max(v, dpp<kDppRor + 1>(v)));
+}
+__device__ inline int row_sum(int v) {
+  v += dpp<kDppRor + 8>(v);
+  v += dpp<kDppRor + 4>(v);
+  v += dpp<kDppRor + 2>(v);
+  return v + dpp<kDppRor + 1>(v);
+}
+// inclusive prefix sum over the row
+__device__ inline int row_scan(int v) {
+  v += dpp<kDppShr + 1>(v);
+  v += dpp<kDppShr + 2>(v);
+  v += dpp<kDppShr + 4>(v);
+  return v + dpp<kDppShr + 8>(v);
+}
+// values of lane `src` of the row; base4 = 4 x the row's first lane
+__device__ inline int row_get(int v, int base4, int src) {
+  return __builtin_amdgcn_ds_bpermute(base4 + 4 * src, v);
+}
+__device__ inline float row_get(float v, int base4, int src) {
+  return __int_as_float(row_get(__float_as_int(v), base4, src));
+}
+__device__ inline double row_get(double v, int base4, int src) {
+  return __hiloint2double(row_get(__double2hiint(v), base4, src),
+                          row_get(__double2loint(v), base4, src));
+}
+
+// Ranges [lo, lo + cnt) of the group's lanes as one stream: f(q, b, valid) is
+// called for 16 consecutive entries at a time, q the entry and b the lane
+// whose range holds it; more() stops the stream.
+template <class F, class M>
+__device__ inline void for_ranges(int base, int l, int32_t lo, int cnt, M &&more, F &&f) {
+  const int inc = row_scan(cnt);
+  const int ex = inc - cnt, tot = dpp<kDppBcast + 15>(inc);
+  for (int s0 = 0; s0 < tot && more(); s0 += kGroup) {
+    const int s = s0 + l;
+    int b = 0;  // the last lane whose range starts at or before s
+#pragma unroll
+    for (int step = 8; step > 0; step >>= 1)
+      if (row_get(ex, 4 * base, b + step) <= s) b += step;
+    const int32_t q = row_get(lo - ex, 4 * base, b) + s;
+    f(q, b, s < tot);
+  }
+}
+
+}  // namespace ma

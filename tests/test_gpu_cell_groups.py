@@ -106,3 +106,44 @@ def test_scales(engine, scale):
     _, g, _ = engine.kantorovich(w * scale ** 2)
     # (the scale is no power of two: positions are rounded once more)
     assert np.abs(g / scale ** 2 - og).max() <= TOL * og.max()
+
+
+@pytest.mark.parametrize("rings", [0, 8])
+@pytest.mark.parametrize("kind", ["warp", "line", "offset", "rough"])
+def test_per_bin_owners(engine, kind, rings):
+    """Cells built from the per-bin owner lists (every cell, with no rings and
+    no walk): far from their Diracs, with Diracs on a line (no gradient to fit
+    to the weights), in a domain far from the origin, and with weights that
+    follow no plane; evaluated twice, from cold and from the last owners."""
+    rng = np.random.default_rng(17)
+    n, shift = 500, 0.0
+    u = rng.uniform(0, 1, (n, 2))
+    X, w = u, np.zeros(n)
+    if kind == "warp":
+        X = u + 0.6 * np.sin(2 * np.pi * u) / (2 * np.pi)
+        psi = X * u - 0.5 * u * u + 0.6 * np.cos(2 * np.pi * u) / (4 * np.pi ** 2)
+        w = (X * X - 2.0 * psi).sum(axis=1)
+    elif kind == "line":
+        X = np.stack([np.full(n, 0.375), u[:, 1]], 1)
+        w = 1e-6 * rng.uniform(-1, 1, n)
+    elif kind == "offset":
+        shift = 64.0
+        w = 1e-4 * rng.uniform(-1, 1, n)
+    else:
+        w = 1e-3 * rng.uniform(-1, 1, n)
+    mesh = _mesh(21)
+    mesh = configs.Mesh(mesh.vxy + shift, mesh.vval, mesh.tri)
+    X = X + shift
+    of, og, oH = oracle.kantorovich(mesh, X, w)
+    engine.set_option("local_rings", rings).set_option("walk_budget", 0 if rings == 0 else 512)
+    try:
+        engine.set_mesh(mesh).set_diracs(X)
+        for _ in range(2):
+            _, g, H = engine.kantorovich(w)
+            # positions about 64 are rounded 64 times coarser
+            assert np.abs(g - og).max() <= TOL * (1 + shift) * og.max()
+            assert abs(H - oH).max() <= TOL * (1 + shift) * abs(oH).max()
+            if rings == 0:
+                assert engine.eval_info()["nbincand"] > 0
+    finally:
+        engine.set_option("local_rings", 8).set_option("walk_budget", 512)
