@@ -9,7 +9,7 @@
 // aggregate map i -> i / kAgg is monotone, a coarse row is the merge of
 // kAgg sorted fine rows.  Cycle: V(1,1) (or V(2,2)) with damped Jacobi
 // (omega, default 0.85), coarse correction scaled by corr (default 1.5:
-// over-correction for piecewise-constant prolongation), dense Cholesky at the
+// over-correction for piecewise-constant prolongation), dense inverse at the
 // coarsest level.  The defaults minimise the linear-solve time of the
 // N = 1M Newton solve over a sweep of omega in [0.6, 1], corr in [1, 2] and
 // both cycles: V(1,1) takes ~55 % more CG iterations than V(2,2) (~440
@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "geom_common.h"
+#include "lanes.h"
 
 namespace ma {
 
@@ -65,11 +66,9 @@ __global__ void k_amg_level0(int64_t n, const int32_t *ptr, const int32_t *col,
 
 // Merge of the kAgg sorted fine rows of coarse row I (columns mapped j/kAgg).
 template <bool FILL, class T>
-__global__ void k_amg_coarse(int64_t nc, int64_t n, const int32_t *ptr, const int32_t *col,
-                             const T *val, int32_t *cnt_or_ptr, int32_t *ccol, T *cval,
-                             T *cdinv) {
-  const int64_t I = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (I >= nc) return;
+__device__ inline void coarse_row(int64_t I, int64_t n, const int32_t *ptr, const int32_t *col,
+                                  const T *val, int32_t *cnt_or_ptr, int32_t *ccol, T *cval,
+                                  T *cdinv) {
   int32_t pos[kAgg], end[kAgg];
 #pragma unroll
   for (int r = 0; r < kAgg; r++) {
@@ -106,32 +105,148 @@ __global__ void k_amg_coarse(int64_t nc, int64_t n, const int32_t *ptr, const in
     cnt_or_ptr[I] = cnt;
 }
 
-// Dense coarsest matrix and its Cholesky factor (one workgroup).
-template <class T>
-__global__ void __launch_bounds__(256) k_amg_dense_chol(int64_t n, const int32_t *ptr,
-                                                        const int32_t *col, const T *val,
-                                                        double *Lf) {
-  for (int64_t q = threadIdx.x; q < n * n; q += blockDim.x) Lf[q] = 0.0;
-  __syncthreads();
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x)
-    for (int32_t q = ptr[i]; q < ptr[i + 1]; q++) Lf[i * n + col[q]] = (double)val[q];
-  __syncthreads();
-  // right-looking Cholesky, lower triangle, row-major
-  for (int64_t k = 0; k < n; k++) {
-    if (threadIdx.x == 0) {
-      const double d = Lf[k * n + k];
-      Lf[k * n + k] = d > 0.0 ? sqrt(d) : 1.0;
-    }
-    __syncthreads();
-    const double lkk = Lf[k * n + k];
-    for (int64_t i = k + 1 + threadIdx.x; i < n; i += blockDim.x) Lf[i * n + k] /= lkk;
-    __syncthreads();
-    for (int64_t q = threadIdx.x; q < (n - k - 1) * (n - k - 1); q += blockDim.x) {
-      const int64_t i = k + 1 + q / (n - k - 1), j = k + 1 + q % (n - k - 1);
-      if (j <= i) Lf[i * n + j] -= Lf[i * n + k] * Lf[j * n + k];
-    }
-    __syncthreads();
+template <bool FILL, class T>
+__global__ void k_amg_coarse(int64_t nc, int64_t n, const int32_t *ptr, const int32_t *col,
+                             const T *val, int32_t *cnt_or_ptr, int32_t *ccol, T *cval,
+                             T *cdinv) {
+  const int64_t I = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (I < nc) coarse_row<FILL, T>(I, n, ptr, col, val, cnt_or_ptr, ccol, cval, cdinv);
+}
+// The same with one wave per coarse row: the kAgg fine rows are consecutive, so
+// lane e takes their e-th entry, sums the entries of its column (in the order
+// of the merge) and, if it is the first of them, writes the column at its rank.
+// A thread's merge is a chain of dependent loads: on levels with few rows it
+// took 35 (count) and 53 us (fill) against 7 and 12 us here; with many rows its
+// fewer instructions win (250k coarse rows: 43 and 73 us, against about 90
+// each), hence kWaveRows.  Rows of more than 64 entries are merged by lane 0.
+constexpr int64_t kWaveRows = 65536;
+template <bool FILL, class T>
+__global__ void __launch_bounds__(kVB2) k_amg_coarse_wave(int64_t nc, int64_t n,
+                                                          const int32_t *ptr, const int32_t *col,
+                                                          const T *val, int32_t *cnt_or_ptr,
+                                                          int32_t *ccol, T *cval, T *cdinv) {
+  const int64_t I = (blockIdx.x * (int64_t)kVB2 + threadIdx.x) >> 6;
+  if (I >= nc) return;
+  const int lane = (int)threadIdx.x & 63;
+  const int32_t p0 = ptr[I * kAgg], p1 = ptr[min(I * kAgg + kAgg, n)];
+  const int tot = __builtin_amdgcn_readfirstlane(p1 - p0);
+  if (tot > 64) {
+    if (lane == 0)
+      coarse_row<FILL, T>(I, n, ptr, col, val, cnt_or_ptr, ccol, cval, cdinv);
+    return;
   }
+  const int key = lane < tot ? col[p0 + lane] / kAgg : INT32_MAX;
+  const double v = FILL && lane < tot ? (double)val[p0 + lane] : 0.0;
+  const int vhi = __double2hiint(v), vlo = __double2loint(v);
+  bool first = lane < tot;
+  double s = 0.0;
+  for (int e = 0; e < tot; e++) {
+    const bool eq = __builtin_amdgcn_readlane(key, e) == key;
+    if (eq && e < lane) first = false;
+    if (FILL) {
+      const double ve = __hiloint2double(__builtin_amdgcn_readlane(vhi, e),
+                                         __builtin_amdgcn_readlane(vlo, e));
+      if (eq) s += ve;
+    }
+  }
+  const unsigned long long heads = __ballot(first);
+  if (!FILL) {
+    if (lane == 0) cnt_or_ptr[I] = __popcll(heads);
+    return;
+  }
+  int rank = 0;
+  for (unsigned long long m = heads; m; m &= m - 1)
+    rank += __builtin_amdgcn_readlane(key, __ffsll((long long)m) - 1) < key;
+  if (first) {
+    const int32_t o = cnt_or_ptr[I] + rank;
+    ccol[o] = key;
+    cval[o] = (T)s;
+  }
+  const unsigned long long dg = __ballot(first && key == (int)I);
+  if (dg ? first && key == (int)I : lane == 0)
+    cdinv[I] = (T)(dg && s > 0.0 ? 1.0 / s : 0.0);
+}
+
+// Inverse of the coarsest matrix (symmetric positive definite) by in-place
+// Gauss-Jordan elimination without pivoting, one workgroup: thread (tx, ty) of
+// 32 x 32 keeps elements (ty + 32 a, tx + 32 b) in registers, and a step
+// passes its pivot row and column through LDS (double buffered: one barrier a
+// step).  A non-positive pivot (a disconnected piece) counts as 1.  Bound by
+// the FP64 rate of its one compute unit; at 157 unknowns 175 us, against 1.7
+// ms for a Cholesky factor in global memory and 2.8 ms for its inverse with
+// one thread per column (serial chains of global loads).
+constexpr int kDenseSide = 32;
+template <int TILES, class T>
+__global__ void __launch_bounds__(kDenseSide *kDenseSide) k_amg_dense_inv(
+    int n, const int32_t *ptr, const int32_t *col, const T *val, double *inv) {
+  __shared__ double srow[2][kDenseSide * TILES], scol[2][kDenseSide * TILES];
+  const int tid = (int)threadIdx.x, tx = tid % kDenseSide, ty = tid / kDenseSide;
+  for (int q = tid; q < n * n; q += kDenseSide * kDenseSide) inv[q] = 0.0;
+  __syncthreads();
+  for (int i = tid; i < n; i += kDenseSide * kDenseSide)
+    for (int32_t q = ptr[i]; q < ptr[i + 1]; q++) inv[i * n + col[q]] = (double)val[q];
+  __syncthreads();
+  double A[TILES][TILES];
+#pragma unroll
+  for (int a = 0; a < TILES; a++)
+#pragma unroll
+    for (int b = 0; b < TILES; b++) {
+      const int i = ty + kDenseSide * a, j = tx + kDenseSide * b;
+      A[a][b] = i < n && j < n ? inv[i * n + j] : 0.0;
+    }
+  // row and column k to LDS
+  auto publish = [&](int k) {
+    const int t = k / kDenseSide, r = k % kDenseSide;
+#pragma unroll
+    for (int c = 0; c < TILES; c++)
+      if (c == t) {
+        if (ty == r) {
+#pragma unroll
+          for (int b = 0; b < TILES; b++) srow[k & 1][tx + kDenseSide * b] = A[c][b];
+        }
+        if (tx == r) {
+#pragma unroll
+          for (int a = 0; a < TILES; a++) scol[k & 1][ty + kDenseSide * a] = A[a][c];
+        }
+      }
+  };
+  publish(0);
+  for (int k = 0; k < n; k++) {
+    __syncthreads();
+    const double d = srow[k & 1][k];
+    const double ip = 1.0 / (d > 0.0 ? d : 1.0);
+    double r[TILES], c[TILES];
+#pragma unroll
+    for (int b = 0; b < TILES; b++) r[b] = srow[k & 1][tx + kDenseSide * b] * ip;
+#pragma unroll
+    for (int a = 0; a < TILES; a++) c[a] = scol[k & 1][ty + kDenseSide * a];
+#pragma unroll
+    for (int a = 0; a < TILES; a++)
+#pragma unroll
+      for (int b = 0; b < TILES; b++) A[a][b] -= c[a] * r[b];
+    const int t = k / kDenseSide, q = k % kDenseSide;
+#pragma unroll
+    for (int e = 0; e < TILES; e++)
+      if (e == t) {
+        if (ty == q) {
+#pragma unroll
+          for (int b = 0; b < TILES; b++) A[e][b] = r[b];
+        }
+        if (tx == q) {
+#pragma unroll
+          for (int a = 0; a < TILES; a++) A[a][e] = -c[a] * ip;
+          if (ty == q) A[e][e] = ip;
+        }
+      }
+    if (k + 1 < n) publish(k + 1);
+  }
+#pragma unroll
+  for (int a = 0; a < TILES; a++)
+#pragma unroll
+    for (int b = 0; b < TILES; b++) {
+      const int i = ty + kDenseSide * a, j = tx + kDenseSide * b;
+      if (i < n && j < n) inv[i * n + j] = A[a][b];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -220,39 +335,39 @@ __global__ void k_amg_smooth_prolong(int64_t n, const int32_t *ptr, const int32_
     y[i] = (TY)(xi + kOmega * ((double)b[i] - ax) * (double)dinv[i]);
   }
 }
-// Inverse of the coarsest matrix from its Cholesky factor L (row-major,
-// lower): thread j solves L L^T x = e_j, column j of the inverse.
-__global__ void __launch_bounds__(256) k_amg_dense_inv(int64_t n, const double *Lf,
-                                                       double *inv) {
-  const int64_t j = threadIdx.x;
-  if (j >= n) return;
-  double *x = inv + j;  // column j, stride n
-  for (int64_t i = 0; i < n; i++) {  // L y = e_j
-    double s = (i == j) ? 1.0 : 0.0;
-    for (int64_t k = j; k < i; k++) s -= Lf[i * n + k] * x[k * n];
-    x[i * n] = (i < j) ? 0.0 : s / Lf[i * n + i];
-  }
-  for (int64_t i = n - 1; i >= 0; i--) {  // L^T x = y
-    double s = x[i * n];
-    for (int64_t k = i + 1; k < n; k++) s -= Lf[k * n + i] * x[k * n];
-    x[i * n] = s / Lf[i * n + i];
-  }
-}
-// coarsest: x = A^-1 b, one row per thread (one workgroup)
+// coarsest: x = A^-1 b, one workgroup, 16 lanes per row
+constexpr int kDenseThreads = 1024;
 template <class TB, class TX>
-__global__ void __launch_bounds__(256) k_amg_dense_solve(int64_t n, const double *inv,
-                                                         const TB *b, TX *x,
-                                                         const double *done) {
+__global__ void __launch_bounds__(kDenseThreads) k_amg_dense_solve(int64_t n, const double *inv,
+                                                                   const TB *b, TX *x,
+                                                                   const double *done) {
   if (*done != 0.0) return;
   __shared__ double sb[kCoarsest];
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) sb[i] = (double)b[i];
+  for (int i = threadIdx.x; i < n; i += kDenseThreads) sb[i] = (double)b[i];
   __syncthreads();
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-    double s = 0.0;
-    for (int64_t k = 0; k < n; k++) s += inv[i * n + k] * sb[k];
-    x[i] = (TX)s;
+  // a group's rows together, so that their loads overlap
+  constexpr int kRows = kCoarsest / (kDenseThreads / kGroup);
+  const int l = (int)threadIdx.x & (kGroup - 1), i0 = (int)threadIdx.x / kGroup;
+  const int N = (int)n;
+  const double *row[kRows];
+  double s[kRows];
+#pragma unroll
+  for (int r = 0; r < kRows; r++) {
+    row[r] = inv + min(i0 + r * (kDenseThreads / kGroup), N - 1) * N;
+    s[r] = 0.0;
+  }
+#pragma unroll 4
+  for (int k = l; k < N; k += kGroup)
+#pragma unroll
+    for (int r = 0; r < kRows; r++) s[r] += row[r][k] * sb[k];
+#pragma unroll
+  for (int r = 0; r < kRows; r++) {
+    const double t = row_sum(s[r]);
+    const int i = i0 + r * (kDenseThreads / kGroup);
+    if (l == 0 && i < N) x[i] = (TX)t;
   }
 }
+static_assert(kCoarsest % (kDenseThreads / kGroup) == 0, "rows of k_amg_dense_solve");
 
 // ---------------------------------------------------------------------------
 // Host side
@@ -270,8 +385,7 @@ struct Amg {
   std::vector<AmgLevel<float>> lvf;  // FP32 hierarchy
   bool fp32 = false;                 // which one the last setup built
   DBuf<int32_t> bad;                 // zero-diagonal flag of the level-0 matrix
-  DBuf<double> dense;                // Cholesky factor of the coarsest matrix
-  DBuf<double> dense_inv;            // its inverse (applied as one matrix-vector product)
+  DBuf<double> dense_inv;            // inverse of the coarsest matrix (one matrix-vector product)
   int nlev = 0;
   const int32_t *ptr0 = nullptr, *col0 = nullptr;  // level-0 pattern (the caller's CSR)
 };
@@ -308,6 +422,7 @@ static ma_status amg_build(ma_engine *e, Amg &A, const CsrView &M) {
   lv[0].n = n;
   MA_HIP_TRY(lv[0].x.ensure((size_t)n));
   MA_HIP_TRY(lv[0].y.ensure((size_t)n));
+  int64_t room = M.nnz;  // bound of the entries of the level being built
   while (lv[used - 1].n > kCoarsest && used < 32) {
     const size_t l = used - 1;
     const int64_t nf = lv[l].n, nc = (nf + kAgg - 1) / kAgg;
@@ -322,30 +437,40 @@ static ma_status amg_build(ma_engine *e, Amg &A, const CsrView &M) {
     MA_HIP_TRY(C.x.ensure((size_t)nc));
     MA_HIP_TRY(C.y.ensure((size_t)nc));
     MA_HIP_TRY(C.b.ensure((size_t)nc));
-    hipLaunchKernelGGL((k_amg_coarse<false, T>), dim3(nb2(nc)), dim3(kVB2), 0, e->stream, nc, nf,
-                       fptr, fcol, fval, C.ptr.p, nullptr, nullptr, nullptr);
+    const bool wave = nc <= kWaveRows;
+    const dim3 grid(nb2(wave ? 64 * nc : nc));
+    hipLaunchKernelGGL((wave ? k_amg_coarse_wave<false, T> : k_amg_coarse<false, T>), grid,
+                       dim3(kVB2), 0, e->stream, nc, nf, fptr, fcol, fval, C.ptr.p, nullptr,
+                       nullptr, nullptr);
     const int32_t zero = 0;
     MA_HIP_TRY(hipMemcpyAsync(C.ptr.p + nc, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
                               e->stream));
     MA_HIP_TRY(exclusive_scan(e, C.ptr.p, C.ptr.p, nc + 1));
-    int32_t nnzc = 0;
-    MA_HIP_TRY(hipMemcpyAsync(&nnzc, C.ptr.p + nc, sizeof(int32_t), hipMemcpyDeviceToHost,
-                              e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
-    MA_HIP_TRY(C.col.ensure((size_t)nnzc + 1));
-    MA_HIP_TRY(C.val.ensure((size_t)nnzc + 1));
-    hipLaunchKernelGGL((k_amg_coarse<true, T>), dim3(nb2(nc)), dim3(kVB2), 0, e->stream, nc, nf,
-                       fptr, fcol, fval, C.ptr.p, C.col.p, C.val.p, C.dinv.p);
+    // small levels take room for as many entries as the level above has,
+    // instead of waiting for their count
+    if (!wave) {
+      int32_t nnzc = 0;
+      MA_HIP_TRY(hipMemcpyAsync(&nnzc, C.ptr.p + nc, sizeof(int32_t), hipMemcpyDeviceToHost,
+                                e->stream));
+      MA_HIP_TRY(hipStreamSynchronize(e->stream));
+      room = nnzc;
+    }
+    room = std::min(room, nc * nc);
+    MA_HIP_TRY(C.col.ensure((size_t)room + 1));
+    MA_HIP_TRY(C.val.ensure((size_t)room + 1));
+    hipLaunchKernelGGL((wave ? k_amg_coarse_wave<true, T> : k_amg_coarse<true, T>), grid,
+                       dim3(kVB2), 0, e->stream, nc, nf, fptr, fcol, fval, C.ptr.p, C.col.p,
+                       C.val.p, C.dinv.p);
   }
   const AmgLevel<T> &Lc = lv[used - 1];
   const int32_t *cptr = (used == 1) ? M.ptr : Lc.ptr.p;
   const int32_t *ccol = (used == 1) ? M.col : Lc.col.p;
-  MA_HIP_TRY(A.dense.ensure((size_t)(Lc.n * Lc.n)));
   MA_HIP_TRY(A.dense_inv.ensure((size_t)(Lc.n * Lc.n)));
-  hipLaunchKernelGGL(k_amg_dense_chol<T>, dim3(1), dim3(256), 0, e->stream, Lc.n, cptr, ccol,
-                     val_of<T>(A, (int)used - 1), A.dense.p);
-  hipLaunchKernelGGL(k_amg_dense_inv, dim3(1), dim3(256), 0, e->stream, Lc.n, A.dense.p,
-                     A.dense_inv.p);
+  auto dense = Lc.n <= 2 * kDenseSide ? k_amg_dense_inv<2, T>
+               : Lc.n <= 4 * kDenseSide ? k_amg_dense_inv<4, T> : k_amg_dense_inv<6, T>;
+  static_assert(kCoarsest <= 6 * kDenseSide, "coarsest matrix in registers");
+  hipLaunchKernelGGL(dense, dim3(1), dim3(kDenseSide * kDenseSide), 0, e->stream, (int)Lc.n, cptr,
+                     ccol, val_of<T>(A, (int)used - 1), A.dense_inv.p);
   A.nlev = (int)used;
   return MA_OK;
 }
@@ -406,8 +531,8 @@ static hipError_t amg_cycle(ma_engine *e, Amg &A, const double *r, double *z, co
   auto ptr_of = [&](int l) { return l == 0 ? A.ptr0 : lv[l].ptr.p; };
   auto col_of = [&](int l) { return l == 0 ? A.col0 : lv[l].col.p; };
   if (nl == 1) {
-    hipLaunchKernelGGL((k_amg_dense_solve<double, double>), dim3(1), dim3(256), 0, e->stream,
-                       lv[0].n, A.dense_inv.p, r, z, done);
+    hipLaunchKernelGGL((k_amg_dense_solve<double, double>), dim3(1), dim3(kDenseThreads), 0,
+                       e->stream, lv[0].n, A.dense_inv.p, r, z, done);
     return hipGetLastError();
   }
   // downward (the first sweep of a coarse level comes from the restriction)
@@ -448,8 +573,8 @@ static hipError_t amg_cycle(ma_engine *e, Amg &A, const double *r, double *z, co
   }
   {
     AmgLevel<T> &Lc = lv[nl - 1];
-    hipLaunchKernelGGL((k_amg_dense_solve<T, T>), dim3(1), dim3(256), 0, e->stream, Lc.n,
-                       A.dense_inv.p, (const T *)Lc.b.p, Lc.x.p, done);
+    hipLaunchKernelGGL((k_amg_dense_solve<T, T>), dim3(1), dim3(kDenseThreads), 0, e->stream,
+                       Lc.n, A.dense_inv.p, (const T *)Lc.b.p, Lc.x.p, done);
   }
   // upward
   for (int l = nl - 2; l >= 0; l--) {

@@ -364,12 +364,6 @@ __device__ inline double plane_bound(const Plane &p, const NodeBox &q, double x,
   const double m = box_min(q, p.ax - 2.0 * x, p.ay - 2.0 * y, mag);
   return p.b + m - kPlaneEps * (fabs(p.b) + mag);
 }
-__device__ inline double row_sum(double v) {
-  v += dpp<kDppRor + 8>(v);
-  v += dpp<kDppRor + 4>(v);
-  v += dpp<kDppRor + 2>(v);
-  return v + dpp<kDppRor + 1>(v);
-}
 
 // One group per node of level lev + 2 (lev + 1 when that is the top: step 1);
 // lane c takes its descendant c of level lev.  lev = 0: from the Diracs of the

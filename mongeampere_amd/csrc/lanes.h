@@ -56,7 +56,8 @@ __device__ inline float row_max_nonneg(float f) {
   v = max(v, dpp<kDppRor + 2>(v));
   return __int_as_float(max(v, dpp<kDppRor + 1>(v)));
 }
-__device__ inline int row_sum(int v) {
+template <class T>
+__device__ inline T row_sum(T v) {
   v += dpp<kDppRor + 8>(v);
   v += dpp<kDppRor + 4>(v);
   v += dpp<kDppRor + 2>(v);
