@@ -133,8 +133,10 @@ struct CellBuf<float> {
 // ---------------------------------------------------------------------------
 static_assert(kMaxFast == kGroup, "one polygon vertex per lane");
 
-// a / b: a reciprocal and one correction (within an ulp), FP64 as the compiler does it
+// a / b: a reciprocal and one correction (within an ulp; not near the ends of
+// the range, which the reciprocal does not cover), FP64 as the compiler does it
 __device__ inline float ratio(float a, float b) {
+  if (!(fabsf(b) > 1e-30f && fabsf(b) < 1e30f)) return a / b;
   const float r = __builtin_amdgcn_rcpf(b), q = a * r;
   return fmaf(fmaf(-b, q, a), r, q);
 }
@@ -1013,16 +1015,20 @@ __device__ inline void acc_add(R &s, R &c, R v) {
   }
 }
 
-// MODE 0: mass, int rho |x - y|^2 and Hessian edge integrals; MODE 1: mass
-// and first moments; MODE 2: MODE 1 plus, per triangle vertex v, the
-// integral of (|x - y_k|^2 - w_k) phi_v(x) over the fragment (phi_v: P1 hat
-// function of v, linear on the triangle), the derivative of the dual value
-// w.r.t. the density value at v.
+// Integrals over a fragment, as a fan of triangles (coordinates local to the
+// Dirac).  MODE 0: mass and int rho |x - y|^2; MODE 1: mass and first moments;
+// MODE 2: MODE 1 plus, per triangle vertex v, the integral of (|x - y_k|^2 -
+// w_k) phi_v(x) over the fragment (phi_v: P1 hat function of v, linear on the
+// triangle), the derivative of the dual value w.r.t. the density value at v;
+// MODE 3: MODE 1 plus the second moments.  The integrands are products of
+// functions linear on the fan triangle, whose integrals are closed forms in
+// the vertex values: with A the area, S the sum of the vertices p_k and R that
+// of the density values r_k there, int rho = A R / 3, int rho x = A/12 (R S +
+// sum r_k p_k), int rho x x^T = A/60 (R (S S^T + sum p_k p_k^T) + W S^T + S W^T
+// + 2 sum r_k p_k p_k^T), W = sum r_k p_k.  (Exact as the 6-point rule of the
+// reference is, at a third of its instructions.)
 template <int MODE, class R>
-struct Integrator {
-  // fragment vertices arrive in order; fan from the first one
-  int cnt;
-  SV<R> first, prev;
+struct Quad {
   R area, mass, intg, mx, my;
   R sxx, syy, sxy;    // second moments (MODE 3)
   R cmass, cintg;     // Kahan compensations (FP32)
@@ -1035,130 +1041,129 @@ struct Integrator {
   double dv[3];
   // extent of the fragment, for the degeneracy test
   R xlo, xhi, ylo, yhi, cmax;
-  // A fragment counts only if its area is positive: the reference clips the
-  // closed triangle by the open cell (ties excluded), so a cell touching a
-  // triangle only along an edge or at a point yields nothing.  Exactly
-  // degenerate fragments come out with areas at rounding level, hence the
-  // scale-aware threshold.  Edge integrals are buffered until the area is
-  // known (named registers rather than arrays, so nothing spills to scratch).
-  int nb;
-  int bl0, bl1, bl2, bl3;
-  R bv0, bv1, bv2, bv3;
-  __device__ bool positive() const {
-    return area > Tol<R>::area * ((xhi - xlo) + (yhi - ylo)) * cmax;
-  }
-  R *eacc;
-  int64_t k;
-  __device__ void commit(int lab, R r) {
-    atomicAdd(&eacc[k * kMaxFast + lab], r);
-  }
-  __device__ void edge(const SV<R> &a, const SV<R> &b) {
-    if (MODE != 0 || a.lab < 0) return;
-    const R ex = b.x - a.x, ey = b.y - a.y;
-    if (ex == R(0) && ey == R(0)) return;  // zero-length piece from a snapped vertex
-    const R r = sqrt(ex * ex + ey * ey) *
-                (r0 + ga * (R(0.5) * (a.x + b.x) - tx) + gb * (R(0.5) * (a.y + b.y) - ty));
-    if (nb == 0) {
-      bl0 = a.lab;
-      bv0 = r;
-    } else if (nb == 1) {
-      bl1 = a.lab;
-      bv1 = r;
-    } else if (nb == 2) {
-      bl2 = a.lab;
-      bv2 = r;
-    } else if (nb == 3) {
-      bl3 = a.lab;
-      bv3 = r;
-    } else {
-      // a degenerate fragment has at most one cell edge of positive length
-      // (plus zero-length edges at tie vertices): five or more means a
-      // genuine fragment
-      commit(a.lab, r);
-    }
-    nb++;
-  }
-  __device__ void fan(const SV<R> &p0, const SV<R> &p1, const SV<R> &p2) {
-    const R x0 = p0.x, y0 = p0.y, x1 = p1.x, y1 = p1.y, x2 = p2.x, y2 = p2.y;
-    const R ar = R(0.5) * ((x1 - x0) * (y2 - y0) - (x2 - x0) * (y1 - y0));
-    const R gx = (x0 + x1 + x2) * R(1.0 / 3.0), gy = (y0 + y1 + y2) * R(1.0 / 3.0);
-    area += ar;
-    acc_add(mass, cmass, ar * (r0 + ga * (gx - tx) + gb * (gy - ty)));
-    AC6T<R> q;
-    ac6_points(x0, y0, x1, y1, x2, y2, q);
-    R a1 = R(0), a9 = R(0), b1 = R(0), b9 = R(0);
-    R u1 = R(0), u9 = R(0), v1 = R(0), v9 = R(0), w1 = R(0), w9 = R(0);
-    double c1[3] = {0.0, 0.0, 0.0}, c9[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-    for (int p = 0; p < 6; p++) {
-      const R rp = r0 + ga * (q.px[p] - tx) + gb * (q.py[p] - ty);
-      if (MODE == 0) {
-        const R f = rp * (q.px[p] * q.px[p] + q.py[p] * q.py[p]);
-        if (p < 3) a1 += f; else a9 += f;
-      } else {
-        if (p < 3) {
-          a1 += rp * q.px[p];
-          b1 += rp * q.py[p];
-        } else {
-          a9 += rp * q.px[p];
-          b9 += rp * q.py[p];
-        }
-      }
-      if (MODE == 2) {
-        const double c = q.px[p] * q.px[p] + q.py[p] * q.py[p] - wk;
-#pragma unroll
-        for (int v = 0; v < 3; v++) {
-          const double f = c * (la[v] * q.px[p] + lb[v] * q.py[p] + lc[v]);
-          if (p < 3) c1[v] += f; else c9[v] += f;
-        }
-      }
-      if (MODE == 3) {
-        const R fx = rp * q.px[p], fy = rp * q.py[p];
-        if (p < 3) {
-          u1 += fx * q.px[p];
-          v1 += fy * q.py[p];
-          w1 += fx * q.py[p];
-        } else {
-          u9 += fx * q.px[p];
-          v9 += fy * q.py[p];
-          w9 += fx * q.py[p];
-        }
-      }
-    }
-    if (MODE == 0) {
-      acc_add(intg, cintg, ar * (a1 * R(1.0 / 30.0) + a9 * R(9.0 / 30.0)));
-    } else {
-      mx += ar * (a1 * R(1.0 / 30.0) + a9 * R(9.0 / 30.0));
-      my += ar * (b1 * R(1.0 / 30.0) + b9 * R(9.0 / 30.0));
-    }
-    if (MODE == 3) {
-      sxx += ar * (u1 * R(1.0 / 30.0) + u9 * R(9.0 / 30.0));
-      syy += ar * (v1 * R(1.0 / 30.0) + v9 * R(9.0 / 30.0));
-      sxy += ar * (w1 * R(1.0 / 30.0) + w9 * R(9.0 / 30.0));
-    }
-    if (MODE == 2) {
-#pragma unroll
-      for (int v = 0; v < 3; v++) dv[v] += ar * (c1[v] * (1.0 / 30.0) + c9[v] * (9.0 / 30.0));
-    }
-  }
-  __device__ void push(const SV<R> &v) {
+
+  struct V {
+    R x, y, r, n;  // density and |x|^2 there
+  };
+  __device__ R rho(R x, R y) const { return r0 + ga * (x - tx) + gb * (y - ty); }
+  __device__ V vertex(R x, R y) const { return {x, y, rho(x, y), x * x + y * y}; }
+  __device__ void extend(const V &v) {
     xlo = fmin(xlo, v.x);
     xhi = fmax(xhi, v.x);
     ylo = fmin(ylo, v.y);
     yhi = fmax(yhi, v.y);
     cmax = fmax(cmax, fmax(fabs(v.x), fabs(v.y)));
-    if (cnt == 0) {
-      first = v;
+  }
+  // A fragment counts only if its area is positive: the reference clips the
+  // closed triangle by the open cell (ties excluded), so a cell touching a
+  // triangle only along an edge or at a point yields nothing.  Exactly
+  // degenerate fragments come out with areas at rounding level, hence the
+  // scale-aware threshold.
+  __device__ bool positive() const {
+    return area > Tol<R>::area * ((xhi - xlo) + (yhi - ylo)) * cmax;
+  }
+  // int rho ds along the edge a -> b
+  __device__ R edge(R ax, R ay, R ra, R bx, R by, R rb) const {
+    const R ex = bx - ax, ey = by - ay;
+    return sqrt(ex * ex + ey * ey) * (R(0.5) * (ra + rb));
+  }
+  __device__ void fan(const V &a, const V &b, const V &c) {
+    const R ar = R(0.5) * ((b.x - a.x) * (c.y - a.y) - (c.x - a.x) * (b.y - a.y));
+    const R Rs = a.r + b.r + c.r, Sx = a.x + b.x + c.x, Sy = a.y + b.y + c.y;
+    const R Wx = a.r * a.x + b.r * b.x + c.r * c.x, Wy = a.r * a.y + b.r * b.y + c.r * c.y;
+    area += ar;
+    acc_add(mass, cmass, ar * (Rs * R(1.0 / 3.0)));
+    if (MODE == 0) {
+      const R q = Rs * (Sx * Sx + Sy * Sy + (a.n + b.n + c.n)) +
+                  R(2) * (Wx * Sx + Wy * Sy + (a.r * a.n + b.r * b.n + c.r * c.n));
+      acc_add(intg, cintg, ar * (q * R(1.0 / 60.0)));
     } else {
-      edge(prev, v);
-      if (cnt >= 2) fan(first, prev, v);
+      mx += ar * (R(1.0 / 12.0) * (Rs * Sx + Wx));
+      my += ar * (R(1.0 / 12.0) * (Rs * Sy + Wy));
     }
-    prev = v;
+    if (MODE == 3) {
+      const R xx = a.x * a.x + b.x * b.x + c.x * c.x, yy = a.y * a.y + b.y * b.y + c.y * c.y;
+      const R xy = a.x * a.y + b.x * b.y + c.x * c.y;
+      const R rxx = a.r * a.x * a.x + b.r * b.x * b.x + c.r * c.x * c.x;
+      const R ryy = a.r * a.y * a.y + b.r * b.y * b.y + c.r * c.y * c.y;
+      const R rxy = a.r * a.x * a.y + b.r * b.x * b.y + c.r * c.x * c.y;
+      const R f = ar * R(1.0 / 60.0);
+      sxx += f * (Rs * (Sx * Sx + xx) + R(2) * (Wx * Sx + rxx));
+      syy += f * (Rs * (Sy * Sy + yy) + R(2) * (Wy * Sy + ryy));
+      sxy += f * (Rs * (Sx * Sy + xy) + Wx * Sy + Wy * Sx + R(2) * rxy);
+    }
+    if (MODE == 2) {
+      const double N = a.n + b.n + c.n, S2 = Sx * Sx + Sy * Sy;
+#pragma unroll
+      for (int v = 0; v < 3; v++) {
+        const double fa = la[v] * a.x + lb[v] * a.y + lc[v], fb = la[v] * b.x + lb[v] * b.y + lc[v];
+        const double fc = la[v] * c.x + lb[v] * c.y + lc[v], F = fa + fb + fc;
+        const double Fx = fa * a.x + fb * b.x + fc * c.x, Fy = fa * a.y + fb * b.y + fc * c.y;
+        const double Fn = fa * a.n + fb * b.n + fc * c.n;
+        dv[v] += ar * ((1.0 / 60.0) * (F * (S2 + N) + 2.0 * (Fx * Sx + Fy * Sy + Fn)) -
+                       (1.0 / 3.0) * wk * F);
+      }
+    }
+  }
+};
+
+// Streaming integration for k_frag_wide: fragment vertices arrive in order.
+template <int MODE, class R>
+struct Integrator : Quad<MODE, R> {
+  using Base = Quad<MODE, R>;
+  using V = typename Base::V;
+  int cnt;
+  V first, prev;
+  int first_lab, prev_lab;
+  // Edge integrals are buffered until the area is known (named registers
+  // rather than arrays, so nothing spills to scratch).
+  int nb;
+  int bl0, bl1, bl2, bl3;
+  R bv0, bv1, bv2, bv3;
+  R *eacc;
+  int64_t k;
+  __device__ void commit(int lab, R r) { atomicAdd(&eacc[k * kMaxFast + lab], r); }
+  __device__ void edge(const V &a, int lab, const V &b) {
+    if (MODE != 0 || lab < 0) return;
+    if (b.x == a.x && b.y == a.y) return;  // zero-length piece from a snapped vertex
+    const R r = Base::edge(a.x, a.y, a.r, b.x, b.y, b.r);
+    if (nb == 0) {
+      bl0 = lab;
+      bv0 = r;
+    } else if (nb == 1) {
+      bl1 = lab;
+      bv1 = r;
+    } else if (nb == 2) {
+      bl2 = lab;
+      bv2 = r;
+    } else if (nb == 3) {
+      bl3 = lab;
+      bv3 = r;
+    } else {
+      // a degenerate fragment has at most one cell edge of positive length
+      // (plus zero-length edges at tie vertices): five or more means a
+      // genuine fragment
+      commit(lab, r);
+    }
+    nb++;
+  }
+  __device__ void push(const SV<R> &v) {
+    const V c = Base::vertex(v.x, v.y);
+    Base::extend(c);
+    if (cnt == 0) {
+      first = c;
+      first_lab = v.lab;
+    } else {
+      edge(prev, prev_lab, c);
+      if (cnt >= 2) Base::fan(first, prev, c);
+    }
+    prev = c;
+    prev_lab = v.lab;
     cnt++;
   }
   __device__ void finish() {
-    if (cnt >= 2) edge(prev, first);
-    if (positive()) {
+    if (cnt >= 2) edge(prev, prev_lab, first);
+    if (Base::positive()) {
       if (nb > 0) commit(bl0, bv0);
       if (nb > 1) commit(bl1, bv1);
       if (nb > 2) commit(bl2, bv2);
@@ -1167,33 +1172,32 @@ struct Integrator {
   }
 };
 
-// Sets up the three clip stages (one per triangle edge, in coordinates local
-// to the Dirac) and the integrator of pair (cell k, triangle t).
+// Corners of triangle t in coordinates local to Dirac k (formed in FP64, then
+// rounded once) and the quadrature of the pair.
+template <class R>
+struct LocalTri {
+  R x[3], y[3];
+};
 template <int MODE, class R>
-__device__ inline void frag_setup(const CellArgs &a, int64_t k, const TriData &t, Stage<R> &s1,
-                                  Stage<R> &s2, Stage<R> &s3, Integrator<MODE, R> &I) {
+__device__ inline void quad_setup(const CellArgs &a, int64_t k, const TriData &t, LocalTri<R> &T,
+                                  Quad<MODE, R> &I) {
   const double yx = a.pos[2 * k], yy = a.pos[2 * k + 1];
-  // triangle in coordinates local to the Dirac (FP64, then rounded once)
-  const R X0 = (R)(t.x[0] - yx), Y0 = (R)(t.y[0] - yy), X1 = (R)(t.x[1] - yx);
-  const R Y1 = (R)(t.y[1] - yy), X2 = (R)(t.x[2] - yx), Y2 = (R)(t.y[2] - yy);
-  s1.init(X0, Y0, X1, Y1);
-  s2.init(X1, Y1, X2, Y2);
-  s3.init(X2, Y2, X0, Y0);
-  I.cnt = 0;
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    T.x[c] = (R)(t.x[c] - yx);
+    T.y[c] = (R)(t.y[c] - yy);
+  }
   I.area = I.mass = I.intg = I.mx = I.my = R(0);
   I.sxx = I.syy = I.sxy = R(0);
   I.cmass = I.cintg = R(0);
   I.r0 = (R)(t.a * t.x[0] + t.b * t.y[0] + t.c);  // the value at vertex 0
   I.ga = (R)t.a;
   I.gb = (R)t.b;
-  I.tx = X0;
-  I.ty = Y0;
-  I.nb = 0;
+  I.tx = T.x[0];
+  I.ty = T.y[0];
   I.xlo = I.ylo = R(kInf);
   I.xhi = I.yhi = R(-kInf);
   I.cmax = R(0);
-  I.eacc = CellBuf<R>::eacc(a);
-  I.k = k;
   if (MODE == 2) {
     // barycentric coordinates of the triangle in coordinates local to the Dirac
     const double X0 = t.x[0] - yx, Y0 = t.y[0] - yy, X1 = t.x[1] - yx, Y1 = t.y[1] - yy;
@@ -1205,6 +1209,21 @@ __device__ inline void frag_setup(const CellArgs &a, int64_t k, const TriData &t
     I.wk = a.w[k];
     I.dv[0] = I.dv[1] = I.dv[2] = 0.0;
   }
+}
+// Sets up the three clip stages (one per triangle edge) and the integrator of
+// pair (cell k, triangle t) for k_frag_wide.
+template <int MODE, class R>
+__device__ inline void frag_setup(const CellArgs &a, int64_t k, const TriData &t, Stage<R> &s1,
+                                  Stage<R> &s2, Stage<R> &s3, Integrator<MODE, R> &I) {
+  LocalTri<R> T;
+  quad_setup<MODE, R>(a, k, t, T, I);
+  s1.init(T.x[0], T.y[0], T.x[1], T.y[1]);
+  s2.init(T.x[1], T.y[1], T.x[2], T.y[2]);
+  s3.init(T.x[2], T.y[2], T.x[0], T.y[0]);
+  I.cnt = 0;
+  I.nb = 0;
+  I.eacc = CellBuf<R>::eacc(a);
+  I.k = k;
 }
 
 // Vertex v of the cell polygon of k (label: v, or -1 on a domain edge) from
@@ -1256,12 +1275,86 @@ __device__ inline void frag_clip(const Src &src, int n, Stage<R> &s1, Stage<R> &
   if (m3 > 1) sink(r1);
 }
 
-// Fragment vertices staged per thread in LDS by k_frag (FP32 / FP64).
+// Vertices per thread that k_frag's LDS holds (FP32 / FP64): cells and
+// fragments with more go to k_frag_wide.  12 is what the label word holds; in
+// FP64 10 keep four workgroups on a compute unit (1M Diracs: 0.78 ms with
+// k_frag_wide, 0.86 with 12, 1.04 with 9).
 template <class R>
 struct FragCap {
-  static constexpr int value = sizeof(R) == sizeof(float) ? 9 : 8;
+  static constexpr int value = sizeof(R) == sizeof(float) ? 12 : 10;
+};
+// The polygon of one thread of k_frag: vertex slots in LDS (a column per
+// thread), their order packed in a word of 4 bits a vertex and the labels of
+// the edges leaving them (the cell edge's index, kNoLabel on a triangle or
+// domain edge) in one of 5 bits.  A clip rotates the two words and moves no
+// vertex; the slots past the last vertex of the order word are free.
+constexpr int kNoLabel = 31;
+template <class R>
+struct FragPoly {
+  R *px, *py;  // this thread's column, 256 apart
+  uint64_t order, labels;
+  int m;
+
+  __device__ int slot(int i) const { return (int)(order >> (4 * i)) & 15; }
+  __device__ int label(int i) const { return (int)(labels >> (5 * i)) & 31; }
+  __device__ R x(int i) const { return px[slot(i) * 256]; }
+  __device__ R y(int i) const { return py[slot(i) * 256]; }
+  // Clip by the closed half-plane left of (ax, ay) -> (bx, by).  Side values
+  // within rounding of zero count as on the line (inside: the triangle is
+  // closed), so a cell edge lying on a mesh edge stays with the triangle on
+  // the cell's side.  Returns false when the polygon outgrows its slots or
+  // rounding breaks the single run of vertices inside.
+  __device__ bool clip(R ax, R ay, R bx, R by) {
+    const R ex = bx - ax, ey = by - ay;
+    const R tol = Tol<R>::snap * sqrt(ex * ex + ey * ey);
+    auto side = [&](R vx, R vy) -> R {
+      const R dx = vx - ax, dy = vy - ay;
+      const R v = ex * dy - ey * dx;
+      return fabs(v) <= tol * (fabs(vx) + fabs(vy) + fabs(dx) + fabs(dy)) ? R(0) : v;
+    };
+    unsigned in = 0u;
+    for (int i = 0; i < m; i++) in |= (side(x(i), y(i)) >= R(0) ? 1u : 0u) << i;
+    const unsigned full = (1u << m) - 1u;
+    if (in == full) return true;
+    if (in == 0u) {
+      m = 0;
+      return true;
+    }
+    const int kept = __popc(in), out = 32 - __clz((int)(~in & full));
+    const int s0 = (in & 1u) ? (out == m ? 0 : out) : __ffs((int)in) - 1;
+    const unsigned run = ((1u << kept) - 1u) << s0;
+    if (((run | (run >> m)) & full) != in || kept + 2 > FragCap<R>::value) return false;
+    // the run first, then the vertices cut off, then the free slots
+    const uint64_t om = (1ull << (4 * m)) - 1ull, lm = (1ull << (5 * m)) - 1ull;
+    const uint64_t lo = order & om, ll = labels & lm;
+    order = (order & ~om) | (((lo >> (4 * s0)) | (lo << (4 * (m - s0)))) & om);
+    labels = ((ll >> (5 * s0)) | (ll << (5 * (m - s0)))) & lm;
+    // edge kept - 1 -> kept leaves, edge m - 1 -> 0 comes back
+    const R ux = x(kept - 1), uy = y(kept - 1), vx = x(kept), vy = y(kept);
+    const R wx = x(m - 1), wy = y(m - 1), zx = x(0), zy = y(0);
+    const R su = side(ux, uy), sv = side(vx, vy), sw = side(wx, wy), sz = side(zx, zy);
+    const R t0 = ratio(su, su - sv), t1 = ratio(sw, sw - sz);
+    const int el = label(m - 1), s1 = slot(kept), s2 = slot(kept + 1);
+    px[s1 * 256] = ux + t0 * (vx - ux);
+    py[s1 * 256] = uy + t0 * (vy - uy);
+    px[s2 * 256] = wx + t1 * (zx - wx);
+    py[s2 * 256] = wy + t1 * (zy - wy);
+    const int at = 5 * kept;
+    labels = (labels & ((1ull << at) - 1ull)) |
+             ((uint64_t)(unsigned)(kNoLabel | (el << 5)) << at);
+    m = kept + 2;
+    return true;
+  }
 };
 
+// One thread per pair: the cell polygon, in LDS, clipped by the triangle's
+// three edges, then integrated in one loop over the fragment.  Every lane runs
+// the same sequence (classify, two crossings, rotate), so the wave is bound by
+// its longest polygon only; a pipeline that streamed the vertices through the
+// three edges took a different branch on every lane (26 % of the lanes active
+// per instruction, 3700 VALU instructions a wave against 2100 and 47 % here).
+// VALU issue bounds it (77 - 82 % busy).  At 10.4M pairs, before and after:
+// FP64 1.38 and 0.68 ms, FP32 0.86 and 0.70 ms.
 template <int MODE, class R>
 __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,
                                               const int32_t *__restrict__ pair_cell,
@@ -1274,49 +1367,72 @@ __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,
   const int64_t k = pair_cell[p];
   const TriData t = a.tri[pair_tri[p]];
   const int n = valid ? a.pn[k] : 0;
-  Stage<R> s1, s2, s3;
-  Integrator<MODE, R> I;
-  frag_setup<MODE, R>(a, k, t, s1, s2, s3, I);
-  // The clip pipeline's output vertices are staged in LDS and integrated
-  // afterwards in one flat loop: calling the integrator from inside the
-  // pipeline's data-dependent branches made every wave execute the
-  // quadrature once per possible path.  Fragments longer than the staging
-  // (rare) go to k_frag_wide.  The same LDS holds the per-cell sums at the end.
+  Quad<MODE, R> I;
+  LocalTri<R> T;
+  quad_setup<MODE, R>(a, k, t, T, I);
+  // the same LDS holds the per-cell sums at the end
   constexpr int kCap = FragCap<R>::value;
-  constexpr int kStageBytes = kCap * 256 * (2 * (int)sizeof(R) + 4);
-  constexpr int kRedBytes = 256 * 4 + 6 * 256 * 8;
+  constexpr int kStageBytes = kCap * 256 * 2 * (int)sizeof(R);
+  constexpr int kRedBytes = 256 * 4 + 6 * 256 * 8 + 16;
   __shared__ __align__(16) unsigned char lds[kStageBytes > kRedBytes ? kStageBytes : kRedBytes];
-  R *ox = reinterpret_cast<R *>(lds);
-  R *oy = ox + kCap * 256;
-  int *ol = reinterpret_cast<int *>(oy + kCap * 256);
-  int nout = 0;
   const int tt = (int)threadIdx.x;
-  frag_clip<R>(PolyGlobal<R>{a, k}, n, s1, s2, s3, [&](const SV<R> &v) {
-    if (nout < kCap) {
-      ox[nout * 256 + tt] = v.x;
-      oy[nout * 256 + tt] = v.y;
-      ol[nout * 256 + tt] = v.lab;
-    }
-    nout++;
-  });
-  const bool wide = nout > kCap;
-  if (wide) {
-    a.ovf[atomicAdd(a.novf, 1)] = (int32_t)p;
-  } else {
-    for (int i = 0; i < nout; i++) {
-      SV<R> v;
-      v.x = ox[i * 256 + tt];
-      v.y = oy[i * 256 + tt];
-      v.lab = ol[i * 256 + tt];
-      I.push(v);
-    }
-    I.finish();
+  FragPoly<R> F;
+  F.px = reinterpret_cast<R *>(lds) + tt;
+  F.py = F.px + kCap * 256;
+  F.order = 0xFEDCBA9876543210ull;
+  F.labels = 0ull;
+  F.m = min(n, kCap);
+  for (int i = 0; i < F.m; i++) {
+    const int64_t at = k * kMaxFast + i;
+    F.px[i * 256] = CellBuf<R>::px(a)[at];
+    F.py[i * 256] = CellBuf<R>::py(a)[at];
+    F.labels |= (uint64_t)(a.plab[at] >= 0 ? i : kNoLabel) << (5 * i);
   }
-  const bool counted = valid && !wide && I.cnt >= 3 && I.positive();
+  bool wide = n > kCap;
+  if (wide) F.m = 0;
+#pragma unroll 1
+  for (int c = 0; c < 3; c++) {
+    const int d = c == 2 ? 0 : c + 1;
+    const R ax = c == 0 ? T.x[0] : c == 1 ? T.x[1] : T.x[2];
+    const R ay = c == 0 ? T.y[0] : c == 1 ? T.y[1] : T.y[2];
+    const R bx = d == 0 ? T.x[0] : d == 1 ? T.x[1] : T.x[2];
+    const R by = d == 0 ? T.y[0] : d == 1 ? T.y[1] : T.y[2];
+    if (F.m > 0 && !F.clip(ax, ay, bx, by)) {
+      wide = true;
+      F.m = 0;
+    }
+  }
+  const int nout = F.m;
+  if (wide) a.ovf[atomicAdd(a.novf, 1)] = (int32_t)p;
+  if (nout > 0) {
+    using V = typename Quad<MODE, R>::V;
+    const V first = I.vertex(F.x(0), F.y(0));
+    I.extend(first);
+    V prev = first;
+    for (int i = 1; i < nout; i++) {
+      const V v = I.vertex(F.x(i), F.y(i));
+      I.extend(v);
+      if (i > 1) I.fan(first, prev, v);
+      prev = v;
+    }
+  }
+  const bool counted = valid && nout >= 3 && I.positive();
+  if (MODE == 0 && counted) {
+    // Hessian edge integrals (include/MA/kantorovich.hpp:109-122)
+    R *eacc = CellBuf<R>::eacc(a) + k * kMaxFast;
+    for (int i = 0; i < nout; i++) {
+      const int lab = F.label(i);
+      if (lab == kNoLabel) continue;
+      const int i1 = i + 1 == nout ? 0 : i + 1;
+      const R ax = F.x(i), ay = F.y(i), bx = F.x(i1), by = F.y(i1);
+      if (ax == bx && ay == by) continue;  // zero-length piece from a snapped vertex
+      atomicAdd(&eacc[lab], I.edge(ax, ay, I.rho(ax, ay), bx, by, I.rho(bx, by)));
+    }
+  }
   if (MODE == 1 && a.fo.count != nullptr) {
     // fragment polygons from the staging (every lane takes part)
-    auto gx = [&](int i) { return ox[i * 256 + tt]; };
-    auto gy = [&](int i) { return oy[i * 256 + tt]; };
+    auto gx = [&](int i) { return F.x(i); };
+    auto gy = [&](int i) { return F.y(i); };
     const double eps = frag_eps(I.xlo, I.xhi, I.ylo, I.yhi);
     const int m = counted ? frag_distinct(nout, eps, gx, gy) : 0;
     unsigned long long f, v;
@@ -1360,7 +1476,7 @@ __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,
     for (int c = 0; c < kQ; c++) sval[c][t] = counted ? q[c] : 0.0;
     // fragment count: per wave into LDS, one global atomic per block (a
     // same-address atomic per wave serialises across the whole grid)
-    __shared__ int wcnt[4];
+    int *wcnt = reinterpret_cast<int *>(lds + 256 * 4 + 6 * 256 * 8);
     const unsigned long long bal = __ballot(counted);
     if ((t & 63) == 0) wcnt[t >> 6] = __popcll(bal);
     __syncthreads();
