@@ -8,7 +8,8 @@
 //                 three-stage Sutherland-Hodgman pipeline (one stage per
 //                 triangle edge) held in registers, fused with the exact
 //                 quadrature of the fragment;
-//   k_rows        one thread per Dirac: Hessian row from the edge integrals.
+//   k_row_count, k_row_fill  Hessian rows from the edge integrals, straight
+//                 into the CSR arrays.
 // Cells that overflow kMaxFast vertices are flagged and evaluated by the
 // general FP64 kernel (k_cells_general).
 //
@@ -24,6 +25,7 @@
 //   per-fragment integrals         include/MA/kantorovich.hpp:109-135, include/MA/lloyd.hpp:45-60
 //   quadrature                     include/MA/quadrature.hpp:23-42,69-85,122-143
 #include <climits>
+#include <type_traits>
 
 #include "geom_common.h"
 #include "lanes.h"
@@ -83,8 +85,10 @@ struct CellArgs {
   double *mass, *intg, *mom;  // mom: local first moments, interleaved (x, y)
   double *mom2;      // local second moments (xx, yy, xy) per Dirac (mode 3)
   int32_t *ovf, *novf;  // pairs left to k_frag_wide, and their count
-  double *eacc;      // edge integrals int rho ds, [k * kMaxFast + v]; -0.0 until an edge is seen
-  float *eaccf;      // FP32 edge integrals (mixed mode)
+  // edge integrals int rho ds, [k * kMaxFast + v]; -0.0 until an edge is seen
+  // (FP64 in both modes: 128 B a cell, so that two cells' atomics do not meet in
+  // a line; k_frag<float> at 10.4M pairs 0.60 ms with FP32 sums, 0.50 with these)
+  double *eacc;
   const int32_t *triv;  // triangle vertex ids (counter-clockwise, as in tri)
   double *dval;      // adjoint w.r.t. vertex density values (mode 2)
   int32_t *flags;
@@ -108,13 +112,11 @@ template <>
 struct CellBuf<double> {
   __device__ static double *px(const CellArgs &a) { return a.px; }
   __device__ static double *py(const CellArgs &a) { return a.py; }
-  __device__ static double *eacc(const CellArgs &a) { return a.eacc; }
 };
 template <>
 struct CellBuf<float> {
   __device__ static float *px(const CellArgs &a) { return a.pxf; }
   __device__ static float *py(const CellArgs &a) { return a.pyf; }
-  __device__ static float *eacc(const CellArgs &a) { return a.eaccf; }
 };
 
 // ---------------------------------------------------------------------------
@@ -489,7 +491,7 @@ __device__ inline void write_cell(const CellArgs &a, int64_t k, double yx, doubl
     CellBuf<R>::px(a)[at] = C.x;
     CellBuf<R>::py(a)[at] = C.y;
     a.plab[at] = C.lab;
-    CellBuf<R>::eacc(a)[at] = R(-0.0);  // "not seen": any contribution (>= 0) clears the sign
+    a.eacc[at] = -0.0;  // "not seen": any contribution (>= 0) clears the sign
   }
   const double bx0 = (double)row_min(C.x) + yx, by0 = (double)row_min(C.y) + yy;
   const double bx1 = (double)row_max(C.x) + yx, by1 = (double)row_max(C.y) + yy;
@@ -566,7 +568,6 @@ __device__ inline bool certify_levels(const Grid &g, const double *pyr3, const P
 }
 
 // -0.0 exactly (an edge integral no fragment has touched)
-__device__ inline bool is_neg_zero(float x) { return __float_as_uint(x) == 0x80000000u; }
 __device__ inline bool is_neg_zero(double x) {
   return (unsigned long long)__double_as_longlong(x) == 0x8000000000000000ull;
 }
@@ -876,52 +877,32 @@ ma_status refine_candidates(ma_engine *e, int64_t total) {
   return MA_OK;
 }
 
-// One wave (one block) per 64 consecutive cells.  Their pair segments are
-// contiguous in the output, so the lanes write the wave's whole range
-// together (coalesced): slot s belongs to the last cell whose offset is <= s
-// (binary search over the 64 offsets in LDS) and takes that cell's kept
-// triangle.  Cells with more than kPadTri candidates were not kept by the
-// cell kernel; the wave's four groups scan the triangle bins of four such
-// cells at a time again.
-__global__ void __launch_bounds__(64) k_pairs(CellArgs a, const int32_t *poff, int32_t *pair_cell,
-                                              int32_t *pair_tri) {
-  __shared__ int32_t soff[65];
-  __shared__ int32_t skeep[64];
-  const int64_t N = a.n;
-  const int64_t k0 = xcd_block(blockIdx.x, gridDim.x) * 64;
-  const int lane = (int)threadIdx.x;
-  const int64_t k = k0 + lane;
-  const int nk = (int)min((int64_t)64, N - k0);
-  const int cnt = lane < nk ? a.tcount[k] : 0;
-  soff[lane] = lane < nk ? poff[k] : poff[k0 + nk];
-  if (lane == 0) soff[64] = poff[k0 + nk];
-  skeep[lane] = cnt <= kPadTri;
-  __syncthreads();
-  const unsigned long long many = __ballot(cnt > kPadTri);
-  for (unsigned long long m = many; m; m &= m - 1, m &= m - 1, m &= m - 1, m &= m - 1) {
-    unsigned long long mine = m;  // this group's cell: the (lane / 16)-th of the next four
-    for (int i = 0; i < lane >> 4; i++) mine &= mine - 1;
-    if (!mine) continue;
-    const int c = __ffsll((long long)mine) - 1;
-    const double *bb = a.bbox + 4 * (k0 + c);
-    const int32_t o = soff[c];
-    group_triangles(a, lane & 48, lane & (kGroup - 1), bb[0], bb[1], bb[2], bb[3],
-                    [&](int32_t ti, int i) {
-                      pair_cell[o + i] = (int32_t)(k0 + c);
-                      pair_tri[o + i] = ti;
-                    });
+// (cell, triangle) pairs: the 16 lanes of a group write the segment of one
+// cell, the segments of consecutive cells being consecutive.  Cells with more
+// than kPadTri candidates were not kept by the cell kernel; their group scans
+// the triangle bins again.  Bound by HBM (8 B written and 4 B read a pair): 1M
+// cells, 10.4M pairs 107 us (one thread per cell's count and a search for each
+// slot's cell, at 1.2 waves per SIMD: 248 us).
+__global__ void __launch_bounds__(kCellThreads) k_pairs(CellArgs a, const int32_t *poff,
+                                                        int32_t *pair_cell, int32_t *pair_tri) {
+  const int64_t k = xcd_block<kCellXcdRun>(blockIdx.x, gridDim.x) * kCellGroups +
+                    threadIdx.x / kGroup;
+  if (k >= a.n) return;
+  const int l = (int)threadIdx.x & (kGroup - 1), base = (int)threadIdx.x & 48;
+  const int cnt = a.tcount[k];
+  const int32_t o = poff[k];
+  if (cnt <= kPadTri) {
+    for (int c = l; c < cnt; c += kGroup) {
+      pair_cell[o + c] = (int32_t)k;
+      pair_tri[o + c] = a.ptri[k * kPadTri + c];
+    }
+    return;
   }
-  const int32_t lo = soff[0], hi = soff[64];
-  for (int32_t slot = lo + lane; slot < hi; slot += 64) {
-    int j = 0;  // last cell with soff[j] <= slot (offsets are non-decreasing)
-#pragma unroll
-    for (int step = 32; step > 0; step >>= 1)
-      if (j + step < nk && soff[j + step] <= slot) j += step;
-    if (!skeep[j]) continue;
-    const int c = slot - soff[j];
-    pair_cell[slot] = (int32_t)(k0 + j);
-    pair_tri[slot] = a.ptri[(k0 + j) * kPadTri + c];
-  }
+  const double *bb = a.bbox + 4 * k;
+  group_triangles(a, base, l, bb[0], bb[1], bb[2], bb[3], [&](int32_t ti, int i) {
+    pair_cell[o + i] = (int32_t)k;
+    pair_tri[o + i] = ti;
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -1120,9 +1101,9 @@ struct Integrator : Quad<MODE, R> {
   int nb;
   int bl0, bl1, bl2, bl3;
   R bv0, bv1, bv2, bv3;
-  R *eacc;
+  double *eacc;
   int64_t k;
-  __device__ void commit(int lab, R r) { atomicAdd(&eacc[k * kMaxFast + lab], r); }
+  __device__ void commit(int lab, R r) { atomicAdd(&eacc[k * kMaxFast + lab], (double)r); }
   __device__ void edge(const V &a, int lab, const V &b) {
     if (MODE != 0 || lab < 0) return;
     if (b.x == a.x && b.y == a.y) return;  // zero-length piece from a snapped vertex
@@ -1222,7 +1203,7 @@ __device__ inline void frag_setup(const CellArgs &a, int64_t k, const TriData &t
   s3.init(T.x[2], T.y[2], T.x[0], T.y[0]);
   I.cnt = 0;
   I.nb = 0;
-  I.eacc = CellBuf<R>::eacc(a);
+  I.eacc = a.eacc;
   I.k = k;
 }
 
@@ -1354,7 +1335,8 @@ struct FragPoly {
 // three edges took a different branch on every lane (26 % of the lanes active
 // per instruction, 3700 VALU instructions a wave against 2100 and 47 % here).
 // VALU issue bounds it (77 - 82 % busy).  At 10.4M pairs, before and after:
-// FP64 1.38 and 0.68 ms, FP32 0.86 and 0.70 ms.
+// FP64 1.38 and 0.68 ms, FP32 0.86 and 0.50 ms (0.70 while every workgroup
+// counted its fragments at one address).
 template <int MODE, class R>
 __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,
                                               const int32_t *__restrict__ pair_cell,
@@ -1419,14 +1401,14 @@ __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,
   const bool counted = valid && nout >= 3 && I.positive();
   if (MODE == 0 && counted) {
     // Hessian edge integrals (include/MA/kantorovich.hpp:109-122)
-    R *eacc = CellBuf<R>::eacc(a) + k * kMaxFast;
+    double *eacc = a.eacc + k * kMaxFast;
     for (int i = 0; i < nout; i++) {
       const int lab = F.label(i);
       if (lab == kNoLabel) continue;
       const int i1 = i + 1 == nout ? 0 : i + 1;
       const R ax = F.x(i), ay = F.y(i), bx = F.x(i1), by = F.y(i1);
       if (ax == bx && ay == by) continue;  // zero-length piece from a snapped vertex
-      atomicAdd(&eacc[lab], I.edge(ax, ay, I.rho(ax, ay), bx, by, I.rho(bx, by)));
+      atomicAdd(&eacc[lab], (double)I.edge(ax, ay, I.rho(ax, ay), bx, by, I.rho(bx, by)));
     }
   }
   if (MODE == 1 && a.fo.count != nullptr) {
@@ -1482,7 +1464,7 @@ __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,
     __syncthreads();
     if (t == 0) {
       const int c4 = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
-      if (c4) atomicAdd(&a.counters[0], (unsigned long long)c4);
+      if (c4) atomicAdd(counter_stripe(a.counters, 0, blockIdx.x), (unsigned long long)c4);
     }
     // runs are keyed by cell; uncounted fragments keep their cell's run
     // boundaries (key -2 - k) but contribute nothing
@@ -1586,91 +1568,124 @@ __global__ void __launch_bounds__(256) k_frag_wide(CellArgs a, const int32_t *__
   }
 }
 
-// Hessian row of every fast-path cell (include/MA/kantorovich.hpp:109-122):
+// Hessian rows of the fast-path cells (include/MA/kantorovich.hpp:109-122):
 // H_kj = -int_{e_kj} rho ds / (2 |y_k - y_j|), H_kk = -sum_j H_kj, in FP64.
-// The row is sorted in LDS (per-thread columns [r][t]; private arrays indexed
-// at run time would live in scratch memory) and staged slot-major,
-// fcol[r * n + k], so that k_csr_fill reads it coalesced.
-template <class R>
-__global__ void __launch_bounds__(kRowBlock) k_rows(CellArgs a, double *fval_part, int32_t *row_cnt,
-                                                    int32_t *fcol, double *fval) {
-  __shared__ int32_t lcol[kMaxFast + 1][kRowBlock];
-  __shared__ double lval[kMaxFast + 1][kRowBlock];
-  const int t = (int)threadIdx.x;
-  const int64_t k = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  const int n = (k < a.n) ? a.pn[k] : -1;  // n < 0: the general kernel writes this row
-  unsigned long long my_max = 0, my_empty = 0, my_nv = 0;
-  if (n >= 0) {
-    const int64_t N = a.n;
-    const R *eacc = CellBuf<R>::eacc(a);
-    const double yx = a.pos[2 * k], yy = a.pos[2 * k + 1];
-    auto cols = [&](int r) -> int32_t & { return lcol[r][t]; };
-    auto vals = [&](int r) -> double & { return lval[r][t]; };
-    int nr = 0;
-    double diag = 0.0;
-    for (int v = 0; v < n; v++) {
-      const int32_t j = a.plab[k * kMaxFast + v];
-      const R ei = eacc[k * kMaxFast + v];
-      if (j < 0 || is_neg_zero(ei)) continue;  // edge met by no fragment
-      const double dx = yx - a.pos[2 * j], dy = yy - a.pos[2 * j + 1];
-      const double val = (double)ei / (2.0 * sqrt(dx * dx + dy * dy));
-      diag += val;
-      int p = 0;
-      while (p < nr && cols(p) < j) p++;
-      if (p < nr && cols(p) == j) {
-        vals(p) -= val;
-        continue;
-      }
-      for (int r = nr; r > p; r--) {
-        cols(r) = cols(r - 1);
-        vals(r) = vals(r - 1);
-      }
-      cols(p) = j;
-      vals(p) = -val;
-      nr++;
-    }
-    int cnt = 0;
-    if (nr > 0) {
-      bool placed = false;
-      for (int r = 0; r < nr; r++) {
-        if (!placed && cols(r) > k) {
-          fcol[cnt * N + k] = (int32_t)k;
-          fval[cnt * N + k] = diag;
-          cnt++;
-          placed = true;
-        }
-        fcol[cnt * N + k] = cols(r);
-        fval[cnt * N + k] = vals(r);
-        cnt++;
-      }
-      if (!placed) {
-        fcol[cnt * N + k] = (int32_t)k;
-        fval[cnt * N + k] = diag;
-        cnt++;
-      }
-    }
-    row_cnt[k] = cnt;
-    const double m = a.mass[k];
-    fval_part[k] = (a.wlo ? a.w[k] + a.wlo[k] : a.w[k]) * m - a.intg[k];
-    my_max = (unsigned long long)n;
-    my_empty = (m <= 0.0) ? 1ull : 0ull;
-    my_nv = (unsigned long long)n;
+// The lanes of a group hold the edges of one cell.  k_row_count finds how many
+// entries each row has; once these are scanned, k_row_fill writes the rows
+// into the CSR arrays, each entry at its rank among the labels.  Two short
+// passes over the edges (12 B an edge and pass) instead of sorted rows staged
+// by one thread per cell and copied by another kernel: 1M cells 77 and 112 us
+// against 364 and 104.
+struct RowLane {
+  int l, base;
+  int32_t j = -1;        // neighbour, -1: no entry
+  bool lead = false;     // the first lane with this neighbour
+  __device__ RowLane() : l((int)threadIdx.x & (kGroup - 1)), base((int)threadIdx.x & 48) {}
+  __device__ unsigned mask(bool p) const { return (unsigned)(__ballot(p) >> base) & 0xffffu; }
+  // calls f(o) with o = 1..15 as compile-time constants, for row rotations
+  template <class F>
+  __device__ static void rotations(F &&f) {
+    f(std::integral_constant<int, 1>{}); f(std::integral_constant<int, 2>{});
+    f(std::integral_constant<int, 3>{}); f(std::integral_constant<int, 4>{});
+    f(std::integral_constant<int, 5>{}); f(std::integral_constant<int, 6>{});
+    f(std::integral_constant<int, 7>{}); f(std::integral_constant<int, 8>{});
+    f(std::integral_constant<int, 9>{}); f(std::integral_constant<int, 10>{});
+    f(std::integral_constant<int, 11>{}); f(std::integral_constant<int, 12>{});
+    f(std::integral_constant<int, 13>{}); f(std::integral_constant<int, 14>{});
+    f(std::integral_constant<int, 15>{});
   }
-  __shared__ unsigned long long s_max, s_empty, s_nv;
-  if (threadIdx.x == 0) {
-    s_max = 0;
-    s_empty = 0;
-    s_nv = 0;
+  // edge l of cell k (n vertices); returns its integral (all slots are read,
+  // so that the loads do not wait for n)
+  __device__ double load(const CellArgs &a, int64_t k, int n) {
+    const int32_t label = a.plab[k * kMaxFast + l];
+    const double e = a.eacc[k * kMaxFast + l];
+    // -0.0: edge met by no fragment
+    j = l < n && label >= 0 && !is_neg_zero(e) ? label : -1;
+    const int key = j >= 0 ? j : -1 - l;
+    lead = j >= 0;
+    rotations([&](auto o) {  // lane l sees lane l - o
+      if (dpp<kDppRor + decltype(o)::value>(key) == key && l >= decltype(o)::value) lead = false;
+    });
+    return j >= 0 ? e : 0.0;
+  }
+};
+
+__global__ void __launch_bounds__(kCellThreads) k_row_count(CellArgs a, double *fval_part,
+                                                            int32_t *row_cnt, int per) {
+  int my_max = 0, my_empty = 0, my_nv = 0;
+  const int64_t k0 = ((int64_t)blockIdx.x * kCellGroups + threadIdx.x / kGroup) * per;
+  for (int64_t k = k0; k < min(k0 + per, a.n); k++) {
+    const int n = a.pn[k];
+    RowLane L;
+    (void)L.load(a, k, n);
+    if (n < 0) continue;  // the general kernels write this row's count
+    const int cnt = __popc(L.mask(L.lead));
+    if (L.l == 0) {
+      row_cnt[k] = cnt > 0 ? cnt + 1 : 0;
+      const double m = a.mass[k];
+      fval_part[k] = (a.wlo ? a.w[k] + a.wlo[k] : a.w[k]) * m - a.intg[k];
+      my_max = max(my_max, n);
+      my_empty += m <= 0.0;
+      my_nv += n;
+    }
+  }
+  __shared__ int s_max, s_empty, s_nv;
+  if (threadIdx.x == 0) s_max = s_empty = s_nv = 0;
+  __syncthreads();
+  if ((threadIdx.x & (kGroup - 1)) == 0) {
+    atomicMax(&s_max, my_max);
+    atomicAdd(&s_empty, my_empty);
+    atomicAdd(&s_nv, my_nv);
   }
   __syncthreads();
-  atomicMax(&s_max, my_max);
-  atomicAdd(&s_empty, my_empty);
-  atomicAdd(&s_nv, my_nv);
-  __syncthreads();
   if (threadIdx.x == 0) {
-    atomicMax(&a.counters[2], s_max);
-    atomicAdd(&a.counters[3], s_empty);
-    atomicAdd(&a.counters[4], s_nv);
+    // (the largest cell is soon known, and few cells are empty)
+    if ((unsigned long long)s_max > __hip_atomic_load(&a.counters[2], __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(&a.counters[2], (unsigned long long)s_max);
+    if (s_empty) atomicAdd(&a.counters[3], (unsigned long long)s_empty);
+    atomicAdd(counter_stripe(a.counters, 1, blockIdx.x), (unsigned long long)s_nv);
+  }
+}
+
+__global__ void __launch_bounds__(kCellThreads) k_row_fill(CellArgs a, const int32_t *ptr,
+                                                           int32_t *col, double *val) {
+  const int64_t k = xcd_block<kCellXcdRun>(blockIdx.x, gridDim.x) * kCellGroups +
+                    threadIdx.x / kGroup;
+  if (k >= a.n) return;
+  const int n = a.pn[k];
+  if (n < 0) return;
+  const int32_t o = ptr[k];
+  if (ptr[k + 1] == o) return;
+  RowLane L;
+  const double e = L.load(a, k, n);
+  double v = 0.0;
+  if (L.j >= 0) {
+    const double dx = a.pos[2 * k] - a.pos[2 * L.j], dy = a.pos[2 * k + 1] - a.pos[2 * L.j + 1];
+    v = e / (2.0 * sqrt(dx * dx + dy * dy));
+  }
+  const double diag = row_sum(v);
+  if (L.mask(L.lead != (L.j >= 0))) {
+    // a label on several edges (degenerate edges): their integrals are one entry
+    double s = v;
+    RowLane::rotations([&](auto r) {
+      const int jr = dpp<kDppRor + decltype(r)::value>(L.j);
+      const double vr = dpp<kDppRor + decltype(r)::value>(v);
+      if (jr == L.j) s += vr;
+    });
+    v = s;
+  }
+  const int key = L.lead ? L.j : INT_MAX;
+  int rank = L.lead && L.j > (int32_t)k ? 1 : 0;
+  RowLane::rotations([&](auto r) { rank += dpp<kDppRor + decltype(r)::value>(key) < key; });
+  if (L.lead) {
+    col[o + rank] = L.j;
+    val[o + rank] = -v;
+  }
+  const int below = __popc(L.mask(L.lead && L.j < (int32_t)k));
+  if (L.l == 0) {
+    col[o + below] = (int32_t)k;
+    val[o + below] = diag;
   }
 }
 
@@ -1757,12 +1772,11 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   if (fp32) {
     MA_HIP_TRY(B.pxf.ensure((size_t)kMaxFast * n));
     MA_HIP_TRY(B.pyf.ensure((size_t)kMaxFast * n));
-    MA_HIP_TRY(B.eaccf.ensure((size_t)kMaxFast * n));
   } else {
     MA_HIP_TRY(B.px.ensure((size_t)kMaxFast * n));
     MA_HIP_TRY(B.py.ensure((size_t)kMaxFast * n));
-    MA_HIP_TRY(B.eacc.ensure((size_t)kMaxFast * n));
   }
+  MA_HIP_TRY(B.eacc.ensure((size_t)kMaxFast * n));
   MA_HIP_TRY(B.plab.ensure((size_t)kMaxFast * n));
   MA_HIP_TRY(B.pn.ensure((size_t)n));
   MA_HIP_TRY(B.bbox.ensure((size_t)(4 * n)));
@@ -1797,7 +1811,6 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   if (mode == 3) MA_HIP_TRY(B.mom2_s.ensure((size_t)(3 * n)));
   a.mom2 = mode == 3 ? B.mom2_s.p : nullptr;
   a.eacc = B.eacc.p;
-  a.eaccf = B.eaccf.p;
   a.flags = B.flags.p;
   a.counters = B.counters.p;
   a.force_general = e->force_general;
@@ -1920,8 +1933,8 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   MA_HIP_TRY(hipStreamSynchronize(e->stream));
   MA_HIP_TRY(B.pair_cell.ensure((size_t)np + 1));
   MA_HIP_TRY(B.pair_tri.ensure((size_t)np + 1));
-  hipLaunchKernelGGL(k_pairs, dim3(nblocks(n, 64)), dim3(64), 0, e->stream, a, B.poff.p,
-                     B.pair_cell.p, B.pair_tri.p);
+  hipLaunchKernelGGL(k_pairs, dim3(nblocks(n, kCellGroups)), dim3(kCellThreads), 0, e->stream, a,
+                     B.poff.p, B.pair_cell.p, B.pair_tri.p);
   MA_HIP_TRY(hipEventRecord(e->ev[4], e->stream));
   if (np > 0) {
     // list of the pairs whose fragment outgrows k_frag's staging (count at [np])
@@ -1949,13 +1962,14 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
     }
   }
   MA_HIP_TRY(hipEventRecord(e->ev[5], e->stream));
-  if (mode == 0 && fp32)
-    hipLaunchKernelGGL(k_rows<float>, dim3(nblocks(n, kRowBlock)), dim3(kRowBlock), 0, e->stream, a,
-                       B.fval_part.p, B.row_cnt.p, B.frow_col.p, B.frow_val.p);
-  else if (mode == 0)
-    hipLaunchKernelGGL(k_rows<double>, dim3(nblocks(n, kRowBlock)), dim3(kRowBlock), 0, e->stream, a,
-                       B.fval_part.p, B.row_cnt.p, B.frow_col.p, B.frow_val.p);
-  else if (mode == 1 || mode == 3)  // mode 2 keeps the moments about the Dirac
+  if (mode == 0) {
+    // cells per group: enough workgroups to fill the chip, few enough that
+    // their counters' atomics do not queue up
+    const int per = (int)std::min<int64_t>(8, std::max<int64_t>(1, n / (2048 * kCellGroups)));
+    hipLaunchKernelGGL(k_row_count, dim3(nblocks(n, kCellGroups * per)), dim3(kCellThreads), 0,
+                       e->stream, a, B.fval_part.p, B.row_cnt.p, per);
+  }
+  if (mode == 1 || mode == 3)  // mode 2 keeps the moments about the Dirac
     hipLaunchKernelGGL(k_mom_finalize, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, a,
                        (int)(mode == 3));
   int32_t ng = 0;
@@ -1971,6 +1985,22 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   MA_HIP_TRY(hipGetLastError());
   *npairs_out = np;
   *ngeneral_out = ng;
+  return MA_OK;
+}
+
+// The CSR rows of the fast-path cells of the last run_cells (mode 0), at the
+// offsets csr_ptr.
+ma_status fill_rows(ma_engine *e) {
+  EvalBuffers &B = e->eb;
+  CellArgs a{};
+  a.n = e->n;
+  a.pos = e->pos.p;
+  a.pn = B.pn.p;
+  a.plab = B.plab.p;
+  a.eacc = B.eacc.p;
+  hipLaunchKernelGGL(k_row_fill, dim3(nblocks(e->n, kCellGroups)), dim3(kCellThreads), 0, e->stream, a,
+                     B.csr_ptr.p, B.csr_col.p, B.csr_val.p);
+  MA_HIP_TRY(hipGetLastError());
   return MA_OK;
 }
 

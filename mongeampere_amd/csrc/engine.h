@@ -101,7 +101,16 @@ constexpr int kPadTri = 24;
 // Polygon capacity of the register/LDS fast path (vertices per cell).
 constexpr int kMaxFast = 16;
 constexpr int kMaxLevels = 12;  // levels of the bin grid above the bins
-constexpr int kRowBlock = 128;  // threads per block of k_rows (its LDS rows)
+
+// Event counts that every workgroup adds to are striped over 16 cache lines
+// (one address takes an atomic every 8 ns or so): stripe `b` mod 16 of count
+// `which` (0: fragments, 1: vertices) behind the plain counters.
+constexpr int kPlainCounters = 16, kCounterStripes = 16;
+constexpr int kCounters = kPlainCounters + 2 * kCounterStripes * 16;
+__host__ __device__ inline unsigned long long *counter_stripe(unsigned long long *counters,
+                                                              int which, unsigned b) {
+  return counters + kPlainCounters + (which * kCounterStripes + (b % kCounterStripes)) * 16;
+}
 
 // Fragment polygons written out by the first-moment kernels while `count` is
 // set (ma_fragments).  Each fragment of positive area reserves one record and
@@ -161,16 +170,15 @@ struct EvalBuffers {
   DBuf<int32_t> row_cnt;     // per Dirac, entries incl. diagonal
   DBuf<int32_t> row_col;     // n x cap_row (rows of the general kernels)
   DBuf<double> row_val;      // n x cap_row
-  DBuf<int32_t> frow_col;    // fast-path rows, slot-major [r * n + k], r <= kMaxFast
-  DBuf<double> frow_val;
   DBuf<int32_t> csr_ptr, csr_col;   // Morton-order CSR
   DBuf<double> csr_val;
-  DBuf<double> diag;
   DBuf<int32_t> flags;       // [0] overflow poly,
                              // [3] cells for the general kernels
   DBuf<unsigned long long> counters;  // [0] fragments, [1] candidates, [2] max poly, [3] empty,
                                       // [4] vertices, [5] FP64 re-decisions, [6] bin-path cells,
-                                      // [7] failing cell (k_cell_huge), [8] long rows
+                                      // [7] failing cell (k_cell_huge), [8] long rows;
+                                      // more fragments and vertices in the stripes
+                                      // (counter_stripe)
   // per-wave event counts of the cell kernel, striped over 16 cache lines
   // (kStripes counters of 16 words each) so that no single address takes
   // an atomic from every wave: [0..15] cells that walked the pyramid,
@@ -181,7 +189,7 @@ struct EvalBuffers {
   DBuf<double> red_tmp;
   // register/LDS fast path
   DBuf<double> px, py, eacc, bbox;
-  DBuf<float> pxf, pyf, eaccf;   // FP32 polygons and edge integrals (mixed mode)
+  DBuf<float> pxf, pyf;          // FP32 polygons (mixed mode)
   DBuf<int32_t> plab, pn, tcount, poff, pair_cell, pair_tri, glist;
   DBuf<int32_t> cstage;  // the first candidates of every bin, kept by the counting walk
   DBuf<int32_t> ptri;         // kPadTri candidate triangles per cell, [k * kPadTri + c]

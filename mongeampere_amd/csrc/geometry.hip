@@ -1674,32 +1674,17 @@ __global__ void __launch_bounds__(kHugeBlock) k_cell_huge(
   }
 }
 
-// Rows longer than cap_row (from k_cell_huge) are read from the long-row
-// staging at the slot stored in their first regular entry.
-// CSR rows from the staged rows: fast-path cells (pn >= 0) slot-major in
-// frow_*, rows of the general kernels per Dirac in row_* (or, past cap_row
-// entries, in the long-row pool hrow_*).
+// CSR rows of the cells evaluated by the general kernels (pn < 0), staged per
+// Dirac in row_*; rows longer than cap_row entries (from k_cell_huge) are read
+// from the long-row pool hrow_* at the slot stored in their first entry.
 __global__ void k_csr_fill(int64_t n, const int32_t *pn, const int32_t *row_cnt,
-                           const int32_t *frow_col, const double *frow_val,
                            const int32_t *row_col, const double *row_val, int cap_row,
                            const int32_t *hrow_col, const double *hrow_val, const int32_t *ptr,
-                           int32_t *col, double *val, double *diag) {
+                           int32_t *col, double *val) {
   const int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k >= n) return;
+  if (k >= n || pn[k] >= 0) return;
   const int c = row_cnt[k];
   const int32_t o = ptr[k];
-  double d = 0.0;
-  if (pn[k] >= 0) {
-    for (int i = 0; i < c; i++) {
-      const int32_t j = frow_col[i * n + k];
-      const double v = frow_val[i * n + k];
-      col[o + i] = j;
-      val[o + i] = v;
-      if (j == k) d = v;
-    }
-    diag[k] = d;
-    return;
-  }
   const int32_t *rc = row_col + k * (int64_t)cap_row;
   const double *rv = row_val + k * (int64_t)cap_row;
   if (c > cap_row) {
@@ -1708,13 +1693,9 @@ __global__ void k_csr_fill(int64_t n, const int32_t *pn, const int32_t *row_cnt,
     rv = hrow_val + s * kHugeRow;
   }
   for (int i = 0; i < c; i++) {
-    const int32_t j = rc[i];
-    const double v = rv[i];
-    col[o + i] = j;
-    val[o + i] = v;
-    if (j == k) d = v;
+    col[o + i] = rc[i];
+    val[o + i] = rv[i];
   }
-  diag[k] = d;
 }
 
 // Deterministic two-stage sum: partials per block, then one block.
@@ -1745,6 +1726,7 @@ hipError_t device_sum(ma_engine *e, const double *x, int64_t n, double *d_out) {
 // One evaluation.
 // ---------------------------------------------------------------------------
 ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out, int32_t *ngeneral_out);
+ma_status fill_rows(ma_engine *e);
 ma_status refine_candidates(ma_engine *e, int64_t total);
 
 // Candidate owners of every domain bin (of the bins with mask[b] set, when
@@ -1839,13 +1821,8 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
   MA_HIP_TRY(B.fval_part.ensure((size_t)n));
   MA_HIP_TRY(B.mom_s.ensure((size_t)(2 * n)));
   MA_HIP_TRY(B.row_cnt.ensure((size_t)n + 1));
-  MA_HIP_TRY(B.row_col.ensure((size_t)n * e->cap_row));
-  MA_HIP_TRY(B.row_val.ensure((size_t)n * e->cap_row));
-  MA_HIP_TRY(B.frow_col.ensure((size_t)n * (kMaxFast + 1)));
-  MA_HIP_TRY(B.frow_val.ensure((size_t)n * (kMaxFast + 1)));
   MA_HIP_TRY(B.flags.ensure(4));
-  MA_HIP_TRY(B.counters.ensure(12));
-  MA_HIP_TRY(B.diag.ensure((size_t)n));
+  MA_HIP_TRY(B.counters.ensure(kCounters));
   MA_HIP_TRY(B.red_tmp.ensure(2048));
   if (!e->owner_init) {
     hipLaunchKernelGGL(k_fill_i32, dim3(nblocks(g.nbins)), dim3(kBlock), 0, e->stream,
@@ -1867,11 +1844,15 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
   }
   MA_HIP_TRY(hipEventRecord(e->ev[1], e->stream));
   MA_HIP_TRY(hipMemsetAsync(B.flags.p, 0, sizeof(int32_t) * 4, e->stream));
-  MA_HIP_TRY(hipMemsetAsync(B.counters.p, 0, sizeof(unsigned long long) * 12, e->stream));
+  MA_HIP_TRY(hipMemsetAsync(B.counters.p, 0, sizeof(unsigned long long) * kCounters, e->stream));
   MA_HIP_TRY(hipEventRecord(e->ev[2], e->stream));
   int32_t npairs = 0, ngen = 0;
   ma_status cs = run_cells(e, mode, fp32, &npairs, &ngen);
   if (cs != MA_OK) return cs;
+  if (ngen > 0 && mode == 0) {  // staging of the general kernels' rows
+    MA_HIP_TRY(B.row_col.ensure((size_t)n * e->cap_row));
+    MA_HIP_TRY(B.row_val.ensure((size_t)n * e->cap_row));
+  }
   int32_t nhuge = 0;
   const int32_t *hl = nullptr;  // list of the cells for k_cell_huge
   if (ngen > 0 && ((ngen <= kHugeRoute && e->force_general != 1) || e->fo.count != nullptr)) {
@@ -1927,17 +1908,19 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
     MA_HIP_TRY(hipStreamSynchronize(e->stream));
     MA_HIP_TRY(B.csr_col.ensure((size_t)nnz + 1));
     MA_HIP_TRY(B.csr_val.ensure((size_t)nnz + 1));
-    hipLaunchKernelGGL(k_csr_fill, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, B.pn.p,
-                       B.row_cnt.p, B.frow_col.p, B.frow_val.p, B.row_col.p, B.row_val.p,
-                       e->cap_row, B.hrow_col.p, B.hrow_val.p, B.csr_ptr.p, B.csr_col.p,
-                       B.csr_val.p, B.diag.p);
+    const ma_status rs = fill_rows(e);
+    if (rs != MA_OK) return rs;
+    if (ngen > 0)
+      hipLaunchKernelGGL(k_csr_fill, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, B.pn.p,
+                         B.row_cnt.p, B.row_col.p, B.row_val.p, e->cap_row, B.hrow_col.p,
+                         B.hrow_val.p, B.csr_ptr.p, B.csr_col.p, B.csr_val.p);
     MA_HIP_TRY(device_sum(e, B.fval_part.p, n, B.red_tmp.p + 1024));
     e->nnz = nnz;  // sizes the CSR buffers now holding this pass's rows
   }
   MA_HIP_TRY(hipEventRecord(e->ev[7], e->stream));
   MA_HIP_TRY(hipGetLastError());
   int32_t fl[4];
-  unsigned long long ct[8];
+  unsigned long long ct[kCounters];
   double fv = 0.0;
   MA_HIP_TRY(hipMemcpyAsync(fl, B.flags.p, sizeof fl, hipMemcpyDeviceToHost, e->stream));
   MA_HIP_TRY(hipMemcpyAsync(ct, B.counters.p, sizeof ct, hipMemcpyDeviceToHost, e->stream));
@@ -1959,6 +1942,10 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
   e->info.ms_cells = t[2] + t[3] + t[4] + t[5];
   e->info.ms_assemble = t[6];
   e->info.ms_total = t[0] + t[1] + t[2] + t[3] + t[4] + t[5] + t[6];
+  for (int b = 0; b < kCounterStripes; b++) {
+    ct[0] += *counter_stripe(ct, 0, b);
+    ct[4] += *counter_stripe(ct, 1, b);
+  }
   e->info.nfrag = (int64_t)ct[0];
   e->info.ncand = (int64_t)ct[1];
   e->info.max_poly = (int64_t)ct[2];
