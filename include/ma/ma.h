@@ -325,7 +325,7 @@ typedef enum {
   MA_OPT_CAP_CAND = 2,
   MA_OPT_GRAPHS = 3,
   MA_OPT_LOCAL_RINGS = 4, /* rings of bins searched around each Dirac (0..64, default 8) */
-  MA_OPT_WALK_BUDGET = 5, /* pyramid nodes per cell before the bin path (default 512) */
+  MA_OPT_WALK_BUDGET = 5, /* pyramid nodes per cell before the bin path (default 1024) */
   MA_OPT_AMG_OMEGA = 6,   /* multigrid Jacobi damping in 1/1000 (100..1000, default 850) */
   MA_OPT_AMG_CORR = 7,    /* coarse-correction scaling in 1/1000 (500..3000, default 1500) */
   MA_OPT_AMG_SWEEPS = 8,  /* Jacobi sweeps before and after the coarse correction (1 or 2, default 1) */

@@ -523,6 +523,15 @@ __device__ inline bool far_enough(double D2, double rho2, double W, double wk) {
   return D2 > rho2 && t > 0.0 && t * t > 4.0 * rho2 * D2;
 }
 
+// From ring kWalkFrom on, a cell whose bound needs kWalkAhead more rings and
+// more than kWalkWeight radii (2 at equal weights: a wide polygon alone is
+// better served by the next ring) walks the pyramid instead.  Cell kernel at 1M
+// Diracs displaced by up to 1, 2 and 3 bins: 3.34, 3.64, 3.86 ms, against 3.35,
+// 4.63, 5.24 ms after all 8 rings and 3.26, 3.77, 4.06 ms after 4; at w = 0 and
+// up to half a bin those who walk early lose (2.57 against 2.16 ms after 4).
+constexpr int kWalkFrom = 3;
+constexpr float kWalkAhead = 4.0f, kWalkWeight = 2.5f;
+
 // Multi-level certificate for the polygon (squared radius rho2 about y_k) once
 // the bins within Chebyshev distance r of the Dirac's bin have been visited.
 // At level l the 3 x 3 block of level-l nodes around the Dirac's node contains
@@ -530,11 +539,12 @@ __device__ inline bool far_enough(double D2, double rho2, double W, double wk) {
 // lie at least as far as the boundary of the covered region (the block one
 // level down, or the visited square) and weigh at most the block's maximum
 // (pyr3).  Blocks are nested and the top one is the whole grid, so every
-// unvisited Dirac is bounded once.  Lane l takes level l.
+// unvisited Dirac is bounded once.  Lane l takes level l.  When some level
+// fails, `need` gets the distance (bins) at which its bound would hold.
 template <class R>
 __device__ inline bool certify_levels(const Grid &g, const double *pyr3, const PyrOff &off, int sbx,
                                       int sby, int r, double yx, double yy, const Cell<R> &C,
-                                      double wk) {
+                                      double wk, float &need) {
   static_assert(kMaxLevels < kGroup, "one lane per level");
   const int G = g.G, l = C.l;
   const int vx0 = max(sbx - r, 0), vx1 = min(sbx + r, G - 1);
@@ -548,6 +558,7 @@ __device__ inline bool certify_levels(const Grid &g, const double *pyr3, const P
     return x0 <= vx0 && x1 >= vx1 && y0 <= vy0 && y1 >= vy1;  // holds the visited square
   };
   bool ok = true;
+  float dist = 0.0f;
   int bx0, by0, bx1, by1;
   if (l <= g.L && block(l, bx0, by0, bx1, by1)) {
     int x0 = vx0, y0 = vy0, x1 = vx1, y1 = vy1;
@@ -562,9 +573,15 @@ __device__ inline bool certify_levels(const Grid &g, const double *pyr3, const P
     if (D != kInf) {
       const double Wb = pyr3[off.o[l] + morton2((uint32_t)(sbx >> l), (uint32_t)(sby >> l))];
       ok = Wb == -kInf || (D > 0.0 && far_enough(D * D, C.rho2(), Wb, wk));
+      if (!ok && r >= kWalkFrom) {
+        const float dw = (float)((Wb - wk) * (C.ih * C.ih));
+        dist = __builtin_amdgcn_sqrtf(C.rb) + __builtin_amdgcn_sqrtf(fmaxf(C.rb + dw, 0.0f));
+      }
     }
   }
-  return C.mask(!ok) == 0u;
+  if (C.mask(!ok) == 0u) return true;
+  need = r >= kWalkFrom ? row_max_nonneg(dist) : 0.0f;
+  return false;
 }
 
 // -0.0 exactly (an edge integral no fragment has touched)
@@ -581,6 +598,43 @@ __device__ inline void wave_count(T *dst, bool flag) {
     atomicAdd(dst, (T)__popcll(bal));
 }
 
+// Whether some Dirac j of a pyramid node may cut the polygon C of the Dirac at
+// (cx, cy) (about the grid's centre): with Y = y_j - y_k in the node's box [x0,
+// x0 + side] x [y0, y0 + side] (bins, from the Dirac) and the node's plane,
+//   pi_j - pi_k = |Y|^2 + w_k - w_j - 2 X.Y
+//               >= b + a.y_k - |y_k|^2 + w_k + (a - 2 y_k - 2 X).Y  at a vertex X,
+// in FP32 and bins, with the rounding of its terms allowed for.  One lane tests
+// one node against all vertices of its group's polygon.
+template <class R>
+__device__ inline bool node_reaches(const Plane &p, const Cell<R> &C, double wk, double cx,
+                                    double cy, float x0, float y0, float side) {
+  const double ih2 = C.ih * C.ih, d = p.ax * cx + p.ay * cy, q = cx * cx + cy * cy;
+  const float c0 = (float)((p.b + d - q + wk) * ih2);
+  const float gx = (float)((p.ax - 2.0 * cx) * C.ih), gy = (float)((p.ay - 2.0 * cy) * C.ih);
+  const float x1 = x0 + side, y1 = y0 + side;
+  const float vx = (float)(C.x * (R)C.ih), vy = (float)(C.y * (R)C.ih);
+  float m = INFINITY;
+#define MA_VERTEX(v)                                                       \
+  {                                                                        \
+    const float tx = gx - 2.0f * dpp<kDppBcast + v>(vx);                   \
+    const float ty = gy - 2.0f * dpp<kDppBcast + v>(vy);                   \
+    m = fminf(m, fminf(tx * x0, tx * x1) + fminf(ty * y0, ty * y1));       \
+  }
+  MA_VERTEX(0) MA_VERTEX(1) MA_VERTEX(2) MA_VERTEX(3) MA_VERTEX(4) MA_VERTEX(5)
+  if (C.n > 6) {
+    MA_VERTEX(6) MA_VERTEX(7) MA_VERTEX(8)
+    if (C.n > 9) {
+      MA_VERTEX(9) MA_VERTEX(10) MA_VERTEX(11) MA_VERTEX(12) MA_VERTEX(13) MA_VERTEX(14)
+      MA_VERTEX(15)
+    }
+  }
+#undef MA_VERTEX
+  const float far = fmaxf(fabsf(x0), fabsf(x1)) + fmaxf(fabsf(y0), fabsf(y1));
+  const float err = 2e-6f * (fabsf(c0) + (fabsf(gx) + fabsf(gy) + 2.0f * __builtin_amdgcn_sqrtf(C.rb)) * far) +
+                    (float)(1e-14 * (fabs(p.b) + fabs(d) + q + fabs(wk)) * ih2);
+  return !(c0 + m > err);
+}
+
 // Site-centric construction: the starting box is clipped by the Diracs of the
 // bins in Chebyshev rings 0..rmax around the Dirac's own bin (rings 0 and 1
 // together).  A lane takes a bin; from ring 2 on a bin whose maximum weight
@@ -594,8 +648,9 @@ __device__ inline void wave_count(T *dst, bool flag) {
 // every pruned Dirac stays unable to cut the final cell.
 template <class R>
 __global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const double *pyr,
-                                                             const double *pyr3, PyrOff off,
-                                                             int rmax) {
+                                                             const double *pyr3,
+                                                             const Plane *__restrict__ planes,
+                                                             PyrOff off, int rmax) {
   __shared__ uint32_t stacks[kCellGroups][kWalkStack];
   const int64_t k = xcd_block<kCellXcdRun>(blockIdx.x, gridDim.x) * kCellGroups +
                     threadIdx.x / kGroup;
@@ -665,8 +720,13 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const d
       clip_ranges<float, false>(a, k, yx, yy, wk, lo, cnt, nullptr, C, fail);
     }
     if (C.n == 0 || fail) break;
-    if (certify_levels(g, pyr3, off, sbx, sby, r, yx, yy, C, wk)) {
+    float need = 0.0f;
+    if (certify_levels(g, pyr3, off, sbx, sby, r, yx, yy, C, wk, need)) {
       certified = true;
+      break;
+    }
+    if (need > (float)r + kWalkAhead && need > kWalkWeight * __builtin_amdgcn_sqrtf(C.rb)) {
+      r++;  // many more rings, because of the weights: the walk is cheaper
       break;
     }
   }
@@ -674,11 +734,15 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const d
   bool over_budget = false;
   if (walk) {
     // bins [sbx - rr, sbx + rr] x [sby - rr, sby + rr] have been visited
-    const int rr = min(r, rmax);
+    const int rr = r - 1;
     const int vx0 = sbx - rr, vx1 = sbx + rr, vy0 = sby - rr, vy1 = sby + rr;
     uint32_t *stack = stacks[threadIdx.x / kGroup];
     int sp = 0, visits = 0;
     uint32_t ent = (uint32_t)g.L << 27;
+    // position about the grid's centre, and in bins from its corner
+    const double half = 0.5 * g.h * (double)g.G;
+    const double cx = yx - g.x0 - half, cy = yy - g.y0 - half;
+    const double bx = (yx - g.x0) * C.ih, by = (yy - g.y0) * C.ih;
     while (true) {
       const int lev = (int)(ent >> 27), st = min(lev, 2), cl = lev - st;
       const uint32_t ch = ((ent & ((1u << 27) - 1u)) << (2 * st)) | (uint32_t)l;
@@ -693,20 +757,26 @@ __global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const d
       bool descend = false;
       int32_t lo = 0;
       int cnt = 0;
-      if (l < nch) {
-        const int nx = (int)(compact1by1(ch) << cl), ny = (int)(compact1by1(ch >> 1) << cl);
-        const int sd = 1 << cl;
-        if (!(nx >= vx0 && nx + sd - 1 <= vx1 && ny >= vy0 && ny + sd - 1 <= vy1)) {
-          const double W = pyr[off.o[cl] + ch];
-          if (W != -kInf && !far_enough(dist2(nx, ny, cl), C.rho2(), W, wk)) {
-            // the Diracs of a node are one contiguous Morton range: a node
-            // holding few of them (sparse regions) is taken whole
-            lo = a.bin_start[(int64_t)ch << (2 * cl)];
-            cnt = a.bin_start[((int64_t)ch + 1) << (2 * cl)] - lo;
-            if (cl > 0 && cnt > kNodeDiracs) {
-              descend = true;
-              cnt = 0;
-            }
+      const int nx = (int)(compact1by1(ch) << cl), ny = (int)(compact1by1(ch >> 1) << cl);
+      const int sd = 1 << cl;
+      bool live = l < nch && !(nx >= vx0 && nx + sd - 1 <= vx1 && ny >= vy0 && ny + sd - 1 <= vy1);
+      if (live) {
+        const double W = pyr[off.o[cl] + ch];
+        live = W != -kInf && !far_enough(dist2(nx, ny, cl), C.rho2(), W, wk);
+      }
+      if (C.mask(live)) {
+        const Plane p = live ? planes[off.o[cl] + ch] : Plane{0.0, 0.0, 0.0, 0.0};
+        // (every lane of the group takes part: it reads their vertices)
+        const bool reaches =
+            node_reaches(p, C, wk, cx, cy, (float)(nx - bx), (float)(ny - by), (float)sd);
+        if (live && reaches) {
+          // the Diracs of a node are one contiguous Morton range: a node
+          // holding few of them (sparse regions) is taken whole
+          lo = a.bin_start[(int64_t)ch << (2 * cl)];
+          cnt = a.bin_start[((int64_t)ch + 1) << (2 * cl)] - lo;
+          if (cl > 0 && cnt > kNodeDiracs) {
+            descend = true;
+            cnt = 0;
           }
         }
       }
@@ -1838,13 +1908,14 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   const int32_t zero = 0;
   PyrOff po{};
   for (int l = 0; l <= e->grid.L; l++) po.o[l] = e->pyr_off[l];
+  const Plane *planes = reinterpret_cast<const Plane *>(B.plane.p);
   MA_HIP_TRY(hipEventRecord(e->ev[10], e->stream));
   if (fp32)
     hipLaunchKernelGGL(k_cell_local<float>, dim3(nblocks(n, kCellGroups)), dim3(kCellThreads), 0,
-                       e->stream, a, B.pyr.p, B.pyr3.p, po, e->local_rings);
+                       e->stream, a, B.pyr.p, B.pyr3.p, planes, po, e->local_rings);
   else
     hipLaunchKernelGGL(k_cell_local<double>, dim3(nblocks(n, kCellGroups)), dim3(kCellThreads), 0,
-                       e->stream, a, B.pyr.p, B.pyr3.p, po, e->local_rings);
+                       e->stream, a, B.pyr.p, B.pyr3.p, planes, po, e->local_rings);
   MA_HIP_TRY(hipEventRecord(e->ev[11], e->stream));
   {
     int32_t fl0[4];

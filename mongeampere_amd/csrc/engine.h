@@ -94,7 +94,7 @@ constexpr int kLongRows = 1024;  // pool of staged rows longer than kMaxRow
 // and pyramid nodes a cell may visit before it is left to the bin path
 // (defaults; MA_OPT_LOCAL_RINGS / MA_OPT_WALK_BUDGET).
 constexpr int kLocalRings = 8;
-constexpr int kWalkBudget = 512;
+constexpr int kWalkBudget = 1024;
 // Candidate triangles per cell kept by the cell kernels for the pair list
 // (cells with more are scanned again).
 constexpr int kPadTri = 24;
@@ -159,7 +159,7 @@ struct EvalBuffers {
   DBuf<int32_t> cbin;        // bin of each candidate entry (before refinement)
   DBuf<int32_t> ckeep;       // keep flags of the entries, then their prefix sums
   DBuf<int32_t> cand2, cstart2;  // refined lists (swapped with cand / cand_cnt)
-  DBuf<double> plane;        // plane pyramid (4 per node) and its sums, built with the lists
+  DBuf<double> plane;        // plane pyramid (4 per node) and its sums
   DBuf<double> node_sums;
   DBuf<int32_t> owner;       // per bin, best competitor of the last evaluation
   DBuf<int32_t> rect;        // per Dirac: bin rectangle (x0, y0, x1, y1)

@@ -286,22 +286,21 @@ hipError_t build_triangle_bins(ma_engine *e) {
 }
 
 // ---------------------------------------------------------------------------
-// Max-weight pyramid: level 0 = bins, level l node m covers the 4^l bins with
-// Morton codes [m 4^l, (m+1) 4^l).  Empty nodes hold -inf.
+// Pyramids over the bins: level l node m covers the 4^l bins with Morton codes
+// [m 4^l, (m+1) 4^l).  pyr: the largest weight of the node's Diracs (-inf: no
+// Diracs); pyr3: the largest over the 3 x 3 nodes around it; and the planes
+// (lanes.h).
 // ---------------------------------------------------------------------------
-__global__ void k_pyr_leaf(const int32_t *bin_start, const double *w, int64_t nb, double *lvl0) {
-  int64_t b = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (b >= nb) return;
-  double m = -kInf;
-  for (int32_t q = bin_start[b]; q < bin_start[b + 1]; q++) m = fmax(m, w[q]);
-  lvl0[b] = m;
-}
-// Neighbourhood maxima: out[m] = max of lvl over the 3 x 3 nodes around node
-// m of a level with `side` nodes per side.
-__global__ void k_pyr3(const double *lvl, int side, int64_t nn, double *out) {
-  const int64_t m = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (m >= nn) return;
-  const int x = (int)compact1by1((uint32_t)m), y = (int)compact1by1((uint32_t)(m >> 1));
+// Neighbourhood maxima, all levels in one launch.
+__global__ void k_pyr3(Grid g, PyrOff off, int64_t nodes, const double *__restrict__ pyr,
+                       double *out) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= nodes) return;
+  int l = 0;
+  while (l < g.L && i >= off.o[l + 1]) l++;
+  const double *lvl = pyr + off.o[l];
+  const uint32_t m = (uint32_t)(i - off.o[l]);
+  const int side = g.G >> l, x = (int)compact1by1(m), y = (int)compact1by1(m >> 1);
   double v = -kInf;
   for (int dy = -1; dy <= 1; dy++)
     for (int dx = -1; dx <= 1; dx++) {
@@ -309,55 +308,9 @@ __global__ void k_pyr3(const double *lvl, int side, int64_t nn, double *out) {
       if (xx >= 0 && xx < side && yy >= 0 && yy < side)
         v = fmax(v, lvl[morton2((uint32_t)xx, (uint32_t)yy)]);
     }
-  out[m] = v;
-}
-__global__ void k_pyr_up(const double *lo, double *hi, int64_t nhi) {
-  int64_t m = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (m >= nhi) return;
-  hi[m] = fmax(fmax(lo[4 * m], lo[4 * m + 1]), fmax(lo[4 * m + 2], lo[4 * m + 3]));
+  out[i] = v;
 }
 
-// ---------------------------------------------------------------------------
-// Plane pyramid.  With coordinates about the grid's centre and v_j = |y_j|^2 -
-// w_j, pi_j(x) = |x|^2 + v_j - 2 x.y_j.  A node keeps a gradient a and b = min
-// over its Diracs of v_j - a.y_j (a lower bound of it above level 0), so that
-//   min_j v_j - 2 x.y_j >= b + min over the node's box of (a - 2 x).y.
-// Where the weights vary smoothly a is close to 2 x for the points x that the
-// node's Diracs own, and the bound is tight to the square of the node's side.
-// (The bound of the max-weight pyramid, dist^2(x, node) - max w, is loose by
-// four times the distance from a Dirac to its cell times the node's side:
-// with clustered Diracs a search for the owners of one bin then met about 500
-// Diracs instead of 10.)
-// a = 2 (centre of the node) - gw, gw the gradient of the weights by least
-// squares over the 16 grandchildren of the node's even-level ancestor.
-// ---------------------------------------------------------------------------
-struct Plane {
-  double ax, ay, b, pad;
-};
-// Diracs of an even-level node: number, sums of y and w.
-struct NodeSums {
-  double n, x, y, w;
-};
-struct NodeBox {
-  double x0, y0, x1, y1;
-};
-__device__ inline NodeBox node_box(const Grid &g, uint32_t m, int lev) {
-  const double side = g.h * (double)(1u << lev), half = 0.5 * g.h * (double)g.G;
-  NodeBox q;
-  q.x0 = compact1by1(m) * side - half;
-  q.y0 = compact1by1(m >> 1) * side - half;
-  q.x1 = q.x0 + side;
-  q.y1 = q.y0 + side;
-  return q;
-}
-// min of t.y over the box; mag gets the magnitude of its terms
-__device__ inline double box_min(const NodeBox &q, double tx, double ty, double &mag) {
-  const double px = tx > 0.0 ? q.x0 : q.x1, py = ty > 0.0 ? q.y0 : q.y1;
-  mag = fabs(tx * px) + fabs(ty * py);
-  return tx * px + ty * py;
-}
-// rounding allowance of a bound: its terms carry errors of a few 1e-16
-constexpr double kPlaneEps = 1e-13;
 // lower bound of v_j - 2 x.y_j over the node's Diracs, rounding allowed for
 __device__ inline double plane_bound(const Plane &p, const NodeBox &q, double x, double y) {
   double mag;
@@ -367,12 +320,14 @@ __device__ inline double plane_bound(const Plane &p, const NodeBox &q, double x,
 
 // One group per node of level lev + 2 (lev + 1 when that is the top: step 1);
 // lane c takes its descendant c of level lev.  lev = 0: from the Diracs of the
-// bins; above: from the records of level lev.
+// bins; above: from the records of level lev.  Writes planes and largest
+// weights.
 __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int step,
                                                         const int32_t *__restrict__ bin_start,
                                                         const double *__restrict__ pos,
                                                         const double *__restrict__ w, PyrOff off,
-                                                        Plane *pl, NodeSums *sums) {
+                                                        Plane *pl, NodeSums *sums,
+                                                        double *pyr) {
   const int top = lev + step;
   const int64_t node = blockIdx.x * (int64_t)kCellGroups + threadIdx.x / kGroup;
   if (node >= (int64_t)1 << (2 * (g.L - top))) return;
@@ -381,6 +336,7 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
   const uint32_t m = ((uint32_t)node << (2 * step)) | (uint32_t)(on ? l : 0);
   const double hx = g.x0 + 0.5 * g.h * g.G, hy = g.y0 + 0.5 * g.h * g.G;
   NodeSums s{0.0, 0.0, 0.0, 0.0};
+  double W = -kInf;  // largest weight
   int32_t q0 = 0, q1 = 0;
   if (on && lev == 0) {
     q0 = bin_start[m];
@@ -389,10 +345,13 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
       s.x += pos[2 * q] - hx;
       s.y += pos[2 * q + 1] - hy;
       s.w += w[q];
+      W = fmax(W, w[q]);
     }
     s.n = (double)(q1 - q0);
+    pyr[off.o[0] + m] = W;
   } else if (on) {
     s = sums[off.o[lev] + m];
+    W = pyr[off.o[lev] + m];
   }
   // gradient of the weights: least squares over the lanes' means
   const double N = row_sum(s.n), Sx = row_sum(s.x), Sy = row_sum(s.y), Sw = row_sum(s.w);
@@ -445,7 +404,12 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
     t = fmin(t, row_get(t, base4, l ^ st));
     t = fmin(t, row_get(t, base4, l ^ (2 * st)));
     u.b = t;
-    if (on && (l & (4 * st - 1)) == 0) pl[off.o[lev + k] + mm] = u;
+    W = fmax(W, row_get(W, base4, l ^ st));
+    W = fmax(W, row_get(W, base4, l ^ (2 * st)));
+    if (on && (l & (4 * st - 1)) == 0) {
+      pl[off.o[lev + k] + mm] = u;
+      pyr[off.o[lev + k] + mm] = W;
+    }
     p = u;
     q = up;
   }
@@ -1738,16 +1702,7 @@ ma_status run_bin_candidates(ma_engine *e, const int32_t *pn, const unsigned cha
   EvalBuffers &B = e->eb;
   PyrOff po{};
   for (int l = 0; l <= g.L; l++) po.o[l] = e->pyr_off[l];
-  const int64_t nodes = e->pyr_off[g.L] + 1;
-  MA_HIP_TRY(B.plane.ensure((size_t)(4 * nodes)));
-  MA_HIP_TRY(B.node_sums.ensure((size_t)(4 * nodes)));
-  Plane *pl = reinterpret_cast<Plane *>(B.plane.p);
-  for (int lev = 0; lev < g.L || lev == 0; lev += 2) {
-    const int step = std::min(2, g.L - lev);
-    hipLaunchKernelGGL(k_plane, dim3(nblocks((int64_t)1 << (2 * (g.L - lev - step)), kCellGroups)),
-                       dim3(kCellThreads), 0, e->stream, g, lev, step, e->bin_start.p, e->pos.p,
-                       B.w_s.p, po, pl, reinterpret_cast<NodeSums *>(B.node_sums.p));
-  }
+  const Plane *pl = reinterpret_cast<const Plane *>(B.plane.p);
   MA_HIP_TRY(B.cand_cnt.ensure((size_t)g.nbins + 1));
   const int32_t zero = 0;
   int32_t total = 0;
@@ -1830,18 +1785,17 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
     e->owner_init = true;
   }
   MA_HIP_TRY(hipEventRecord(e->ev[0], e->stream));
-  hipLaunchKernelGGL(k_pyr_leaf, dim3(nblocks(g.nbins)), dim3(kBlock), 0, e->stream,
-                     e->bin_start.p, B.w_s.p, g.nbins, B.pyr.p);
-  for (int l = 1; l <= g.L; l++) {
-    int64_t nh = (int64_t)1 << (2 * (g.L - l));
-    hipLaunchKernelGGL(k_pyr_up, dim3(nblocks(nh)), dim3(kBlock), 0, e->stream,
-                       B.pyr.p + e->pyr_off[l - 1], B.pyr.p + e->pyr_off[l], nh);
+  MA_HIP_TRY(B.plane.ensure((size_t)(4 * tot)));
+  MA_HIP_TRY(B.node_sums.ensure((size_t)(4 * tot)));
+  for (int lev = 0; lev < g.L || lev == 0; lev += 2) {
+    const int step = std::min(2, g.L - lev);
+    hipLaunchKernelGGL(k_plane, dim3(nblocks((int64_t)1 << (2 * (g.L - lev - step)), kCellGroups)),
+                       dim3(kCellThreads), 0, e->stream, g, lev, step, e->bin_start.p, e->pos.p,
+                       B.w_s.p, po, reinterpret_cast<Plane *>(B.plane.p),
+                       reinterpret_cast<NodeSums *>(B.node_sums.p), B.pyr.p);
   }
-  for (int l = 0; l <= g.L; l++) {
-    const int64_t nn = (int64_t)1 << (2 * (g.L - l));
-    hipLaunchKernelGGL(k_pyr3, dim3(nblocks(nn)), dim3(kBlock), 0, e->stream,
-                       B.pyr.p + e->pyr_off[l], g.G >> l, nn, B.pyr3.p + e->pyr_off[l]);
-  }
+  hipLaunchKernelGGL(k_pyr3, dim3(nblocks(tot)), dim3(kBlock), 0, e->stream, g, po, tot, B.pyr.p,
+                     B.pyr3.p);
   MA_HIP_TRY(hipEventRecord(e->ev[1], e->stream));
   MA_HIP_TRY(hipMemsetAsync(B.flags.p, 0, sizeof(int32_t) * 4, e->stream));
   MA_HIP_TRY(hipMemsetAsync(B.counters.p, 0, sizeof(unsigned long long) * kCounters, e->stream));

@@ -100,4 +100,45 @@ __device__ inline void for_ranges(int base, int l, int32_t lo, int cnt, M &&more
   }
 }
 
+// ---------------------------------------------------------------------------
+// Plane pyramid.  With coordinates about the grid's centre and v_j = |y_j|^2 -
+// w_j, pi_j(x) = |x|^2 + v_j - 2 x.y_j.  A node keeps a gradient a and b = min
+// over its Diracs of v_j - a.y_j (a lower bound of it above level 0), so that
+//   min_j v_j - 2 x.y_j >= b + min over the node's box of (a - 2 x).y.
+// Where the weights vary smoothly a is close to 2 x for the points x that the
+// node's Diracs own, and the bound is tight to the square of the node's side.
+// (The bound of the max-weight pyramid, dist^2(x, node) - max w, is loose by
+// four times the distance from a Dirac to its cell times the node's side:
+// with clustered Diracs a search for the owners of one bin then met about 500
+// Diracs instead of 10.)
+// a = 2 (centre of the node) - gw, gw the gradient of the weights by least
+// squares over the 16 grandchildren of the node's even-level ancestor.
+// ---------------------------------------------------------------------------
+struct Plane {
+  double ax, ay, b, pad;
+};
+// Diracs of an even-level node: number, sums of y and w.
+struct NodeSums {
+  double n, x, y, w;
+};
+struct NodeBox {
+  double x0, y0, x1, y1;
+};
+__device__ inline NodeBox node_box(const Grid &g, uint32_t m, int lev) {
+  const double side = g.h * (double)(1u << lev), half = 0.5 * g.h * (double)g.G;
+  NodeBox q;
+  q.x0 = compact1by1(m) * side - half;
+  q.y0 = compact1by1(m >> 1) * side - half;
+  q.x1 = q.x0 + side;
+  q.y1 = q.y0 + side;
+  return q;
+}
+// min of t.y over the box; mag gets the magnitude of its terms
+__device__ inline double box_min(const NodeBox &q, double tx, double ty, double &mag) {
+  const double px = tx > 0.0 ? q.x0 : q.x1, py = ty > 0.0 ? q.y0 : q.y1;
+  mag = fabs(tx * px) + fabs(ty * py);
+  return tx * px + ty * py;
+}
+// rounding allowance of a bound: its terms carry errors of a few 1e-16
+constexpr double kPlaneEps = 1e-13;
 }  // namespace ma
