@@ -254,120 +254,277 @@ __global__ void __launch_bounds__(kDenseSide *kDenseSide) k_amg_dense_inv(
 // converged: done[0] != 0).  T: values, diagonals and coarse vectors; TB,
 // TX, TY: right-hand side, iterate and output (FP64 at level 0, where they
 // are the conjugate gradient's r and z).
+//
+// Up to a few hundred thousand rows a cycle is bound by the number of its
+// launches (3-5 us each on the coarse levels, most of it the chain row pointer
+// -> entry -> gather and the gap to the next launch), so that what fits into a
+// neighbour is part of it: level 0's first sweep comes from the residual update of the
+// conjugate gradient, a coarse level's from the restriction above it, r.z
+// from level 0's last sweep, and the levels of at most kTailRows rows with
+// the dense solve are one workgroup's work.
 // ---------------------------------------------------------------------------
-// Sparse row times vector by a group of kRowLanes lanes, FP64 accumulation.
-template <class T, class TX>
-__device__ inline double row_dot_t(const int32_t *__restrict__ ptr,
-                                   const int32_t *__restrict__ col, const T *__restrict__ val,
-                                   const TX *__restrict__ x, int64_t i, bool valid, int lane) {
-  double s = 0.0;
-  if (valid)
-    for (int32_t q = ptr[i] + lane; q < ptr[i + 1]; q += kRowLanes)
-      s += (double)val[q] * (double)x[col[q]];
-  for (int o = 1; o < kRowLanes; o <<= 1) s += __shfl_xor(s, o, kRowLanes);
-  return s;
-}
-// x = omega * b / D   (first sweep from x = 0)
-template <class T, class TB>
-__global__ void k_amg_smooth0(int64_t n, const T *dinv, const TB *b, T *x, const double *done,
-                              double kOmega) {
-  if (*done != 0.0) return;
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) x[i] = (T)(kOmega * (double)b[i] * (double)dinv[i]);
-}
 // y = x + omega (b - A x) / D; rows are read by groups of kRowLanes lanes
-// (consecutive entries of consecutive rows: coalesced)
-template <class T, class TB, class TX, class TY>
-__global__ void k_amg_smooth(int64_t n, const int32_t *ptr, const int32_t *col, const T *val,
-                             const T *dinv, const TB *b, const TX *x, TY *y, const double *done,
-                             double kOmega) {
+// (consecutive entries of consecutive rows: coalesced).  With xc the first
+// sweep after the coarse correction: x' = x + corr xc[. / kAgg], formed on
+// the fly, takes the place of x.  DOT: cg_grid(n) workgroups of
+// kCgThreads threads, and the partial sums of b.y go to part.
+template <bool DOT, bool CORR, class T, class TB, class TX, class TY>
+__global__ void __launch_bounds__(DOT ? kCgThreads : kVB2)
+    k_amg_smooth(int64_t n, const int32_t *ptr, const int32_t *col, const T *val, const T *dinv,
+                 const TB *b, const TX *x, const T *xc, TY *y, double *part, const double *done,
+                 double kOmega, double kCorr) {
+  const int lane = (int)threadIdx.x % kRowLanes;
+  auto at = [&](int64_t j) {
+    return CORR ? (double)x[j] + kCorr * (double)xc[j / kAgg] : (double)x[j];
+  };
+  int64_t i = xcd_share(blockIdx.x, gridDim.x) * (kVB2 / kRowLanes), last = n;
+  if (DOT) cg_rows(n, i, last);
+  i += threadIdx.x / kRowLanes;
+  RowHead<T> row;
+  row.load(ptr, col, val, i, i < last, lane);
   if (*done != 0.0) return;
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t i = t / kRowLanes;
-  const int lane = (int)(t % kRowLanes);
-  const double ax = row_dot_t(ptr, col, val, x, i, i < n, lane);
-  if (i < n && lane == 0)
-    y[i] = (TY)((double)x[i] + kOmega * ((double)b[i] - ax) * (double)dinv[i]);
+  double acc = 0.0;
+  while (i < last) {  // a group's lanes go together
+    const double ax = row.dot(col, val, at);
+    if (lane == 0) {
+      const double bi = (double)b[i];
+      const TY v = (TY)(at(i) + kOmega * (bi - ax) * (double)dinv[i]);
+      y[i] = v;
+      acc += bi * (double)v;
+    }
+    if (!DOT) return;
+    i += kCgGroups;
+    row.load(ptr, col, val, i, i < last, lane);
+  }
+  if (DOT) {
+    __shared__ double s[kCgThreads / 64];
+    acc = cg_block_sum(acc, s);
+    if (threadIdx.x == 0) part[blockIdx.x] = acc;
+  }
 }
 // bc[I] = sum over the aggregate of (b - A x): kAgg rows x kRowLanes lanes;
 // with dinv_c, also the coarse level's first smoothing sweep from zero,
 // yc = omega bc / Dc (saves that level a launch)
 template <class T, class TB, class TX>
-__global__ void k_amg_restrict(int64_t nc, int64_t n, const int32_t *ptr, const int32_t *col,
-                               const T *val, const TB *b, const TX *x, T *bc, const T *dinv_c,
-                               T *yc, const double *done, double kOmega) {
-  if (*done != 0.0) return;
-  constexpr int kGroup = kAgg * kRowLanes;
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t I = t / kGroup;
-  const int lane = (int)(t % kGroup);
+__global__ void __launch_bounds__(kVB2)
+    k_amg_restrict(int64_t nc, int64_t n, const int32_t *ptr, const int32_t *col, const T *val,
+                   const TB *b, const TX *x, T *bc, const T *dinv_c, T *yc, const double *done,
+                   double kOmega) {
+  constexpr int kLanes = kAgg * kRowLanes;
+  const int64_t t = xcd_share(blockIdx.x, gridDim.x) * kVB2 + threadIdx.x;
+  const int64_t I = t / kLanes;
+  const int lane = (int)(t % kLanes);
   const int64_t i = I * kAgg + lane / kRowLanes;
   const bool valid = I < nc && i < n;
-  const double ax = row_dot_t(ptr, col, val, x, i, valid, lane % kRowLanes);
+  RowHead<T> row;
+  row.load(ptr, col, val, i, valid, lane % kRowLanes);
+  if (*done != 0.0) return;
+  const double ax = row.dot(col, val, [&](int64_t j) { return (double)x[j]; });
   double s = (valid && lane % kRowLanes == 0) ? (double)b[i] - ax : 0.0;
-  for (int o = kRowLanes; o < kGroup; o <<= 1) s += __shfl_xor(s, o, kGroup);
+  for (int o = kRowLanes; o < kLanes; o <<= 1) s += __shfl_xor(s, o, kLanes);
   if (I < nc && lane == 0) {
     bc[I] = (T)s;
     if (dinv_c) yc[I] = (T)(kOmega * s * (double)dinv_c[I]);
   }
 }
-// First post-smoothing sweep fused with the prolongation: with
-// x' = x + corr * xc[. / kAgg] (the corrected iterate, formed on the fly),
-// y = x' + omega (b - A x') / D
-template <class T, class TB, class TX, class TY>
-__global__ void k_amg_smooth_prolong(int64_t n, const int32_t *ptr, const int32_t *col,
-                                     const T *val, const T *dinv, const TB *b, const TX *x,
-                                     const T *xc, TY *y, const double *done, double kOmega,
-                                     double kCorr) {
-  if (*done != 0.0) return;
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  const int64_t i = t / kRowLanes;
-  const int lane = (int)(t % kRowLanes);
-  double ax = 0.0;
-  if (i < n)
-    for (int32_t q = ptr[i] + lane; q < ptr[i + 1]; q += kRowLanes) {
-      const int32_t j = col[q];
-      ax += (double)val[q] * ((double)x[j] + kCorr * (double)xc[j / kAgg]);
+
+// The last levels of a cycle, one workgroup: the smoothed levels lv[0 .. nlev)
+// (at most kTailRows rows, each level a kAgg-th of the one before) and the
+// dense solve below them, with the vectors in LDS.  b, y: the first level's
+// right-hand side and first sweep (nlev = 0: the dense solve's right-hand
+// side); x: its result.  With part the one partial sum of b.x goes there
+// (nlev = 0).  Bound by the chain of its steps (load, residual, restriction,
+// dense solve, correction): 8.7 us for 250 + 63 rows in FP32, 13.8 us for
+// 586 + 147 in FP64, against the three or five launches it replaces.  More
+// rows would not fit the registers of one pass and take a second one of about
+// the length of a launch.
+constexpr int kTailRows = 1024, kTailLevels = 2, kTailThreads = 1024;
+static_assert(kTailRows <= kCoarsest * kAgg * kAgg, "smoothed levels of the tail");
+template <class T>
+struct TailLevel {
+  int n;
+  const int32_t *ptr, *col;
+  const T *val, *dinv;
+};
+template <class T>
+struct Tail {
+  TailLevel<T> lv[kTailLevels];
+  int nlev, nd;          // smoothed levels; rows of the dense level
+  const double *inv;
+  double omega, corr;
+  int two;               // V(2,2)
+};
+// A level's rows, all of them at once and kept in registers: groups of
+// kRowLanes lanes, N rows each, two entries of a row per lane (rows of more
+// entries, few, are read on from memory).
+constexpr int kTailGroups = kTailThreads / kRowLanes;
+template <int N, class T>
+struct TailRows {
+  int32_t c[N][2];
+  T v[N][2];
+  unsigned lng = 0;  // bit r: row r goes on
+  __device__ inline void load(const TailLevel<T> &L, int lane) {
+    const int i0 = (int)threadIdx.x / kRowLanes;
+    int32_t q[N], e[N];
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+      const int i = min(i0 + r * kTailGroups, L.n - 1);
+      q[r] = L.ptr[i] + lane;
+      e[r] = L.ptr[i + 1];
     }
-  for (int o = 1; o < kRowLanes; o <<= 1) ax += __shfl_xor(ax, o, kRowLanes);
-  if (i < n && lane == 0) {
-    const double xi = (double)x[i] + kCorr * (double)xc[i / kAgg];
-    y[i] = (TY)(xi + kOmega * ((double)b[i] - ax) * (double)dinv[i]);
+#pragma unroll
+    for (int r = 0; r < N; r++)
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        // (an empty slot: 0 times the row's own unknown)
+        c[r][k] = min(i0 + r * kTailGroups, L.n - 1);
+        v[r][k] = (T)0;
+        if (q[r] + k * kRowLanes < e[r]) {
+          c[r][k] = L.col[q[r] + k * kRowLanes];
+          v[r][k] = L.val[q[r] + k * kRowLanes];
+        }
+        if (q[r] + 2 * kRowLanes < e[r]) lng |= 1u << r;
+      }
   }
-}
-// coarsest: x = A^-1 b, one workgroup, 16 lanes per row
-constexpr int kDenseThreads = 1024;
-template <class TB, class TX>
-__global__ void __launch_bounds__(kDenseThreads) k_amg_dense_solve(int64_t n, const double *inv,
-                                                                   const TB *b, TX *x,
-                                                                   const double *done) {
+  // f(i, A x at row i) on lane 0 of row i's group
+  template <class X, class F>
+  __device__ inline void each(const TailLevel<T> &L, X &&x, F &&f) const {
+    const int i0 = (int)threadIdx.x / kRowLanes, lane = (int)threadIdx.x % kRowLanes;
+    double s[N];
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+      s[r] = (double)v[r][0] * x(c[r][0]);
+      s[r] += (double)v[r][1] * x(c[r][1]);
+    }
+    if (lng)
+#pragma unroll
+      for (int r = 0; r < N; r++)
+        if (lng >> r & 1) {
+          const int i = min(i0 + r * kTailGroups, L.n - 1);
+          for (int32_t k = L.ptr[i] + lane + 2 * kRowLanes; k < L.ptr[i + 1]; k += kRowLanes)
+            s[r] += (double)L.val[k] * x(L.col[k]);
+        }
+#pragma unroll
+    for (int r = 0; r < N; r++) {
+      s[r] = oct_sum(s[r]);
+      if (lane == 0 && i0 + r * kTailGroups < L.n) f(i0 + r * kTailGroups, s[r]);
+    }
+  }
+};
+template <class T, class TB, class TX>
+__global__ void __launch_bounds__(kTailThreads)
+    k_amg_tail(Tail<T> t, const TB *b, const T *y, TX *x, double *part, const double *done) {
+  // every level's vectors after those of the one before
+  constexpr int kAll = kTailRows + kTailRows / kAgg + kCoarsest;
+  __shared__ T sy[kAll], sx[kAll], sd[kTailRows + kTailRows / kAgg];
+  __shared__ double sb[kAll], res[kTailRows];
+  const int tid = (int)threadIdx.x, lane = tid % kRowLanes;
+  const int n0 = t.nlev ? t.lv[0].n : t.nd, n1 = t.nlev > 1 ? t.lv[1].n : 0;
+  const double om = t.omega, co = t.corr;
+  // the levels' first entries, loaded with the vectors and kept for the way up
+  TailRows<kTailRows / kTailGroups, T> rows0;
+  TailRows<kTailRows / kTailGroups / kAgg, T> rows1;
+  if (t.nlev) rows0.load(t.lv[0], lane);
+  if (t.nlev > 1) rows1.load(t.lv[1], lane);
+  for (int i = tid; i < n0; i += kTailThreads) {
+    sb[i] = (double)b[i];
+    if (t.nlev) {
+      sy[i] = y[i];
+      sd[i] = t.lv[0].dinv[i];
+    }
+  }
+  for (int i = tid; i < n1; i += kTailThreads) sd[n0 + i] = t.lv[1].dinv[i];
   if (*done != 0.0) return;
-  __shared__ double sb[kCoarsest];
-  for (int i = threadIdx.x; i < n; i += kDenseThreads) sb[i] = (double)b[i];
   __syncthreads();
-  // a group's rows together, so that their loads overlap
-  constexpr int kRows = kCoarsest / (kDenseThreads / kGroup);
-  const int l = (int)threadIdx.x & (kGroup - 1), i0 = (int)threadIdx.x / kGroup;
-  const int N = (int)n;
-  const double *row[kRows];
-  double s[kRows];
+  // down from a level at off: smooth (V(2,2)), residual, restriction
+  auto down = [&](const TailLevel<T> &L, const auto &rows, int off, int nc, bool smoothed) {
+    const T *v = sy + off;
+    if (t.two) {
+      rows.each(L, [&](int j) { return (double)sy[off + j]; }, [&](int i, double ax) {
+        sx[off + i] = (T)((double)sy[off + i] + om * (sb[off + i] - ax) * (double)sd[off + i]);
+      });
+      __syncthreads();
+      v = sx + off;
+    }
+    rows.each(L, [&](int j) { return (double)v[j]; },
+              [&](int i, double ax) { res[i] = sb[off + i] - ax; });
+    __syncthreads();
+    const int oc = off + L.n;
+    for (int I = tid; I < nc; I += kTailThreads) {
+      double a[kAgg];
 #pragma unroll
-  for (int r = 0; r < kRows; r++) {
-    row[r] = inv + min(i0 + r * (kDenseThreads / kGroup), N - 1) * N;
-    s[r] = 0.0;
+      for (int k = 0; k < kAgg; k++) a[k] = I * kAgg + k < L.n ? res[I * kAgg + k] : 0.0;
+      static_assert(kAgg == 4, "sum of an aggregate in the order of k_amg_restrict");
+      const double s = (a[0] + a[1]) + (a[2] + a[3]);
+      sb[oc + I] = (double)(T)s;
+      if (smoothed) sy[oc + I] = (T)(om * s * (double)sd[oc + I]);
+    }
+    __syncthreads();
+  };
+  // up to a level at off: correction from the level after it, smooth; the
+  // first level's result goes to x
+  auto up = [&](const TailLevel<T> &L, const auto &rows, int off, bool out) {
+    __syncthreads();
+    const T *xc = sx + off + L.n, *v = t.two ? sx + off : sy + off;
+    auto at = [&](int j) { return (double)v[j] + co * (double)xc[j / kAgg]; };
+    rows.each(L, at, [&](int i, double ax) {
+      const T u = (T)(at(i) + om * (sb[off + i] - ax) * (double)sd[off + i]);
+      if (t.two)
+        sy[off + i] = u;
+      else if (out)
+        x[i] = (TX)u;
+      else
+        sx[off + i] = u;
+    });
+    if (!t.two) return;
+    __syncthreads();
+    rows.each(L, [&](int j) { return (double)sy[off + j]; }, [&](int i, double ax) {
+      const T u = (T)((double)sy[off + i] + om * (sb[off + i] - ax) * (double)sd[off + i]);
+      if (out)
+        x[i] = (TX)u;
+      else
+        sx[off + i] = u;
+    });
+  };
+  if (t.nlev) down(t.lv[0], rows0, 0, t.nlev > 1 ? n1 : t.nd, t.nlev > 1);
+  if (t.nlev > 1) down(t.lv[1], rows1, n0, t.nd, false);
+  {
+    // coarsest: x = A^-1 b, 16 lanes per row, a group's rows together
+    constexpr int kGroups = kTailThreads / kGroup, kRows = kCoarsest / kGroups;
+    static_assert(kCoarsest % kGroups == 0, "rows of the dense solve");
+    const int l = tid & (kGroup - 1), i0 = tid / kGroup, N = t.nd;
+    const int off = t.nlev ? n0 + n1 : 0;
+    const double *row[kRows];
+    double s[kRows], dot = 0.0;
+#pragma unroll
+    for (int r = 0; r < kRows; r++) {
+      row[r] = t.inv + min(i0 + r * kGroups, N - 1) * N;
+      s[r] = 0.0;
+    }
+#pragma unroll 6
+    for (int k = l; k < N; k += kGroup)
+#pragma unroll
+      for (int r = 0; r < kRows; r++) s[r] += row[r][k] * sb[off + k];
+#pragma unroll
+    for (int r = 0; r < kRows; r++) {
+      const double v = row_sum(s[r]);
+      const int i = i0 + r * kGroups;
+      if (l == 0 && i < N) {
+        if (t.nlev)
+          sx[off + i] = (T)v;
+        else
+          x[i] = (TX)v;
+        dot += sb[off + i] * v;
+      }
+    }
+    if (part) {
+      dot = cg_block_sum(dot, res);
+      if (tid == 0) part[0] = dot;
+    }
   }
-#pragma unroll 4
-  for (int k = l; k < N; k += kGroup)
-#pragma unroll
-    for (int r = 0; r < kRows; r++) s[r] += row[r][k] * sb[k];
-#pragma unroll
-  for (int r = 0; r < kRows; r++) {
-    const double t = row_sum(s[r]);
-    const int i = i0 + r * (kDenseThreads / kGroup);
-    if (l == 0 && i < N) x[i] = (TX)t;
-  }
+  if (t.nlev > 1) up(t.lv[1], rows1, n0, false);
+  if (t.nlev) up(t.lv[0], rows0, 0, true);
 }
-static_assert(kCoarsest % (kDenseThreads / kGroup) == 0, "rows of k_amg_dense_solve");
 
 // ---------------------------------------------------------------------------
 // Host side
@@ -420,7 +577,6 @@ static ma_status amg_build(ma_engine *e, Amg &A, const CsrView &M) {
   lv.reserve(32);
   size_t used = 1;
   lv[0].n = n;
-  MA_HIP_TRY(lv[0].x.ensure((size_t)n));
   MA_HIP_TRY(lv[0].y.ensure((size_t)n));
   int64_t room = M.nnz;  // bound of the entries of the level being built
   while (lv[used - 1].n > kCoarsest && used < 32) {
@@ -520,50 +676,70 @@ ma_status amg_setup(ma_engine *e, Amg &A, const CsrView &M, int32_t gi, int max_
   return MA_OK;
 }
 
-// z = M^-1 r (one V-cycle) with the hierarchy in T; level 0 reads r and
-// keeps its iterate in z (FP64), its smoother output in lv[0].y (T).
+// First level of the tail: the first one below level 0 with at most kTailRows
+// rows (the coarsest level at the latest).
 template <class T>
-static hipError_t amg_cycle(ma_engine *e, Amg &A, const double *r, double *z, const double *done) {
+static int tail_start(Amg &A) {
+  std::vector<AmgLevel<T>> &lv = levels_of(A, (T *)nullptr);
+  int l = 1;
+  while (l < A.nlev - 1 && lv[l].n > kTailRows) l++;
+  return l;
+}
+
+// z = M^-1 r (one V-cycle) with the hierarchy in T; level 0 reads r and its
+// first sweep (amg_head, written with r), and writes z (FP64).  V(2,2) keeps
+// level 0's iterate in z.
+template <class T>
+static hipError_t amg_cycle(ma_engine *e, Amg &A, const double *r, double *z, double *part,
+                            const double *done) {
   std::vector<AmgLevel<T>> &lv = levels_of(A, (T *)nullptr);
   const int nl = A.nlev;
   const double om = e->amg_omega, co = e->amg_corr;  // Jacobi damping, coarse over-correction
   const bool two = e->amg_sweeps != 1;                 // V(2,2), else V(1,1)
-  auto ptr_of = [&](int l) { return l == 0 ? A.ptr0 : lv[l].ptr.p; };
-  auto col_of = [&](int l) { return l == 0 ? A.col0 : lv[l].col.p; };
+  Tail<T> t{};
+  t.inv = A.dense_inv.p;
+  t.omega = om;
+  t.corr = co;
+  t.two = two;
+  t.nd = (int)lv[nl - 1].n;
   if (nl == 1) {
-    hipLaunchKernelGGL((k_amg_dense_solve<double, double>), dim3(1), dim3(kDenseThreads), 0,
-                       e->stream, lv[0].n, A.dense_inv.p, r, z, done);
+    hipLaunchKernelGGL((k_amg_tail<T, double, double>), dim3(1), dim3(kTailThreads), 0, e->stream,
+                       t, r, (const T *)nullptr, z, part, done);
     return hipGetLastError();
   }
+  auto ptr_of = [&](int l) { return l == 0 ? A.ptr0 : lv[l].ptr.p; };
+  auto col_of = [&](int l) { return l == 0 ? A.col0 : lv[l].col.p; };
+  const T *none = nullptr;
+  double *no_part = nullptr;
+  const int lt = tail_start<T>(A);
   // downward (the first sweep of a coarse level comes from the restriction)
-  for (int l = 0; l < nl - 1; l++) {
+  for (int l = 0; l < lt; l++) {
     AmgLevel<T> &L = lv[l];
     AmgLevel<T> &Ln = lv[l + 1];
     const bool seed = l + 1 < nl - 1;  // the coarsest level is solved directly
-    const T *dc = seed ? Ln.dinv.p : (const T *)nullptr;
+    const T *dc = seed ? Ln.dinv.p : none;
     T *yc = seed ? Ln.y.p : nullptr;
     const unsigned gr = nb2(Ln.n * kAgg * kRowLanes), gs = nb2(L.n * kRowLanes);
+    const T *x = L.y.p;
     if (l == 0) {
-      hipLaunchKernelGGL((k_amg_smooth0<T, double>), dim3(nb2(L.n)), dim3(kVB2), 0, e->stream,
-                         L.n, dinv_of<T>(A, 0), r, L.y.p, done, om);
       if (two) {
-        hipLaunchKernelGGL((k_amg_smooth<T, double, T, double>), dim3(gs), dim3(kVB2), 0,
-                           e->stream, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0),
-                           dinv_of<T>(A, 0), r, (const T *)L.y.p, z, done, om);
+        hipLaunchKernelGGL((k_amg_smooth<false, false, T, double, T, double>), dim3(gs),
+                           dim3(kVB2), 0, e->stream, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0),
+                           dinv_of<T>(A, 0), r, x, none, z, no_part, done, om, co);
         hipLaunchKernelGGL((k_amg_restrict<T, double, double>), dim3(gr), dim3(kVB2), 0,
                            e->stream, Ln.n, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0), r,
                            (const double *)z, Ln.b.p, dc, yc, done, om);
       } else {  // V(1,1): the one downward sweep is the iterate
         hipLaunchKernelGGL((k_amg_restrict<T, double, T>), dim3(gr), dim3(kVB2), 0, e->stream,
-                           Ln.n, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0), r,
-                           (const T *)L.y.p, Ln.b.p, dc, yc, done, om);
+                           Ln.n, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0), r, x, Ln.b.p, dc,
+                           yc, done, om);
       }
     } else {
-      const T *x = L.y.p;
       if (two) {
-        hipLaunchKernelGGL((k_amg_smooth<T, T, T, T>), dim3(gs), dim3(kVB2), 0, e->stream, L.n,
-                           ptr_of(l), col_of(l), val_of<T>(A, l), dinv_of<T>(A, l),
-                           (const T *)L.b.p, (const T *)L.y.p, L.x.p, done, om);
+        hipLaunchKernelGGL((k_amg_smooth<false, false, T, T, T, T>), dim3(gs), dim3(kVB2), 0,
+                           e->stream, L.n, ptr_of(l), col_of(l), val_of<T>(A, l),
+                           dinv_of<T>(A, l), (const T *)L.b.p, x, none, L.x.p, no_part, done, om,
+                           co);
         x = L.x.p;
       }
       hipLaunchKernelGGL((k_amg_restrict<T, T, T>), dim3(gr), dim3(kVB2), 0, e->stream, Ln.n,
@@ -571,52 +747,70 @@ static hipError_t amg_cycle(ma_engine *e, Amg &A, const double *r, double *z, co
                          Ln.b.p, dc, yc, done, om);
     }
   }
-  {
-    AmgLevel<T> &Lc = lv[nl - 1];
-    hipLaunchKernelGGL((k_amg_dense_solve<T, T>), dim3(1), dim3(kDenseThreads), 0, e->stream,
-                       Lc.n, A.dense_inv.p, (const T *)Lc.b.p, Lc.x.p, done);
-  }
+  for (int l = lt; l < nl - 1; l++)
+    t.lv[t.nlev++] = {(int)lv[l].n, ptr_of(l), col_of(l), val_of<T>(A, l), dinv_of<T>(A, l)};
+  hipLaunchKernelGGL((k_amg_tail<T, T, T>), dim3(1), dim3(kTailThreads), 0, e->stream, t,
+                     (const T *)lv[lt].b.p, (const T *)lv[lt].y.p, lv[lt].x.p, no_part, done);
   // upward
-  for (int l = nl - 2; l >= 0; l--) {
+  for (int l = lt - 1; l >= 0; l--) {
     AmgLevel<T> &L = lv[l];
     const T *xc = lv[l + 1].x.p;
     const unsigned gs = nb2(L.n * kRowLanes);
+    const dim3 gd(cg_grid(L.n)), bd(kCgThreads);
     if (l == 0) {
       if (two) {
-        hipLaunchKernelGGL((k_amg_smooth_prolong<T, double, double, T>), dim3(gs), dim3(kVB2), 0,
+        hipLaunchKernelGGL((k_amg_smooth<false, true, T, double, double, T>), dim3(gs),
+                           dim3(kVB2), 0, e->stream, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0),
+                           dinv_of<T>(A, 0), r, (const double *)z, xc, L.y.p, no_part, done, om,
+                           co);
+        hipLaunchKernelGGL((k_amg_smooth<true, false, T, double, T, double>), gd, bd, 0,
                            e->stream, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0),
-                           dinv_of<T>(A, 0), r, (const double *)z, xc, L.y.p, done, om, co);
-        hipLaunchKernelGGL((k_amg_smooth<T, double, T, double>), dim3(gs), dim3(kVB2), 0,
-                           e->stream, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0),
-                           dinv_of<T>(A, 0), r, (const T *)L.y.p, z, done, om);
+                           dinv_of<T>(A, 0), r, (const T *)L.y.p, none, z, part, done, om, co);
       } else {
-        hipLaunchKernelGGL((k_amg_smooth_prolong<T, double, T, double>), dim3(gs), dim3(kVB2), 0,
+        hipLaunchKernelGGL((k_amg_smooth<true, true, T, double, T, double>), gd, bd, 0,
                            e->stream, L.n, ptr_of(0), col_of(0), val_of<T>(A, 0),
-                           dinv_of<T>(A, 0), r, (const T *)L.y.p, xc, z, done, om, co);
+                           dinv_of<T>(A, 0), r, (const T *)L.y.p, xc, z, part, done, om, co);
       }
     } else {
       if (two) {
-        hipLaunchKernelGGL((k_amg_smooth_prolong<T, T, T, T>), dim3(gs), dim3(kVB2), 0,
+        hipLaunchKernelGGL((k_amg_smooth<false, true, T, T, T, T>), dim3(gs), dim3(kVB2), 0,
                            e->stream, L.n, ptr_of(l), col_of(l), val_of<T>(A, l),
                            dinv_of<T>(A, l), (const T *)L.b.p, (const T *)L.x.p, xc, L.y.p,
-                           done, om, co);
-        hipLaunchKernelGGL((k_amg_smooth<T, T, T, T>), dim3(gs), dim3(kVB2), 0, e->stream, L.n,
-                           ptr_of(l), col_of(l), val_of<T>(A, l), dinv_of<T>(A, l),
-                           (const T *)L.b.p, (const T *)L.y.p, L.x.p, done, om);
+                           no_part, done, om, co);
+        hipLaunchKernelGGL((k_amg_smooth<false, false, T, T, T, T>), dim3(gs), dim3(kVB2), 0,
+                           e->stream, L.n, ptr_of(l), col_of(l), val_of<T>(A, l),
+                           dinv_of<T>(A, l), (const T *)L.b.p, (const T *)L.y.p, none, L.x.p,
+                           no_part, done, om, co);
       } else {
-        hipLaunchKernelGGL((k_amg_smooth_prolong<T, T, T, T>), dim3(gs), dim3(kVB2), 0,
+        hipLaunchKernelGGL((k_amg_smooth<false, true, T, T, T, T>), dim3(gs), dim3(kVB2), 0,
                            e->stream, L.n, ptr_of(l), col_of(l), val_of<T>(A, l),
                            dinv_of<T>(A, l), (const T *)L.b.p, (const T *)L.y.p, xc, L.x.p,
-                           done, om, co);
+                           no_part, done, om, co);
       }
     }
   }
   return hipGetLastError();
 }
 
-// z = M^-1 r (one V-cycle); done: device flag, cycles are skipped once set.
-hipError_t amg_apply(ma_engine *e, Amg &A, const double *r, double *z, const double *done) {
-  return A.fp32 ? amg_cycle<float>(e, A, r, z, done) : amg_cycle<double>(e, A, r, z, done);
+AmgHead amg_head(ma_engine *e, Amg &A) {
+  AmgHead h;
+  h.fp32 = A.fp32;
+  h.omega = e->amg_omega;
+  h.partials = 1;  // the tail's own sum
+  if (A.nlev > 1) {
+    h.partials = cg_grid(A.fp32 ? A.lvf[0].n : A.lv[0].n);
+    h.dinv = A.fp32 ? (const void *)dinv_of<float>(A, 0) : (const void *)dinv_of<double>(A, 0);
+    h.y = A.fp32 ? (void *)A.lvf[0].y.p : (void *)A.lv[0].y.p;
+  }
+  return h;
+}
+
+// z = M^-1 r (one V-cycle) and the partial sums of r.z; done: device flag,
+// cycles are skipped once set.
+hipError_t amg_apply(ma_engine *e, Amg &A, const double *r, double *z, double *part,
+                     const double *done) {
+  return A.fp32 ? amg_cycle<float>(e, A, r, z, part, done)
+                : amg_cycle<double>(e, A, r, z, part, done);
 }
 
 }  // namespace ma

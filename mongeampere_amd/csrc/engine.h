@@ -202,9 +202,8 @@ struct EvalBuffers {
 };
 
 struct SolverBuffers {
-  DBuf<double> w, m, nu, g, d, x, r, z, p, Ap, wtrial, red;
+  DBuf<double> w, m, nu, g, d, x, r, z, p, q, Ap, wtrial, red;
   DBuf<double> stage;         // host <-> device staging of per-Dirac arrays
-  DBuf<double> red_sp;        // partial sums of the sparse products
   DBuf<int32_t> hptr, hcol;   // caller-supplied CSR (ma_solve_laplacian_csr)
   DBuf<double> hval, hg, hd;
   DBuf<int32_t> moved;        // set when a trial point differs from the iterate
@@ -341,7 +340,19 @@ void amg_destroy(Amg *a);
 // Returns MA_SINGULAR when a row other than gi has a non-positive diagonal.
 ma_status amg_setup(ma_engine *e, Amg &A, const CsrView &M, int32_t gi, int max_levels,
                     bool fp32);
-hipError_t amg_apply(ma_engine *e, Amg &A, const double *r, double *z, const double *done);
+// What the conjugate gradient does for the cycle where it writes r: level 0's
+// first sweep y = omega r / D (in the hierarchy's precision; y = null: the
+// cycle has none).  partials: partial sums of r.z that amg_apply leaves.
+struct AmgHead {
+  bool fp32 = false;
+  const void *dinv = nullptr;
+  void *y = nullptr;
+  double omega = 1.0;
+  int partials = 0;
+};
+AmgHead amg_head(ma_engine *e, Amg &A);
+hipError_t amg_apply(ma_engine *e, Amg &A, const double *r, double *z, double *part,
+                     const double *done);
 const double *amg_level0_values(const Amg &a);
 const double *amg_level0_dinv(const Amg &a);
 

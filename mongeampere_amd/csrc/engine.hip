@@ -10,6 +10,7 @@
 #include <mutex>
 
 #include "geom_common.h"
+#include "lanes.h"
 
 namespace ma {
 
@@ -17,7 +18,6 @@ hipError_t device_sum(ma_engine *e, const double *x, int64_t n, double *d_out);
 
 constexpr int kVB = 256;      // threads per block for vector kernels
 constexpr int kVGrid = 512;   // fixed grid => fixed number of partial sums
-constexpr int kSpGrid = 4096; // blocks of the sparse products (gathers need more waves in flight)
 
 // ---------------------------------------------------------------------------
 // Mesh preparation: ccw orientation and per-face linear density a x + b y + c
@@ -76,156 +76,173 @@ __device__ inline double block_sum(double v, double *s) {
   __syncthreads();
   return r;
 }
-// sum of kVGrid partials, computed identically by every block
-__device__ inline double reduce_partials(const double *part, double *s) {
-  double v = 0.0;
-  for (int i = threadIdx.x; i < kVGrid; i += kVB) v += part[i];
-  return block_sum(v, s);
-}
-
 // The conjugate gradient runs on A0 = the Hessian with row and column gi
 // replaced by the identity (symmetric positive definite for a connected
 // diagram); with b[gi] = 0 its solution has x[gi] = 0, the gauge of
 // include/MA/optimal_transport.hpp:82-86.  Scalars live on the device:
-// scal = [rz (ping-pong, 2), rr, -, bb, done, iterations, breakdown].
+// scal = [rz (of the iteration's parity, 2), rr, -, bb, done, iterations,
+// breakdown].
+//
+// An iteration is k_cg_spmv, k_cg_update and the preconditioner.  Below a few
+// hundred thousand rows its time is the number of launches (about 5 us each),
+// so the direction p = z + beta p is formed inside the product (p of a
+// neighbour on the fly from z and the last p; two buffers of p take turns),
+// and what the preconditioner needs at each r is written where r is.  With
+// the cycle's own fusions an iteration on 150k rows went from 17 launches to
+// 11 and from 89 to 73 us (10.1 k_cg_spmv, 5.1 k_cg_update, 58 the cycle).
 
-// y = A0 x, partial sums of x.y.  gz >= 0: the matrix holds the Hessian's
-// own values and row gz is the gauge row, y[gz] = 0 (every vector of the
-// iteration has a zero there, so column gz contributes nothing either);
-// gz < 0: the values are already gauge-fixed.
-__global__ void __launch_bounds__(kVB) k_spmv_dot(int64_t n, const int32_t *ptr,
-                                                  const int32_t *col, const double *val,
-                                                  const double *x, double *y, double *part,
-                                                  const double *scal, int32_t gz) {
-  __shared__ double s[kVB];
-  if (scal[5] != 0.0) return;
-  double acc = 0.0;
-  const int lane = (int)(threadIdx.x % kRowLanes);
-  const int64_t stride = (int64_t)kSpGrid * kVB / kRowLanes;
-  // the kRowLanes lanes of a group share i, so they iterate together
-  for (int64_t i = (blockIdx.x * (int64_t)kVB + threadIdx.x) / kRowLanes; i < n; i += stride) {
-    const double v = (i == gz) ? 0.0 : row_dot(ptr, col, val, x, i, true, lane);
-    if (lane == 0) {
-      y[i] = v;
-      acc += x[i] * v;
-    }
+// The head of the preconditioner at unknown i: y = omega r / D, and its
+// share of r.y
+template <class TY>
+struct Head {
+  const TY *dinv;
+  TY *y;  // null: no head
+  double omega;
+  __device__ inline double operator()(int64_t i, double r) const {
+    if (!y) return 0.0;
+    const TY v = (TY)(omega * r * (double)dinv[i]);
+    y[i] = v;
+    return r * (double)v;
   }
-  acc = block_sum(acc, s);
-  if (threadIdx.x == 0) part[blockIdx.x] = acc;
-}
-// Folds the kSpGrid partial sums of k_spmv_dot into kVGrid partials (in a
-// fixed order, so that sums stay deterministic).
-__global__ void k_fold_partials(const double *in, double *out, const double *scal) {
-  if (scal[5] != 0.0) return;
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= kVGrid) return;
-  double v = 0.0;
-  for (int i = 0; i < kSpGrid / kVGrid; i++) v += in[b * (kSpGrid / kVGrid) + i];
-  out[b] = v;
-}
-// x = 0, r = b (r[gi] = 0), partial sums of r.r; clears the done flag
-__global__ void __launch_bounds__(kVB) k_cg_begin(int64_t n, const double *b, int32_t gi,
-                                                  double *x, double *r, double *part_rr,
-                                                  double *scal) {
-  __shared__ double s[kVB];
-  double rr = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)kVB + threadIdx.x; i < n; i += (int64_t)kVGrid * kVB) {
+};
+
+// x = 0, r = b (r[gi] = 0), partial sums of r.r and (part_rz) of r.y; clears
+// the scalars
+template <class TY>
+__global__ void __launch_bounds__(kCgThreads)
+    k_cg_begin(int64_t n, const double *b, int32_t gi, double *x, double *r, Head<TY> head,
+               double *part_rr, double *part_rz, double *scal) {
+  __shared__ double s[2 * kCgThreads / 64];
+  double c[2] = {0.0, 0.0};
+  int64_t first, last;
+  cg_rows(n, first, last);
+  for (int64_t i = first + threadIdx.x; i < last; i += kCgThreads) {
     const double ri = (i == gi) ? 0.0 : b[i];
     x[i] = 0.0;
     r[i] = ri;
-    rr += ri * ri;
+    c[0] += ri * ri;
+    c[1] += head(i, ri);
   }
-  rr = block_sum(rr, s);
-  if (threadIdx.x == 0) part_rr[blockIdx.x] = rr;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    scal[5] = 0.0;
-    scal[6] = 0.0;
-    scal[7] = 0.0;
-  }
-}
-// z = r / D
-__global__ void k_jacobi(int64_t n, const double *dinv, const double *r, double *z,
-                         const double *scal) {
-  if (scal[5] != 0.0) return;
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) z[i] = r[i] * dinv[i];
-}
-// partial sums of r.z; optionally p = z
-__global__ void __launch_bounds__(kVB) k_dot_rz(int64_t n, const double *r, const double *z,
-                                                double *p, double *part, const double *scal) {
-  __shared__ double s[kVB];
-  if (scal[5] != 0.0) return;
-  double a = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)kVB + threadIdx.x; i < n; i += (int64_t)kVGrid * kVB) {
-    a += r[i] * z[i];
-    if (p) p[i] = z[i];
-  }
-  a = block_sum(a, s);
-  if (threadIdx.x == 0) part[blockIdx.x] = a;
-}
-__global__ void __launch_bounds__(kVB) k_cg_scal_init(const double *part_rz, const double *part_rr,
-                                                      double *scal) {
-  __shared__ double s[kVB];
-  double rz = reduce_partials(part_rz, s);
-  double rr = reduce_partials(part_rr, s);
+  cg_block_sums(c, s);
   if (threadIdx.x == 0) {
-    scal[0] = rz;
+    part_rr[blockIdx.x] = c[0];
+    if (part_rz) part_rz[blockIdx.x] = c[1];
+    if (blockIdx.x == 0)
+      for (int k = 0; k < 8; k++) scal[k] = 0.0;
+  }
+}
+// bb = r.r; done when it is 0
+__global__ void __launch_bounds__(kCgThreads) k_cg_scal_init(const double *part_rr, int np,
+                                                             double *scal) {
+  __shared__ double s[kCgThreads / 64];
+  const double rr = cg_block_sum(threadIdx.x < np ? part_rr[threadIdx.x] : 0.0, s);
+  if (threadIdx.x == 0) {
     scal[2] = rr;
     scal[4] = rr;
     if (rr == 0.0) scal[5] = 1.0;
   }
 }
-// x += alpha p, r -= alpha Ap; partial sums of r.r
-__global__ void __launch_bounds__(kVB) k_cg_update(int64_t n, int parity, const double *part_pap,
-                                                   double *scal, double *x, double *r,
-                                                   const double *p, const double *Ap,
-                                                   double *part_rr) {
-  __shared__ double s[kVB];
+static_assert(kCgGrid <= kCgThreads, "one partial sum per thread");
+// Start of iteration: nrz partial sums of r.z give beta, those of r.r the
+// stopping test; then p = z + beta p_old, Ap = A0 p and partial sums of p.Ap.
+// gz >= 0: the matrix holds the Hessian's own values and row gz is the gauge
+// row, Ap[gz] = 0 (every vector of the iteration has a zero there, so column
+// gz contributes nothing either); gz < 0: the values are already gauge-fixed.
+__global__ void __launch_bounds__(kCgThreads)
+    k_cg_spmv(int64_t n, int parity, const int32_t *__restrict__ ptr,
+              const int32_t *__restrict__ col, const double *__restrict__ val,
+              const double *__restrict__ z, const double *__restrict__ p_old,
+              double *__restrict__ p, double *__restrict__ Ap, const double *part_rz, int nrz,
+              const double *part_rr, double *part_pap, double *scal, double tol2, int32_t gz) {
+  __shared__ double s[2 * kCgThreads / 64];
+  const int t = (int)threadIdx.x, lane = t % kRowLanes;
+  double v[2] = {t < nrz ? part_rz[t] : 0.0, t < gridDim.x ? part_rr[t] : 0.0};
+  int64_t i, last;
+  cg_rows(n, i, last);
+  i += t / kRowLanes;
+  RowHead<double> row;
+  row.load(ptr, col, val, i, i < last, lane);
   if (scal[5] != 0.0) return;
-  const double pap = reduce_partials(part_pap, s);
-  const double rz = scal[parity];
-  const double alpha = (pap > 0.0) ? rz / pap : 0.0;
-  if (!(pap > 0.0)) {
-    // p.Ap <= 0 (or NaN) with a nonzero residual: the matrix is not
-    // positive definite on the search space.  Stop with a breakdown flag
-    // (alpha = 0 leaves x and r unchanged in every block).
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+  cg_block_sums(v, s);
+  const double rz = v[0], rr = v[1], rz_old = scal[1 - parity];
+  const bool end = scal[7] != 0.0 || (scal[6] != 0.0 && rr <= tol2 * scal[4]);
+  if (blockIdx.x == 0 && t == 0) {
+    scal[parity] = rz;
+    scal[2] = rr;
+    if (end) scal[5] = 1.0;
+  }
+  if (end) return;
+  const double beta = (rz_old > 0.0) ? rz / rz_old : 0.0;
+  // (the first iteration has no p_old: what the buffer holds is not read)
+  auto at = [&](int64_t j) { return beta != 0.0 ? fma(beta, p_old[j], z[j]) : z[j]; };
+  double acc = 0.0;
+  // the kRowLanes lanes of a group share i, so they iterate together
+  while (i < last) {
+    const double a = row.dot(col, val, at);
+    if (lane == 0) {
+      const double pi = at(i), ai = i == gz ? 0.0 : a;
+      p[i] = pi;
+      Ap[i] = ai;
+      acc += pi * ai;
+    }
+    i += kCgGroups;
+    row.load(ptr, col, val, i, i < last, lane);
+  }
+  acc = cg_block_sum(acc, s);
+  if (t == 0) part_pap[blockIdx.x] = acc;
+}
+// x += alpha p, r -= alpha Ap; the preconditioner's head; partial sums of r.r
+// and (part_rz) of r.y
+template <class TY>
+__global__ void __launch_bounds__(kCgThreads)
+    k_cg_update(int64_t n, int parity, const double *part_pap, double *scal, double *x, double *r,
+                const double *p, const double *Ap, Head<TY> head, double *part_rr,
+                double *part_rz) {
+  __shared__ double s[2 * kCgThreads / 64];
+  const double part = threadIdx.x < gridDim.x ? part_pap[threadIdx.x] : 0.0;
+  if (scal[5] != 0.0) return;
+  const double pap = cg_block_sum(part, s);
+  const double alpha = (pap > 0.0) ? scal[parity] / pap : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (pap > 0.0) {
+      scal[6] += 1.0;
+    } else {
+      // p.Ap <= 0 (or NaN) with a nonzero residual: the matrix is not
+      // positive definite on the search space.  The breakdown flag ends the
+      // iteration at the next stopping test (alpha = 0 leaves x and r
+      // unchanged in every block).
       scal[7] = 1.0;
-      scal[5] = 1.0;
     }
   }
-  double c = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)kVB + threadIdx.x; i < n; i += (int64_t)kVGrid * kVB) {
+  double c[2] = {0.0, 0.0};
+  int64_t first, last;
+  cg_rows(n, first, last);
+  for (int64_t i = first + threadIdx.x; i < last; i += kCgThreads) {
     x[i] += alpha * p[i];
     const double ri = r[i] - alpha * Ap[i];
     r[i] = ri;
-    c += ri * ri;
+    c[0] += ri * ri;
+    c[1] += head(i, ri);
   }
-  c = block_sum(c, s);
-  if (threadIdx.x == 0) part_rr[blockIdx.x] = c;
+  cg_block_sums(c, s);
+  if (threadIdx.x == 0) {
+    part_rr[blockIdx.x] = c[0];
+    if (part_rz) part_rz[blockIdx.x] = c[1];
+  }
+}
+// The stopping test after the last iteration of a batch (k_cg_spmv of the
+// next one would make the same).
+__global__ void __launch_bounds__(kCgThreads)
+    k_cg_end(const double *part_rr, int np, double *scal, double tol2) {
+  __shared__ double s[kCgThreads / 64];
+  if (scal[5] != 0.0) return;
+  const double rr = cg_block_sum(threadIdx.x < np ? part_rr[threadIdx.x] : 0.0, s);
+  if (threadIdx.x == 0) {
+    scal[2] = rr;
+    if (scal[7] != 0.0 || rr <= tol2 * scal[4]) scal[5] = 1.0;
+  }
 }
 __global__ void k_set_zero_at(double *x, int32_t i) { x[i] = 0.0; }
-// p = z + beta p; writes the new r.z into the other parity slot
-__global__ void __launch_bounds__(kVB) k_cg_dir(int64_t n, int parity, const double *part_rz,
-                                                const double *part_rr, double *scal, double tol2,
-                                                const double *z, double *p) {
-  __shared__ double s[kVB];
-  if (scal[5] != 0.0) return;
-  const double rz_new = reduce_partials(part_rz, s);
-  const double rr = reduce_partials(part_rr, s);
-  const double rz = scal[parity];
-  const double beta = (rz > 0.0) ? rz_new / rz : 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)kVB + threadIdx.x; i < n; i += (int64_t)kVGrid * kVB)
-    p[i] = z[i] + beta * p[i];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    scal[1 - parity] = rz_new;
-    scal[2] = rr;
-    scal[6] += 1.0;
-    if (rr <= tol2 * scal[4]) scal[5] = 1.0;
-  }
-}
-// Stop the remaining launches of a batch once converged.
-__global__ void k_noop() {}
 
 // Reductions for the Newton driver: min m, ||m - nu||^2, max |m-nu|/nu, nu.w,
 // sum(m - nu).  g = m - nu is written.
@@ -392,37 +409,40 @@ static ma_status weight_floor(ma_engine *e, const double *w, const double *nu, d
   return MA_OK;
 }
 
-// Work vectors and scalars of one conjugate-gradient solve (n entries each;
-// part_*: kVGrid partial sums, part_sp: kSpGrid; scal: 8 scalars).
+// Work vectors and scalars of one conjugate-gradient solve (n entries each,
+// p twice; part_*: up to kCgGrid partial sums; scal: 8 scalars).
 struct CgWork {
-  double *r, *z, *p, *Ap, *part_a, *part_b, *part_c, *part_sp, *scal;
+  double *r, *z, *p[2], *Ap, *part_rz, *part_rr, *part_pap, *scal;
 };
 
 // The iterations of the preconditioned conjugate gradient on M0 (see
-// k_spmv_dot for gz), from x = 0, on the engine's stream.  precondition()
-// launches z = P r.  Iterations run in batches; the scalars stay on the
+// k_cg_spmv for gz), from x = 0, on the engine's stream.  head: what the
+// preconditioner takes from the kernels that write r; precondition() launches
+// the rest of z = P r and leaves nrz partial sums of r.z (0: the head is the
+// whole preconditioner).  Iterations run in batches; the scalars stay on the
 // device and the host checks the converged flag once per batch.  With
-// use_graph a batch is recorded once into a HIP graph (kernel nodes only)
-// and replayed.  Returns MA_SINGULAR on a breakdown (p.Ap <= 0) and
+// use_graph the batches of a long solve are recorded once into a HIP graph
+// (kernel nodes only) and replayed.  Returns MA_SINGULAR on a breakdown (p.Ap <= 0) and
 // MA_LINEAR_FAIL when maxiter iterations end above rel_tol (the residual
 // check of include/MA/optimal_transport.hpp:67-79); x, *iters and *rel_res
 // are set in every case.
-template <class Precond>
+template <class TY, class Precond>
 static ma_status cg_iterate(ma_engine *e, int64_t n, const int32_t *ptr, const int32_t *col,
                             const double *val, int32_t gz, const double *b, int32_t gi,
-                            double *x, const CgWork &W, Precond precondition, double rel_tol,
-                            int maxiter, int batch, bool use_graph, int64_t *iters,
-                            double *rel_res) {
+                            double *x, const CgWork &W, Head<TY> head, int nrz,
+                            Precond precondition, double rel_tol, int maxiter, int batch,
+                            bool use_graph, int64_t *iters, double *rel_res) {
   *iters = 0;
   *rel_res = 0.0;
   double *scal = W.scal;
-  hipLaunchKernelGGL(k_cg_begin, dim3(kVGrid), dim3(kVB), 0, e->stream, n, b, gi, x, W.r,
-                     W.part_b, scal);
+  const int np = cg_grid(n);
+  const dim3 grid(np), block(kCgThreads);
+  double *head_rz = nrz ? nullptr : W.part_rz;  // r.y is r.z
+  if (!nrz) nrz = np;
+  hipLaunchKernelGGL(k_cg_begin<TY>, grid, block, 0, e->stream, n, b, gi, x, W.r, head, W.part_rr,
+                     head_rz, scal);
+  hipLaunchKernelGGL(k_cg_scal_init, dim3(1), block, 0, e->stream, W.part_rr, np, scal);
   MA_HIP_TRY(precondition());
-  hipLaunchKernelGGL(k_dot_rz, dim3(kVGrid), dim3(kVB), 0, e->stream, n, W.r, W.z, W.p,
-                     W.part_a, scal);
-  hipLaunchKernelGGL(k_cg_scal_init, dim3(1), dim3(kVB), 0, e->stream, W.part_a, W.part_b,
-                     scal);
   const double tol2 = rel_tol * rel_tol;
   double sc[8];
   MA_HIP_TRY(hipMemcpyAsync(sc, scal, sizeof sc, hipMemcpyDeviceToHost, e->stream));
@@ -432,36 +452,38 @@ static ma_status cg_iterate(ma_engine *e, int64_t n, const int32_t *ptr, const i
   auto launch = [&](int it0, int count) -> hipError_t {
     for (int q = 0; q < count; q++) {
       const int parity = (it0 + q) & 1;
-      hipLaunchKernelGGL(k_spmv_dot, dim3(kSpGrid), dim3(kVB), 0, e->stream, n, ptr, col, val,
-                         W.p, W.Ap, W.part_sp, scal, gz);
-      hipLaunchKernelGGL(k_fold_partials, dim3(kVGrid / kVB), dim3(kVB), 0, e->stream,
-                         W.part_sp, W.part_c, scal);
-      hipLaunchKernelGGL(k_cg_update, dim3(kVGrid), dim3(kVB), 0, e->stream, n, parity,
-                         W.part_c, scal, x, W.r, W.p, W.Ap, W.part_b);
+      hipLaunchKernelGGL(k_cg_spmv, grid, block, 0, e->stream, n, parity, ptr, col, val, W.z,
+                         W.p[1 - parity], W.p[parity], W.Ap, W.part_rz, nrz, W.part_rr,
+                         W.part_pap, scal, tol2, gz);
+      hipLaunchKernelGGL(k_cg_update<TY>, grid, block, 0, e->stream, n, parity, W.part_pap, scal,
+                         x, W.r, W.p[parity], W.Ap, head, W.part_rr, head_rz);
       MA_HIP_RET(precondition());
-      hipLaunchKernelGGL(k_dot_rz, dim3(kVGrid), dim3(kVB), 0, e->stream, n, W.r, W.z,
-                         (double *)nullptr, W.part_a, scal);
-      hipLaunchKernelGGL(k_cg_dir, dim3(kVGrid), dim3(kVB), 0, e->stream, n, parity, W.part_a,
-                         W.part_b, scal, tol2, W.z, W.p);
     }
+    hipLaunchKernelGGL(k_cg_end, dim3(1), block, 0, e->stream, W.part_rr, np, scal, tol2);
     return hipGetLastError();
   };
+  // Recording and instantiating a graph costs as much as some 20 replays of it
+  // (60-90 launches each) save: with the graph from the first batch a Newton
+  // solve of N = 1000 took 17.6 ms against 16.8 ms without, from the 8th of 18
+  // batches on 150k rows 11.1 against 11.0 ms.  Solves that have run longer
+  // than that replay the rest.
+  constexpr int kGraphFrom = 32;  // batches launched one by one before
   hipGraphExec_t exec = nullptr;
-  if (use_graph && maxiter >= batch) {
-    hipGraph_t graph = nullptr;
-    MA_HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    const hipError_t le = launch(0, batch);
-    const hipError_t ce = hipStreamEndCapture(e->stream, &graph);
-    MA_HIP_TRY(le);
-    MA_HIP_TRY(ce);
-    const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    MA_HIP_TRY(ie);
-  }
   int it = 0;
   hipError_t err = hipSuccess;
   while (it < maxiter) {
     const int count = std::min(batch, maxiter - it);
+    if (use_graph && !exec && it >= kGraphFrom * batch && count == batch) {
+      hipGraph_t graph = nullptr;
+      MA_HIP_TRY(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
+      const hipError_t le = launch(0, batch);
+      const hipError_t ce = hipStreamEndCapture(e->stream, &graph);
+      MA_HIP_TRY(le);
+      MA_HIP_TRY(ce);
+      const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+      (void)hipGraphDestroy(graph);
+      MA_HIP_TRY(ie);
+    }
     if (exec && count == batch)
       err = hipGraphLaunch(exec, e->stream);
     else
@@ -512,11 +534,12 @@ static ma_status pcg(ma_engine *e, const CsrView &M, int32_t gi, const double *b
   MA_HIP_TRY(S.r.ensure((size_t)n));
   MA_HIP_TRY(S.z.ensure((size_t)n));
   MA_HIP_TRY(S.p.ensure((size_t)n));
+  MA_HIP_TRY(S.q.ensure((size_t)n));
   MA_HIP_TRY(S.Ap.ensure((size_t)n));
-  MA_HIP_TRY(S.red.ensure(4 * kVGrid + 16));
-  MA_HIP_TRY(S.red_sp.ensure(kSpGrid));
-  CgWork W{S.r.p, S.z.p, S.p.p, S.Ap.p, S.red.p, S.red.p + kVGrid, S.red.p + 2 * kVGrid,
-           S.red_sp.p, S.red.p + 4 * kVGrid};
+  MA_HIP_TRY(S.red.ensure(5 * kVGrid + 16));
+  static_assert(3 * kCgGrid <= 5 * kVGrid, "partial sums");
+  CgWork W{S.r.p, S.z.p, {S.p.p, S.q.p}, S.Ap.p, S.red.p, S.red.p + kCgGrid,
+           S.red.p + 2 * kCgGrid, S.red.p + 5 * kVGrid};
   if (!e->amg) e->amg = amg_create();
   {
     const int levels = precond == 0 ? 0 : 1;  // Jacobi needs level 0 only
@@ -527,28 +550,33 @@ static ma_status pcg(ma_engine *e, const CsrView &M, int32_t gi, const double *b
     if (st != MA_OK) return st;
   }
   const double *val = amg_level0_values(*e->amg), *dinv = amg_level0_dinv(*e->amg);
-  auto precondition = [&]() -> hipError_t {
-    if (precond == 0) return amg_apply(e, *e->amg, W.r, W.z, W.scal + 5);
-    hipLaunchKernelGGL(k_jacobi, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, n,
-                       dinv, W.r, W.z, W.scal);
-    return hipGetLastError();
-  };
-  return cg_iterate(e, n, M.ptr, M.col, val, -1, b, gi, x, W, precondition, rel_tol, maxiter,
-                    precond == 0 ? 8 : 32, e->use_graphs != 0, iters, rel_res);
+  if (precond != 0)
+    return cg_iterate(e, n, M.ptr, M.col, val, -1, b, gi, x, W, Head<double>{dinv, W.z, 1.0}, 0,
+                      [] { return hipGetLastError(); }, rel_tol, maxiter, 32, e->use_graphs != 0,
+                      iters, rel_res);
+  auto cycle = [&]() { return amg_apply(e, *e->amg, W.r, W.z, W.part_rz, W.scal + 5); };
+  const AmgHead h = amg_head(e, *e->amg);
+  if (h.fp32)
+    return cg_iterate(e, n, M.ptr, M.col, val, -1, b, gi, x, W,
+                      Head<float>{(const float *)h.dinv, (float *)h.y, h.omega}, h.partials, cycle,
+                      rel_tol, maxiter, 8, e->use_graphs != 0, iters, rel_res);
+  return cg_iterate(e, n, M.ptr, M.col, val, -1, b, gi, x, W,
+                    Head<double>{(const double *)h.dinv, (double *)h.y, h.omega}, h.partials,
+                    cycle, rel_tol, maxiter, 8, e->use_graphs != 0, iters, rel_res);
 }
 
 // ---------------------------------------------------------------------------
 // ma_solve_laplacian_csr_noalloc: the work memory of its conjugate gradient
 // is this fixed device array (one copy per GPU, held until the process
-// ends), carved into the Jacobi diagonal, four vectors of MA_NOALLOC_MAX_N
+// ends), carved into the Jacobi diagonal, five vectors of MA_NOALLOC_MAX_N
 // entries, the partial sums, the scalars and two status flags.  Host code
 // never passes `scratch` itself to a kernel (in host code the name is a
 // stand-in, not a device address): ma_create looks up its address on each
 // device once (scratch_ptr) and every launch uses that address.
 // ---------------------------------------------------------------------------
 constexpr int64_t kNaN = MA_NOALLOC_MAX_N;
-constexpr size_t kNaVec = 5 * (size_t)kNaN;                 // dinv, r, z, p, Ap
-constexpr size_t kNaDoubles = kNaVec + kSpGrid + 4 * kVGrid + 16 + 2;
+constexpr size_t kNaVec = 6 * (size_t)kNaN;                 // dinv, r, z, p (2), Ap
+constexpr size_t kNaDoubles = kNaVec + 3 * kCgGrid + 16 + 2;
 static __device__ __align__(256) double scratch[kNaDoubles];
 
 constexpr int kMaxDevices = 64;
@@ -1117,11 +1145,10 @@ ma_status ma_solve_laplacian_csr_noalloc(ma_engine *e, int64_t n, int64_t nnz,
     return MA_HIP_ERROR;
   }
   double *dinv = base;
-  CgWork W{base + kNaN,     base + 2 * kNaN,          base + 3 * kNaN,
-           base + 4 * kNaN, base + kNaVec,            base + kNaVec + kVGrid,
-           base + kNaVec + 2 * kVGrid, base + kNaVec + 4 * kVGrid + 16,
-           base + kNaVec + 4 * kVGrid};
-  int32_t *flags = reinterpret_cast<int32_t *>(base + kNaVec + 4 * kVGrid + 16 + kSpGrid);
+  double *sums = base + kNaVec;
+  CgWork W{base + kNaN, base + 2 * kNaN, {base + 3 * kNaN, base + 4 * kNaN}, base + 5 * kNaN, sums,
+           sums + kCgGrid, sums + 2 * kCgGrid, sums + 3 * kCgGrid};
+  int32_t *flags = reinterpret_cast<int32_t *>(sums + 3 * kCgGrid + 16);
   const int32_t gi = (int32_t)(n - 1);  // gauge: the last unknown, as ma_solve_laplacian_csr
   hipLaunchKernelGGL(k_na_clear, dim3(1), dim3(64), 0, e->stream, flags);
   hipLaunchKernelGGL(k_na_check, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, n,
@@ -1138,15 +1165,11 @@ ma_status ma_solve_laplacian_csr_noalloc(ma_engine *e, int64_t n, int64_t nnz,
     e->err = "singular matrix: a row other than the gauge row has no positive diagonal entry";
     return MA_SINGULAR;
   }
-  auto precondition = [&]() -> hipError_t {
-    hipLaunchKernelGGL(k_jacobi, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, n,
-                       dinv, W.r, W.z, W.scal);
-    return hipGetLastError();
-  };
   int64_t it = 0;
   double rr = 0.0;
   const ma_status st = cg_iterate(e, n, d_rowptr, d_col, d_val, gi, d_g, gi, d_d, W,
-                                  precondition, rel_tol > 0 ? rel_tol : 1e-12,
+                                  Head<double>{dinv, W.z, 1.0}, 0,
+                                  [] { return hipGetLastError(); }, rel_tol > 0 ? rel_tol : 1e-12,
                                   maxiter > 0 ? maxiter : 100000, 32, false, &it, &rr);
   if (res) *res = rr;
   if (iters) *iters = it;

@@ -68,21 +68,6 @@ __device__ inline double wdiff(const double *lo, double hk, int64_t k, double hj
   return s + (err + (lo[k] - lo[j]));
 }
 
-// Sparse row times vector by a group of kRowLanes consecutive lanes: lane l
-// takes entries l, l + kRowLanes, ... of row i, so a wave reads consecutive
-// entries of consecutive rows (coalesced); every lane of the group returns
-// the sum.  All lanes of the group must call it (valid = false: no row).
-constexpr int kRowLanes = 8;
-__device__ inline double row_dot(const int32_t *__restrict__ ptr, const int32_t *__restrict__ col,
-                                 const double *__restrict__ val, const double *__restrict__ x,
-                                 int64_t i, bool valid, int lane) {
-  double s = 0.0;
-  if (valid)
-    for (int32_t q = ptr[i] + lane; q < ptr[i + 1]; q += kRowLanes) s += val[q] * x[col[q]];
-  for (int o = 1; o < kRowLanes; o <<= 1) s += __shfl_xor(s, o, kRowLanes);
-  return s;
-}
-
 __device__ inline void tri_bbox(const TriData &t, double &x0, double &y0, double &x1,
                                 double &y1) {
   x0 = fmin(t.x[0], fmin(t.x[1], t.x[2]));

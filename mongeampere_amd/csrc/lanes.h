@@ -4,6 +4,8 @@
 // independent.
 #pragma once
 
+#include <algorithm>
+
 #include "geom_common.h"
 
 namespace ma {
@@ -62,6 +64,13 @@ __device__ inline T row_sum(T v) {
   v += dpp<kDppRor + 4>(v);
   v += dpp<kDppRor + 2>(v);
   return v + dpp<kDppRor + 1>(v);
+}
+// sum over aligned groups of 8 lanes (quad permutations, then the mirror
+// image within 8)
+__device__ inline double oct_sum(double v) {
+  v += dpp<0xB1>(v);   // quad_perm 1,0,3,2
+  v += dpp<0x4E>(v);   // quad_perm 2,3,0,1
+  return v + dpp<0x141>(v);  // row_half_mirror
 }
 // inclusive prefix sum over the row
 __device__ inline int row_scan(int v) {
@@ -141,4 +150,86 @@ __device__ inline double box_min(const NodeBox &q, double tx, double ty, double 
 }
 // rounding allowance of a bound: its terms carry errors of a few 1e-16
 constexpr double kPlaneEps = 1e-13;
+
+// ---------------------------------------------------------------------------
+// Sparse rows and sums of the conjugate gradient.  A row is read by a group
+// of kRowLanes consecutive lanes, lane l taking entries l, l + kRowLanes, ...,
+// so that a wave reads consecutive entries of consecutive rows.  The kernels
+// that leave partial sums run cg_grid(n) workgroups of kCgThreads threads: at
+// most all of the chip's wave slots at once, and few enough partial sums that
+// every workgroup of the next kernel can add all of them up itself (in the
+// same order: the scalars agree everywhere and from run to run).  4096
+// workgroups of 256 threads took a launch of their own to fold the sums.
+// Several rows of a group at once (2 or 4) made the kernels slower: 150k rows
+// 10.2 -> 10.9 -> 14.9 us, 1k rows 4.0 -> 5.4 -> 6.6.
+// ---------------------------------------------------------------------------
+constexpr int kRowLanes = 8;
+constexpr int kCgGrid = 512, kCgThreads = 1024;
+constexpr int kCgGroups = kCgThreads / kRowLanes;  // rows of a workgroup at a time
+static inline int cg_grid(int64_t n) {
+  return (int)std::min<int64_t>(kCgGrid, (n + kCgGroups / 8 - 1) / (kCgGroups / 8));
+}
+// Workgroup b's share of nb when every XCD takes a run of consecutive ones:
+// neighbouring rows, and the same rows in kernel after kernel, meet in one L2.
+__device__ inline int64_t xcd_share(int64_t b, int64_t nb) {
+  const int64_t x = b % kXcds, q = nb / kXcds, r = nb % kXcds;
+  return x * q + min(x, r) + b / kXcds;
+}
+// the workgroup's rows [first, last) of n
+__device__ inline void cg_rows(int64_t n, int64_t &first, int64_t &last) {
+  const int64_t nb = gridDim.x, b = xcd_share(blockIdx.x, nb);
+  first = n * b / nb;
+  last = n * (b + 1) / nb;
+}
+// A row's first entries, loaded ahead of what decides whether they are needed
+// (the done flag, the scalars of the iteration).
+template <class T>
+struct RowHead {
+  int32_t q, e, c;
+  T v;
+  __device__ inline void load(const int32_t *__restrict__ ptr, const int32_t *__restrict__ col,
+                              const T *__restrict__ val, int64_t i, bool valid, int lane) {
+    q = e = c = 0;
+    v = (T)0;
+    if (!valid) return;
+    q = ptr[i] + lane;
+    e = ptr[i + 1];
+    if (q < e) {  // (the matrix may hold no entry at all)
+      c = col[q];
+      v = val[q];
+    }
+  }
+  // the row times x(j), FP64 accumulation, on every lane of the group
+  template <class X>
+  __device__ inline double dot(const int32_t *__restrict__ col, const T *__restrict__ val,
+                               X &&x) const {
+    double s = q < e ? (double)v * x(c) : 0.0;
+    for (int32_t k = q + kRowLanes; k < e; k += kRowLanes) s += (double)val[k] * x(col[k]);
+    return oct_sum(s);
+  }
+};
+// sums over the workgroup (kCgThreads threads), on every thread; s holds N
+// values per wave
+template <int N>
+__device__ inline void cg_block_sums(double (&v)[N], double *s) {
+  constexpr int kWaves = kCgThreads / 64;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    v[k] = row_sum(v[k]);
+    v[k] += __shfl_xor(v[k], 16);
+    v[k] += __shfl_xor(v[k], 32);
+    if (threadIdx.x % 64 == 0) s[k * kWaves + threadIdx.x / 64] = v[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; k++) v[k] = row_sum(s[k * kWaves + threadIdx.x % kWaves]);
+  __syncthreads();
+}
+static_assert(kCgThreads / 64 == kGroup, "one row of lanes adds up the waves");
+__device__ inline double cg_block_sum(double v, double *s) {
+  double a[1] = {v};
+  cg_block_sums(a, s);
+  return a[0];
+}
+
 }  // namespace ma
