@@ -598,17 +598,12 @@ static ma_status amg_build(ma_engine *e, Amg &A, const CsrView &M) {
     hipLaunchKernelGGL((wave ? k_amg_coarse_wave<false, T> : k_amg_coarse<false, T>), grid,
                        dim3(kVB2), 0, e->stream, nc, nf, fptr, fcol, fval, C.ptr.p, nullptr,
                        nullptr, nullptr);
-    const int32_t zero = 0;
-    MA_HIP_TRY(hipMemcpyAsync(C.ptr.p + nc, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
-                              e->stream));
-    MA_HIP_TRY(exclusive_scan(e, C.ptr.p, C.ptr.p, nc + 1));
+    MA_HIP_TRY(exclusive_scan(e, C.ptr.p, C.ptr.p, nc));
     // small levels take room for as many entries as the level above has,
     // instead of waiting for their count
     if (!wave) {
       int32_t nnzc = 0;
-      MA_HIP_TRY(hipMemcpyAsync(&nnzc, C.ptr.p + nc, sizeof(int32_t), hipMemcpyDeviceToHost,
-                                e->stream));
-      MA_HIP_TRY(hipStreamSynchronize(e->stream));
+      MA_HIP_TRY(read_back(e, {{&nnzc, C.ptr.p + nc, sizeof(int32_t)}}));
       room = nnzc;
     }
     room = std::min(room, nc * nc);
@@ -656,8 +651,7 @@ ma_status amg_setup(ma_engine *e, Amg &A, const CsrView &M, int32_t gi, int max_
   hipLaunchKernelGGL(k_amg_level0, dim3(nb2(n)), dim3(kVB2), 0, e->stream, n, M.ptr, M.col,
                      M.val, gi, A.val0.p, A.dinv0.p, valf, dinvf, A.bad.p);
   int32_t bad = 0;
-  MA_HIP_TRY(hipMemcpyAsync(&bad, A.bad.p, sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(read_back(e, {{&bad, A.bad.p, sizeof(int32_t)}}));
   if (bad) {
     // include/MA/optimal_transport.hpp:48-58 reports zero diagonal entries
     // of the gauge-fixed matrix the same way (its Cholesky cannot proceed)

@@ -1905,7 +1905,6 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   a.fo = e->fo;
   if (mode != 1) a.fo.count = nullptr;
   for (int i = 0; i < 4; i++) a.dom[i] = e->dom[i];
-  const int32_t zero = 0;
   PyrOff po{};
   for (int l = 0; l <= e->grid.L; l++) po.o[l] = e->pyr_off[l];
   const Plane *planes = reinterpret_cast<const Plane *>(B.plane.p);
@@ -1920,10 +1919,9 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
   {
     int32_t fl0[4];
     unsigned long long ct0[8], st[48 * 16];
-    MA_HIP_TRY(hipMemcpyAsync(fl0, B.flags.p, sizeof fl0, hipMemcpyDeviceToHost, e->stream));
-    MA_HIP_TRY(hipMemcpyAsync(ct0, B.counters.p, sizeof ct0, hipMemcpyDeviceToHost, e->stream));
-    MA_HIP_TRY(hipMemcpyAsync(st, B.stripes.p, sizeof st, hipMemcpyDeviceToHost, e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
+    MA_HIP_TRY(read_back(e, {{fl0, B.flags.p, sizeof fl0},
+                             {ct0, B.counters.p, sizeof ct0},
+                             {st, B.stripes.p, sizeof st}}));
     unsigned long long nwalk = 0, nbins = 0, nfail = 0;
     for (int i = 0; i < 16; i++) {
       nwalk += st[i * 16];
@@ -1963,9 +1961,7 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
         MA_HIP_TRY(hipMemsetAsync(B.flags.p + 2, 0, sizeof(int32_t), e->stream));
         hipLaunchKernelGGL(k_mask_check, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, e->grid, n,
                            e->pos.p, B.pn.p, B.rect.p, B.flags.p + 2);
-        MA_HIP_TRY(hipMemcpyAsync(&outside, B.flags.p + 2, sizeof(int32_t), hipMemcpyDeviceToHost,
-                                  e->stream));
-        MA_HIP_TRY(hipStreamSynchronize(e->stream));
+        MA_HIP_TRY(read_back(e, {{&outside, B.flags.p + 2, sizeof(int32_t)}}));
         if (outside) {
           e->mask_ok = false;
           s = run_bin_candidates(e, B.pn.p, nullptr);
@@ -1977,8 +1973,7 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
       a.cand_start = B.cand_cnt.p;  // (re)allocated by the candidate search
       a.cand = B.cand.p;
       if (ct0[6]) {
-        MA_HIP_TRY(hipMemcpyAsync(B.glist.p + n, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
-                                  e->stream));
+        MA_HIP_TRY(hipMemsetAsync(B.glist.p + n, 0, sizeof(int32_t), e->stream));
         hipLaunchKernelGGL(k_collect, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, B.pn.p,
                            -2, B.glist.p, B.glist.p + n);
         const unsigned nb = nblocks((int64_t)ct0[6], kCellGroups);
@@ -1994,14 +1989,9 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
     }
   }
   MA_HIP_TRY(hipEventRecord(e->ev[3], e->stream));
-  MA_HIP_TRY(hipMemcpyAsync(B.tcount.p + n, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
-                            e->stream));
-  MA_HIP_TRY(exclusive_scan(e, B.tcount.p, B.poff.p, n + 1));
+  MA_HIP_TRY(exclusive_scan(e, B.tcount.p, B.poff.p, n));
   int32_t np = 0, fl[4];
-  MA_HIP_TRY(hipMemcpyAsync(&np, B.poff.p + n, sizeof(int32_t), hipMemcpyDeviceToHost,
-                            e->stream));
-  MA_HIP_TRY(hipMemcpyAsync(fl, B.flags.p, sizeof fl, hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(read_back(e, {{&np, B.poff.p + n, sizeof np}, {fl, B.flags.p, sizeof fl}}));
   MA_HIP_TRY(B.pair_cell.ensure((size_t)np + 1));
   MA_HIP_TRY(B.pair_tri.ensure((size_t)np + 1));
   hipLaunchKernelGGL(k_pairs, dim3(nblocks(n, kCellGroups)), dim3(kCellThreads), 0, e->stream, a,
@@ -2045,13 +2035,10 @@ ma_status run_cells(ma_engine *e, int mode, bool fp32, int32_t *npairs_out,
                        (int)(mode == 3));
   int32_t ng = 0;
   if (fl[3]) {
-    MA_HIP_TRY(hipMemcpyAsync(B.glist.p + n, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
-                              e->stream));
+    MA_HIP_TRY(hipMemsetAsync(B.glist.p + n, 0, sizeof(int32_t), e->stream));
     hipLaunchKernelGGL(k_collect, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, B.pn.p, -1,
                        B.glist.p, B.glist.p + n);
-    MA_HIP_TRY(hipMemcpyAsync(&ng, B.glist.p + n, sizeof(int32_t), hipMemcpyDeviceToHost,
-                              e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
+    MA_HIP_TRY(read_back(e, {{&ng, B.glist.p + n, sizeof(int32_t)}}));
   }
   MA_HIP_TRY(hipGetLastError());
   *npairs_out = np;

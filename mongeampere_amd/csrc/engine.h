@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -201,6 +202,15 @@ struct EvalBuffers {
   DBuf<unsigned char> binmask;  // bins whose candidate owners are built (few cells left over)
 };
 
+// What the calls that copy Diracs in and results out work in.
+struct CopyBuffers {
+  DBuf<double> xy;            // positions (2 n) in the caller's layout, column (n) or results
+  DBuf<double> xi;            // positions, interleaved
+  DBuf<int32_t> bin, cnt;     // bin of a Dirac; entries per bin
+  DBuf<int32_t> ptr, col;     // the Hessian in the caller's order
+  DBuf<double> val;
+};
+
 struct SolverBuffers {
   DBuf<double> w, m, nu, g, d, x, r, z, p, q, Ap, wtrial, red;
   DBuf<double> stage;         // host <-> device staging of per-Dirac arrays
@@ -267,6 +277,8 @@ struct ma_engine {
   int cap_row = ma::kMaxRow;
 
   ma::EvalBuffers eb;
+  ma::CopyBuffers cb;
+  uint32_t *pinned = nullptr;  // kReadBytes of host memory (read_back)
   ma::SolverBuffers sb;
   ma::OutBuffers ob;
   ma::FragOut fo;  // set only while ma_fragments / ma_draw_laguerre run
@@ -325,9 +337,23 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32 = false);
 // Copy helpers between caller order and Morton order.
 hipError_t to_morton(ma_engine *e, const double *src_caller, double *dst_morton, bool src_on_device);
 hipError_t from_morton(ma_engine *e, const double *src_morton, double *dst_caller, bool dst_on_device);
+// out[i] = in[0] + ... + in[i - 1] for i = 0 .. n (out may be in).
 hipError_t exclusive_scan(ma_engine *e, const int32_t *in, int32_t *out, int64_t n);
 hipError_t csr_to_caller(ma_engine *e, int32_t *rowptr, int32_t *col, double *val);
 ma_status adjoint(ma_engine *e, double *dY_caller, double *dval);
+// Words of device memory to the host, up to kReadBytes together: one kernel
+// writes them into the engine's pinned page and the stream is waited for.  (A
+// copy into pageable memory takes a launch, a wait and a host copy each, about
+// 10 us; an evaluation of N = 1000 reads eleven such values.)
+struct ReadPart {
+  void *dst;
+  const void *src;
+  size_t bytes;  // a multiple of 4
+};
+constexpr int kReadParts = 4;
+constexpr size_t kReadBytes = 32768;
+hipError_t read_back(ma_engine *e, std::initializer_list<ReadPart> parts);
+
 // A square CSR matrix on the device.
 struct CsrView {
   int64_t n = 0, nnz = 0;

@@ -335,9 +335,11 @@ __global__ void k_add_const(int64_t n, double *x, double c) {
   if (i < n) x[i] += c;
 }
 
-__global__ void k_split(const double *m, int64_t n, int ncol, int c, double *o) {
-  int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (k < n) o[k] = m[ncol * k + c];
+// rows of ncol components from Morton to the caller's order
+__global__ void k_columns(const double *src, const int32_t *perm, int64_t n, int ncol,
+                          double *out) {
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (t < ncol * n) out[(int64_t)perm[t / ncol] * ncol + t % ncol] = src[t];
 }
 
 struct NewtonStats {
@@ -351,9 +353,7 @@ static hipError_t newton_stats(ma_engine *e, const double *m, const double *nu, 
   hipLaunchKernelGGL(k_newton_stats, dim3(kVGrid), dim3(kVB), 0, e->stream, e->n, m, nu, w, g,
                      S.red.p);
   std::vector<double> h(5 * kVGrid);
-  MA_HIP_RET(hipMemcpyAsync(h.data(), S.red.p, sizeof(double) * 5 * kVGrid,
-                            hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_RET(hipStreamSynchronize(e->stream));
+  MA_HIP_RET(read_back(e, {{h.data(), S.red.p, sizeof(double) * 5 * kVGrid}}));
   st.minm = HUGE_VAL;
   st.maxrel = 0.0;
   double ss = 0.0, dot = 0.0, sg = 0.0;
@@ -402,9 +402,7 @@ static ma_status weight_floor(ma_engine *e, const double *w, const double *nu, d
   hipLaunchKernelGGL(k_weight_floor, dim3(kVGrid), dim3(kVB), 0, e->stream, e->n,
                      e->eb.csr_ptr.p, e->eb.csr_col.p, e->eb.csr_val.p, w, nu, S.red.p);
   std::vector<double> h(kVGrid);
-  MA_HIP_TRY(hipMemcpyAsync(h.data(), S.red.p, sizeof(double) * kVGrid, hipMemcpyDeviceToHost,
-                            e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(read_back(e, {{h.data(), S.red.p, sizeof(double) * kVGrid}}));
   *floor = *std::max_element(h.begin(), h.end());
   return MA_OK;
 }
@@ -445,8 +443,7 @@ static ma_status cg_iterate(ma_engine *e, int64_t n, const int32_t *ptr, const i
   MA_HIP_TRY(precondition());
   const double tol2 = rel_tol * rel_tol;
   double sc[8];
-  MA_HIP_TRY(hipMemcpyAsync(sc, scal, sizeof sc, hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(read_back(e, {{sc, scal, sizeof sc}}));
   if (sc[4] == 0.0) return MA_OK;
   // iterations it0 .. it0 + count - 1 (batch is even: the parity pattern repeats)
   auto launch = [&](int it0, int count) -> hipError_t {
@@ -490,8 +487,7 @@ static ma_status cg_iterate(ma_engine *e, int64_t n, const int32_t *ptr, const i
       err = launch(it, count);
     if (err != hipSuccess) break;
     it += count;
-    err = hipMemcpyAsync(sc, scal, sizeof sc, hipMemcpyDeviceToHost, e->stream);
-    if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
+    err = read_back(e, {{sc, scal, sizeof sc}});
     if (err != hipSuccess || sc[5] != 0.0) break;
   }
   if (exec) (void)hipGraphExecDestroy(exec);
@@ -677,16 +673,12 @@ static ma_status diagram_connected(ma_engine *e, bool *connected) {
     for (int k = 0; k < 32; k++)
       hipLaunchKernelGGL(k_cc_step, dim3(nb), dim3(256), 0, e->stream, n, ptr, col, val, S.cc.p,
                          S.moved.p);
-    MA_HIP_TRY(hipMemcpyAsync(&changed, S.moved.p, sizeof(int32_t), hipMemcpyDeviceToHost,
-                              e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
+    MA_HIP_TRY(read_back(e, {{&changed, S.moved.p, sizeof(int32_t)}}));
   }
   int32_t other = 0;
   MA_HIP_TRY(hipMemsetAsync(S.moved.p, 0, sizeof(int32_t), e->stream));
   hipLaunchKernelGGL(k_cc_any_nonzero, dim3(nb), dim3(256), 0, e->stream, n, S.cc.p, S.moved.p);
-  MA_HIP_TRY(hipMemcpyAsync(&other, S.moved.p, sizeof(int32_t), hipMemcpyDeviceToHost,
-                            e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(read_back(e, {{&other, S.moved.p, sizeof(int32_t)}}));
   *connected = other == 0;
   return MA_OK;
 }
@@ -697,9 +689,7 @@ static hipError_t eval_csr(ma_engine *e, CsrView &M, int32_t &gi) {
   M.ptr = e->eb.csr_ptr.p;
   M.col = e->eb.csr_col.p;
   M.val = e->eb.csr_val.p;
-  MA_HIP_RET(hipMemcpyAsync(&gi, e->iperm.p + (e->n - 1), sizeof(int32_t), hipMemcpyDeviceToHost,
-                            e->stream));
-  return hipStreamSynchronize(e->stream);
+  return read_back(e, {{&gi, e->iperm.p + (e->n - 1), sizeof(int32_t)}});
 }
 
 }  // namespace ma
@@ -790,6 +780,12 @@ ma_status ma_create(int device, ma_engine **out) {
     delete e;
     return MA_HIP_ERROR;
   }
+  if (hipHostMalloc(reinterpret_cast<void **>(&e->pinned), kReadBytes, hipHostMallocDefault) !=
+      hipSuccess) {
+    hipStreamDestroy(e->stream);
+    delete e;
+    return MA_HIP_ERROR;
+  }
   for (auto &ev : e->ev) hipEventCreate(&ev);
   *out = e;
   return MA_OK;
@@ -801,6 +797,7 @@ void ma_destroy(ma_engine *e) {
   hipStreamSynchronize(e->stream);
   for (auto &ev : e->ev) hipEventDestroy(ev);
   hipStreamDestroy(e->stream);
+  (void)hipHostFree(e->pinned);
   if (e->amg) amg_destroy(e->amg);
   // every device buffer is released by its owner's destructor
   delete e;
@@ -910,11 +907,10 @@ ma_status ma_set_diracs(ma_engine *e, int64_t n, const double *X, int layout) {
   e->many_far = false;
   e->n = n;
   choose_grid(e, X, n, layout);
-  DBuf<double> dX;
+  DBuf<double> &dX = e->cb.xy;
   MA_HIP_TRY(dX.ensure((size_t)(2 * n)));
   MA_HIP_TRY(hipMemcpyAsync(dX.p, X, sizeof(double) * 2 * n, hipMemcpyHostToDevice, e->stream));
   MA_HIP_TRY(build_dirac_grid(e, dX.p, layout));
-  dX.release();
   e->have_diracs = true;
   return MA_OK;
 }
@@ -1006,16 +1002,14 @@ ma_status ma_cell_costs(ma_engine *e, double *cost) {
 // Copies an interleaved per-Dirac array of `ncol` components from Morton
 // order on the device to the caller's order on the host.
 static hipError_t columns_to_host(ma_engine *e, const double *src, int ncol, double *dst) {
-  std::vector<double> col((size_t)e->n);
-  DBuf<double> tmp;
-  MA_HIP_RET(tmp.ensure((size_t)e->n));
-  for (int c = 0; c < ncol; c++) {
-    hipLaunchKernelGGL(k_split, dim3((unsigned)((e->n + 127) / 128)), dim3(128), 0, e->stream,
-                       src, e->n, ncol, c, tmp.p);
-    MA_HIP_RET(from_morton(e, tmp.p, col.data(), false));
-    for (int64_t i = 0; i < e->n; i++) dst[ncol * i + c] = col[i];
-  }
-  return hipSuccess;
+  DBuf<double> &out = e->cb.xy;
+  MA_HIP_RET(out.ensure((size_t)(ncol * e->n)));
+  hipLaunchKernelGGL(k_columns, dim3((unsigned)((ncol * e->n + 127) / 128)), dim3(128), 0,
+                     e->stream, src, e->perm.p, e->n, ncol, out.p);
+  MA_HIP_RET(hipGetLastError());
+  MA_HIP_RET(hipMemcpyAsync(dst, out.p, sizeof(double) * ncol * e->n, hipMemcpyDeviceToHost,
+                            e->stream));
+  return hipStreamSynchronize(e->stream);
 }
 
 ma_status ma_first_moment(ma_engine *e, const double *w, double *mass, double *mom) {
@@ -1154,8 +1148,7 @@ ma_status ma_solve_laplacian_csr_noalloc(ma_engine *e, int64_t n, int64_t nnz,
   hipLaunchKernelGGL(k_na_check, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, e->stream, n,
                      nnz, d_rowptr, d_col, d_val, gi, dinv, flags);
   int32_t hf[2] = {0, 0};
-  MA_HIP_TRY(hipMemcpyAsync(hf, flags, sizeof hf, hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(read_back(e, {{hf, flags, sizeof hf}}));
   if (hf[0]) {
     e->err = "CSR matrix: row pointers must run from 0 to nnz without decreasing and columns "
              "must lie in [0, n)";
@@ -1368,9 +1361,7 @@ ma_status ma_ot_solve_x(ma_engine *e, const double *nu, double *w, double *w_lo,
         hipLaunchKernelGGL(k_axpy_to, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                            e->stream, n, S.w.p, alpha, S.d.p, S.wtrial.p, S.moved.p);
       int32_t moved = 0;
-      MA_HIP_TRY(hipMemcpyAsync(&moved, S.moved.p, sizeof(int32_t), hipMemcpyDeviceToHost,
-                                e->stream));
-      MA_HIP_TRY(hipStreamSynchronize(e->stream));
+      MA_HIP_TRY(read_back(e, {{&moved, S.moved.p, sizeof(int32_t)}}));
       if (!moved) {
         // alpha d is below half an ulp of every weight: the trial point is
         // the iterate itself, and so is every shorter step (the weights'
@@ -1572,14 +1563,13 @@ ma_status adjoint(ma_engine *e, double *dY, double *dval) {
   ma_status s = evaluate(e, 2, nullptr);
   if (s != MA_OK) return s;
   if (dY) {
-    DBuf<double> tmp;
+    DBuf<double> &tmp = e->cb.xy;
     MA_HIP_TRY(tmp.ensure((size_t)(2 * e->n)));
     hipLaunchKernelGGL(k_adjoint_dy, dim3((unsigned)((e->n + 127) / 128)), dim3(128), 0,
                        e->stream, e->n, e->perm.p, B.mom_s.p, tmp.p);
     MA_HIP_TRY(hipMemcpyAsync(dY, tmp.p, sizeof(double) * 2 * e->n, hipMemcpyDeviceToHost,
                               e->stream));
     MA_HIP_TRY(hipStreamSynchronize(e->stream));
-    tmp.release();
   }
   if (dval) {
     MA_HIP_TRY(hipMemcpyAsync(dval, B.dval.p, sizeof(double) * e->nv, hipMemcpyDeviceToHost,

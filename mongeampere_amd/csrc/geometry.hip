@@ -12,6 +12,7 @@
 #include <cfloat>
 #include <climits>
 #include <cmath>
+#include <cstring>
 
 #include "geom_common.h"
 #include "lanes.h"
@@ -21,7 +22,8 @@ namespace ma {
 // ---------------------------------------------------------------------------
 // Exclusive prefix sum of int32 (wave64 shuffles, 1024 elements per block).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_scan_block(const int32_t *in, int32_t *out,
+// (entries from nin on count as 0)
+__global__ void __launch_bounds__(256) k_scan_block(const int32_t *in, int64_t nin, int32_t *out,
                                                      int32_t *sums, int64_t n) {
   __shared__ int32_t ws[8];
   const int tid = threadIdx.x;
@@ -31,7 +33,7 @@ __global__ void __launch_bounds__(256) k_scan_block(const int32_t *in, int32_t *
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     int64_t idx = base + i;
-    v[i] = idx < n ? in[idx] : 0;
+    v[i] = idx < nin ? in[idx] : 0;
     s += v[i];
   }
   const int lane = tid & 63, wid = tid >> 6;
@@ -72,8 +74,7 @@ __global__ void __launch_bounds__(256) k_scan_add(int32_t *out, const int32_t *o
 }
 
 hipError_t exclusive_scan(ma_engine *e, const int32_t *in, int32_t *out, int64_t n) {
-  if (n <= 0) return hipSuccess;
-  std::vector<int64_t> len{n};
+  std::vector<int64_t> len{n + 1};
   while (len.back() > 1024) len.push_back((len.back() + 1023) / 1024);
   int64_t tmp = 0;
   for (size_t l = 1; l < len.size(); l++) tmp += len[l];
@@ -89,7 +90,7 @@ hipError_t exclusive_scan(ma_engine *e, const int32_t *in, int32_t *out, int64_t
     const int32_t *src = (l == 0) ? in : buf[l];
     int32_t *sums = (l + 1 < len.size()) ? buf[l + 1] : nullptr;
     hipLaunchKernelGGL(k_scan_block, dim3((unsigned)((len[l] + 1023) / 1024)), dim3(256), 0,
-                       e->stream, src, buf[l], sums, len[l]);
+                       e->stream, src, l == 0 ? n : len[l], buf[l], sums, len[l]);
   }
   for (size_t l = len.size() - 1; l-- > 0;) {
     hipLaunchKernelGGL(k_scan_add, dim3((unsigned)((len[l] + 1023) / 1024)), dim3(256), 0,
@@ -101,6 +102,34 @@ hipError_t exclusive_scan(ma_engine *e, const int32_t *in, int32_t *out, int64_t
 // ---------------------------------------------------------------------------
 // Small helpers
 // ---------------------------------------------------------------------------
+struct ReadSrc {
+  const uint32_t *src[kReadParts];
+  int words[kReadParts];
+};
+__global__ void __launch_bounds__(256) k_read_back(ReadSrc s, uint32_t *out) {
+  for (int k = 0; k < kReadParts; out += s.words[k++])
+    for (int i = threadIdx.x; i < s.words[k]; i += 256) out[i] = s.src[k][i];
+}
+hipError_t read_back(ma_engine *e, std::initializer_list<ReadPart> parts) {
+  ReadSrc s{};
+  int k = 0;
+  size_t bytes = 0;
+  for (const ReadPart &p : parts) {
+    bytes += p.bytes;
+    if (k == kReadParts || bytes > kReadBytes || p.bytes % 4) return hipErrorInvalidValue;
+    s.src[k] = static_cast<const uint32_t *>(p.src);
+    s.words[k++] = (int)(p.bytes / 4);
+  }
+  hipLaunchKernelGGL(k_read_back, dim3(1), dim3(256), 0, e->stream, s, e->pinned);
+  MA_HIP_RET(hipGetLastError());
+  MA_HIP_RET(hipStreamSynchronize(e->stream));
+  const char *h = reinterpret_cast<const char *>(e->pinned);
+  for (const ReadPart &p : parts) {
+    std::memcpy(p.dst, h, p.bytes);
+    h += p.bytes;
+  }
+  return hipSuccess;
+}
 __global__ void k_fill_i32(int32_t *p, int32_t v, int64_t n) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -152,11 +181,13 @@ __global__ void k_dirac_bin(const double *X, int64_t n, Grid g, int32_t *bin, in
   bin[i] = b;
   atomicAdd(&cnt[b], 1);
 }
-__global__ void k_dirac_scatter(const int32_t *bin, int64_t n, int32_t *cursor, int32_t *perm) {
+// cnt counts down to 0 (k_sort_bins orders the bin afterwards)
+__global__ void k_dirac_scatter(const int32_t *bin, int64_t n, const int32_t *start, int32_t *cnt,
+                                int32_t *perm) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  int32_t s = atomicAdd(&cursor[bin[i]], 1);
-  perm[s] = (int32_t)i;
+  const int32_t b = bin[i];
+  perm[start[b] + atomicSub(&cnt[b], 1) - 1] = (int32_t)i;
 }
 // Sort each bin's item list ascending (lists are short; insertion sort).
 __global__ void k_sort_bins(const int32_t *start, int64_t nb, int32_t *items) {
@@ -192,8 +223,8 @@ __global__ void k_colmajor_to_xy(const double *Xc, int64_t n, double *Xi) {
 hipError_t build_dirac_grid(ma_engine *e, const double *d_X, int layout) {
   const int64_t n = e->n;
   const Grid &g = e->grid;
-  DBuf<double> xi;
-  DBuf<int32_t> bin, cnt;
+  DBuf<double> &xi = e->cb.xi;
+  DBuf<int32_t> &bin = e->cb.bin, &cnt = e->cb.cnt;
   const double *X = d_X;
   if (layout == MA_XY_COLMAJOR) {
     MA_HIP_RET(xi.ensure((size_t)(2 * n)));
@@ -207,29 +238,18 @@ hipError_t build_dirac_grid(ma_engine *e, const double *d_X, int layout) {
   MA_HIP_RET(e->perm.ensure((size_t)n));
   MA_HIP_RET(e->iperm.ensure((size_t)n));
   MA_HIP_RET(e->pos.ensure((size_t)(2 * n)));
-  MA_HIP_RET(hipMemsetAsync(cnt.p, 0, sizeof(int32_t) * (g.nbins + 1), e->stream));
+  MA_HIP_RET(hipMemsetAsync(cnt.p, 0, sizeof(int32_t) * g.nbins, e->stream));
   hipLaunchKernelGGL(k_dirac_bin, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, X, n, g, bin.p,
                      cnt.p);
-  MA_HIP_RET(exclusive_scan(e, cnt.p, e->bin_start.p, g.nbins + 1));
-  MA_HIP_RET(hipMemcpyAsync(cnt.p, e->bin_start.p, sizeof(int32_t) * g.nbins,
-                            hipMemcpyDeviceToDevice, e->stream));
-  DBuf<int32_t> tmp;
-  MA_HIP_RET(tmp.ensure((size_t)n));
+  MA_HIP_RET(exclusive_scan(e, cnt.p, e->bin_start.p, g.nbins));
   hipLaunchKernelGGL(k_dirac_scatter, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, bin.p, n,
-                     cnt.p, tmp.p);
+                     e->bin_start.p, cnt.p, e->perm.p);
   hipLaunchKernelGGL(k_sort_bins, dim3(nblocks(g.nbins)), dim3(kBlock), 0, e->stream,
-                     e->bin_start.p, g.nbins, tmp.p);
-  MA_HIP_RET(hipMemcpyAsync(e->perm.p, tmp.p, sizeof(int32_t) * n, hipMemcpyDeviceToDevice,
-                            e->stream));
+                     e->bin_start.p, g.nbins, e->perm.p);
   hipLaunchKernelGGL(k_gather_pos, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, X, e->perm.p, n,
                      e->pos.p, e->iperm.p);
   MA_HIP_RET(hipGetLastError());
-  MA_HIP_RET(hipStreamSynchronize(e->stream));
-  xi.release();
-  bin.release();
-  cnt.release();
-  tmp.release();
-  return hipSuccess;
+  return hipStreamSynchronize(e->stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -238,8 +258,8 @@ hipError_t build_dirac_grid(ma_engine *e, const double *d_X, int layout) {
 template <bool FILL>
 // A triangle is listed in every bin its FP32 (outward-rounded) bounding box
 // meets (the box group_triangles tests).
-__global__ void k_tbin(const float4 *tbox, int64_t nt, Grid g, int32_t *cnt_or_cursor,
-                       int32_t *items) {
+__global__ void k_tbin(const float4 *tbox, int64_t nt, Grid g, int32_t *cnt,
+                       const int32_t *start, int32_t *items) {
   int64_t f = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (f >= nt) return;
   const float4 tb = tbox[f];
@@ -250,39 +270,33 @@ __global__ void k_tbin(const float4 *tbox, int64_t nt, Grid g, int32_t *cnt_or_c
     for (int bx = bx0; bx <= bx1; bx++) {
       uint32_t b = morton2((uint32_t)bx, (uint32_t)by);
       if (FILL) {
-        int32_t s = atomicAdd(&cnt_or_cursor[b], 1);
+        const int32_t s = start[b] + atomicSub(&cnt[b], 1) - 1;
         items[s] = ((int32_t)f << kTriShift) | (bx == bx0 ? kTriFirstX : 0) |
                    (by == by0 ? kTriFirstY : 0);
       } else {
-        atomicAdd(&cnt_or_cursor[b], 1);
+        atomicAdd(&cnt[b], 1);
       }
     }
 }
 
 hipError_t build_triangle_bins(ma_engine *e) {
   const Grid &g = e->grid;
-  DBuf<int32_t> cnt;
+  DBuf<int32_t> &cnt = e->cb.cnt;
   MA_HIP_RET(cnt.ensure((size_t)g.nbins + 1));
   MA_HIP_RET(e->tbin_start.ensure((size_t)g.nbins + 1));
-  MA_HIP_RET(hipMemsetAsync(cnt.p, 0, sizeof(int32_t) * (g.nbins + 1), e->stream));
+  MA_HIP_RET(hipMemsetAsync(cnt.p, 0, sizeof(int32_t) * g.nbins, e->stream));
   hipLaunchKernelGGL(k_tbin<false>, dim3(nblocks(e->nt)), dim3(kBlock), 0, e->stream, e->tbox.p,
-                     e->nt, g, cnt.p, nullptr);
-  MA_HIP_RET(exclusive_scan(e, cnt.p, e->tbin_start.p, g.nbins + 1));
+                     e->nt, g, cnt.p, nullptr, nullptr);
+  MA_HIP_RET(exclusive_scan(e, cnt.p, e->tbin_start.p, g.nbins));
   int32_t total = 0;
-  MA_HIP_RET(hipMemcpyAsync(&total, e->tbin_start.p + g.nbins, sizeof(int32_t),
-                            hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_RET(hipStreamSynchronize(e->stream));
+  MA_HIP_RET(read_back(e, {{&total, e->tbin_start.p + g.nbins, sizeof(int32_t)}}));
   MA_HIP_RET(e->tbin_items.ensure((size_t)total + 1));
-  MA_HIP_RET(hipMemcpyAsync(cnt.p, e->tbin_start.p, sizeof(int32_t) * g.nbins,
-                            hipMemcpyDeviceToDevice, e->stream));
   hipLaunchKernelGGL(k_tbin<true>, dim3(nblocks(e->nt)), dim3(kBlock), 0, e->stream, e->tbox.p,
-                     e->nt, g, cnt.p, e->tbin_items.p);
+                     e->nt, g, cnt.p, e->tbin_start.p, e->tbin_items.p);
   hipLaunchKernelGGL(k_sort_bins, dim3(nblocks(g.nbins)), dim3(kBlock), 0, e->stream,
                      e->tbin_start.p, g.nbins, e->tbin_items.p);
   MA_HIP_RET(hipGetLastError());
-  MA_HIP_RET(hipStreamSynchronize(e->stream));
-  cnt.release();
-  return hipSuccess;
+  return hipStreamSynchronize(e->stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1704,7 +1718,6 @@ ma_status run_bin_candidates(ma_engine *e, const int32_t *pn, const unsigned cha
   for (int l = 0; l <= g.L; l++) po.o[l] = e->pyr_off[l];
   const Plane *pl = reinterpret_cast<const Plane *>(B.plane.p);
   MA_HIP_TRY(B.cand_cnt.ensure((size_t)g.nbins + 1));
-  const int32_t zero = 0;
   int32_t total = 0;
   // walks of the pyramid per bin: owners and counts (keeping the first
   // kCandStage candidates), then the lists of the bins with more (one walk
@@ -1716,12 +1729,8 @@ ma_status run_bin_candidates(ma_engine *e, const int32_t *pn, const unsigned cha
                      e->bin_start.p, e->pos.p, B.w_s.p, pl, po, B.owner.p, B.cand_cnt.p,
                      (int32_t *)nullptr, (int32_t *)nullptr, B.cstage.p, B.counters.p, mask);
   // offsets, and the total to the host
-  MA_HIP_TRY(hipMemcpyAsync(B.cand_cnt.p + g.nbins, &zero, sizeof(int32_t),
-                            hipMemcpyHostToDevice, e->stream));
-  MA_HIP_TRY(exclusive_scan(e, B.cand_cnt.p, B.cand_cnt.p, g.nbins + 1));
-  MA_HIP_TRY(hipMemcpyAsync(&total, B.cand_cnt.p + g.nbins, sizeof(int32_t),
-                            hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(exclusive_scan(e, B.cand_cnt.p, B.cand_cnt.p, g.nbins));
+  MA_HIP_TRY(read_back(e, {{&total, B.cand_cnt.p + g.nbins, sizeof(int32_t)}}));
   MA_HIP_TRY(B.cand.ensure((size_t)total + 1));
   MA_HIP_TRY(B.cbin.ensure((size_t)total + 1));
   hipLaunchKernelGGL(k_cand_list<true>, grid, block, 0, e->stream, g, e->tbin_start.p,
@@ -1735,7 +1744,7 @@ ma_status run_bin_candidates(ma_engine *e, const int32_t *pn, const unsigned cha
     MA_HIP_TRY(B.cstart2.ensure((size_t)g.nbins + 1));
     ma_status rs = refine_candidates(e, total);
     if (rs != MA_OK) return rs;
-    MA_HIP_TRY(exclusive_scan(e, B.ckeep.p, B.ckeep.p, total + 1));
+    MA_HIP_TRY(exclusive_scan(e, B.ckeep.p, B.ckeep.p, total));
     hipLaunchKernelGGL(k_refine_starts, dim3(nblocks(g.nbins + 1)), dim3(kBlock), 0, e->stream,
                        g.nbins, B.cand_cnt.p, B.ckeep.p, B.cstart2.p);
     hipLaunchKernelGGL(k_refine_move, dim3(nblocks(total)), dim3(kBlock), 0, e->stream,
@@ -1830,9 +1839,7 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
                        B.mass_s.p, B.intg_s.p, B.fval_part.p, B.mom_s.p, B.mom2_s.p, B.row_cnt.p,
                        B.row_col.p, B.row_val.p, e->cap_row, e->triv.p, B.dval.p, B.hlist.p,
                        (int)(e->force_general == 2), B.flags.p, B.counters.p);
-    MA_HIP_TRY(hipMemcpyAsync(&nhuge, B.hlist.p + n, sizeof(int32_t), hipMemcpyDeviceToHost,
-                              e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
+    MA_HIP_TRY(read_back(e, {{&nhuge, B.hlist.p + n, sizeof(int32_t)}}));
   }
   if (nhuge > 0) {
     // the few cells beyond the general kernel: one workgroup each
@@ -1852,14 +1859,9 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
   MA_HIP_TRY(hipEventRecord(e->ev[6], e->stream));
   if (mode == 0) {
     MA_HIP_TRY(B.csr_ptr.ensure((size_t)n + 1));
-    int32_t zero = 0;
-    MA_HIP_TRY(hipMemcpyAsync(B.row_cnt.p + n, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
-                              e->stream));
-    MA_HIP_TRY(exclusive_scan(e, B.row_cnt.p, B.csr_ptr.p, n + 1));
+    MA_HIP_TRY(exclusive_scan(e, B.row_cnt.p, B.csr_ptr.p, n));
     int32_t nnz = 0;
-    MA_HIP_TRY(hipMemcpyAsync(&nnz, B.csr_ptr.p + n, sizeof(int32_t), hipMemcpyDeviceToHost,
-                              e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
+    MA_HIP_TRY(read_back(e, {{&nnz, B.csr_ptr.p + n, sizeof(int32_t)}}));
     MA_HIP_TRY(B.csr_col.ensure((size_t)nnz + 1));
     MA_HIP_TRY(B.csr_val.ensure((size_t)nnz + 1));
     const ma_status rs = fill_rows(e);
@@ -1876,12 +1878,9 @@ ma_status evaluate(ma_engine *e, int mode, double *fval_out, bool fp32) {
   int32_t fl[4];
   unsigned long long ct[kCounters];
   double fv = 0.0;
-  MA_HIP_TRY(hipMemcpyAsync(fl, B.flags.p, sizeof fl, hipMemcpyDeviceToHost, e->stream));
-  MA_HIP_TRY(hipMemcpyAsync(ct, B.counters.p, sizeof ct, hipMemcpyDeviceToHost, e->stream));
-  if (mode == 0)
-    MA_HIP_TRY(hipMemcpyAsync(&fv, B.red_tmp.p + 1024, sizeof(double), hipMemcpyDeviceToHost,
-                              e->stream));
-  MA_HIP_TRY(hipStreamSynchronize(e->stream));
+  MA_HIP_TRY(read_back(e, {{fl, B.flags.p, sizeof fl},
+                           {ct, B.counters.p, sizeof ct},
+                           {&fv, B.red_tmp.p + 1024, mode == 0 ? sizeof fv : 0}}));
   float t[7] = {0, 0, 0, 0, 0, 0, 0}, tc = 0.0f;
   for (int i = 0; i < 7; i++) MA_HIP_TRY(hipEventElapsedTime(&t[i], e->ev[i], e->ev[i + 1]));
   if (e->ran_candidates) MA_HIP_TRY(hipEventElapsedTime(&tc, e->ev[8], e->ev[9]));
@@ -1961,16 +1960,14 @@ __global__ void k_caller_fill(int64_t n, const int32_t *iperm, const int32_t *pe
 
 hipError_t csr_to_caller(ma_engine *e, int32_t *rowptr, int32_t *col, double *val) {
   const int64_t n = e->n;
-  DBuf<int32_t> cnt, optr, ocol;
-  DBuf<double> oval;
-  MA_HIP_RET(cnt.ensure((size_t)n + 1));
+  DBuf<int32_t> &optr = e->cb.ptr, &ocol = e->cb.col;
+  DBuf<double> &oval = e->cb.val;
   MA_HIP_RET(optr.ensure((size_t)n + 1));
   MA_HIP_RET(ocol.ensure((size_t)e->nnz + 1));
   MA_HIP_RET(oval.ensure((size_t)e->nnz + 1));
-  MA_HIP_RET(hipMemsetAsync(cnt.p, 0, sizeof(int32_t) * (n + 1), e->stream));
   hipLaunchKernelGGL(k_caller_cnt, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, e->iperm.p,
-                     e->eb.csr_ptr.p, cnt.p);
-  MA_HIP_RET(exclusive_scan(e, cnt.p, optr.p, n + 1));
+                     e->eb.csr_ptr.p, optr.p);
+  MA_HIP_RET(exclusive_scan(e, optr.p, optr.p, n));
   hipLaunchKernelGGL(k_caller_fill, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, e->iperm.p,
                      e->perm.p, e->eb.csr_ptr.p, e->eb.csr_col.p, e->eb.csr_val.p, optr.p,
                      ocol.p, oval.p);
@@ -1980,12 +1977,7 @@ hipError_t csr_to_caller(ma_engine *e, int32_t *rowptr, int32_t *col, double *va
                             e->stream));
   MA_HIP_RET(hipMemcpyAsync(val, oval.p, sizeof(double) * e->nnz, hipMemcpyDeviceToHost,
                             e->stream));
-  MA_HIP_RET(hipStreamSynchronize(e->stream));
-  cnt.release();
-  optr.release();
-  ocol.release();
-  oval.release();
-  return hipSuccess;
+  return hipStreamSynchronize(e->stream);
 }
 
 }  // namespace ma

@@ -84,8 +84,7 @@ static ma_status emit_fragments(ma_engine *e, int64_t *nf_out, int64_t *nv_out) 
     e->fo = FragOut{};
     if (s != MA_OK) return s;
     unsigned long long c[2];
-    MA_HIP_TRY(hipMemcpyAsync(c, O.fcount.p, sizeof c, hipMemcpyDeviceToHost, e->stream));
-    MA_HIP_TRY(hipStreamSynchronize(e->stream));
+    MA_HIP_TRY(read_back(e, {{c, O.fcount.p, sizeof c}}));
     if ((int64_t)c[0] <= cf && (int64_t)c[1] <= cv) {
       *nf_out = (int64_t)c[0];
       *nv_out = (int64_t)c[1];
