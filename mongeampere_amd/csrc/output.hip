@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "geom_common.h"
+#include "lanes.h"
 
 namespace ma {
 
@@ -260,9 +261,22 @@ struct RasterArgs {
   int32_t *big_n;
 };
 
-constexpr int kRasterSmall = 16;  // pixels a thread covers by itself
+// A fragment of up to this many pixels is covered by a group of 16 lanes, a
+// pixel per lane at a time.  560k fragments on 1024 x 1024 pixels: 333 us,
+// where a thread per fragment of at most 16 pixels (its vertices in private
+// memory) and a workgroup per larger one took 522 + 210 us.
+constexpr int kRasterPixels = 512;
 constexpr int kRasterMaxV = 128;  // fragment vertices staged by k_raster_big
 
+// Pixel range [i0, i1] x [j0, j1] of image coordinates within [ulo, uhi] x
+// [vlo, vhi].
+__device__ inline void raster_range(const RasterArgs &r, double ulo, double uhi, double vlo,
+                                    double vhi, int &i0, int &i1, int &j0, int &j1) {
+  i0 = max((int)floor(fmax(ulo, -1.0)), 0);
+  i1 = min((int)floor(fmin(uhi, (double)r.W)), r.W - 1);
+  j0 = max((int)floor(fmax(vlo, -1.0)), 0);
+  j1 = min((int)floor(fmin(vhi, (double)r.H)), r.H - 1);
+}
 // Pixel range of fragment f and its weight: the mean of the density over its
 // vertices (rasterization.hpp:528-534).
 __device__ inline void raster_setup(const RasterArgs &r, int64_t f, int &i0, int &i1, int &j0,
@@ -281,10 +295,7 @@ __device__ inline void raster_setup(const RasterArgs &r, int64_t f, int &i0, int
     vhi = fmax(vhi, v);
   }
   ff = acc / m;
-  i0 = max((int)floor(fmax(ulo, -1.0)), 0);
-  i1 = min((int)floor(fmin(uhi, (double)r.W)), r.W - 1);
-  j0 = max((int)floor(fmax(vlo, -1.0)), 0);
-  j1 = min((int)floor(fmin(vhi, (double)r.H)), r.H - 1);
+  raster_range(r, ulo, uhi, vlo, vhi, i0, i1, j0, j1);
 }
 
 // uv(q, u, v): image coordinates of vertex q of fragment f.
@@ -309,32 +320,41 @@ __device__ inline void raster_pixel(const RasterArgs &r, int64_t f, UV uv, int m
   for (int c = 0; c < r.nc; c++) atomicAdd(&dst[c], s * col[c]);
 }
 
-// One thread per fragment covering at most kRasterSmall pixels; larger ones
-// are listed for k_raster_big.
-__global__ void __launch_bounds__(256) k_raster_small(RasterArgs r, int64_t nf) {
-  const int64_t f = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+// One group of 16 lanes per fragment; those of more than kRasterPixels pixels
+// or 16 vertices are listed for k_raster_big.
+__global__ void __launch_bounds__(kCellThreads) k_raster(RasterArgs r, int64_t nf) {
+  __shared__ double su[kCellThreads], sv[kCellThreads];
+  const int l = (int)threadIdx.x % kGroup, base = (int)threadIdx.x - l;
+  const int64_t f = (int64_t)blockIdx.x * kCellGroups + threadIdx.x / kGroup;
   if (f >= nf) return;
-  int i0, i1, j0, j1;
-  double ff;
-  raster_setup(r, f, i0, i1, j0, j1, ff);
-  if (i1 < i0 || j1 < j0) return;
   const int m = r.nv[f];
-  if ((int64_t)(i1 - i0 + 1) * (j1 - j0 + 1) > kRasterSmall || m > 32) {
-    r.big[atomicAdd(r.big_n, 1)] = (int32_t)f;
+  const double *p = r.xy + 2 * r.start[f];
+  const TriData *t = r.T + r.tri[f];
+  double u = INFINITY, v = INFINITY, uh = -INFINITY, vh = -INFINITY, acc = 0.0;
+  if (l < m) {
+    const double x = p[2 * l], y = p[2 * l + 1];
+    acc = t->a * x + t->b * y + t->c;
+    uh = u = r.sx * (x - r.x0);
+    vh = v = r.sy * (y - r.y0);
+  }
+  su[base + l] = u;
+  sv[base + l] = v;
+  __threadfence_block();  // (the group is part of one wave)
+  const double ff = row_sum(acc) / m;
+  int i0, i1, j0, j1;
+  raster_range(r, row_min(u), row_max(uh), row_min(v), row_max(vh), i0, i1, j0, j1);
+  if (m > kGroup || (i1 >= i0 && j1 >= j0 &&
+                     (int64_t)(i1 - i0 + 1) * (j1 - j0 + 1) > kRasterPixels)) {
+    if (l == 0) r.big[atomicAdd(r.big_n, 1)] = (int32_t)f;
     return;
   }
-  double u[32], v[32];
-  const double *p = r.xy + 2 * r.start[f];
-  for (int q = 0; q < m; q++) {
-    u[q] = r.sx * (p[2 * q] - r.x0);
-    v[q] = r.sy * (p[2 * q + 1] - r.y0);
-  }
+  if (i1 < i0 || j1 < j0) return;
+  const int w = i1 - i0 + 1, npix = w * (j1 - j0 + 1);
   auto uv = [&](int q, double &uq, double &vq) {
-    uq = u[q];
-    vq = v[q];
+    uq = su[base + q];
+    vq = sv[base + q];
   };
-  for (int j = j0; j <= j1; j++)
-    for (int i = i0; i <= i1; i++) raster_pixel(r, f, uv, m, i, j, ff);
+  for (int q = l; q < npix; q += kGroup) raster_pixel(r, f, uv, m, i0 + q % w, j0 + q / w, ff);
 }
 
 // One workgroup per listed fragment, its threads striding over the pixels.
@@ -576,7 +596,7 @@ ma_status ma_draw_laguerre(ma_engine *e, const double *w, const double *colors, 
     r.img = dimg;
     r.big = O.idx.p;
     r.big_n = O.idx.p + nf;
-    hipLaunchKernelGGL(k_raster_small, dim3(nblocks(nf, 256)), dim3(256), 0, e->stream, r, nf);
+    hipLaunchKernelGGL(k_raster, dim3(nblocks(nf, kCellGroups)), dim3(kCellThreads), 0, e->stream, r, nf);
     hipLaunchKernelGGL(k_raster_big, dim3(1024), dim3(256), 0, e->stream, r);
   }
   if (!device_ptrs)
