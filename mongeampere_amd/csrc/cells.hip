@@ -1482,13 +1482,13 @@ __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,
     }
   }
   if (MODE == 1 && a.fo.count != nullptr) {
-    // fragment polygons from the staging (every lane takes part)
+    // fragment polygons from the staging (every thread takes part)
     auto gx = [&](int i) { return F.x(i); };
     auto gy = [&](int i) { return F.y(i); };
     const double eps = frag_eps(I.xlo, I.xhi, I.ylo, I.yhi);
     const int m = counted ? frag_distinct(nout, eps, gx, gy) : 0;
     unsigned long long f, v;
-    frag_reserve_wave(a.fo, m, f, v);
+    frag_reserve_block(a.fo, m, f, v);
     if (m > 0)
       frag_write(a.fo, f, v, m, a.perm[k], pair_tri[p], a.pos[2 * k], a.pos[2 * k + 1], nout,
                  eps, gx, gy);

@@ -48,3 +48,23 @@ def test_vertices_of_a_fragment(engine, edges, size):
 def test_outside_the_image(engine):
     X = np.random.default_rng(3).uniform(0.05, 0.95, (200, 2))
     _draw(engine, _mesh(9), X, np.zeros(200), (0.9, 0.9, 1.7, 1.3), 20, 11)
+
+
+@pytest.mark.parametrize("n", [1, 7, 31, 60, 300, 3000])
+def test_fragment_slots(engine, n):
+    """Slots reserved by whole workgroups: fragments from less than one wave
+    to many workgroups, none lost or written twice."""
+    X = np.random.default_rng(n).uniform(0.05, 0.95, (n, 2))
+    mesh = _mesh(6)
+    engine.set_mesh(mesh).set_diracs(X)
+    cell, tri, start, xy = engine.fragments(np.zeros(n))
+    assert len(set(zip(cell.tolist(), tri.tolist()))) == len(cell)  # one per pair
+    assert start[0] == 0 and np.all(np.diff(start) >= 3) and start[-1] == len(xy)
+    area = 0.0
+    for a, b in zip(start[:-1], start[1:]):
+        p = xy[a:b]
+        q = np.roll(p, -1, axis=0)
+        s = 0.5 * (p[:, 0] * q[:, 1] - p[:, 1] * q[:, 0]).sum()
+        assert s > 0
+        area += s
+    assert abs(area - 1.0) <= 1e-12
