@@ -1937,24 +1937,36 @@ __global__ void k_caller_cnt(int64_t n, const int32_t *iperm, const int32_t *ptr
   const int32_t k = iperm[i];
   cnt[i] = ptr[k + 1] - ptr[k];
 }
-__global__ void k_caller_fill(int64_t n, const int32_t *iperm, const int32_t *perm,
-                              const int32_t *ptr, const int32_t *col, const double *val,
-                              const int32_t *optr, int32_t *ocol, double *oval) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+// 16 lanes per row: every entry goes to its rank among the row's columns (all
+// different).  Rows of up to 16 entries stay in registers; longer ones, rare,
+// count ranks from memory.  (A thread per row that sorted by insertion in the
+// output waited for its own stores: N = 1000 19.9 us instead of 3.7.)
+__global__ void __launch_bounds__(kCellThreads)
+    k_caller_fill(int64_t n, const int32_t *iperm, const int32_t *perm, const int32_t *ptr,
+                  const int32_t *col, const double *val, const int32_t *optr, int32_t *ocol,
+                  double *oval) {
+  const int l = (int)threadIdx.x % kGroup, base = (int)threadIdx.x % 64 - l;
+  const int64_t i = (int64_t)blockIdx.x * kCellGroups + threadIdx.x / kGroup;
   if (i >= n) return;
   const int32_t k = iperm[i];
   const int32_t s = ptr[k], c = ptr[k + 1] - s, o = optr[i];
-  for (int r = 0; r < c; r++) {
-    const int32_t j = perm[col[s + r]];
-    const double v = val[s + r];
-    int p = r;
-    while (p > 0 && ocol[o + p - 1] > j) {
-      ocol[o + p] = ocol[o + p - 1];
-      oval[o + p] = oval[o + p - 1];
-      p--;
+  if (c <= kGroup) {
+    const bool have = l < c;
+    const int32_t j = have ? perm[col[s + l]] : INT32_MAX;
+    int rank = 0;
+    for (int q = 0; q < c; q++) rank += row_get(j, 4 * base, q) < j;
+    if (have) {
+      ocol[o + rank] = j;
+      oval[o + rank] = val[s + l];
     }
-    ocol[o + p] = j;
-    oval[o + p] = v;
+    return;
+  }
+  for (int32_t r = l; r < c; r += kGroup) {
+    const int32_t j = perm[col[s + r]];
+    int rank = 0;
+    for (int32_t q = 0; q < c; q++) rank += perm[col[s + q]] < j;
+    ocol[o + rank] = j;
+    oval[o + rank] = val[s + r];
   }
 }
 
@@ -1968,7 +1980,8 @@ hipError_t csr_to_caller(ma_engine *e, int32_t *rowptr, int32_t *col, double *va
   hipLaunchKernelGGL(k_caller_cnt, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, e->iperm.p,
                      e->eb.csr_ptr.p, optr.p);
   MA_HIP_RET(exclusive_scan(e, optr.p, optr.p, n));
-  hipLaunchKernelGGL(k_caller_fill, dim3(nblocks(n)), dim3(kBlock), 0, e->stream, n, e->iperm.p,
+  hipLaunchKernelGGL(k_caller_fill, dim3(nblocks(n, kCellGroups)), dim3(kCellThreads), 0,
+                     e->stream, n, e->iperm.p,
                      e->perm.p, e->eb.csr_ptr.p, e->eb.csr_col.p, e->eb.csr_val.p, optr.p,
                      ocol.p, oval.p);
   MA_HIP_RET(hipMemcpyAsync(rowptr, optr.p, sizeof(int32_t) * (n + 1), hipMemcpyDeviceToHost,
