@@ -1383,6 +1383,9 @@ ma_status ma_ot_solve_x(ma_engine *e, const double *nu, double *w, double *w_lo,
         const ma_status fs = weight_floor(e, S.w.p, S.nu.p, &floor);
         if (fs != MA_OK) return fs;
         if (ns0.maxrel <= kFloorMargin * floor) {
+          // (the norm of the error is rounding here and need not halve while
+          // the last cells above the tolerance come below it)
+          if (ns.minm >= eps0 && !keep_going(ns)) break;
           result = MA_LINESEARCH_FAIL;
           char msg[160];
           snprintf(msg, sizeof msg,
