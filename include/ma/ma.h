@@ -198,7 +198,7 @@ ma_status ma_solve_laplacian_csr(ma_engine *e, int64_t n, const int32_t *rowptr,
  * in device memory (d_rowptr n + 1 entries from 0 to nnz, d_col and d_val
  * nnz entries), right-hand side d_g and solution d_d (n entries each, device
  * memory), by Jacobi-preconditioned conjugate gradients.  It allocates
- * nothing: its work memory is one fixed array per GPU (about 5 x 8 bytes x
+ * nothing: its work memory is one fixed array per GPU (about 6 x 8 bytes x
  * MA_NOALLOC_MAX_N, held until the process ends) whose address ma_create
  * looks up, so n may not exceed MA_NOALLOC_MAX_N (MA_BAD_INPUT otherwise).
  * Every call on a GPU uses that GPU's one array: calls that overlap on one
@@ -319,7 +319,7 @@ ma_status ma_cell_paths(ma_engine *e, int64_t count, const int64_t *ids, int32_t
  * one-workgroup-per-cell kernel for large cells (2) (for testing the overflow
  * paths); MA_OPT_CAP_CAND: initial capacity of the per-bin candidate
  * lists (grows automatically on overflow); MA_OPT_GRAPHS (0/1, default 1):
- * replay batches of conjugate-gradient iterations from a HIP graph. */
+ * replay the batches of a long conjugate-gradient solve from a HIP graph. */
 typedef enum {
   MA_OPT_FORCE_GENERAL = 1,
   MA_OPT_CAP_CAND = 2,
