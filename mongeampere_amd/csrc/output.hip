@@ -264,7 +264,8 @@ struct RasterArgs {
 // A fragment of up to this many pixels is covered by a group of 16 lanes, a
 // pixel per lane at a time.  560k fragments on 1024 x 1024 pixels: 333 us,
 // where a thread per fragment of at most 16 pixels (its vertices in private
-// memory) and a workgroup per larger one took 522 + 210 us.
+// memory) and a workgroup per larger one took 522 + 210 us.  Filling the lanes
+// that small fragments leave idle, 16 fragments' pixels as one stream, took 377.
 constexpr int kRasterPixels = 512;
 constexpr int kRasterMaxV = 128;  // fragment vertices staged by k_raster_big
 
