@@ -332,10 +332,15 @@ __device__ inline double plane_bound(const Plane &p, const NodeBox &q, double x,
   return p.b + m - kPlaneEps * (fabs(p.b) + mag);
 }
 
+// A bound with infinite terms may be no number: then it bounds nothing.  A node
+// with Diracs stays below the +inf that marks the empty ones.
+__device__ inline double node_bound(double t) { return t != t ? -kInf : fmin(t, DBL_MAX); }
+
 // One group per node of level lev + 2 (lev + 1 when that is the top: step 1);
 // lane c takes its descendant c of level lev.  lev = 0: from the Diracs of the
 // bins; above: from the records of level lev.  Writes planes and largest
-// weights.
+// weights.  Weights need not be finite: -inf (or NaN) is no Dirac here, as in
+// pyr; +inf gives its nodes the bound -inf; neither enters the fits.
 __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int step,
                                                         const int32_t *__restrict__ bin_start,
                                                         const double *__restrict__ pos,
@@ -356,12 +361,13 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
     q0 = bin_start[m];
     q1 = bin_start[m + 1];
     for (int32_t q = q0; q < q1; q++) {
+      W = fmax(W, w[q]);
+      if (!(fabs(w[q]) < kInf)) continue;
+      s.n += 1.0;
       s.x += pos[2 * q] - hx;
       s.y += pos[2 * q + 1] - hy;
       s.w += w[q];
-      W = fmax(W, w[q]);
     }
-    s.n = (double)(q1 - q0);
     pyr[off.o[0] + m] = W;
   } else if (on) {
     s = sums[off.o[lev] + m];
@@ -381,6 +387,8 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
       gx = (xw * yy - yw * xy) / det;
       gy = (yw * xx - xw * xy) / det;
     }
+    // (finite weights may be too large for their sums)
+    if (!(fabs(gx) + fabs(gy) < kInf)) gx = gy = 0.0;
   }
   auto gradient = [&](const NodeBox &q, Plane &p) {
     p.ax = (q.x0 + q.x1) - gx;
@@ -394,8 +402,9 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
     for (int32_t i = q0; i < q1; i++) {
       const double x = pos[2 * i] - hx, y = pos[2 * i + 1] - hy;
       const double v = x * x + y * y - w[i], d = p.ax * x + p.ay * y;
-      p.b = fmin(p.b, v - d - kPlaneEps * (x * x + y * y + fabs(w[i]) + fabs(p.ax * x) +
-                                           fabs(p.ay * y)));
+      if (w[i] > -kInf)
+        p.b = fmin(p.b, node_bound(v - d - kPlaneEps * (x * x + y * y + fabs(w[i]) +
+                                                        fabs(p.ax * x) + fabs(p.ay * y))));
     }
     if (on) pl[off.o[0] + m] = p;
   } else if (on) {
@@ -412,7 +421,7 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
     if (on && p.b < kInf) {
       double mag;
       const double d = box_min(q, p.ax - u.ax, p.ay - u.ay, mag);
-      t = p.b + d - kPlaneEps * (fabs(p.b) + mag);
+      t = node_bound(p.b + d - kPlaneEps * (fabs(p.b) + mag));
     }
     const int st = k == 1 ? 1 : 4;  // lanes of the children: l, l ^ st, ...
     t = fmin(t, row_get(t, base4, l ^ st));
@@ -431,7 +440,9 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
 }
 
 // true if pi_j - pi_k (affine) can be <= 0 somewhere in the bin (min over
-// corners); corners in absolute coordinates
+// corners); corners in absolute coordinates.  Beside an infinite weight only
+// the order counts: a Dirac of weight -inf, or beside one of weight +inf, owns
+// nothing and is not listed.
 __device__ inline bool may_beat(double x0, double y0, double h, double jx, double jy, double wj,
                                 double kx, double ky, double wk) {
   bool ok = false;
@@ -440,7 +451,8 @@ __device__ inline bool may_beat(double x0, double y0, double h, double jx, doubl
     const double cx = x0 + (c & 1 ? h : 0.0), cy = y0 + (c & 2 ? h : 0.0);
     const double dj = (cx - jx) * (cx - jx) + (cy - jy) * (cy - jy) - wj;
     const double dk = (cx - kx) * (cx - kx) + (cy - ky) * (cy - ky) - wk;
-    ok |= (dj - dk) <= 1e-12 * (fabs(dj) + fabs(dk));
+    ok |= fabs(dj) < kInf && fabs(dk) < kInf ? (dj - dk) <= 1e-12 * (fabs(dj) + fabs(dk))
+                                             : dj < dk;
   }
   return ok;
 }
@@ -540,9 +552,10 @@ __global__ void __launch_bounds__(kCellThreads) k_cand_list(
         best = row_get(q, 4 * base, __ffs((unsigned)(__ballot(h == m) >> base) & 0xffffu) - 1);
       }
     };
-    if (best >= 0) {
-      U = value(best);
-    } else {
+    if (best >= 0) U = value(best);
+    if (!(U < kInf)) {  // no last owner, or its weight is -inf or NaN now
+      U = kInf;
+      best = -1;
       // greedy descent to the bin with the smallest lower bound
       uint32_t m = 0;
       for (int lev = g.L; lev > 0;) {
@@ -564,17 +577,24 @@ __global__ void __launch_bounds__(kCellThreads) k_cand_list(
              [&](const Plane &p, const NodeBox &q) { return !(plane_bound(p, q, mx, my) > U); },
              better);
     if (l == 0) owner[b] = best;
+    if (best < 0) {  // no Dirac has a weight above -inf
+      if (l == 0) cand_start[b] = 0;
+      return;
+    }
   }
   const double kx = pos[2 * best], ky = pos[2 * best + 1], kw = w[best];
-  // the owner's v - 2 x.y at the corners, rounding allowed for
+  // the owner's v - 2 x.y at the corners, rounding allowed for (weight +inf:
+  // only its like may share the bin)
   double thr[4];
   {
     const double x = kx - hx, y = ky - hy, v = x * x + y * y - kw;
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       const double cx = c & 1 ? B.x1 : B.x0, cy = c & 2 ? B.y1 : B.y0;
-      thr[c] = v - 2.0 * (cx * x + cy * y) +
-               kPlaneEps * (x * x + y * y + fabs(kw) + 2.0 * (fabs(cx * x) + fabs(cy * y)));
+      thr[c] = kw < kInf ? v - 2.0 * (cx * x + cy * y) +
+                               kPlaneEps * (x * x + y * y + fabs(kw) +
+                                            2.0 * (fabs(cx * x) + fabs(cy * y)))
+                         : -kInf;
     }
   }
   const double ox = B.x0 + hx, oy = B.y0 + hy;  // the bin's lower corner
