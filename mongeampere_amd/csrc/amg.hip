@@ -599,8 +599,9 @@ static ma_status amg_build(ma_engine *e, Amg &A, const CsrView &M) {
                        dim3(kVB2), 0, e->stream, nc, nf, fptr, fcol, fval, C.ptr.p, nullptr,
                        nullptr, nullptr);
     MA_HIP_TRY(exclusive_scan(e, C.ptr.p, C.ptr.p, nc));
-    // small levels take room for as many entries as the level above has,
-    // instead of waiting for their count
+    // small levels take room for as many entries as the level above has (or a
+    // full matrix: rows in column order give every column once), instead of
+    // waiting for their count
     if (!wave) {
       int32_t nnzc = 0;
       MA_HIP_TRY(read_back(e, {{&nnzc, C.ptr.p + nc, sizeof(int32_t)}}));
