@@ -42,7 +42,8 @@ constexpr int kVB2 = 256;
 
 // Level 0: the Hessian with row and column gi removed (identity there), so
 // the system is SPD and the solution keeps x[gi] = 0.  A row other than gi
-// without a positive diagonal (a cell sharing no edge, or a NaN) sets *bad.
+// without a positive diagonal (a cell sharing no edge, or a NaN) sets bit 0 of
+// *bad, one that is not in column order bit 1.
 // With outf, also an FP32 copy of the values and inverse diagonal.
 __global__ void k_amg_level0(int64_t n, const int32_t *ptr, const int32_t *col,
                              const double *val, int32_t gi, double *out, double *dinv,
@@ -50,8 +51,12 @@ __global__ void k_amg_level0(int64_t n, const int32_t *ptr, const int32_t *col,
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
   double d = 0.0;
+  int32_t last = 0;
+  bool descends = false;
   for (int32_t q = ptr[i]; q < ptr[i + 1]; q++) {
     const int32_t j = col[q];
+    descends |= j < last;
+    last = j;
     double v = val[q];
     if (i == gi || j == gi) v = (i == j) ? 1.0 : 0.0;
     out[q] = v;
@@ -62,6 +67,39 @@ __global__ void k_amg_level0(int64_t n, const int32_t *ptr, const int32_t *col,
   dinv[i] = d > 0.0 ? 1.0 / d : 0.0;
   if (dinvf) dinvf[i] = (float)dinv[i];
   if (!(d > 0.0)) atomicOr(bad, 1);
+  if (descends) atomicOr(bad, 2);
+}
+
+// Brings the rows of M into column order, on the host (a caller's matrix may
+// come in any order; the engine's rows never take this).  Coarse rows are
+// merges of rows in that order: of others they would hold columns twice, more
+// entries than amg_build has room for.
+static hipError_t sort_rows(ma_engine *e, const CsrView &M) {
+  std::vector<int32_t> ptr((size_t)M.n + 1), col((size_t)M.nnz);
+  std::vector<double> val((size_t)M.nnz);
+  MA_HIP_RET(hipMemcpyAsync(ptr.data(), M.ptr, sizeof(int32_t) * ptr.size(),
+                            hipMemcpyDeviceToHost, e->stream));
+  MA_HIP_RET(hipMemcpyAsync(col.data(), M.col, sizeof(int32_t) * col.size(),
+                            hipMemcpyDeviceToHost, e->stream));
+  MA_HIP_RET(hipMemcpyAsync(val.data(), M.val, sizeof(double) * val.size(),
+                            hipMemcpyDeviceToHost, e->stream));
+  MA_HIP_RET(hipStreamSynchronize(e->stream));
+  std::vector<std::pair<int32_t, double>> row;
+  for (int64_t i = 0; i < M.n; i++) {
+    row.clear();
+    for (int32_t q = ptr[i]; q < ptr[i + 1]; q++) row.emplace_back(col[q], val[q]);
+    std::stable_sort(row.begin(), row.end(),
+                     [](const auto &a, const auto &b) { return a.first < b.first; });
+    for (size_t q = 0; q < row.size(); q++) {
+      col[ptr[i] + q] = row[q].first;
+      val[ptr[i] + q] = row[q].second;
+    }
+  }
+  MA_HIP_RET(hipMemcpyAsync(M.own_col, col.data(), sizeof(int32_t) * col.size(),
+                            hipMemcpyHostToDevice, e->stream));
+  MA_HIP_RET(hipMemcpyAsync(M.own_val, val.data(), sizeof(double) * val.size(),
+                            hipMemcpyHostToDevice, e->stream));
+  return hipStreamSynchronize(e->stream);
 }
 
 // Merge of the kAgg sorted fine rows of coarse row I (columns mapped j/kAgg).
@@ -648,12 +686,16 @@ ma_status amg_setup(ma_engine *e, Amg &A, const CsrView &M, int32_t gi, int max_
     dinvf = A.lvf[0].dinv.p;
   }
   MA_HIP_TRY(A.bad.ensure(1));
-  MA_HIP_TRY(hipMemsetAsync(A.bad.p, 0, sizeof(int32_t), e->stream));
-  hipLaunchKernelGGL(k_amg_level0, dim3(nb2(n)), dim3(kVB2), 0, e->stream, n, M.ptr, M.col,
-                     M.val, gi, A.val0.p, A.dinv0.p, valf, dinvf, A.bad.p);
   int32_t bad = 0;
-  MA_HIP_TRY(read_back(e, {{&bad, A.bad.p, sizeof(int32_t)}}));
-  if (bad) {
+  for (int pass = 0; pass < 2; pass++) {
+    MA_HIP_TRY(hipMemsetAsync(A.bad.p, 0, sizeof(int32_t), e->stream));
+    hipLaunchKernelGGL(k_amg_level0, dim3(nb2(n)), dim3(kVB2), 0, e->stream, n, M.ptr, M.col,
+                       M.val, gi, A.val0.p, A.dinv0.p, valf, dinvf, A.bad.p);
+    MA_HIP_TRY(read_back(e, {{&bad, A.bad.p, sizeof(int32_t)}}));
+    if (!(bad & 2) || !M.own_col) break;
+    MA_HIP_TRY(sort_rows(e, M));
+  }
+  if (bad & 1) {
     // include/MA/optimal_transport.hpp:48-58 reports zero diagonal entries
     // of the gauge-fixed matrix the same way (its Cholesky cannot proceed)
     e->err = "singular Hessian: a cell other than the gauge cell has no positive diagonal "

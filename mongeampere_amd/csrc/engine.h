@@ -359,6 +359,9 @@ struct CsrView {
   int64_t n = 0, nnz = 0;
   const int32_t *ptr = nullptr, *col = nullptr;
   const double *val = nullptr;
+  // col and val once more where amg_setup may bring the rows into column order
+  int32_t *own_col = nullptr;
+  double *own_val = nullptr;
 };
 // Multigrid preconditioner (amg.hip)
 Amg *amg_create();

@@ -1087,29 +1087,6 @@ ma_status ma_solve_laplacian_csr(ma_engine *e, int64_t n, const int32_t *rowptr,
       e->err = "column index out of range";
       return MA_BAD_INPUT;
     }
-  // Coarse rows are merges of rows in column order; of others they would hold
-  // columns twice, more entries than the room made for them.
-  std::vector<int32_t> scol;
-  std::vector<double> sval;
-  for (int64_t i = 0; i < n; i++) {
-    if (std::is_sorted(col + hp[i], col + hp[i + 1])) continue;
-    if (scol.empty()) {
-      scol.assign(col, col + nnz);
-      sval.assign(val, val + nnz);
-    }
-    std::vector<std::pair<int32_t, double>> row;
-    for (int32_t q = hp[i]; q < hp[i + 1]; q++) row.emplace_back(col[q], val[q]);
-    std::stable_sort(row.begin(), row.end(),
-                     [](const auto &a, const auto &b) { return a.first < b.first; });
-    for (size_t q = 0; q < row.size(); q++) {
-      scol[hp[i] + q] = row[q].first;
-      sval[hp[i] + q] = row[q].second;
-    }
-  }
-  if (!scol.empty()) {
-    col = scol.data();
-    val = sval.data();
-  }
   SolverBuffers &S = e->sb;
   MA_HIP_TRY(S.hptr.ensure((size_t)n + 1));
   MA_HIP_TRY(S.hcol.ensure((size_t)nnz + 1));
@@ -1129,6 +1106,8 @@ ma_status ma_solve_laplacian_csr(ma_engine *e, int64_t n, const int32_t *rowptr,
   M.ptr = S.hptr.p;
   M.col = S.hcol.p;
   M.val = S.hval.p;
+  M.own_col = S.hcol.p;
+  M.own_val = S.hval.p;
   int64_t it = 0;
   double rr = 0.0;
   const ma_status ps = pcg(e, M, (int32_t)(n - 1), S.hg.p, S.hd.p,
