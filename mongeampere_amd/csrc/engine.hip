@@ -80,8 +80,11 @@ __device__ inline double block_sum(double v, double *s) {
 // replaced by the identity (symmetric positive definite for a connected
 // diagram); with b[gi] = 0 its solution has x[gi] = 0, the gauge of
 // include/MA/optimal_transport.hpp:82-86.  Scalars live on the device:
-// scal = [rz (of the iteration's parity, 2), rr, -, bb, done, iterations,
-// breakdown].
+// scal = [rz (of the iteration's parity, 2), rr, ended, bb, done, iterations,
+// breakdown].  No launch of more than one workgroup writes a flag that it
+// returns on: its waves would read it before or after that write, and some of
+// a workgroup would miss the others' barriers.  So k_cg_spmv returns on done
+// and sets ended, k_cg_update returns on ended and sets done.
 //
 // An iteration is k_cg_spmv, k_cg_update and the preconditioner.  Below a few
 // hundred thousand rows its time is the number of launches (about 5 us each),
@@ -139,7 +142,7 @@ __global__ void __launch_bounds__(kCgThreads) k_cg_scal_init(const double *part_
   if (threadIdx.x == 0) {
     scal[2] = rr;
     scal[4] = rr;
-    if (rr == 0.0) scal[5] = 1.0;
+    if (rr == 0.0) scal[3] = scal[5] = 1.0;
   }
 }
 static_assert(kCgGrid <= kCgThreads, "one partial sum per thread");
@@ -169,7 +172,7 @@ __global__ void __launch_bounds__(kCgThreads)
   if (blockIdx.x == 0 && t == 0) {
     scal[parity] = rz;
     scal[2] = rr;
-    if (end) scal[5] = 1.0;
+    if (end) scal[3] = 1.0;
   }
   if (end) return;
   const double beta = (rz_old > 0.0) ? rz / rz_old : 0.0;
@@ -200,7 +203,10 @@ __global__ void __launch_bounds__(kCgThreads)
                 double *part_rz) {
   __shared__ double s[2 * kCgThreads / 64];
   const double part = threadIdx.x < gridDim.x ? part_pap[threadIdx.x] : 0.0;
-  if (scal[5] != 0.0) return;
+  if (scal[3] != 0.0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[5] = 1.0;
+    return;
+  }
   const double pap = cg_block_sum(part, s);
   const double alpha = (pap > 0.0) ? scal[parity] / pap : 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -239,7 +245,7 @@ __global__ void __launch_bounds__(kCgThreads)
   const double rr = cg_block_sum(threadIdx.x < np ? part_rr[threadIdx.x] : 0.0, s);
   if (threadIdx.x == 0) {
     scal[2] = rr;
-    if (scal[7] != 0.0 || rr <= tol2 * scal[4]) scal[5] = 1.0;
+    if (scal[7] != 0.0 || rr <= tol2 * scal[4]) scal[3] = scal[5] = 1.0;
   }
 }
 __global__ void k_set_zero_at(double *x, int32_t i) { x[i] = 0.0; }
