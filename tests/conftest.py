@@ -97,3 +97,37 @@ def engine():
     e = Engine(0)
     yield e
     e.close()
+
+
+def option_defaults():
+    """{option: default} of Engine.set_option, from the engine's own header."""
+    import re
+
+    with open(os.path.join(ROOT, "mongeampere_amd", "csrc", "engine.h")) as f:
+        text = f.read()
+    constant = dict(re.findall(r"constexpr int (k\w+) = (\d+);", text))
+
+    def default(member):
+        v = re.search(r"\b%s = (?:ma::)?([\w.]+);" % member, text).group(1)
+        return float(constant.get(v, v))
+
+    return {"force_general": int(default("force_general")), "cap_cand": int(default("cap_cand")),
+            "graphs": int(default("use_graphs")), "local_rings": int(default("local_rings")),
+            "walk_budget": int(default("walk_budget")),
+            "amg_omega_permille": round(1000 * default("amg_omega")),
+            "amg_corr_permille": round(1000 * default("amg_corr")),
+            "amg_sweeps": int(default("amg_sweeps")), "far_cells": int(default("far_cells"))}
+
+
+def restore_options(engine):
+    for name, value in option_defaults().items():
+        engine.set_option(name, value)
+
+
+@pytest.fixture(autouse=True)
+def _default_options(request):
+    """The engine is shared by the session: every test starts from the options
+    a caller gets, whatever the test before it left."""
+    if "engine" in request.fixturenames:
+        restore_options(request.getfixturevalue("engine"))
+    yield
