@@ -940,9 +940,6 @@ ma_status refine_candidates(ma_engine *e, int64_t total) {
   a.cand = B.cand.p;
   hipLaunchKernelGGL(k_cand_refine, dim3(nblocks(total, kCellGroups)), dim3(kCellThreads), 0,
                      e->stream, a, B.cbin.p, total, B.ckeep.p);
-  const int32_t zero = 0;
-  MA_HIP_TRY(hipMemcpyAsync(B.ckeep.p + total, &zero, sizeof(int32_t), hipMemcpyHostToDevice,
-                            e->stream));
   MA_HIP_TRY(hipGetLastError());
   return MA_OK;
 }
