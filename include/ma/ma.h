@@ -181,8 +181,8 @@ ma_status ma_solve_laplacian(ma_engine *e, const double *g, double *d, double re
                              int maxiter, double *res, int64_t *iters);
 
 /* Same gauge-fixed solve for a caller-supplied symmetric CSR matrix (n x n,
- * 0-based rowptr/col; e.g. a Hessian copied out earlier or assembled by the
- * caller), the solve_laplacian_matrix(h, g) call shape of
+ * 0-based rowptr/col, the columns of a row in any order; e.g. a Hessian copied
+ * out earlier or assembled by the caller), the solve_laplacian_matrix(h, g) call shape of
  * include/MA/optimal_transport.hpp:41-44.  Needs no mesh or Diracs.  The
  * multigrid aggregates follow the index order, so a spatially coherent
  * numbering converges fastest. */

@@ -2,12 +2,12 @@
 //   k_cell_local  16 lanes per Dirac: power cell clipped in place, one vertex
 //                 per lane (at most kMaxFast), by the Diracs of the
 //                 surrounding bins, certified ring by ring or through the
-//                 max-weight pyramid, written once to HBM;
+//                 pyramids, written once to HBM;
 //   k_pairs       (cell, triangle) pairs whose bounding boxes meet;
-//   k_frag        one thread per pair: the cell polygon streamed through a
-//                 three-stage Sutherland-Hodgman pipeline (one stage per
-//                 triangle edge) held in registers, fused with the exact
-//                 quadrature of the fragment;
+//   k_frag        one thread per pair: the cell polygon, in LDS, clipped in
+//                 place by the triangle's three edges and integrated exactly
+//                 in closed form; fragments that outgrow its slots stream
+//                 through three clip stages in registers (k_frag_wide);
 //   k_row_count, k_row_fill  Hessian rows from the edge integrals, straight
 //                 into the CSR arrays.
 // Cells that overflow kMaxFast vertices are flagged and evaluated by the
@@ -125,13 +125,13 @@ struct CellBuf<float> {
 // pyramid node at a time, and all control flow is uniform in the group.
 // Candidates, bins and nodes are loaded 16 at a time, reductions and
 // broadcasts are DPP moves, and no LDS limits the waves in flight; what bounds
-// k_cell_local is VALU issue (84 % busy, 61 % of the lanes active).  One
+// k_cell_local is VALU issue (75 - 80 % busy, 61 % of the lanes active).  One
 // thread per cell with its polygon in LDS waited instead on dependent gathers
 // and its wave's slowest lane (24 % of the lanes active, 1.4 - 1.8 waves per
-// SIMD).  Measured, before and after: 1M Diracs at w = 0 in FP32 2.49 and
-// 1.55 ms, 1M in FP64 at weights up to 1.6 bins off 8.5 and 3.0 ms, 2M on an
-// annulus in FP64 13.0 and 2.8 ms, 1000 Diracs (too few threads before) 278
-// and 33 us.
+// SIMD).  Measured, before and now: 1M Diracs at w = 0 in FP32 2.49 and
+// 1.80 ms, 1M in FP64 at weights up to 1.6 bins off 8.5 and 3.35 ms, 2M on an
+// annulus in FP64 13.0 and 2.94 ms, 1000 Diracs (too few threads before) 278
+// and 27 us.
 // ---------------------------------------------------------------------------
 static_assert(kMaxFast == kGroup, "one polygon vertex per lane");
 
@@ -640,12 +640,13 @@ __device__ inline bool node_reaches(const Plane &p, const Cell<R> &C, double wk,
 // together).  A lane takes a bin; from ring 2 on a bin whose maximum weight
 // and distance cannot reach the polygon is skipped.  After each ring the cell
 // is final if every unvisited Dirac is far_enough (certify_levels).  Otherwise
-// the remaining Diracs are reached through the max-weight pyramid: a
-// depth-first walk that tests the 16 grandchildren of a node at once, skips
-// nodes inside the visited square, prunes nodes that are far_enough for their
-// own maximum weight and clips by the Diracs of the nodes it keeps.  Pruning
-// uses the polygon radius at the time of the test, which only shrinks, so
-// every pruned Dirac stays unable to cut the final cell.
+// the remaining Diracs are reached through the pyramids: a depth-first walk
+// that tests the 16 grandchildren of a node at once, skips nodes inside the
+// visited square, prunes nodes that are far_enough for their own maximum weight
+// or whose plane does not reach the polygon (node_reaches) and clips by the
+// Diracs of the nodes it keeps.  Pruning uses the polygon at the time of the
+// test, which only shrinks, so every pruned Dirac stays unable to cut the final
+// cell.
 template <class R>
 __global__ void __launch_bounds__(kCellThreads) k_cell_local(CellArgs a, const double *pyr,
                                                              const double *pyr3,
@@ -1401,8 +1402,8 @@ struct FragPoly {
 // its longest polygon only; a pipeline that streamed the vertices through the
 // three edges took a different branch on every lane (26 % of the lanes active
 // per instruction, 3700 VALU instructions a wave against 2100 and 47 % here).
-// VALU issue bounds it (77 - 82 % busy).  At 10.4M pairs, before and after:
-// FP64 1.38 and 0.68 ms, FP32 0.86 and 0.50 ms (0.70 while every workgroup
+// VALU issue bounds it (75 - 84 % busy).  At 10.4M pairs, before and after:
+// FP64 1.38 and 0.68 ms, FP32 0.86 and 0.48 ms (0.70 while every workgroup
 // counted its fragments at one address).
 template <int MODE, class R>
 __global__ void __launch_bounds__(256) k_frag(CellArgs a, int64_t npairs,

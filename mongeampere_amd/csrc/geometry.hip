@@ -503,10 +503,11 @@ __device__ inline void row_walk(const Grid &g, const int32_t *bin_start, const P
 // (stage[b * kCandStage + i], 512 B per bin, allocated only when lists are
 // built).  Filling pass, into exactly sized CSR lists: copies those, and walks
 // again only for the bins with more (48 kept candidates left C2's converged
-// cells a third slower).  VALU work of the node tests bounds it.  200k
-// clustered Diracs, 512 x 512 bins: 16.5 ms with one thread per bin walking the
-// max-weight pyramid, 3.1 ms with a group per bin on that pyramid, 0.93 ms
-// with the planes (their five launches take 0.03 ms).
+// cells a third slower).  VALU work of the node tests bounds it (81 % busy,
+// 77 % of the lanes active; the count of all bins at one address hides behind
+// it).  200k clustered Diracs, 512 x 512 bins: 16.5 ms with one thread per bin
+// walking the max-weight pyramid, 3.1 ms with a group per bin on that pyramid,
+// 0.93 ms with the planes (their five launches take 0.03 ms).
 constexpr int kCandStage = 128;
 template <bool FILL>
 __global__ void __launch_bounds__(kCellThreads) k_cand_list(
