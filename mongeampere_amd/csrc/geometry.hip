@@ -361,12 +361,13 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
     q0 = bin_start[m];
     q1 = bin_start[m + 1];
     for (int32_t q = q0; q < q1; q++) {
-      W = fmax(W, w[q]);
-      if (!(fabs(w[q]) < kInf)) continue;
-      s.n += 1.0;
-      s.x += pos[2 * q] - hx;
-      s.y += pos[2 * q + 1] - hy;
-      s.w += w[q];
+      const double x = pos[2 * q] - hx, y = pos[2 * q + 1] - hy, wq = w[q];
+      const bool fits = fabs(wq) < kInf;  // (selects: a branch would hold up the loads)
+      s.n += fits ? 1.0 : 0.0;
+      s.x += fits ? x : 0.0;
+      s.y += fits ? y : 0.0;
+      s.w += fits ? wq : 0.0;
+      W = fmax(W, wq);
     }
     pyr[off.o[0] + m] = W;
   } else if (on) {
@@ -401,10 +402,10 @@ __global__ void __launch_bounds__(kCellThreads) k_plane(Grid g, int lev, int ste
     gradient(q, p);
     for (int32_t i = q0; i < q1; i++) {
       const double x = pos[2 * i] - hx, y = pos[2 * i + 1] - hy;
-      const double v = x * x + y * y - w[i], d = p.ax * x + p.ay * y;
-      if (w[i] > -kInf)
-        p.b = fmin(p.b, node_bound(v - d - kPlaneEps * (x * x + y * y + fabs(w[i]) +
-                                                        fabs(p.ax * x) + fabs(p.ay * y))));
+      const double wi = w[i], v = x * x + y * y - wi, d = p.ax * x + p.ay * y;
+      const double t = node_bound(v - d - kPlaneEps * (x * x + y * y + fabs(wi) +
+                                                       fabs(p.ax * x) + fabs(p.ay * y)));
+      p.b = fmin(p.b, wi > -kInf ? t : kInf);
     }
     if (on) pl[off.o[0] + m] = p;
   } else if (on) {
